@@ -171,17 +171,53 @@ __global__ __launch_bounds__(256) void gn_fold_quads_kernel(float *__restrict__ 
     }
 }
 
+/* Both stages in one launch, for images whose convolutions leave few partial rows: a workgroup owns one group and sums its
+ * quads over every row in double precision. Up to 2048 rows (512 x 512 positions) that is one launch of 5 us instead of
+ * two of 4.7; beyond, the strided 8- to 32-byte reads of 32 workgroups take longer than the two coalesced passes
+ * (16448 rows, 1024 x 1024 positions: 6.4 + 4.8 us). */
+#define GN_ONE_PASS_ROWS 2048
+__global__ __launch_bounds__(256) void gn_stats_kernel(float *__restrict__ stats, const float *__restrict__ conv, int prows, int C, double count,
+                                                       float eps) {
+    __shared__ double sh[4][2];
+    const int g = blockIdx.x, quads = C >> 2, qpg = quads >> 5, sub = threadIdx.x & (qpg - 1), step = 256 / qpg; /* qpg = 1, 2 or 4 */
+    double a = 0.0, b = 0.0;
+#pragma unroll 4
+    for (int r = threadIdx.x / qpg; r < prows; r += step) {
+        const f32x2 v = *(const f32x2 *)(conv + ((size_t)r * quads + g * qpg + sub) * 2);
+        a += (double)v[0];
+        b += (double)v[1];
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        a += __shfl_xor(a, o);
+        b += __shfl_xor(b, o);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        sh[threadIdx.x >> 6][0] = a;
+        sh[threadIdx.x >> 6][1] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const double mean = ((sh[0][0] + sh[1][0]) + (sh[2][0] + sh[3][0])) / count;
+        double var = ((sh[0][1] + sh[1][1]) + (sh[2][1] + sh[3][1])) / count - mean * mean;
+        if (var < 0.0) var = 0.0;
+        stats[g * 2 + 0] = (float)mean;
+        stats[g * 2 + 1] = (float)(1.0 / sqrt(var + (double)eps));
+    }
+}
+
 /* out bf16 = [swish](gamma * (x - mean) * rstd + beta), zeros on the border; raw (optional)
  * receives x itself as bf16, the input of a residual block's 1x1 shortcut convolution. Same
- * thread-to-data map as the partial-sum pass. */
+ * thread-to-data map as the partial-sum pass, over `span` positions per workgroup: with 256 of them a 32 x 32 image of 512
+ * channels was five workgroups and 32 us, with 8 it is 145 and a few; images that give every compute unit several
+ * workgroups either way keep 256. */
 template <typename T>
 __global__ __launch_bounds__(256) void gn_apply_kernel(bf16 *__restrict__ out, bf16 *__restrict__ raw, const T *__restrict__ x,
                                                        const float *__restrict__ stats, const float *__restrict__ gamma,
                                                        const float *__restrict__ beta, int rows, int C, int hp, int wp,
-                                                       unsigned long long magic, int swish) {
+                                                       unsigned long long magic, int swish, int span) {
     const int quads = C >> 2, rpi = 256 / quads;
     const int q = threadIdx.x % quads, r0 = threadIdx.x / quads;
-    const int row_begin = blockIdx.x * GN_ROWS, row_end = min(rows, row_begin + GN_ROWS);
+    const int row_begin = blockIdx.x * span, row_end = min(rows, row_begin + span);
     const int g = (q * 4) / (C >> 5);
     const float mean = stats[g * 2], rstd = stats[g * 2 + 1];
     const f32x4 gm = *(const f32x4 *)(gamma + q * 4), bt = *(const f32x4 *)(beta + q * 4);
@@ -453,7 +489,10 @@ static int group_norm_run(void *out_bf16, void *raw_bf16, const T *x, const floa
     float *partial = scratch + 64, *stats = scratch;
     hipStream_t st = flux_hip_stream_handle();
     const double count = (double)(hp - 2) * (wp - 2) * (C / 32);
-    if (conv_stats) {
+    if (conv_stats && conv_stats_rows <= GN_ONE_PASS_ROWS) {
+        hipLaunchKernelGGL(gn_stats_kernel, dim3(32), dim3(256), 0, st, stats, conv_stats, conv_stats_rows, C, count, eps);
+        LAUNCH_OK("gn_stats_kernel");
+    } else if (conv_stats) {
         const int rpi = 256 / (C / 4);
         int nb = (conv_stats_rows + 8 * rpi - 1) / (8 * rpi); /* about eight trips per thread, at most as many workgroups as the scratch has rows */
         nb = nb < 1 ? 1 : nb > nblocks ? nblocks : nb > 256 ? 256 : nb;
@@ -468,8 +507,11 @@ static int group_norm_run(void *out_bf16, void *raw_bf16, const T *x, const floa
         LAUNCH_OK("gn_finalize_kernel");
     }
     const unsigned long long magic = ((1ull << 40) + (unsigned)wp - 1) / (unsigned)wp;
-    hipLaunchKernelGGL(gn_apply_kernel<T>, dim3(nblocks), dim3(256), 0, st, (bf16 *)out_bf16, (bf16 *)raw_bf16, x, stats, gamma, beta, rows, C, hp,
-                       wp, magic, swish);
+    /* as many positions per workgroup as leave 2048 workgroups, at least four per thread */
+    int span = GN_ROWS;
+    while (span > 4 * (256 / (C / 4)) && (rows + span - 1) / span < 2048) span >>= 1;
+    hipLaunchKernelGGL(gn_apply_kernel<T>, dim3((rows + span - 1) / span), dim3(256), 0, st, (bf16 *)out_bf16, (bf16 *)raw_bf16, x, stats, gamma, beta, rows, C, hp,
+                       wp, magic, swish, span);
     LAUNCH_OK("gn_apply_kernel");
     return 1;
 }

@@ -217,6 +217,30 @@ def test_group_norm_from_convolution_statistics(hip, oracle_mod, tile, epi_bf16)
     hip.lib().flux_hip_linear_force_tile(-1)
 
 
+@pytest.mark.parametrize("prows,C", [(1, 128), (5, 256), (37, 512), (63, 512), (2048, 128), (2049, 128), (4100, 256)])
+def test_group_norm_statistics_in_one_or_two_launches(hip, prows, C):
+    """Partial sums of any number of rows, on both sides of the switch between one launch and two: the statistics are
+    the same sums, so the normed image may differ from numpy's (float64) by its rounding to bf16 alone (2^-9)."""
+    H = W = 34                                          # not a multiple of the positions a workgroup covers
+    rows = (H + 2) * (W + 2)
+    x = normal_f32((C, H, W), 58, 1, 0.3, 1.0)
+    part = np.abs(normal_f32((prows, C // 4, 2), 58, 2))
+    part *= np.array([0.3, 1.09], np.float32) * 4 * H * W / part.sum(0, keepdims=True)     # mean 0.3, mean square 1.09 per quad
+    gm, bt = normal_f32((C,), 58, 5, 1.0, 0.2), normal_f32((C,), 58, 6)
+    dx, dp = hip.DevBuf.from_array(to_padded(x)), hip.DevBuf.from_array(part)
+    dg, dbt = hip.DevBuf.from_array(gm), hip.DevBuf.from_array(bt)
+    out = hip.DevBuf.from_array(np.full((rows, C), 0x4040, np.uint16))
+    scratch = hip.DevBuf(hip.lib().flux_hip_group_norm_scratch_floats(H + 2, W + 2) * 4)
+    hip.check(hip.lib().flux_hip_group_norm_stats(out.ptr, None, dx.ptr, 0, dg.ptr, dbt.ptr, scratch.ptr, H + 2, W + 2, C, 1e-4, 0, dp.ptr, prows))
+    got = bf16_to_f32(out.to_array(np.uint16, (rows, C)))
+    sums = part.astype(np.float64).sum(0).reshape(32, -1, 2).sum(1) / (H * W * C // 32)
+    mean, var = np.repeat(sums[:, 0], C // 32), np.repeat(sums[:, 1] - sums[:, 0] ** 2, C // 32)
+    want = (x - mean[:, None, None]) / np.sqrt(var + 1e-4)[:, None, None] * gm[:, None, None] + bt[:, None, None]
+    assert border_is_zero(got, H, W)
+    assert np.abs(from_padded(got, H, W) - want).max() <= 2.0 ** -8 * np.abs(want).max()
+    assert rel_l2(from_padded(got, H, W), want) < 2.0 ** -8
+
+
 def test_upsample(hip, oracle_mod):
     C, H, W = 128, 5, 7
     x = normal_f32((C, H, W), 55, 1)
