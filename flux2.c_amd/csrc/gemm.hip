@@ -68,6 +68,7 @@
  * side: each lane fetches the chunk that belongs at its LDS position.
  */
 #include "common.h"
+#include <type_traits>
 #include "../../include/flux_hip.h"
 #include "../../include/flux_hip_debug.h"
 
@@ -92,28 +93,47 @@ struct GemmArgs {
     int ksplit, kt_per;
     float *ws;
     int moff[GEMM_MAX_PARTS], ws_rows;
-    /* convolution epilogues (see flux_hip_conv): rows are the positions of a zero-bordered
-     * conv_hp x conv_wp image with channels contiguous. With 9 taps K runs over
+    /* convolution epilogues (see flux_hip_conv): the operand's rows are the conv_rows positions of a zero-bordered
+     * image conv_wp wide, channels contiguous; the GEMM's rows are its interior positions alone (conv_row), so that an
+     * image of 2^n positions is a whole number of tiles (with the border rows computed and thrown away, 256 x 256 positions
+     * x 512 channels were 522 tiles of 256 x 256, three rounds of 256 compute units instead of two). conv_wp = 0:
+     * every row is computed. With 9 taps K runs over
      * [cin / 64 channel chunks][9 taps][64 channels]: K step kt = 9 * chunk + tap reads the
      * activation rows shifted by its tap's (dy, dx). The nine taps of a chunk follow each other so
      * that what one tap fetched is still in L2 when the next asks for the neighbouring rows
      * (tap-major order re-fetched wide images 3 to 10 times from HBM). */
-    int conv_taps, conv_wp, conv_hp;
+    int conv_taps, conv_wp, conv_rows;
+    unsigned conv_magic; /* (2^32 - 1) / (conv_wp - 2) */
     const float *bias, *res;
     /* optional: per (row-tile half, 4-channel group) sums and sums of squares of what a convolution
      * epilogue writes, [prow][N/4][2], for the group norm that follows */
     float *stats;
 };
 
-template <int EPI> struct IsConv { static constexpr bool value = EPI == FLUX_HIP_EPI_CONV_BF16 || EPI == FLUX_HIP_EPI_CONV_F32; };
+/* internal epilogue: fp32 partial sums of one K slice of a convolution, rows = interior positions */
+#define EPI_CONV_PARTIAL 9
+template <int EPI> struct IsConv { static constexpr bool value = EPI == FLUX_HIP_EPI_CONV_BF16 || EPI == FLUX_HIP_EPI_CONV_F32 || EPI == EPI_CONV_PARTIAL; };
+
+/* m / (conv_wp - 2): the product with the truncated reciprocal is the quotient or one less for every 32-bit m */
+__device__ __forceinline__ int conv_div(const GemmArgs &g, int m) {
+    const unsigned w = g.conv_wp - 2, q = __umulhi((unsigned)m, g.conv_magic);
+    return (int)(q + ((unsigned)m - q * w >= w));
+}
+/* operand row of GEMM row m: the m-th interior position of the bordered image */
+template <int EPI>
+__device__ __forceinline__ int conv_row(const GemmArgs &g, int m) {
+    if (!IsConv<EPI>::value || g.conv_wp == 0) return m;
+    return m + 2 * conv_div(g, m) + g.conv_wp + 1;
+}
 
 /* Element offset of K step kt within an activation row. Plain GEMM: kt * 64. 3x3 convolution:
  * kt = 9 * chunk + tap; the tap selects a neighbour dy*Wp + dx rows away (uniform for the whole
  * launch, because border positions are rows of the matrix too), the chunk a 64-channel slice. */
 template <int EPI>
 __device__ __forceinline__ int a_step_offset(const GemmArgs &g, int kt) {
-    if (IsConv<EPI>::value && g.conv_taps == 9) {
-        const int chunk = (kt * 7282) >> 16, tap = kt - 9 * chunk; /* kt / 9, kt % 9 for kt < 2048 */
+    if (IsConv<EPI>::value) {
+        /* kt / 9, kt % 9 for kt < 2048; a 1x1 convolution's step is a chunk at the middle tap. No branch: this stands in the K loops */
+        const int nine = -(int)(g.conv_taps == 9), q = (kt * 7282) >> 16, chunk = kt + (nine & (q - kt)), tap = 4 + (nine & (kt - 9 * q - 4));
         const int dy = (tap * 11) >> 5, dx = tap - dy * 3;         /* tap / 3, tap % 3 for tap < 9 */
         return ((dy - 1) * g.conv_wp + (dx - 1)) * g.lda + chunk * 64;
     }
@@ -133,12 +153,26 @@ __device__ __forceinline__ int lds_swz(int r) { return ((r >> 1) & 7) ^ ((r & 1)
 /* s_waitcnt vmcnt(0) only (expcnt and lgkmcnt fields left at their maxima) */
 #define WAIT_VMCNT0() __builtin_amdgcn_s_waitcnt(0x0F70)
 
+/* A convolution kernel's arguments, read anew: what only the epilogue and the step to the next tile need (and what the compiler
+ * derives from it for their divisions) is more than the scalar registers hold across the K loops. */
+__device__ __forceinline__ GemmArgs conv_args_again() {
+    auto *ka = (const __attribute__((address_space(4))) GemmArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(ka));
+    GemmArgs a = {};
+    a.M[0] = ka->M[0]; a.C[0] = ka->C[0]; a.bias = ka->bias; a.res = ka->res; a.stats = ka->stats;
+    a.N = ka->N; a.ldc = ka->ldc; a.mtiles = ka->mtiles; a.ntiles = ka->ntiles; a.total_tiles = ka->total_tiles; a.vgrid = ka->vgrid;
+    a.ksplit = ka->ksplit;
+    a.conv_wp = ka->conv_wp; a.conv_rows = ka->conv_rows; a.conv_magic = ka->conv_magic;
+    return a;
+}
+
 /* Which tile (and K slice) a workgroup owns. Workgroups are dealt round-robin to the 8 XCDs;
  * each XCD gets a contiguous run of tiles so that its L2 sees the reuse, and tiles are walked in
  * groups of GROUP_M rows. */
 struct TileId {
     int ks, tm, tn, prob, tml;
 };
+template <bool ONE> /* one matrix, not parts */
 __device__ __forceinline__ bool decode_tile(const GemmArgs &g, int vb, TileId &t) {
     int per_xcd = g.vgrid >> 3;
     int logical = (vb & 7) * per_xcd + (vb >> 3);
@@ -152,6 +186,11 @@ __device__ __forceinline__ bool decode_tile(const GemmArgs &g, int vb, TileId &t
     int in_grp = logical - grp * per_group;
     t.tm = first_m + in_grp % gsz;
     t.tn = in_grp / gsz;
+    if (ONE) {
+        t.prob = 0;
+        t.tml = t.tm;
+        return true;
+    }
     t.prob = (t.tm >= g.mt_end[0]) + (t.tm >= g.mt_end[1]) + (t.tm >= g.mt_end[2]);
     t.tml = t.prob ? t.tm - g.mt_end[t.prob - 1] : t.tm;
     return true;
@@ -191,7 +230,7 @@ __device__ __forceinline__ int weight_row(const GemmArgs &g, int tn, int v) {
         return ((blk & 1) ? g.w_row1 : g.w_row0) + tn * (BN / 2) + idx;
     }
     int col;
-    if (EPI == FLUX_HIP_EPI_BF16 || EPI == EPI_QKV_SWIGLU) col = tn * BN + wv * WN + bf16_feature<TN>(blk, r);
+    if (EPI == FLUX_HIP_EPI_BF16 || EPI == EPI_QKV_SWIGLU || EPI == FLUX_HIP_EPI_CONV_BF16) col = tn * BN + wv * WN + bf16_feature<TN>(blk, r);
     else col = tn * BN + v;
     if (CutTile<BN>::value) col = min(col, g.N - 1);
     return g.w_row0 + col;
@@ -274,9 +313,6 @@ __device__ __forceinline__ void store_tile_to(const GemmArgs &g, const TileId &t
         else rows(BoolC<false>{});
         return;
     }
-    float st_s[TN], st_q[TN]; /* convolutions with statistics: this lane's sums per 16-column block */
-#pragma unroll
-    for (int i = 0; i < TN; i++) st_s[i] = st_q[i] = 0.0f;
 #pragma unroll
     for (int j = 0; j < TM; j++) {
         const int m = m0 + wm * WM + j * 16 + l15;
@@ -287,11 +323,6 @@ __device__ __forceinline__ void store_tile_to(const GemmArgs &g, const TileId &t
                 acc[i][j] = acc_in[i][j];
                 asm volatile("" : "+v"(acc[i][j]));
             }
-        }
-        bool inside = true; /* convolutions: border positions of the image are written as zeros */
-        if (IsConv<EPI>::value && g.conv_wp > 0) {
-            const int y = m / g.conv_wp, x = m - y * g.conv_wp;
-            inside = y >= 1 && y < g.conv_hp - 1 && x >= 1 && x < g.conv_wp - 1;
         }
         if (EPI == FLUX_HIP_EPI_SWIGLU) {
             /* see swiglu_feature: two (gate, up) pairs give eight consecutive features, a last odd pair four */
@@ -326,7 +357,7 @@ __device__ __forceinline__ void store_tile_to(const GemmArgs &g, const TileId &t
             for (int i = 0; i < TN; i++) {
                 if (CutTile<BN>::value && n0 + wn * WN + i * 16 >= g.N) continue; /* the same for the whole wave */
                 const int n = n0 + wn * WN + i * 16 + lq * 4;
-                if (EPI == EPI_PARTIAL) {
+                if (EPI == EPI_PARTIAL || EPI == EPI_CONV_PARTIAL) {
                     *(f32x4 *)(g.ws + ((size_t)ks * g.ws_rows + g.moff[prob] + m) * g.N + n) = acc[i][j];
                 } else if (EPI == FLUX_HIP_EPI_F32) {
                     *(f32x4 *)((float *)Cp + (size_t)m * ldc + n) = acc[i][j];
@@ -340,56 +371,128 @@ __device__ __forceinline__ void store_tile_to(const GemmArgs &g, const TileId &t
 #pragma unroll
                     for (int e = 0; e < 4; e++) x[e] += gt[e] * acc[i][j][e];
                     *(f32x4 *)p = x;
-                } else if (EPI == FLUX_HIP_EPI_CONV_BF16) {
-                    const f32x4 bv = *(const f32x4 *)(g.bias + n);
-                    bf16x4 o;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float v = inside ? acc[i][j][e] + bv[e] : 0.0f;
-                        o[e] = (bf16)v;
-                        st_s[i] += v;
-                        st_q[i] += v * v;
-                    }
-                    *(bf16x4 *)((bf16 *)Cp + (size_t)m * ldc + n) = o;
-                } else if (EPI == FLUX_HIP_EPI_CONV_F32) {
-                    const f32x4 bv = *(const f32x4 *)(g.bias + n);
-                    f32x4 r = {0.0f, 0.0f, 0.0f, 0.0f};
-                    if (g.res) r = *(const f32x4 *)(g.res + (size_t)m * ldc + n);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        r[e] = inside ? r[e] + acc[i][j][e] + bv[e] : 0.0f;
-                        st_s[i] += r[e];
-                        st_q[i] += r[e] * r[e];
-                    }
-                    *(f32x4 *)((float *)Cp + (size_t)m * ldc + n) = r;
                 }
             }
         }
     }
-    if (IsConv<EPI>::value && g.stats) {
-        /* sum over the 16 rows held by lanes of equal lane/16, then one lane per column quad stores */
+}
+
+/* What a convolution's tile stores: acc + bias [+ residual] at the interior positions, zeros at the border, and (g.stats) the
+ * sums for the group norm that follows. Two column blocks at a time over all row blocks, so that bias and sums of the
+ * whole tile never sit in registers beside the accumulators and the next tile's fragments; as in the residual epilogue above,
+ * the residual of the next row blocks is requested before the present ones are touched. bf16 outputs leave as 16-byte
+ * stores (bf16_pair_feature). The border is not computed: the positions behind the last pixel of an image row go with the
+ * tile that holds that pixel, the rows above and below the image are shared out over all row tiles. */
+template <int BN, int WM, int WN, int EPI, int WGM, bool HERE>
+__device__ __forceinline__ void store_conv_tile(const GemmArgs &g, const TileId &t, f32x4 (&acc_in)[WN / 16][WM / 16], int m0, int M,
+                                                int wm, int wn, int l15, int lq, int prow) {
+    constexpr int TM = WM / 16, TN = WN / 16, BM = WM * WGM;
+    constexpr bool F32 = EPI == FLUX_HIP_EPI_CONV_F32;
+    static_assert(TN % 2 == 0, "bf16 outputs pair 16-column blocks");
+    const int nw = t.tn * BN + wn * WN, ldc = g.ldc;
+    constexpr int RB = TM * TN * 4 > 224 ? 1 : 2, UPP = (TM + RB - 1) / RB, NU = TN / 2 * UPP; /* a unit: RB row blocks of one pair of column blocks */
+    using Off = std::conditional_t<HERE, unsigned, size_t>; /* (conv_launch sends outputs beyond 2^32 elements to the small tiles) */
+    Off off[TM]; /* first element of the wave's columns in each of this lane's rows; rows beyond M repeat the last one */
 #pragma unroll
-        for (int i = 0; i < TN; i++) {
+    for (int j = 0; j < TM; j++) off[j] = (Off)conv_row<EPI>(g, min(m0 + wm * WM + j * 16 + l15, M - 1)) * (Off)ldc + nw;
+    const auto rows = [&](auto res_c) {
+        constexpr bool RES = decltype(res_c)::value;
+        f32x4 xb[2][RB][2];
+        const auto fetch = [&](int u) {
+            const int i0 = u / UPP * 2, j0 = u % UPP * RB;
 #pragma unroll
-            for (int o = 1; o < 16; o <<= 1) {
-                st_s[i] += __shfl_xor(st_s[i], o);
-                st_q[i] += __shfl_xor(st_q[i], o);
+            for (int r = 0; r < RB; r++)
+#pragma unroll
+                for (int k = 0; k < 2; k++)
+                    if (j0 + r < TM) xb[u & 1][r][k] = *(const f32x4 *)(g.res + (size_t)off[j0 + r] + (i0 + k) * 16 + lq * 4);
+        };
+        if (RES) fetch(0);
+#pragma unroll
+        for (int ip = 0; ip < TN / 2; ip++) {
+            const int c0 = F32 ? ip * 32 + lq * 4 : ip * 32 + lq * 8, cs = F32 ? 16 : 4; /* columns of block 2 ip, and block 2 ip + 1 behind it */
+            const f32x4 bv[2] = {*(const f32x4 *)(g.bias + nw + c0), *(const f32x4 *)(g.bias + nw + c0 + cs)};
+            float st[2][2] = {{0.0f, 0.0f}, {0.0f, 0.0f}};
+            int left = M - (m0 + wm * WM + l15); /* rows of this lane's column of row blocks below M, compared anew per pair: TM kept lane masks are spilled */
+            asm volatile("" : "+v"(left));
+#pragma unroll
+            for (int ju = 0; ju < UPP; ju++) {
+                const int u = ip * UPP + ju;
+                if (RES && u + 1 < NU) fetch(u + 1);
+#pragma unroll
+                for (int r = 0; r < RB; r++) {
+                    const int j = ju * RB + r;
+                    if (j >= TM) continue;
+                    const bool ok = j * 16 < left;
+                    f32x4 v[2];
+#pragma unroll
+                    for (int k = 0; k < 2; k++) {
+                        f32x4 a = acc_in[2 * ip + k][j];
+                        if (HERE) asm volatile("" : "+v"(a)); /* out of its AGPRs here, one block at a time */
+                        float s = 0.0f, q = 0.0f;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            v[k][e] = RES ? xb[u & 1][r][k][e] + a[e] + bv[k][e] : a[e] + bv[k][e];
+                            s += v[k][e];
+                            q += v[k][e] * v[k][e];
+                        }
+                        st[k][0] += ok ? s : 0.0f;
+                        st[k][1] += ok ? q : 0.0f;
+                    }
+                    if (F32) {
+                        float *p = (float *)g.C[0] + (size_t)off[j] + c0;
+                        if (ok) {
+                            *(f32x4 *)p = v[0];
+                            *(f32x4 *)(p + 16) = v[1];
+                        }
+                    } else {
+                        bf16x4 o[2];
+#pragma unroll
+                        for (int e = 0; e < 4; e++) { o[0][e] = (bf16)v[0][e]; o[1][e] = (bf16)v[1][e]; }
+                        if (ok) store_bf16x8((bf16 *)g.C[0] + (size_t)off[j] + c0, o[0], o[1], true);
+                    }
+                }
             }
-            if (l15 == 0) {
-                const int n = n0 + wn * WN + i * 16 + lq * 4;
-                f32x2 v = {st_s[i], st_q[i]};
-                *(f32x2 *)(g.stats + ((size_t)prow * (g.N >> 2) + (n >> 2)) * 2) = v;
+            if (g.stats) {
+                /* sum over the 16 rows held by lanes of equal lane/16, then one lane per column quad stores */
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+#pragma unroll
+                    for (int o = 1; o < 16; o <<= 1) {
+                        st[k][0] += __shfl_xor(st[k][0], o);
+                        st[k][1] += __shfl_xor(st[k][1], o);
+                    }
+                    const f32x2 v = {st[k][0], st[k][1]};
+                    if (l15 == 0) *(f32x2 *)(g.stats + ((size_t)prow * (g.N >> 2) + ((nw + c0 + k * cs) >> 2)) * 2) = v;
+                }
             }
+        }
+    };
+    if (F32 && g.res) rows(BoolC<F32>{});
+    else rows(BoolC<false>{});
+    const int lane = lq * 16 + l15;
+    if (g.conv_wp > 0) {
+        constexpr int QPW = WN / 4, PPI = 64 / QPW; /* lanes per position, positions per instruction */
+        const int wp = g.conv_wp, y0 = conv_div(g, m0), y1 = conv_div(g, min(m0 + BM, M));
+        const int nside = 2 * (y1 - y0), nedge = 2 * wp + 1, per = (nedge + g.mtiles - 1) / g.mtiles;
+        const int e0 = min(nedge, t.tm * per), total = nside + min(nedge - e0, per);
+        for (int k = wm * PPI + lane / QPW; k < total; k += WGM * PPI) {
+            const int e = e0 + k - nside;
+            const int p = k < nside ? (y0 + (k >> 1) + 2) * wp - 1 + (k & 1) : e <= wp ? e : g.conv_rows - wp + (e - wp - 1);
+            const size_t at = (size_t)p * ldc + nw + (lane % QPW) * 4;
+            if (F32) *(f32x4 *)((float *)g.C[0] + at) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            else *(bf16x4 *)((bf16 *)g.C[0] + at) = bf16x4{(bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f};
         }
     }
 }
 
 /* Cp, ldc, tn: where the tile goes - the part's output, or for the fused [Q|K|V|gate|up] projection the output of the
  * side of the boundary the tile lies on (the tile width divides nq_cols, so a tile is wholly on one side) */
-template <int BN, int WM, int WN, int EPI, bool PINNED = false>
+template <int BN, int WM, int WN, int EPI, int WGM, bool PINNED = false>
 __device__ __forceinline__ void store_tile(const GemmArgs &g, const TileId &t, f32x4 (&acc)[WN / 16][WM / 16], int m0, int M,
                                            int wm, int wn, int l15, int lq, int prow) {
-    if constexpr (EPI == EPI_QKV_SWIGLU) {
+    if constexpr (EPI == FLUX_HIP_EPI_CONV_BF16 || EPI == FLUX_HIP_EPI_CONV_F32) {
+        store_conv_tile<BN, WM, WN, EPI, WGM, PINNED>(g, t, acc, m0, M, wm, wn, l15, lq, prow);
+    } else if constexpr (EPI == EPI_QKV_SWIGLU) {
         /* HERE = true: each side reads the accumulators through an empty asm statement, row by row. The conversions
          * are then work of that side; left to itself the compiler converted the whole tile to bf16 in front of the
          * branch, for both sides, and kept the hundred results in registers next to the other side's work, past
@@ -415,7 +518,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_kernel(GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     TileId t;
-    if (!decode_tile(g, blockIdx.x, t)) return;
+    if (!decode_tile<IsConv<EPI>::value>(g, blockIdx.x, t)) return;
     const int ks = t.ks, tn = t.tn, prob = t.prob;
     const bf16 *__restrict__ A = g.A[prob];
     const bf16 *__restrict__ W = g.W[prob];
@@ -434,7 +537,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_kernel(GemmArgs g) {
 #pragma unroll
     for (int i = 0; i < PA; i++) {
         int r = lrow + i * RPP;
-        int gm = min(m0 + r, M - 1);
+        int gm = conv_row<EPI>(g, min(m0 + r, M - 1));
         a_ptr[i] = A + (size_t)gm * g.lda + ((lchunk ^ lds_swz(r)) << 3);
         a_lds[i] = (wave * 8 + i * RPP) * 128;
     }
@@ -509,7 +612,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_kernel(GemmArgs g) {
         cur = cur == NS - 1 ? 0 : cur + 1;
     }
 
-    store_tile<BN, WM, WN, EPI>(g, t, acc, m0, M, wm, wn, l15, lq, t.tm * WGM + wm);
+    store_tile<BN, WM, WN, EPI, WGM>(g, t, acc, m0, M, wm, wn, l15, lq, t.tm * WGM + wm);
 }
 
 /* The large tiles: 4 waves (2 x 2), one per SIMD, each owning a (16 TM) x (16 TN) part of a
@@ -545,9 +648,8 @@ __device__ __forceinline__ void acc_fence(f32x4 (&acc)[TN][TM]) {
     }
 }
 
-/* whether a workgroup of gemm4w_kernel goes on to further tiles (the 4-wave form of the transformer's epilogues;
- * with the convolution epilogues the values kept across tiles would spill) */
-template <int EPI, int WAVES> struct Walks4w { static constexpr bool value = !IsConv<EPI>::value && WAVES == 4; };
+/* whether a workgroup of gemm4w_kernel goes on to further tiles: the 4-wave form */
+template <int WAVES> struct Walks4w { static constexpr bool value = WAVES == 4; };
 
 template <int TM, int TN, int EPI, int WGM = 2, int WGN = 2>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm4w_kernel(GemmArgs g) {
@@ -584,7 +686,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm4w_kernel(GemmArgs g) {
      * start of the next on a compute unit cost 5-14 us of a 60 us tile). */
     int vb = blockIdx.x;
     TileId t;
-    if (!decode_tile(g, vb, t)) return;
+    if (!decode_tile<IsConv<EPI>::value>(g, vb, t)) return;
 
     /* Load i of a stage by this wave covers tile rows lrow + RPP i (8 rows of 128 bytes per wave
      * instruction): activation rows for i < LA, weight rows after. Rows RPP apart share a swizzle.
@@ -603,9 +705,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm4w_kernel(GemmArgs g) {
 #pragma unroll
         for (int i = 0; i < LB; i++) voff[LA + i] = ((unsigned)weight_row<BN, WN, EPI>(g, tt.tn, lrow + i * RPP) * (unsigned)g.ldw + chunk) * 2u;
     };
-    /* (convolutions never split K, so for them kt below is the absolute K step) */
     auto issue1 = [&](int kt, int stage, int i) {
-        const char *base = i < LA ? baseA + (ptrdiff_t)a_step_offset<EPI>(g, kt) * 2 : baseW + kt * 128;
+        const char *base = (i < LA ? baseA : baseW) + kt * 128;
         asm volatile("" : "+v"(voff[i])); /* keeps the load in its scalar base + 32-bit lane offset form, see gemm4d_kernel */
         __builtin_amdgcn_global_load_lds(GLOBAL_PTR(base + voff[i]), LDS_PTR(smem + stage * STAGE + (wave * 8 + i * RPP) * 128), 16, 0, 0);
     };
@@ -681,7 +782,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm4w_kernel(GemmArgs g) {
          * its last fragments out of LDS once it is past this barrier. */
         const TileId done = t;
         vb += gridDim.x;
-        const bool again = Walks4w<EPI, WGM * WGN>::value && vb < g.vgrid && decode_tile(g, vb, t);
+        const bool again = Walks4w<WGM * WGN>::value && vb < g.vgrid && decode_tile<IsConv<EPI>::value>(g, vb, t);
         if (again) {
             __syncthreads();
             set_sources(t);
@@ -697,7 +798,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm4w_kernel(GemmArgs g) {
          * across the K loops, beyond what the register file holds beside the accumulators and fragments. */
         int l15e = l15, lqe = lq;
         asm volatile("" : "+v"(l15e), "+v"(lqe));
-        store_tile<BN, WM, WN, EPI, true>(g, done, acc, done.tml * BM, g.M[done.prob], wm, wn, l15e, lqe, done.tm * WGM + wm);
+        store_tile<BN, WM, WN, EPI, WGM, true>(g, done, acc, done.tml * BM, g.M[done.prob], wm, wn, l15e, lqe, done.tm * WGM + wm);
         if (!again) break;
     }
 }
@@ -727,7 +828,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm4w_kernel(GemmArgs g) {
 template <int EPI, int TM, int TN>
 struct EpilogueOps { /* vector memory instructions a wave issues in the epilogue of a tile whose rows are all valid */
     static constexpr int value = EPI == FLUX_HIP_EPI_SWIGLU || EPI == EPI_QKV_SWIGLU ? TM * (TN / 4 + TN / 2 % 2) /* 16-byte stores + a last 8-byte one */
-                                 : EPI == FLUX_HIP_EPI_BF16 ? TM * (TN / 2 + TN % 2) : EPI == FLUX_HIP_EPI_F32_T ? 4 * TM * TN : TM * TN;
+                                 : EPI == FLUX_HIP_EPI_BF16 || EPI == FLUX_HIP_EPI_CONV_BF16 ? TM * (TN / 2 + TN % 2) : EPI == FLUX_HIP_EPI_F32_T ? 4 * TM * TN : TM * TN;
 };
 
 template <int TM, int TN, int EPI, int NSA, int NSW>
@@ -764,7 +865,7 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
 
     int vb = blockIdx.x;
     TileId t;
-    if (!decode_tile(g, vb, t)) return;
+    if (!decode_tile<IsConv<EPI>::value>(g, vb, t)) return;
 
     /* Sources of a tile's loads: a uniform base per operand (the tile's matrix + this workgroup's K slice) and a 32-bit
      * byte offset per lane and load, so that stepping along K is scalar work. Two sets: the tile being multiplied and
@@ -772,6 +873,7 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
     struct Src {
         unsigned voff[NL];
         const char *baseA, *baseW;
+        int k0; /* convolutions: the first K step of the slice (the rows' offset is a function of the absolute step) */
     };
     Src cur, nxt;
     auto set_sources = [&](Src &sc, const TileId &tt) {
@@ -782,20 +884,23 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
         int lr = lrow;
         asm volatile("" : "+v"(lr));
         const int chunk = (lchunk ^ lds_swz(lr)) << 3;
-        sc.baseA = (const char *)(g.A[tt.prob] + tt.ks * g.kt_per * 64);
+        sc.k0 = IsConv<EPI>::value ? tt.ks * g.kt_per : 0;
+        sc.baseA = (const char *)(g.A[tt.prob] + (IsConv<EPI>::value ? 0 : tt.ks * g.kt_per * 64));
         sc.baseW = (const char *)(g.W[tt.prob] + tt.ks * g.kt_per * 64);
 #pragma unroll
-        for (int i = 0; i < LA; i++) sc.voff[i] = ((unsigned)min(m0 + lr + i * RPP, M - 1) * (unsigned)g.lda + chunk) * 2u;
+        for (int i = 0; i < LA; i++) sc.voff[i] = ((unsigned)conv_row<EPI>(g, min(m0 + lr + i * RPP, M - 1)) * (unsigned)g.lda + chunk) * 2u;
 #pragma unroll
         for (int i = 0; i < LB; i++) sc.voff[LA + i] = ((unsigned)weight_row<BN, WN, EPI>(g, tt.tn, lr + i * RPP) * (unsigned)g.ldw + chunk) * 2u;
     };
-    /* load i of K step kt of the tile whose sources are (baseA, baseW, vo): activation rows for i < LA (into slot sa
+    /* where K step kt of an operand starts */
+    auto step_a = [&](const Src &sc, int kt) { return sc.baseA + (ptrdiff_t)a_step_offset<EPI>(g, sc.k0 + kt) * 2; };
+    auto step_w = [&](const Src &sc, int kt) { return sc.baseW + (ptrdiff_t)kt * 128; };
+    /* load i of the K step that starts at base: activation rows for i < LA (into slot sa
      * of their ring), weight rows after (slot sw). The offset passes through an empty asm statement where it is used: the
      * load is then selected in its "scalar base + 32-bit lane offset" form. Without it the compiler widens every offset
      * to 64 bits once, outside the K loop, keeps NL register pairs instead of NL registers, and adds the base with a
      * 64-bit vector addition in front of every load. */
-    auto issue1 = [&](const char *baseA, const char *baseW, unsigned &vo, int kt, int sa, int sw, int i) {
-        const char *base = (i < LA ? baseA : baseW) + (ptrdiff_t)kt * 128;
+    auto issue1 = [&](const char *base, unsigned &vo, int sa, int sw, int i) {
         const int dst = i < LA ? sa * ASZ + (wave * 8 + i * RPP) * 128 : NSA * ASZ + sw * WSZ + (wave * 8 + (i - LA) * RPP) * 128;
         asm volatile("" : "+v"(vo));
         __builtin_amdgcn_global_load_lds(GLOBAL_PTR(base + vo), LDS_PTR(smem + dst), 16, 0, 0);
@@ -808,12 +913,12 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
         for (int s = 0; s < 2; s++) {
             if (s < KTn) {
 #pragma unroll
-                for (int i = 0; i < NL; i++) issue1(sc.baseA, sc.baseW, sc.voff[i], s, s, s, i);
+                for (int i = 0; i < NL; i++) issue1(i < LA ? step_a(sc, s) : step_w(sc, s), sc.voff[i], s, s, i);
             }
         }
         if (NS2 == 3 && KTn > 2) {
 #pragma unroll
-            for (int n = 0; n < LS; n++) issue1(sc.baseA, sc.baseW, sc.voff[(FIRST_A ? LA : 0) + n], 2, 2, 2, (FIRST_A ? LA : 0) + n);
+            for (int n = 0; n < LS; n++) issue1(FIRST_A ? step_w(sc, 2) : step_a(sc, 2), sc.voff[(FIRST_A ? LA : 0) + n], 2, 2, (FIRST_A ? LA : 0) + n);
         }
     };
 
@@ -847,22 +952,27 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
             auto &accr = acc;
             const int na = ca == NSA - 1 ? 0 : ca + 1, nw = cw == NSW - 1 ? 0 : cw + 1;
             const unsigned van = a_frag + na * ASZ, vwn = w_frag + nw * WSZ;
-            auto load = [&](int ks, int sa, int sw, int i) {
+            const auto start = [&](int ks, bool a) {
+                const bool over = TAIL && ks >= KT;
+                const Src &sc = over ? nxt : cur;
+                return a ? step_a(sc, over ? ks - KT : ks) : step_w(sc, over ? ks - KT : ks);
+            };
+            auto load = [&](const char *base, int ks, int sa, int sw, int i) {
                 if (!TAIL) {
-                    issue1(cur.baseA, cur.baseW, cur.voff[i], ks, sa, sw, i);
+                    issue1(base, cur.voff[i], sa, sw, i);
                 } else {
-                    const bool over = ks >= KT;
-                    unsigned vo = over ? nxt.voff[i] : cur.voff[i];
-                    issue1(over ? nxt.baseA : cur.baseA, over ? nxt.baseW : cur.baseW, vo, over ? ks - KT : ks, sa, sw, i);
+                    unsigned vo = ks >= KT ? nxt.voff[i] : cur.voff[i];
+                    issue1(base, vo, sa, sw, i);
                 }
             };
+            const char *first = start(kt + 2, FIRST_A), *second = start(kt + NS2, !FIRST_A); /* the K steps requested in the two halves */
 #pragma unroll
             for (int b = 0; b < NM; b++) {
                 if (FIRST) MFMA_AGPR_NEW(accr[serp(b)][b / TN], f0[serp(b)], f0[TN + b / TN]);
                 else MFMA_AGPR(accr[serp(b)][b / TN], f0[serp(b)], f0[TN + b / TN]);
                 if (b % RD == 0 && b / RD < NF) f1[b / RD] = frag(va, vw, coff1, b / RD);
                 /* step kt + 2 of the first operand, into the slot that step kt - 1 left */
-                if (b % SF == 1 && b / SF < LF) load(kt + 2, ca == 0 ? 2 : ca - 1, cw == 0 ? 2 : cw - 1, (FIRST_A ? 0 : LA) + b / SF);
+                if (b % SF == 1 && b / SF < LF) load(first, kt + 2, ca == 0 ? 2 : ca - 1, cw == 0 ? 2 : cw - 1, (FIRST_A ? 0 : LA) + b / SF);
             }
             /* step kt + 1 has landed for this wave and its reads of step kt are complete; past the barrier both hold
              * for all */
@@ -873,7 +983,7 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
                 MFMA_AGPR(accr[serp(b)][b / TN], f1[serp(b)], f1[TN + b / TN]);
                 if (b % RD == 0 && b / RD < NF) f0[b / RD] = frag(van, vwn, coff0, b / RD);
                 /* step kt + NS2 of the second operand, into the slot of step kt */
-                if (b % SS == 1 && b / SS < LS) load(kt + NS2, ca, cw, (FIRST_A ? LA : 0) + b / SS);
+                if (b % SS == 1 && b / SS < LS) load(second, kt + NS2, ca, cw, (FIRST_A ? LA : 0) + b / SS);
             }
             ca = na;
             cw = nw;
@@ -890,7 +1000,13 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
          * request this tile's first steps once more, into slots that nobody reads again. */
         const TileId done = t;
         vb += gridDim.x;
-        const bool again = vb < g.vgrid && decode_tile(g, vb, t);
+        bool again;
+        if constexpr (IsConv<EPI>::value) {
+            const GemmArgs gd = conv_args_again();
+            again = vb < gd.vgrid && decode_tile<true>(gd, vb, t);
+        } else {
+            again = vb < g.vgrid && decode_tile<IsConv<EPI>::value>(g, vb, t);
+        }
         if (again) set_sources(nxt, t);
         else nxt = cur;
         for (; kt < KT; kt++) step(kt, BoolC<true>{}, IntC<AHEAD>{}, BoolC<false>{});
@@ -904,7 +1020,12 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
          * across the K loops, beyond what the register file holds beside the accumulators and fragments. */
         int l15e = l15, lqe = lq;
         asm volatile("" : "+v"(l15e), "+v"(lqe));
-        store_tile<BN, WM, WN, EPI, true>(g, done, acc, done.tml * BM, g.M[done.prob], wm, wn, l15e, lqe, done.tm * WGM + wm);
+        if constexpr (EPI == FLUX_HIP_EPI_CONV_BF16 || EPI == FLUX_HIP_EPI_CONV_F32) {
+            const GemmArgs ge = conv_args_again();
+            store_tile<BN, WM, WN, EPI, WGM, true>(ge, done, acc, done.tml * BM, ge.M[0], wm, wn, l15e, lqe, done.tm * WGM + wm);
+        } else {
+            store_tile<BN, WM, WN, EPI, WGM, true>(g, done, acc, done.tml * BM, g.M[done.prob], wm, wn, l15e, lqe, done.tm * WGM + wm);
+        }
         if (!again) break;
         /* not every row of this wave's part of the stored tile was valid, or not every column: it issued fewer than
          * EpilogueOps operations */
@@ -978,7 +1099,7 @@ static int launch_4w(GemmArgs &g) {
     if (span >= ((size_t)1 << 32)) return g.N % 128 == 0 ? launch_cfg<128, 128, 2, 2, EPI>(g) : launch_cfg<64, 64, 2, 2, EPI>(g);
     /* one workgroup fits on a compute unit (registers, LDS): launch at most that many, each walks its share of the tiles */
     g.vgrid = (g.total_tiles * g.ksplit + 7) & ~7;
-    const int grid = g_persistent && Walks4w<EPI, WGM * WGN>::value ? min(g.vgrid, compute_units() & ~7) : g.vgrid;
+    const int grid = g_persistent && Walks4w<WGM * WGN>::value ? min(g.vgrid, compute_units() & ~7) : g.vgrid;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * WGM * WGN), LDS, flux_hip_stream_handle(), g);
     HIP_OK(hipGetLastError());
     return 1;
@@ -1003,7 +1124,8 @@ static int launch_4d(GemmArgs &g) {
     g.total_tiles = g.mtiles * g.ntiles;
     size_t span = ((size_t)max(max(g.w_row0, g.w_row1), g.w_row2) + g.N) * g.ldw * 2;
     for (int i = 0; i < GEMM_MAX_PARTS; i++) span = max(span, (size_t)g.M[i] * g.lda * 2);
-    if (span >= ((size_t)1 << 32)) return g.N % 128 == 0 ? launch_cfg<128, 128, 2, 2, EPI>(g) : launch_cfg<64, 64, 2, 2, EPI>(g);
+    if constexpr (!IsConv<EPI>::value) /* (conv_launch has looked) */
+        if (span >= ((size_t)1 << 32)) return g.N % 128 == 0 ? launch_cfg<128, 128, 2, 2, EPI>(g) : launch_cfg<64, 64, 2, 2, EPI>(g);
     g.vgrid = (g.total_tiles * g.ksplit + 7) & ~7;
     const int grid = min(g.vgrid, compute_units() & ~7);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), LDS, flux_hip_stream_handle(), g);
@@ -1043,18 +1165,6 @@ static int launch_epi(GemmArgs &g, int tile) {
         case 8: return launch_cfg<64, 128, 2, 2, EPI, 6>(g);  /* few rows: the same tiles with a ring that fills the LDS */
         case 9: return launch_cfg<128, 128, 2, 2, EPI, 5>(g);
         case 10: return launch_cfg<96, 128, 2, 2, EPI, 5>(g);
-        default: return launch_cfg<64, 128, 2, 2, EPI>(g);
-    }
-}
-
-/* The convolution epilogues exist for the tiles whose width divides 64, 128, 256 or 512 output
- * channels. */
-template <int EPI>
-static int launch_conv(GemmArgs &g, int tile) {
-    switch (tile) {
-        case 2: return launch_4w<8, 8, EPI>(g);
-        case 1: return launch_cfg<128, 128, 2, 2, EPI>(g);
-        case 3: return launch_cfg<64, 64, 2, 2, EPI>(g);
         default: return launch_cfg<64, 128, 2, 2, EPI>(g);
     }
 }
@@ -1100,6 +1210,69 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(GemmArgs g) {
 #pragma unroll
         for (int e = 0; e < 4; e++) o[e] = (bf16)(EPI == FLUX_HIP_EPI_SWIGLU ? silu_f(sum[e]) * sum2[e] : sum[e]);
         *(bf16x4 *)((bf16 *)g.C[prob] + (size_t)m * g.ldc + n) = o;
+    }
+}
+
+/* Second pass of a convolution that ran as K slices: sums the slices of 32 positions x 64 channels in slice order, adds bias and
+ * residual, writes the interior and the zero border, and leaves the sums for the group norm that follows, one row of
+ * them per 32 positions. ksplit = 0 (an image without interior) writes zeros. */
+template <int EPI>
+__global__ __launch_bounds__(256) void conv_finish_kernel(GemmArgs g) {
+    __shared__ float sh[4 * 16 * 2];
+    constexpr bool F32 = EPI == FLUX_HIP_EPI_CONV_F32;
+    const int q = threadIdx.x & 15, r = threadIdx.x >> 4, n = blockIdx.y * 64 + q * 4, wp = g.conv_wp;
+    const size_t slice = (size_t)g.M[0] * g.N;
+    float s1 = 0.0f, s2 = 0.0f;
+    const f32x4 bv = *(const f32x4 *)(g.bias + n);
+#pragma unroll
+    for (int it = 0; it < 2; it++) {
+        const int p = blockIdx.x * 32 + it * 16 + r;
+        if (p >= g.conv_rows) break;
+        int m = p;
+        bool inside = g.ksplit > 0;
+        if (wp > 0) {
+            const int y = p / wp, x = p - y * wp;
+            inside = inside && y >= 1 && p < g.conv_rows - wp && x >= 1 && x < wp - 1;
+            m = (y - 1) * (wp - 2) + x - 1;
+        }
+        f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (inside) {
+            f32x4 a = v;
+            if (F32 && g.res) v = *(const f32x4 *)(g.res + (size_t)p * g.ldc + n);
+            const float *w = g.ws + (size_t)m * g.N + n;
+#pragma unroll 8
+            for (int s = 0; s < g.ksplit; s++) {
+                const f32x4 t = *(const f32x4 *)(w + s * slice);
+#pragma unroll
+                for (int e = 0; e < 4; e++) a[e] += t[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                v[e] = v[e] + a[e] + bv[e];
+                s1 += v[e];
+                s2 += v[e] * v[e];
+            }
+        }
+        if (F32) {
+            *(f32x4 *)((float *)g.C[0] + (size_t)p * g.ldc + n) = v;
+        } else {
+            bf16x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = (bf16)v[e];
+            *(bf16x4 *)((bf16 *)g.C[0] + (size_t)p * g.ldc + n) = o;
+        }
+    }
+    if (g.stats) {
+        s1 += __shfl_xor(s1, 16); s2 += __shfl_xor(s2, 16);
+        s1 += __shfl_xor(s1, 32); s2 += __shfl_xor(s2, 32);
+        const int wave = threadIdx.x >> 6;
+        if ((threadIdx.x & 63) < 16) { sh[(wave * 16 + q) * 2] = s1; sh[(wave * 16 + q) * 2 + 1] = s2; }
+        __syncthreads();
+        if (threadIdx.x < 16) {
+            const float *c = sh + q * 2;
+            const f32x2 o = {(c[0] + c[32]) + (c[64] + c[96]), (c[1] + c[33]) + (c[65] + c[97])};
+            *(f32x2 *)(g.stats + ((size_t)blockIdx.x * (g.N >> 2) + (n >> 2)) * 2) = o;
+        }
     }
 }
 
@@ -1493,8 +1666,6 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
             break;
         case FLUX_HIP_EPI_SWIGLU: ok = split ? launch_split<FLUX_HIP_EPI_SWIGLU>(g, tile) : launch_epi<FLUX_HIP_EPI_SWIGLU>(g, tile); break;
         case EPI_QKV_SWIGLU: ok = launch_epi<EPI_QKV_SWIGLU>(g, tile); break;
-        case FLUX_HIP_EPI_CONV_BF16: ok = launch_conv<FLUX_HIP_EPI_CONV_BF16>(g, tile); break;
-        case FLUX_HIP_EPI_CONV_F32: ok = launch_conv<FLUX_HIP_EPI_CONV_F32>(g, tile); break;
         default: return flux_hip_fail("flux_hip_linear: unknown epilogue %d", epilogue);
     }
     if (slot >= 0) (void)hipEventRecord(g_probe_ev[slot][1], flux_hip_stream_handle());
@@ -1609,6 +1780,87 @@ extern "C" int flux_hip_linear_resid_adaln(int nparts, const flux_hip_linear_par
 
 
 
+/* Tiles of a convolution: ids 0 to 3 as above (64 x 128, 128 x 128, 256 x 256, 64 x 64), 12 = 256 x 128. The two with 256
+ * rows run in the ring kernel: 128 x 128 in two stages reached 700 to 870 TFLOP/s on 3x3 layers of 128 to 512 channels over
+ * 128 x 128 to 1024 x 1024 positions, 256 x 128 reaches 920 to 1230 and 256 x 256 1200 to 1390 (bf16 output). */
+template <int EPI>
+static int conv_tile_launch(GemmArgs &g, int tile) {
+    switch (tile) {
+        case 2: return launch_4d<8, 8, EPI, 2, 3>(g);
+        case 12: return launch_4d<8, 4, EPI, 3, 3>(g);
+        case 1: return launch_cfg<128, 128, 2, 2, EPI>(g);
+        case 3: return launch_cfg<64, 64, 2, 2, EPI>(g);
+        default: return launch_cfg<64, 128, 2, 2, EPI>(g);
+    }
+}
+
+#define CONV_TILES 13
+static const int conv_bm[CONV_TILES] = {64, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 256}, conv_bn[CONV_TILES] = {128, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 128};
+
+template <int EPI>
+static int conv_finish(GemmArgs &g) {
+    hipLaunchKernelGGL(conv_finish_kernel<EPI>, dim3((g.conv_rows + 31) / 32, g.N / 64), dim3(256), 0, flux_hip_stream_handle(), g);
+    HIP_OK(hipGetLastError());
+    return 1;
+}
+
+/* Tile and K split of a convolution by the same kind of model as gemm_dispatch's: rounds of workgroups, each a tile's time at
+ * its measured rate plus the bytes of its epilogue at a compute unit's share of the memory rate (nothing overlaps those where one
+ * workgroup owns the unit). K slices, which add a second pass and its partial sums, are what small images need: 32 x 32
+ * positions x 512 channels are 32 tiles of 128 x 128 for 256 units, 57 us in one piece and 24 in slices; at 96 x 96 positions
+ * one piece wins (54 us against 69). */
+static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
+    static const int occ[CONV_TILES] = {3, 2, 1, 4, 0, 0, 0, 0, 0, 0, 0, 0, 1};
+    static const double rate[CONV_TILES] = {2.0e12, 3.3e12, 5.4e12, 1.5e12, 0, 0, 0, 0, 0, 0, 0, 0, 4.8e12}; /* FLOP/s of one CU */
+    static const int splits[] = {1, 2, 3, 4, 6, 8, 12, 16};
+    const int M = g.M[0], N = g.N, kt_total = g.K >> 6, f = g_force_tile;
+    const bool forced = f >= 0 && f < CONV_TILES && conv_bm[f] && N % conv_bn[f] == 0; /* a forced tile that this layer cannot use is ignored */
+    const bool ring_ok = g_ring && (size_t)g.conv_rows * g.lda * 2 < ((size_t)1 << 32) && (size_t)N * g.ldw * 2 < ((size_t)1 << 32) &&
+                         (size_t)g.conv_rows * N < ((size_t)1 << 32);
+    int tile = -1, split = 1;
+    double best = 1e30;
+    for (int t = 0; t < CONV_TILES; t++) {
+        const bool ring = t == 2 || t >= 12;
+        if (!conv_bm[t] || N % conv_bn[t] || (forced && t != f)) continue;
+        if (t == 0 && !forced) continue; /* (for comparison runs) */
+        if (ring && (!ring_ok || kt_total < 4)) continue;
+        const long tiles = (long)((M + conv_bm[t] - 1) / conv_bm[t]) * (N / conv_bn[t]);
+        for (int sp : splits) {
+            const int per = (kt_total + sp - 1) / sp, used = (kt_total + per - 1) / per, last = kt_total - (used - 1) * per;
+            if (sp > 1 && (!g_splitk_enabled || per < 4 || last < 4 || used != sp || N % 64)) continue;
+            if (g_force_split && kt_total / g_force_split >= 4 && sp != g_force_split) continue;
+            const double ws = (double)sp * M * N * 4.0;
+            if (sp > 1 && ws > 256e6) continue;
+            const long blocks = tiles * sp, slots = 256L * occ[t], rounds = (blocks + slots - 1) / slots;
+            const long per_cu = (min(blocks, slots) + 255) / 256;
+            double est = rounds * (2.0 * conv_bm[t] * conv_bn[t] * 64.0 * per / (rate[t] / per_cu) + 2.5e-6 +
+                                   (double)conv_bm[t] * conv_bn[t] * (sp > 1 ? 0 : epilogue == FLUX_HIP_EPI_CONV_BF16 ? 2 : g.res ? 8 : 4) / 2.0e10);
+            if (sp > 1) est += 4.0e-6 + 2.0 * ws / 4.0e12;
+            if (est < best) { best = est; tile = t; split = sp; }
+        }
+    }
+    if (tile < 0) tile = N % 128 == 0 ? 1 : 3; /* (a forced ring tile that cannot run) */
+    g.kt_per = (kt_total + split - 1) / split;
+    g.ksplit = split;
+    const bool bf = epilogue == FLUX_HIP_EPI_CONV_BF16;
+    int ok;
+    if (M == 0) { /* nothing but border */
+        g.ksplit = 0;
+        if (stats_rows) *stats_rows = (g.conv_rows + 31) / 32;
+        return bf ? conv_finish<FLUX_HIP_EPI_CONV_BF16>(g) : conv_finish<FLUX_HIP_EPI_CONV_F32>(g);
+    }
+    if (split > 1) {
+        if (!ensure_ws((size_t)split * M * N * sizeof(float))) return 0;
+        g.ws = g_ws;
+        g.ws_rows = M;
+        ok = conv_tile_launch<EPI_CONV_PARTIAL>(g, tile) && (bf ? conv_finish<FLUX_HIP_EPI_CONV_BF16>(g) : conv_finish<FLUX_HIP_EPI_CONV_F32>(g));
+        if (stats_rows) *stats_rows = (g.conv_rows + 31) / 32;
+        return ok;
+    }
+    if (stats_rows) *stats_rows = 2 * ((M + conv_bm[tile] - 1) / conv_bm[tile]);
+    return bf ? conv_tile_launch<FLUX_HIP_EPI_CONV_BF16>(g, tile) : conv_tile_launch<FLUX_HIP_EPI_CONV_F32>(g, tile);
+}
+
 /* Convolution over a zero-bordered channels-last image as one GEMM, see the header. */
 extern "C" int flux_hip_conv_stats(int epilogue, const void *in, const void *w, const float *bias, const float *res, void *out, int rows,
                                    int wp, int cin, int cout, int taps, float *stats, int *stats_rows);
@@ -1637,27 +1889,14 @@ extern "C" int flux_hip_conv_stats(int epilogue, const void *in, const void *w, 
     g.A[0] = (const bf16 *)in;
     g.W[0] = (const bf16 *)w;
     g.C[0] = out;
-    g.M[0] = rows;
     g.N = cout; g.K = taps * cin; g.lda = cin; g.ldw = taps * cin; g.ldc = cout;
-    g.conv_taps = taps; g.conv_wp = wp; g.conv_hp = wp > 0 ? rows / wp : 0;
+    g.conv_taps = taps; g.conv_wp = wp; g.conv_rows = rows;
+    g.M[0] = rows;
+    if (wp > 0) {
+        g.M[0] = wp > 2 && rows / wp > 2 ? (rows / wp - 2) * (wp - 2) : 0;
+        g.conv_magic = wp > 2 ? 0xFFFFFFFFu / (unsigned)(wp - 2) : 0;
+    }
     g.bias = bias; g.res = res; g.stats = stats;
     if (stats && (!stats_rows || ((uintptr_t)stats & 7))) return flux_hip_fail("flux_hip_conv_stats: stats needs stats_rows and 8-byte alignment");
-    const unsigned conv_tiles = 0x0F; /* 64x128, 128x128, 256x256 (4 waves), 64x64 */
-    static const int width[4] = {128, 128, 256, 64};
-    unsigned allowed;
-    if (g_force_tile >= 0 && g_force_tile < 4 && cout % width[g_force_tile] == 0) {
-        allowed = 1u << g_force_tile; /* a forced tile that this layer cannot use is ignored */
-    } else {
-        /* These layers move many bytes per FLOP (fp32 image in and out of the epilogue), which a
-         * second resident workgroup hides and the one-workgroup-per-CU 256 x 256 tile does not:
-         * measured over the decoder's layers, 128 x 128 wins (3-15 %) until the launch is at least
-         * eight full rounds of 256 x 256 tiles, where the big tile's higher MFMA rate takes over. */
-        const long big_tiles = cout % 256 ? 0 : (long)((rows + 255) / 256) * (cout / 256);
-        allowed = big_tiles >= 2048 ? 1u << 2 : cout % 128 == 0 ? 1u << 1 : 1u << 3;
-    }
-    int tile = -1;
-    if (!gemm_dispatch(g, 1, epilogue, allowed & conv_tiles, &tile)) return 0;
-    static const int tile_rows[4] = {64, 128, 256, 64}; /* every convolution tile is two waves high */
-    if (stats_rows) *stats_rows = 2 * ((rows + tile_rows[tile & 3] - 1) / tile_rows[tile & 3]);
-    return 1;
+    return conv_launch(g, epilogue, stats_rows);
 }

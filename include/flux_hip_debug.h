@@ -20,7 +20,7 @@ extern "C" {
  * with a ring of 6 / 5 / 5 LDS stages, only for row ranges of at most 64 / 128 / 96 rows; 11 = 256x224, whose last column
  * tile is cut off at N: for the residual and bf16 epilogues with at least four 64-wide K steps and no K slices), -1
  * restores the automatic choice (a tile whose width does not divide N is skipped, tile 11 apart; if none is left the
- * 128x128 tile runs). */
+ * 128x128 tile runs). Convolutions know tiles 0 to 3 and 12 (256x128) and ignore one whose width does not divide cout. */
 void flux_hip_linear_force_tile(int tile);
 /* bit t set = the automatic choice may use tile t (default 0xFEF: all but tile 4; 0 restores it) */
 void flux_hip_linear_tile_mask(unsigned mask);

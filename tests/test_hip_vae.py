@@ -141,6 +141,63 @@ def test_conv1x1(hip, oracle_mod):
     np.testing.assert_allclose(got[0], b, rtol=1e-6)
 
 
+@pytest.mark.parametrize("H,W,cin,cout", [(1, 1, 64, 256), (1, 40, 128, 256), (301, 1, 64, 256), (17, 31, 512, 256), (16, 16, 512, 512),
+                                          (280, 281, 64, 128), (200, 190, 64, 256)])
+def test_conv_tiles_and_slices(hip, H, W, cin, cout):
+    """The ring tiles (2: 256 x 256, 12: 256 x 128) against the 128 x 128 one, which test_conv3x3 ties to the oracle: the same
+    K order, so the same bits, at images smaller than a tile, one pixel wide, with cut-off last tiles, and with more tiles
+    than compute units (280 x 281: 308 tiles). K slices regroup an fp32 sum of 9 cin products: at most cin * 9 roundings
+    of 2^-24 of the sum of magnitudes, in practice their root. The statistics are sums of what was written."""
+    import ctypes
+    L = hip.lib()
+    rows, wp = (H + 2) * (W + 2), W + 2
+    x, w = q(normal_f32((cin, H, W), 59, 1)), q(normal_f32((cout, cin, 3, 3), 59, 2, 0.0, 0.05))
+    b, res = normal_f32((cout,), 59, 3), normal_f32((cout, H, W), 59, 4)
+    din = Guarded(hip, to_padded(x), wp)
+    dw, db, dres = hip.DevBuf.from_array(conv_weight(w)), hip.DevBuf.from_array(b), hip.DevBuf.from_array(to_padded(res))
+
+    def run(tile, split, epi, r):
+        L.flux_hip_linear_force_tile(tile)
+        L.flux_hip_linear_force_split(split)
+        bf = epi == hip.EPI_CONV_BF16
+        out = hip.DevBuf.from_array(np.full((rows, cout), 3.0, np.float32))
+        stats = hip.DevBuf.from_array(np.full(((rows // 32 + 2) * (cout // 4) * 2,), np.nan, np.float32))
+        n = ctypes.c_int(0)
+        try:
+            hip.check(L.flux_hip_conv_stats(epi, din.ptr, dw.ptr, db.ptr, r, out.ptr, rows, wp, cin, cout, 9, stats.ptr, ctypes.byref(n)))
+        finally:
+            L.flux_hip_linear_force_tile(-1)
+            L.flux_hip_linear_force_split(0)
+        assert 0 < n.value <= rows // 32 + 2
+        got = bf16_to_f32(out.to_array(np.uint16, (rows, cout))) if bf else out.to_array(np.float32, (rows, cout))
+        assert border_is_zero(got, H, W)
+        st = stats.to_array(np.float32, (n.value, cout // 4, 2)).astype(np.float64).sum(0)
+        quads = got.astype(np.float64).reshape(rows, cout // 4, 4)
+        tol = 2.0 ** -8 if bf else 1e-5       # bf16: sums of the unrounded values
+        np.testing.assert_allclose(st[:, 1], (quads ** 2).sum((0, 2)), rtol=2 * tol)
+        np.testing.assert_allclose(st[:, 0], quads.sum((0, 2)), atol=tol * np.abs(quads).sum((0, 2)).max() + 1e-30)
+        return got
+
+    for epi, r in ((hip.EPI_CONV_F32, None), (hip.EPI_CONV_F32, dres.ptr), (hip.EPI_CONV_BF16, None)):
+        want = run(1, 0, epi, r) if H * W >= 4096 else run(3, 0, epi, r)
+        for tile, split in ((12, 0), (2, 0), (12, 2), (2, 2), (1, 4), (-1, 0), (-1, 8)):
+            if tile == 2 and cout % 256:
+                continue
+            got = run(tile, split, epi, r)
+            if split == 0 and H * W >= 4096:
+                np.testing.assert_array_equal(got, want)
+            else:
+                assert rel_l2(got, want) < (2.0 ** -9 if epi == hip.EPI_CONV_BF16 else 2e-6)
+
+
+def test_conv_of_an_image_without_interior(hip):
+    """Two columns of border and nothing between them: the output is zeros."""
+    d = hip.DevBuf.from_array(np.zeros(1 << 14, np.uint16))
+    out = hip.DevBuf.from_array(np.full((8, 64), 3.0, np.float32))
+    hip.check(hip.lib().flux_hip_conv(hip.EPI_CONV_F32, d.ptr, d.ptr, d.ptr, None, out.ptr, 8, 2, 64, 64, 1))
+    assert not out.to_array(np.float32, (8, 64)).any()
+
+
 def test_conv_rejects_bad_arguments(hip):
     L = hip.lib()
     d = hip.DevBuf(1 << 16)
