@@ -1147,13 +1147,16 @@ static int launch_epi(GemmArgs &g, int tile) {
             case 5: return launch_4d<9, 6, EPI, 2, 3>(g);
             case 6: return launch_4d<6, 6, EPI, 3, 3>(g);
             case 7: return launch_4d<8, 6, EPI, 2, 3>(g);
+            case 12: return launch_4d<8, 4, EPI, 3, 3>(g);
+            case 13: return launch_4d<4, 4, EPI, 3, 3>(g);
+            case 14: return launch_4d<6, 8, EPI, 2, 3>(g);
             case 11:
                 if constexpr (EPI == FLUX_HIP_EPI_RESID || EPI == FLUX_HIP_EPI_BF16) return launch_4d<8, 7, EPI, 2, 3>(g);
                 break;
             default: break;
         }
     }
-    if (tile == 11) tile = g.N % 256 == 0 ? 2 : 1; /* (the dispatch offers 256 x 224 only where the ring kernel takes it) */
+    if (tile >= 11) tile = g.N % 256 == 0 ? 2 : 1; /* (the dispatch offers these only where the ring kernel takes them) */
     switch (tile) {
         case 2: return launch_4w<8, 8, EPI>(g);
         case 5: return launch_4w<9, 6, EPI>(g);
@@ -1481,10 +1484,11 @@ extern "C" void flux_hip_linear_release(void) {
 }
 
 static int g_force_tile = -1;
-static unsigned g_tile_mask = 0xFEF; /* tiles the automatic choice may use: all but the 8-wave form of 256 x 256 */
+#define TILE_MASK_ALL 0x7FEFu /* tiles the automatic choice may use: all but the 8-wave form of 256 x 256 */
+static unsigned g_tile_mask = TILE_MASK_ALL;
 static int g_splitk_enabled = 1;
 extern "C" void flux_hip_linear_force_tile(int tile) { g_force_tile = tile; }
-extern "C" void flux_hip_linear_tile_mask(unsigned mask) { g_tile_mask = mask ? mask : 0xFEF; }
+extern "C" void flux_hip_linear_tile_mask(unsigned mask) { g_tile_mask = mask ? mask : TILE_MASK_ALL; }
 extern "C" void flux_hip_linear_enable_splitk(int on) { g_splitk_enabled = on; }
 static int g_force_split = 0; /* > 1: every projection that can run as K slices runs as this many (comparison runs and tests) */
 extern "C" void flux_hip_linear_force_split(int slices) { g_force_split = slices > 1 ? slices : 0; }
@@ -1559,11 +1563,14 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
      * forced, for comparison runs), 5 = 288 x 192, 6 = 192 x 192, 7 = 256 x 192, 8, 9 and 10 = 64 x 128, 128 x 128 and
      * 96 x 128 with a ring of 6, 5 and 5 stages instead of 2 (one workgroup per compute unit; for parts of at most that
      * many rows), 11 = 256 x 224 (4096 + 512 rows x 3072 columns are 252 such tiles, one round of workgroups on 256
-     * compute units of which each does 7/8 of a 256 x 256 tile's work; 216 tiles of 256 x 256 are one round as well) */
-    constexpr int NT = 12;
-    static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 64, 128, 96, 256}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 128, 128, 128, 224};
-    static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1}, ahead[NT] = {1, 1, 1, 1, 1, 1, 1, 1, 5, 4, 4, 1}; /* stages a workgroup keeps in flight */
-    static const double rate[NT] = {2.0e12, 2.9e12, 6.05e12, 1.5e12, 4.6e12, 6.0e12, 5.7e12, 5.75e12, 1.6e12, 3.0e12, 2.4e12, 5.9e12}; /* FLOP/s of one CU running this tile */
+     * compute units of which each does 7/8 of a 256 x 256 tile's work; 216 tiles of 256 x 256 are one round as well),
+     * 12 = 256 x 128, 13 = 128 x 128 and 14 = 192 x 256 in the ring kernel, for launches of about one round: the two-stage 128 x 128
+     * tile waits for memory in every K step when it has a compute unit to itself (512 x 6144 x 2560: 31 us, in the ring 21;
+     * 1202 x 3072 x 3072: 40 and 28; 512 x 19456 x 2560 on 228 tiles of 192 x 256 51, on 152 of 256 x 256 59) */
+    constexpr int NT = 15;
+    static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 64, 128, 96, 256, 256, 128, 192}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 128, 128, 128, 224, 128, 128, 256};
+    static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, ahead[NT] = {1, 1, 1, 1, 1, 1, 1, 1, 5, 4, 4, 1, 1, 1, 1}; /* stages a workgroup keeps in flight */
+    static const double rate[NT] = {2.0e12, 2.9e12, 6.05e12, 1.5e12, 4.6e12, 6.0e12, 5.7e12, 5.75e12, 1.6e12, 3.0e12, 2.4e12, 5.9e12, 5.3e12, 4.4e12, 5.5e12}; /* FLOP/s of one CU running this tile */
     const int kt_total = g.K >> 6;
     int tile = -1, best_split = 1;
     {
@@ -1586,6 +1593,7 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
             if (cut && epilogue == FLUX_HIP_EPI_BF16 && (N % 224) % 112 % 32 != 0) continue;
             if (!cut && (N % bn[t] || g.nq_cols % bn[t])) continue;
             if (!((allowed >> t) & 1)) continue;
+            if (t >= 12 && !(g_ring && g_persistent && kt_total >= 4)) continue;
             if (ahead[t] > 1) { /* the deep rings stream the weights once: every part in one row tile */
                 bool fits = true;
                 for (int i = 0; i < np; i++) fits = fits && g.M[i] <= bm[t];
@@ -1622,6 +1630,7 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
                 if (bw > bw_cap) bw = bw_cap;
                 double est = t_compute > bytes / bw ? t_compute : bytes / bw;
                 if (sp > 1) est += 3.0e-6 + (sp + 2.0) * rows * N * 4.0 / 4.0e12;
+                else if (adaln) est += 3.0e-6 + rows * N * 6.0 / 4.0e12; /* the norm that the second pass would have taken along */
                 if (est < best) { best = est; tile = t; best_split = sp; }
             }
         }
@@ -1716,7 +1725,7 @@ static int linear_impl(int epilogue, int nparts, const flux_hip_linear_part *par
     g.N = N; g.K = K; g.lda = lda; g.ldw = ldw; g.ldc = ldc; g.w_row0 = w_row0; g.w_row1 = w_row1;
     a.ldo = N;
     a.eps = eps;
-    return gemm_dispatch(g, np, epilogue, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0xFFFu, nullptr, norm ? &a : nullptr, fused,
+    return gemm_dispatch(g, np, epilogue, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7FFFu, nullptr, norm ? &a : nullptr, fused,
                          fixed_ws, fixed_ws_bytes);
 }
 
@@ -1744,7 +1753,7 @@ extern "C" int flux_hip_linear_qkv_swiglu(const void *A, const void *W, void *qk
     int tile = -1;
     const int saved = g_splitk_enabled;
     g_splitk_enabled = 0;
-    const int ok = gemm_dispatch(g, 1, EPI_QKV_SWIGLU, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0xFFFu, &tile);
+    const int ok = gemm_dispatch(g, 1, EPI_QKV_SWIGLU, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7FFFu, &tile);
     g_splitk_enabled = saved;
     return ok;
 }

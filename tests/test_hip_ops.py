@@ -150,6 +150,44 @@ def test_linear_tile_with_cut_last_column_tile(hip, oracle_mod, N, K):
     L.flux_hip_linear_force_tile(-1)
 
 
+@pytest.mark.parametrize("tile", [12, 13, 14])
+@pytest.mark.parametrize("M0,M1,N,K", [(1, 0, 256, 256), (300, 70, 768, 448), (129, 257, 512, 320), (2000, 30, 3072, 256), (40, 90, 256, 192)])
+def test_linear_small_ring_tiles(hip, oracle_mod, tile, M0, M1, N, K):
+    """256 x 128, 128 x 128 and 192 x 256 in the ring kernel: four to seven K steps, one or several tiles per workgroup (2030 x 3072
+    is 408 tiles of 128 x 128), two row ranges; three K steps are too few for it and run elsewhere. Every epilogue bit for
+    bit what the two-stage 128 x 128 tile gives (the same K order), which is held against the oracle here as well."""
+    L = hip.lib()
+    M = M0 + M1
+    a = q(normal_f32((M, K), 42, 1))
+    W0, W1 = q(normal_f32((N, K), 42, 2, 0.0, 0.1)), q(normal_f32((N, K), 42, 3, 0.0, 0.1))
+    res, g = normal_f32((M, N), 42, 4), normal_f32((N,), 42, 5)
+    da, dW0, dW1, dg = dev_bf16(hip, a), dev_bf16(hip, W0), dev_bf16(hip, W1), hip.DevBuf.from_array(g)
+
+    def run(t, epi, dtype, cols, row1=0):
+        L.flux_hip_linear_force_tile(t)
+        L.flux_hip_linear_enable_splitk(0)
+        out = hip.DevBuf.from_array(np.concatenate([res[:, :cols], np.full((1, cols), 7.0, np.float32)]).astype(np.float32) if dtype == np.float32
+                                    else np.full((M + 1, cols), 0x4242, np.uint16))
+        size = np.dtype(dtype).itemsize
+        parts = [(da.ptr, dW0.ptr, out.ptr, dg.ptr, M0), (da.at(M0 * K * 2), dW1.ptr, out.at(M0 * cols * size), dg.ptr, M1)]
+        try:
+            hip.linear(epi, parts, N, K, K, K, cols, 0, row1)
+        finally:
+            L.flux_hip_linear_force_tile(-1)
+            L.flux_hip_linear_enable_splitk(1)
+        full = out.to_array(dtype, (M + 1, cols))
+        assert (full[-1] == (7.0 if dtype == np.float32 else 0x4242)).all()     # nothing behind the output
+        return full[:-1]
+
+    plain = np.concatenate([oracle_mod.linear(a[:M0], W0)] + ([oracle_mod.linear(a[M0:], W1)] if M1 else []))
+    for epi, dtype, cols, row1, want in ((hip.EPI_BF16, np.uint16, N, 0, plain), (hip.EPI_F32, np.float32, N, 0, plain),
+                                         (hip.EPI_RESID, np.float32, N, 0, res + g * plain),
+                                         (hip.EPI_SWIGLU, np.uint16, N // 2, N // 2, oracle_mod.silu(plain[:, :N // 2]) * plain[:, N // 2:])):
+        ref, got = run(1, epi, dtype, cols, row1), run(tile, epi, dtype, cols, row1)
+        assert np.array_equal(got, ref), epi
+        assert rel_l2(bf16_to_f32(ref) if dtype == np.uint16 else ref, want) < (4e-3 if dtype == np.uint16 else 2e-6), epi
+
+
 @pytest.mark.parametrize("epi,N", [("resid", 3072), ("bf16", 9216)])
 def test_linear_cut_tile_at_the_double_stream_shapes(hip, epi, N):
     """256 x 224 where the model uses it: 4096 image + 512 text rows with weights of their own, K = 3072, the gated residual
