@@ -49,30 +49,86 @@ __global__ __launch_bounds__(256) void qwen3_rms_norm_kernel(bf16 *__restrict__ 
 /* In place on the fused projection output qkv bf16 [seq, (heads + 2 kv_heads) * 128]: every q and k
  * head gets RMS norm * weight over its 128 values (qwen3_head_rms_norm, flux_qwen3.c:199-220)
  * and rotate-half RoPE, pairs (i, i + 64) with the table's angle for (position, i)
- * (apply_rope, flux_qwen3.c:264-307). One wave per (token, head): lane i holds the pair.
- * The v heads are written transposed to vt [kv_heads * 128, ldv] (keys contiguous), the layout the
- * attention kernel's second product reads. */
-__global__ __launch_bounds__(64) void qwen3_qk_rope_kernel(bf16 *__restrict__ qkv, bf16 *__restrict__ vt, int ldv, const float *__restrict__ q_w,
-                                                           const float *__restrict__ k_w, const float *__restrict__ rope_cos,
-                                                           const float *__restrict__ rope_sin, int heads, int kv_heads, float eps) {
-    const int s = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-    const int width = (heads + 2 * kv_heads) * 128;
-    bf16 *p = qkv + (size_t)s * width + h * 128;
-    if (h >= heads + kv_heads) { /* a v head: transpose */
-        const int vh = h - heads - kv_heads;
-        vt[(size_t)(vh * 128 + lane) * ldv + s] = p[lane];
-        vt[(size_t)(vh * 128 + lane + 64) * ldv + s] = p[lane + 64];
+ * (apply_rope, flux_qwen3.c:264-307). The v heads are written transposed to vt [kv_heads * 128, ldv] (keys contiguous), the
+ * layout the attention kernel's second product reads.
+ * 16 lanes share a head's row, four pairs each (8-byte accesses), 16 rows per workgroup; the v heads go through LDS in blocks of
+ * 64 tokens, so that a dim's tokens leave as 16-byte stores. With one wave per row and a 2-byte store per lane and token
+ * for V the launch took 10.8 us at 512 tokens x 48 heads. VEC = false: pointers or ldv that do not allow the wide accesses. */
+template <bool VEC, typename V4, typename T>
+__device__ __forceinline__ V4 qw_load4(const T *p) {
+    if (VEC) return *(const V4 *)p;
+    V4 v;
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = p[e];
+    return v;
+}
+template <bool VEC>
+__device__ __forceinline__ void qw_store4(bf16 *p, bf16x4 v) {
+    if (VEC) {
+        *(bf16x4 *)p = v;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++) p[e] = v[e];
+    }
+}
+template <bool VEC>
+__global__ __launch_bounds__(256) void qwen3_qk_rope_kernel(bf16 *__restrict__ qkv, bf16 *__restrict__ vt, int ldv, const float *__restrict__ q_w,
+                                                            const float *__restrict__ k_w, const float *__restrict__ rope_cos,
+                                                            const float *__restrict__ rope_sin, int seq, int heads, int kv_heads, float eps) {
+    __shared__ bf16 tile[64][130]; /* (rows of 65 words: a column's reads fall on different banks) */
+    const int width = (heads + 2 * kv_heads) * 128, nqk = heads + kv_heads, rows = seq * nqk, qk_blocks = (rows + 15) / 16;
+    if ((int)blockIdx.x >= qk_blocks) { /* 64 tokens of a v head: transpose */
+        const int vb = blockIdx.x - qk_blocks, vh = vb % kv_heads, s0 = vb / kv_heads * 64;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int idx = i * 256 + threadIdx.x, r = idx >> 5, c = (idx & 31) * 4, s = min(s0 + r, seq - 1);
+            const bf16x4 v = qw_load4<VEC, bf16x4>(qkv + (size_t)s * width + (nqk + vh) * 128 + c);
+#pragma unroll
+            for (int e = 0; e < 4; e++) tile[r][c + e] = v[e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int idx = i * 256 + threadIdx.x, d = idx >> 3, c = (idx & 7) * 8;
+            bf16 *o = vt + (size_t)(vh * 128 + d) * ldv + s0 + c;
+            bf16x8 v;
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = tile[c + e][d];
+            if (VEC && s0 + c + 8 <= seq) {
+                *(bf16x8 *)o = v;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (s0 + c + e < seq) o[e] = v[e];
+            }
+        }
         return;
     }
-    const float *w = h < heads ? q_w : k_w;
-    const float x0 = (float)p[lane], x1 = (float)p[lane + 64];
-    float ss = x0 * x0 + x1 * x1;
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    const int row = min((int)blockIdx.x * 16 + (int)(threadIdx.x >> 4), rows - 1), i0 = (threadIdx.x & 15) * 4;
+    const bool mine = (int)blockIdx.x * 16 + (int)(threadIdx.x >> 4) < rows;
+    const int s = row / nqk, h = row - s * nqk;
+    bf16 *p = qkv + (size_t)s * width + h * 128 + i0;
+    const float *w = (h < heads ? q_w : k_w) + i0;
+    const bf16x4 lo = qw_load4<VEC, bf16x4>(p), hi = qw_load4<VEC, bf16x4>(p + 64);
+    const f32x4 w0 = qw_load4<VEC, f32x4>(w), w1 = qw_load4<VEC, f32x4>(w + 64);
+    const f32x4 cs = qw_load4<VEC, f32x4>(rope_cos + s * 64 + i0), sn = qw_load4<VEC, f32x4>(rope_sin + s * 64 + i0);
+    float ss = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; e++) ss += (float)lo[e] * (float)lo[e] + (float)hi[e] * (float)hi[e];
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
     const float inv = 1.0f / sqrtf(ss / 128.0f + eps);
-    const float a = x0 * inv * w[lane], b = x1 * inv * w[lane + 64];
-    const float cs = rope_cos[s * 64 + lane], sn = rope_sin[s * 64 + lane];
-    p[lane] = (bf16)(a * cs - b * sn);
-    p[lane + 64] = (bf16)(a * sn + b * cs);
+    bf16x4 olo, ohi;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const float a = (float)lo[e] * inv * w0[e], b = (float)hi[e] * inv * w1[e];
+        olo[e] = (bf16)(a * cs[e] - b * sn[e]);
+        ohi[e] = (bf16)(a * sn[e] + b * cs[e]);
+    }
+    if (mine) {
+        qw_store4<VEC>(p, olo);
+        qw_store4<VEC>(p + 64, ohi);
+    }
 }
 
 /*
@@ -82,9 +138,10 @@ __global__ __launch_bounds__(64) void qwen3_qk_rope_kernel(bf16 *__restrict__ qk
  * seq columns, exactly as in the reference); softmax over all seq columns; out = P v.
  *
  * One workgroup per (16 queries, kv head): its waves are the query heads that share that kv head,
- * so each 32-key tile of K and of V^T is fetched once and shared through LDS (two slots; the next
- * tile travels global -> registers while the current one is multiplied, then registers -> LDS,
- * one barrier per tile). A wave keeps all scores of its 16 queries against all keys in registers
+ * so each 32-key tile of K and of V^T is fetched once and shared through LDS (two slots; tiles travel global -> registers, D
+ * of them on their way, then registers -> LDS, one barrier per tile). A tile is 16 MFMAs per wave, far less than the time
+ * its load takes: with one tile on its way every step waited for memory, 22 us at 512 tokens x 32 heads. The V^T tiles continue
+ * the K tiles' sequence, so the first ones arrive during the softmax. A wave keeps all scores of its 16 queries against all keys in registers
  * (S^T = K Q^T as 16 x 16 blocks, keys x queries: 32 blocks of 4 registers), so the softmax is
  * the plain three-step one. Inside each group of 32 keys the K rows are assigned to MFMA rows so
  * that a lane ends up with 8 consecutive keys of one query: that is the B-operand layout of the
@@ -114,49 +171,60 @@ __device__ __forceinline__ void qwen3_attend(bf16 *__restrict__ out, const bf16 
 #pragma unroll
     for (int ks = 0; ks < 4; ks++) qf[ks] = *(const bf16x8 *)(qkv + (size_t)qrow * width + h * 128 + ks * 32 + lq * 8);
 
-    bf16x8 stage[per_lane];
+    constexpr int D = NT < 8 / per_lane || per_lane > 8 ? NT : 8 / per_lane; /* tiles on their way: 32 registers */
+    bf16x8 stage[D][per_lane];
     /* K tile t: LDS row j = key 32 t + j, 16 chunks of 8 dims, chunk c stored at c ^ kswz(j) */
-    auto fetch_k = [&](int t) {
+    auto fetch_k = [&](int t) { /* into stage[t % D] */
 #pragma unroll
         for (int u = 0; u < per_lane; u++)
             {
                 const int idx = tid + u * nthreads, j = idx >> 4, c = idx & 15;
-                stage[u] = *(const bf16x8 *)(qkv + (size_t)min(32 * t + j, seq - 1) * width + (heads + kh) * 128 + c * 8);
+                stage[t % D][u] = *(const bf16x8 *)(qkv + (size_t)min(32 * t + j, seq - 1) * width + (heads + kh) * 128 + c * 8);
             }
     };
-    auto put_k = [&](int slot) {
+    auto put_k = [&](int t) {
 #pragma unroll
         for (int u = 0; u < per_lane; u++)
             {
                 const int idx = tid + u * nthreads, j = idx >> 4, c = idx & 15;
-                *(bf16x8 *)(smem + slot * 8192 + j * 256 + ((c ^ qw_kswz(j)) << 4)) = stage[u];
+                *(bf16x8 *)(smem + (t & 1) * 8192 + j * 256 + ((c ^ qw_kswz(j)) << 4)) = stage[t % D][u];
             }
     };
     /* V^T tile t: LDS row d = head dim, 4 chunks of 8 keys, chunk c stored at c ^ vswz(d) */
-    auto fetch_v = [&](int t) {
+    auto fetch_v = [&](int t) { /* into stage[(NT + t) % D] */
 #pragma unroll
         for (int u = 0; u < per_lane; u++)
             {
                 const int idx = tid + u * nthreads, d = idx >> 2, c = idx & 3;
-                stage[u] = *(const bf16x8 *)(vt + (size_t)(kh * 128 + d) * ldv + min(32 * t, ldv - 32) + c * 8);
+                stage[(NT + t) % D][u] = *(const bf16x8 *)(vt + (size_t)(kh * 128 + d) * ldv + min(32 * t, ldv - 32) + c * 8);
             }
     };
-    auto put_v = [&](int slot) {
+    auto put_v = [&](int t) {
 #pragma unroll
         for (int u = 0; u < per_lane; u++)
             {
                 const int idx = tid + u * nthreads, d = idx >> 2, c = idx & 3;
-                *(bf16x8 *)(smem + 16384 + slot * 8192 + d * 64 + ((c ^ qw_vswz(d)) << 4)) = stage[u];
+                *(bf16x8 *)(smem + 16384 + (t & 1) * 8192 + d * 64 + ((c ^ qw_vswz(d)) << 4)) = stage[(NT + t) % D][u];
             }
     };
 
     f32x4 sc[2 * NT];
-    fetch_k(0);
+    /* padding mask, requested ahead of everything (behind the scores its words were one round trip to memory after the other) */
+    int mv[(NT + 1) / 2];
+#pragma unroll
+    for (int w = 0; w < (NT + 1) / 2; w++) mv[w] = mask ? mask[min(64 * w + lane, seq - 1)] : 1;
+#pragma unroll
+    for (int t = 0; t < D; t++) fetch_k(t);
+    /* as bits: word w covers keys [64 w, 64 w + 64), one ballot per word */
+    unsigned long long keep[(NT + 1) / 2];
+#pragma unroll
+    for (int w = 0; w < (NT + 1) / 2; w++) keep[w] = __ballot(64 * w + lane < seq && mv[w] != 0);
     put_k(0);
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-        if (t + 1 < NT) fetch_k(t + 1);
+        if (t + D < NT) fetch_k(t + D);
+        else fetch_v(t + D - NT);
         const char *kt = smem + (t & 1) * 8192;
 #pragma unroll
         for (int half = 0; half < 2; half++) {
@@ -171,19 +239,11 @@ __device__ __forceinline__ void qwen3_attend(bf16 *__restrict__ out, const bf16 
             sc[2 * t + half] = acc;
         }
         if (t + 1 < NT) {
-            put_k((t + 1) & 1);
+            put_k(t + 1);
             __syncthreads();
         }
     }
-    fetch_v(0); /* in flight during the softmax */
 
-    /* padding mask as bits: word w covers keys [64 w, 64 w + 64), one ballot per word */
-    unsigned long long keep[(NT + 1) / 2];
-#pragma unroll
-    for (int w = 0; w < (NT + 1) / 2; w++) {
-        const int key = 64 * w + lane;
-        keep[w] = __ballot(key < seq && (!mask || mask[key] != 0));
-    }
     /* accumulator element e of block (t, half): query l15, key 32 t + 8 lq + 4 half + e */
     const int qi = q0 + l15;
     float mx = -3.0e38f;
@@ -228,7 +288,7 @@ __device__ __forceinline__ void qwen3_attend(bf16 *__restrict__ out, const bf16 
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-        if (t + 1 < NT) fetch_v(t + 1);
+        if (t + D < NT) fetch_v(t + D);
         const char *vtile = smem + 16384 + (t & 1) * 8192;
         bf16x8 pf;
 #pragma unroll
@@ -243,7 +303,7 @@ __device__ __forceinline__ void qwen3_attend(bf16 *__restrict__ out, const bf16 
             o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[d], 0, 0, 0);
         }
         if (t + 1 < NT) {
-            put_v((t + 1) & 1);
+            put_v(t + 1);
             __syncthreads();
         }
     }
@@ -302,8 +362,10 @@ extern "C" int flux_hip_rms_norm(void *out_bf16, const float *x, const float *w,
 extern "C" int flux_hip_qwen3_qk_rope(void *qkv_bf16, void *vt_bf16, int ldv, const float *q_w, const float *k_w, const float *rope_cos,
                                       const float *rope_sin, int seq, int heads, int kv_heads, float eps) {
     if (seq <= 0 || heads <= 0 || kv_heads <= 0 || ldv < seq) return flux_hip_fail("flux_hip_qwen3_qk_rope: bad shape");
-    hipLaunchKernelGGL(qwen3_qk_rope_kernel, dim3(seq, heads + 2 * kv_heads), dim3(64), 0, flux_hip_stream_handle(), (bf16 *)qkv_bf16,
-                       (bf16 *)vt_bf16, ldv, q_w, k_w, rope_cos, rope_sin, heads, kv_heads, eps);
+    const bool vec = !((((uintptr_t)qkv_bf16 | (uintptr_t)vt_bf16 | (uintptr_t)q_w | (uintptr_t)k_w | (uintptr_t)rope_cos | (uintptr_t)rope_sin) & 15) | (ldv & 7));
+    const dim3 grid((seq * (heads + kv_heads) + 15) / 16 + (seq + 63) / 64 * kv_heads);
+    hipLaunchKernelGGL(vec ? qwen3_qk_rope_kernel<true> : qwen3_qk_rope_kernel<false>, grid, dim3(256), 0, flux_hip_stream_handle(),
+                       (bf16 *)qkv_bf16, (bf16 *)vt_bf16, ldv, q_w, k_w, rope_cos, rope_sin, seq, heads, kv_heads, eps);
     LAUNCH_OK("qwen3_qk_rope_kernel");
     return 1;
 }

@@ -72,6 +72,36 @@ def test_causal_attention(hip, oracle_mod, seq, heads, kv, masked):
         assert rel_l2(got[0, :128], vv[:, :128].mean(axis=0)) < 6e-3     # uniform over ALL columns
 
 
+@pytest.mark.parametrize("seq,heads,kv,ldv", [(1, 2, 1, 32), (7, 4, 2, 512), (64, 8, 2, 64), (65, 3, 1, 96), (135, 4, 2, 137)])
+def test_qk_norm_rope_and_v_transpose(hip, seq, heads, kv, ldv):
+    """Rows that fill no workgroup, token counts around the 64 of a V block and the 8 of a store, a row stride of V^T that
+    forbids the wide stores; float64 numpy as reference, one rounding to bf16 (2^-9). V^T is copied: the same bits, and
+    nothing behind its last token."""
+    import ctypes
+    rng = np.random.default_rng(75)
+    width = (heads + 2 * kv) * 128
+    x = q(normal_f32((seq, width), 75, 1))
+    qw, kw = normal_f32((128,), 75, 2, 1.0, 0.2), normal_f32((128,), 75, 3, 1.0, 0.2)
+    ang = rng.uniform(-3, 3, (seq, 64))
+    cos, sin = np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)
+    d = [hip.DevBuf.from_array(a) for a in (f32_to_bf16(x), np.full((kv * 128, ldv), 0x4242, np.uint16), qw, kw, cos, sin)]
+    vp, ci = ctypes.c_void_p, ctypes.c_int
+    f = hip.lib().flux_hip_qwen3_qk_rope
+    f.argtypes = [vp, vp, ci, vp, vp, vp, vp, ci, ci, ci, ctypes.c_float]
+    hip.check(f(d[0].ptr, d[1].ptr, ldv, d[2].ptr, d[3].ptr, d[4].ptr, d[5].ptr, seq, heads, kv, 1e-6))
+    got = bf16_to_f32(d[0].to_array(np.uint16, (seq, width))).reshape(seq, -1, 128)
+    h = x.astype(np.float64).reshape(seq, -1, 128)
+    w = np.concatenate([np.tile(qw, (heads, 1)), np.tile(kw, (kv, 1))]).astype(np.float64)
+    n = h[:, :heads + kv] / np.sqrt((h[:, :heads + kv] ** 2).mean(-1, keepdims=True) + 1e-6) * w
+    c, s = cos[:, None].astype(np.float64), sin[:, None].astype(np.float64)
+    want = np.concatenate([n[..., :64] * c - n[..., 64:] * s, n[..., :64] * s + n[..., 64:] * c], -1)
+    assert rel_l2(got[:, :heads + kv], want) < 2.0 ** -8
+    assert np.array_equal(got[:, heads + kv:], x.reshape(seq, -1, 128)[:, heads + kv:])
+    vt = d[1].to_array(np.uint16, (kv * 128, ldv))
+    assert np.array_equal(bf16_to_f32(vt[:, :seq]), x[:, (heads + kv) * 128:].T)
+    assert (vt[:, seq:] == 0x4242).all()
+
+
 MID = QwenConfig(hidden=512, intermediate=1152, heads=8, kv_heads=2, layers=6, vocab=1000, out_layers=(0, 3, 5))
 
 
