@@ -34,7 +34,11 @@ int flux_hip_vae_latent_in(void *out_bf16, const float *latent, const float *bn_
 int flux_hip_vae_key_bias(float *bias, int n, int hp, int wp);
 int flux_hip_vae_image_out(uint8_t *rgb, float *rgb_f32, const float *x, int ldx, int H, int W);
 int flux_hip_vae_image_in(void *out_bf16, const float *img, int H, int W);
-int flux_hip_downsample_gather(void *out_bf16, const float *x, int hp, int wp, int C);
+int flux_hip_vae_upsample2x_bf16(void *out_bf16, const void *x_bf16, int hp, int wp, int C);
+/* gemm.hip */
+int flux_hip_conv_image(int epilogue, const void *in, int in_wp, const void *w, const float *bias, const float *res, void *out, int rows, int wp,
+                        int cin, int cout, int taps, float *stats, int *stats_rows);
+/* vae.hip */
 int flux_hip_vae_latent_out(float *latent, const float *x, int ldx, const float *bn_mean, const float *bn_var, int h, int w, float eps);
 
 enum { K_VEC, K_CONV3, K_CONV1, K_RAW, K_CONV3_PACKED };
@@ -351,7 +355,7 @@ void flux_hip_vae_free(flux_hip_vae *v) {
 }
 
 /* Test hook: upper bound on the query rows per attention chunk (0 = the buffer's own bound,
- * 1 GB of fp32 scores). */
+ * 2 GB of fp32 scores). */
 static int g_att_chunk_limit = 0;
 void flux_hip_vae_set_attention_chunk(int rows) { g_att_chunk_limit = rows > 0 ? rows : 0; }
 
@@ -361,13 +365,11 @@ void flux_hip_vae_set_attention_chunk(int rows) { g_att_chunk_limit = rows > 0 ?
 static int ensure_work(flux_hip_vae *v, int h, int w) {
     const size_t hp0 = 16 * (size_t)h + 2, wp0 = 16 * (size_t)w + 2, mp0 = hp0 * wp0;
     const size_t hpm = 2 * (size_t)h + 2, wpm = 2 * (size_t)w + 2, mpm = hpm * wpm;
-    const size_t ld = (mpm + 127) & ~(size_t)127;
+    const size_t ld = (mpm + 255) & ~(size_t)255; /* whole tiles of 256 x 256: 16900 rows of scores took 430 us in tiles of 128 x 128 */
     size_t f32_elems = mp0 * 256, guard = (wp0 + 2) * 512;
     size_t bf16_elems = mp0 * 256;
     if (bf16_elems < ld * 1536) bf16_elems = ld * 1536; /* R also holds q, k, v of the attention */
-    const size_t mp_half = (8 * (size_t)h + 2) * (8 * (size_t)w + 2);
-    if (bf16_elems < mp_half * 9 * 128) bf16_elems = mp_half * 9 * 128; /* the encoder's first downsampling step: nine taps of 128 channels per half-size position */
-    size_t chunk = ((size_t)1 << 28) / ld;               /* at most 1 GB of fp32 scores at a time */
+    size_t chunk = ((size_t)1 << 29) / ld;               /* at most 2 GB of fp32 scores at a time: a 1024x1024 picture's in one piece */
     if (chunk < 128) chunk = 128;
     if (chunk > mpm) chunk = mpm;
     const size_t gn_floats = flux_hip_group_norm_scratch_floats((int)hp0, (int)wp0);
@@ -422,9 +424,14 @@ static int run_conv(vstate *s, const vconv *c, int epi, const void *in, const fl
                                stats_rows);
 }
 
+static int conv_to_bf16(vstate *s, const vconv *c, const float *res, void *out_bf16) {
+    return flux_hip_conv_image(FLUX_HIP_EPI_CONV_BF16, s->A, 0, c->w, c->b, res, out_bf16, s->hp * s->wp, s->wp, c->cin_pad, c->cout_pad, c->taps, NULL, NULL);
+}
+
 /* resblock_forward, flux_vae.c:179-219. Every group norm takes its statistics from the epilogue of
- * the convolution that produced its input. */
-static int run_res(vstate *s, const vres *r) {
+ * the convolution that produced its input. out_bf16: the last block of a level, whose result only a resampling convolution reads, and
+ * that as bf16, leaves it there in that form and not in s->x. */
+static int run_res(vstate *s, const vres *r, void *out_bf16) {
     flux_hip_vae *v = s->v;
     const int differ = r->cin != r->cout;
     if (!flux_hip_group_norm_stats(s->A, differ ? v->R : NULL, s->x, 0, r->n1g, r->n1b, v->gn, s->hp, s->wp, r->cin, v->eps, 1, v->st_x, s->x_rows)) return 0;
@@ -432,17 +439,19 @@ static int run_res(vstate *s, const vres *r) {
     if (!flux_hip_group_norm_stats(s->A, NULL, v->Hb, 1, r->n2g, r->n2b, v->gn, s->hp, s->wp, r->cout, v->eps, 1, v->st_h, s->h_rows)) return 0;
     if (differ) {
         if (!run_conv(s, &r->skip, FLUX_HIP_EPI_CONV_F32, v->R, NULL, s->y, 1, NULL, NULL)) return 0;
+        if (out_bf16) return conv_to_bf16(s, &r->c2, s->y, out_bf16);
         if (!run_conv(s, &r->c2, FLUX_HIP_EPI_CONV_F32, s->A, s->y, s->y, 1, v->st_x, &s->x_rows)) return 0;
         float *t = s->x; s->x = s->y; s->y = t;
         return 1;
     }
+    if (out_bf16) return conv_to_bf16(s, &r->c2, s->x, out_bf16);
     return run_conv(s, &r->c2, FLUX_HIP_EPI_CONV_F32, s->A, s->x, s->x, 1, v->st_x, &s->x_rows);
 }
 
 /* attnblock_forward, flux_vae.c:223-313 */
 static int run_attn(vstate *s, const vattn *a) {
     flux_hip_vae *v = s->v;
-    const int C = 512, rows = s->hp * s->wp, ld = (rows + 127) & ~127;
+    const int C = 512, rows = s->hp * s->wp, ld = (rows + 255) & ~255;
     if (!flux_hip_group_norm_stats(s->A, NULL, s->x, 0, a->g, a->b, v->gn, s->hp, s->wp, C, v->eps, 0, v->st_x, s->x_rows)) return 0;
     /* key rows between the image and the padded width are read by the score GEMM: zero them */
     if (ld > rows && !flux_hip_memset((char *)v->R + (size_t)rows * 3 * C * 2, 0, (size_t)(ld - rows) * 3 * C * 2)) return 0;
@@ -476,21 +485,21 @@ int flux_hip_vae_decode(flux_hip_vae *v, const float *latent, int h, int w, uint
     if (!run_conv(&s, &v->conv_in, FLUX_HIP_EPI_CONV_F32, s.A, NULL, s.x, 1, v->st_x, &s.x_rows)) return 0;
     int done = 0;
     const int total = 15;
-    if (!run_res(&s, &v->mid[0])) return 0;
+    if (!run_res(&s, &v->mid[0], NULL)) return 0;
     if (flux_hip_vae_progress) flux_hip_vae_progress(done++, total);
     if (!run_attn(&s, &v->attn)) return 0;
     if (flux_hip_vae_progress) flux_hip_vae_progress(done++, total);
-    if (!run_res(&s, &v->mid[1])) return 0;
+    if (!run_res(&s, &v->mid[1], NULL)) return 0;
     if (flux_hip_vae_progress) flux_hip_vae_progress(done++, total);
     int bi = 0;
     for (int level = 3; level >= 0; level--) {
         for (int r = 0; r < 3; r++) {
-            if (!run_res(&s, &v->up[bi++])) return 0;
+            if (!run_res(&s, &v->up[bi++], level > 0 && r == 2 ? v->R : NULL)) return 0;
             if (flux_hip_vae_progress) flux_hip_vae_progress(done++, total);
         }
         if (level > 0) {
             const vconv *c = &v->up_conv[3 - level];
-            if (!flux_hip_upsample2x(s.A, s.x, s.hp, s.wp, c->cin)) return 0;
+            if (!flux_hip_vae_upsample2x_bf16(s.A, v->R, s.hp, s.wp, c->cin)) return 0;
             s.hp = 2 * (s.hp - 2) + 2;
             s.wp = 2 * (s.wp - 2) + 2;
             if (!run_conv(&s, c, FLUX_HIP_EPI_CONV_F32, s.A, NULL, s.x, 1, v->st_x, &s.x_rows)) return 0;
@@ -521,25 +530,25 @@ int flux_hip_vae_encode(flux_hip_vae *v, const float *img, int H, int W, float *
     const int total = 11; /* 8 down + 3 mid, the reference's count (flux_vae.c:343) */
     for (int level = 0; level < 4; level++) {
         for (int r = 0; r < 2; r++) {
-            if (!run_res(&s, &v->enc_down[bi++])) return 0;
+            if (!run_res(&s, &v->enc_down[bi++], level < 3 && r == 1 ? v->R : NULL)) return 0;
             if (flux_hip_vae_progress) flux_hip_vae_progress(done++, total);
         }
         if (level < 3) {
             const vconv *c = &v->enc_down_conv[level];
-            if (!flux_hip_downsample_gather(s.A, s.x, s.hp, s.wp, c->cin)) return 0;
+            const int in_wp = s.wp;
             s.hp = (s.hp - 2) / 2 + 2;
             s.wp = (s.wp - 2) / 2 + 2;
-            /* the nine taps sit side by side in every row of A, in the weights' K order: a 1x1 convolution over 9 * cin channels */
-            if (!flux_hip_conv_stats(FLUX_HIP_EPI_CONV_F32, s.A, c->w, c->b, NULL, s.x, s.hp * s.wp, s.wp, 9 * c->cin_pad, c->cout_pad, 1, v->st_x,
+            /* stride 2, straight from the bordered image (gathering nine taps per position first was 250 us at 720 x 1296 x 128) */
+            if (!flux_hip_conv_image(FLUX_HIP_EPI_CONV_F32, v->R, in_wp, c->w, c->b, NULL, s.x, s.hp * s.wp, s.wp, c->cin_pad, c->cout_pad, 9, v->st_x,
                                      &s.x_rows))
                 return 0;
         }
     }
-    if (!run_res(&s, &v->enc_mid[0])) return 0;
+    if (!run_res(&s, &v->enc_mid[0], NULL)) return 0;
     if (flux_hip_vae_progress) flux_hip_vae_progress(done++, total);
     if (!run_attn(&s, &v->enc_attn)) return 0;
     if (flux_hip_vae_progress) flux_hip_vae_progress(done++, total);
-    if (!run_res(&s, &v->enc_mid[1])) return 0;
+    if (!run_res(&s, &v->enc_mid[1], NULL)) return 0;
     if (flux_hip_vae_progress) flux_hip_vae_progress(done++, total);
     if (!flux_hip_group_norm_stats(s.A, NULL, s.x, 0, v->enc_out_g, v->enc_out_b, v->gn, s.hp, s.wp, 512, v->eps, 1, v->st_x, s.x_rows)) return 0;
     if (!run_conv(&s, &v->enc_conv_out, FLUX_HIP_EPI_CONV_BF16, s.A, NULL, v->R, 1, NULL, NULL)) return 0;

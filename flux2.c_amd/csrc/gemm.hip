@@ -103,6 +103,7 @@ struct GemmArgs {
      * that what one tap fetched is still in L2 when the next asks for the neighbouring rows
      * (tap-major order re-fetched wide images 3 to 10 times from HBM). */
     int conv_taps, conv_wp, conv_rows;
+    int conv_stride, conv_in_wp; /* the operand's image: the same one, or for the downsampling steps one twice as large */
     unsigned conv_magic; /* (2^32 - 1) / (conv_wp - 2) */
     const float *bias, *res;
     /* optional: per (row-tile half, 4-channel group) sums and sums of squares of what a convolution
@@ -119,11 +120,21 @@ __device__ __forceinline__ int conv_div(const GemmArgs &g, int m) {
     const unsigned w = g.conv_wp - 2, q = __umulhi((unsigned)m, g.conv_magic);
     return (int)(q + ((unsigned)m - q * w >= w));
 }
-/* operand row of GEMM row m: the m-th interior position of the bordered image */
+/* row of GEMM row m in the output: the m-th interior position of the bordered image */
 template <int EPI>
 __device__ __forceinline__ int conv_row(const GemmArgs &g, int m) {
     if (!IsConv<EPI>::value || g.conv_wp == 0) return m;
     return m + 2 * conv_div(g, m) + g.conv_wp + 1;
+}
+
+/* ... and in the operand, where the 3x3 window is centred. With stride 2 (flux_vae.c:363-377: a row of zeros below and a column on
+ * the right, no padding above and left) the window of output (y, x) starts at input (2 y, 2 x), so its centre is
+ * (2 y + 2, 2 x + 2) of the bordered input; with stride 1 it is (y + 1, x + 1). */
+template <int EPI>
+__device__ __forceinline__ int conv_in_row(const GemmArgs &g, int m) {
+    if (!IsConv<EPI>::value || g.conv_wp == 0) return m;
+    const int y = conv_div(g, m), x = m - y * (g.conv_wp - 2);
+    return g.conv_stride * ((y + 1) * g.conv_in_wp + x + 1);
 }
 
 /* Element offset of K step kt within an activation row. Plain GEMM: kt * 64. 3x3 convolution:
@@ -135,7 +146,7 @@ __device__ __forceinline__ int a_step_offset(const GemmArgs &g, int kt) {
         /* kt / 9, kt % 9 for kt < 2048; a 1x1 convolution's step is a chunk at the middle tap. No branch: this stands in the K loops */
         const int nine = -(int)(g.conv_taps == 9), q = (kt * 7282) >> 16, chunk = kt + (nine & (q - kt)), tap = 4 + (nine & (kt - 9 * q - 4));
         const int dy = (tap * 11) >> 5, dx = tap - dy * 3;         /* tap / 3, tap % 3 for tap < 9 */
-        return ((dy - 1) * g.conv_wp + (dx - 1)) * g.lda + chunk * 64;
+        return ((dy - 1) * g.conv_in_wp + (dx - 1)) * g.lda + chunk * 64;
     }
     return kt * 64;
 }
@@ -404,7 +415,7 @@ __device__ __forceinline__ void store_conv_tile(const GemmArgs &g, const TileId 
             for (int r = 0; r < RB; r++)
 #pragma unroll
                 for (int k = 0; k < 2; k++)
-                    if (j0 + r < TM) xb[u & 1][r][k] = *(const f32x4 *)(g.res + (size_t)off[j0 + r] + (i0 + k) * 16 + lq * 4);
+                    if (j0 + r < TM) xb[u & 1][r][k] = *(const f32x4 *)(g.res + (size_t)off[j0 + r] + i0 * 16 + (F32 ? k * 16 + lq * 4 : lq * 8 + k * 4));
         };
         if (RES) fetch(0);
 #pragma unroll
@@ -467,7 +478,7 @@ __device__ __forceinline__ void store_conv_tile(const GemmArgs &g, const TileId 
             }
         }
     };
-    if (F32 && g.res) rows(BoolC<F32>{});
+    if (g.res) rows(BoolC<true>{});
     else rows(BoolC<false>{});
     const int lane = lq * 16 + l15;
     if (g.conv_wp > 0) {
@@ -537,7 +548,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_kernel(GemmArgs g) {
 #pragma unroll
     for (int i = 0; i < PA; i++) {
         int r = lrow + i * RPP;
-        int gm = conv_row<EPI>(g, min(m0 + r, M - 1));
+        int gm = conv_in_row<EPI>(g, min(m0 + r, M - 1));
         a_ptr[i] = A + (size_t)gm * g.lda + ((lchunk ^ lds_swz(r)) << 3);
         a_lds[i] = (wave * 8 + i * RPP) * 128;
     }
@@ -888,7 +899,7 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
         sc.baseA = (const char *)(g.A[tt.prob] + (IsConv<EPI>::value ? 0 : tt.ks * g.kt_per * 64));
         sc.baseW = (const char *)(g.W[tt.prob] + tt.ks * g.kt_per * 64);
 #pragma unroll
-        for (int i = 0; i < LA; i++) sc.voff[i] = ((unsigned)conv_row<EPI>(g, min(m0 + lr + i * RPP, M - 1)) * (unsigned)g.lda + chunk) * 2u;
+        for (int i = 0; i < LA; i++) sc.voff[i] = ((unsigned)conv_in_row<EPI>(g, min(m0 + lr + i * RPP, M - 1)) * (unsigned)g.lda + chunk) * 2u;
 #pragma unroll
         for (int i = 0; i < LB; i++) sc.voff[LA + i] = ((unsigned)weight_row<BN, WN, EPI>(g, tt.tn, lr + i * RPP) * (unsigned)g.ldw + chunk) * 2u;
     };
@@ -1241,7 +1252,7 @@ __global__ __launch_bounds__(256) void conv_finish_kernel(GemmArgs g) {
         f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
         if (inside) {
             f32x4 a = v;
-            if (F32 && g.res) v = *(const f32x4 *)(g.res + (size_t)p * g.ldc + n);
+            if (g.res) v = *(const f32x4 *)(g.res + (size_t)p * g.ldc + n);
             const float *w = g.ws + (size_t)m * g.N + n;
 #pragma unroll 8
             for (int s = 0; s < g.ksplit; s++) {
@@ -1789,22 +1800,23 @@ extern "C" int flux_hip_linear_resid_adaln(int nparts, const flux_hip_linear_par
 
 
 
-/* Tiles of a convolution: ids 0 to 3 as above (64 x 128, 128 x 128, 256 x 256, 64 x 64), 12 = 256 x 128. The two with 256
- * rows run in the ring kernel: 128 x 128 in two stages reached 700 to 870 TFLOP/s on 3x3 layers of 128 to 512 channels over
+/* Tiles of a convolution: ids 0 to 3 as above (64 x 128, 128 x 128, 256 x 256, 64 x 64), 12 = 256 x 128, 13 =
+ * 128 x 128 in the ring kernel, as is 2: 128 x 128 in two stages reached 700 to 870 TFLOP/s on 3x3 layers of 128 to 512 channels over
  * 128 x 128 to 1024 x 1024 positions, 256 x 128 reaches 920 to 1230 and 256 x 256 1200 to 1390 (bf16 output). */
 template <int EPI>
 static int conv_tile_launch(GemmArgs &g, int tile) {
     switch (tile) {
         case 2: return launch_4d<8, 8, EPI, 2, 3>(g);
         case 12: return launch_4d<8, 4, EPI, 3, 3>(g);
+        case 13: return launch_4d<4, 4, EPI, 3, 3>(g);
         case 1: return launch_cfg<128, 128, 2, 2, EPI>(g);
         case 3: return launch_cfg<64, 64, 2, 2, EPI>(g);
         default: return launch_cfg<64, 128, 2, 2, EPI>(g);
     }
 }
 
-#define CONV_TILES 13
-static const int conv_bm[CONV_TILES] = {64, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 256}, conv_bn[CONV_TILES] = {128, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 128};
+#define CONV_TILES 14
+static const int conv_bm[CONV_TILES] = {64, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 256, 128}, conv_bn[CONV_TILES] = {128, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 128, 128};
 
 template <int EPI>
 static int conv_finish(GemmArgs &g) {
@@ -1819,12 +1831,12 @@ static int conv_finish(GemmArgs &g) {
  * positions x 512 channels are 32 tiles of 128 x 128 for 256 units, 57 us in one piece and 24 in slices; at 96 x 96 positions
  * one piece wins (54 us against 69). */
 static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
-    static const int occ[CONV_TILES] = {3, 2, 1, 4, 0, 0, 0, 0, 0, 0, 0, 0, 1};
-    static const double rate[CONV_TILES] = {2.0e12, 3.3e12, 5.4e12, 1.5e12, 0, 0, 0, 0, 0, 0, 0, 0, 4.8e12}; /* FLOP/s of one CU */
+    static const int occ[CONV_TILES] = {3, 2, 1, 4, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1};
+    static const double rate[CONV_TILES] = {2.0e12, 3.3e12, 5.4e12, 1.5e12, 0, 0, 0, 0, 0, 0, 0, 0, 4.8e12, 4.2e12}; /* FLOP/s of one CU */
     static const int splits[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int M = g.M[0], N = g.N, kt_total = g.K >> 6, f = g_force_tile;
     const bool forced = f >= 0 && f < CONV_TILES && conv_bm[f] && N % conv_bn[f] == 0; /* a forced tile that this layer cannot use is ignored */
-    const bool ring_ok = g_ring && (size_t)g.conv_rows * g.lda * 2 < ((size_t)1 << 32) && (size_t)N * g.ldw * 2 < ((size_t)1 << 32) &&
+    const bool ring_ok = g_ring && (size_t)g.conv_rows * g.conv_stride * g.conv_stride * g.lda * 2 < ((size_t)1 << 32) && (size_t)N * g.ldw * 2 < ((size_t)1 << 32) &&
                          (size_t)g.conv_rows * N < ((size_t)1 << 32);
     int tile = -1, split = 1;
     double best = 1e30;
@@ -1843,7 +1855,7 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
             const long blocks = tiles * sp, slots = 256L * occ[t], rounds = (blocks + slots - 1) / slots;
             const long per_cu = (min(blocks, slots) + 255) / 256;
             double est = rounds * (2.0 * conv_bm[t] * conv_bn[t] * 64.0 * per / (rate[t] / per_cu) + 2.5e-6 +
-                                   (double)conv_bm[t] * conv_bn[t] * (sp > 1 ? 0 : epilogue == FLUX_HIP_EPI_CONV_BF16 ? 2 : g.res ? 8 : 4) / 2.0e10);
+                                   (double)conv_bm[t] * conv_bn[t] * (sp > 1 ? 0 : (epilogue == FLUX_HIP_EPI_CONV_BF16 ? 2 : 4) + (g.res ? 4 : 0)) / 2.0e10);
             if (sp > 1) est += 4.0e-6 + 2.0 * ws / 4.0e12;
             if (est < best) { best = est; tile = t; split = sp; }
         }
@@ -1870,6 +1882,9 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
     return bf ? conv_tile_launch<FLUX_HIP_EPI_CONV_BF16>(g, tile) : conv_tile_launch<FLUX_HIP_EPI_CONV_F32>(g, tile);
 }
 
+extern "C" int flux_hip_conv_image(int epilogue, const void *in, int in_wp, const void *w, const float *bias, const float *res, void *out,
+                                   int rows, int wp, int cin, int cout, int taps, float *stats, int *stats_rows);
+
 /* Convolution over a zero-bordered channels-last image as one GEMM, see the header. */
 extern "C" int flux_hip_conv_stats(int epilogue, const void *in, const void *w, const float *bias, const float *res, void *out, int rows,
                                    int wp, int cin, int cout, int taps, float *stats, int *stats_rows);
@@ -1894,12 +1909,20 @@ extern "C" int flux_hip_conv_stats(int epilogue, const void *in, const void *w, 
     if ((((uintptr_t)in | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)res | (uintptr_t)out) & 15))
         return flux_hip_fail("flux_hip_conv: operands must be 16-byte aligned");
     if (res && epilogue != FLUX_HIP_EPI_CONV_F32) return flux_hip_fail("flux_hip_conv: only the fp32 epilogue adds a residual");
+    return flux_hip_conv_image(epilogue, in, 0, w, bias, res, out, rows, wp, cin, cout, taps, stats, stats_rows);
+}
+
+/* flux_hip_conv_stats without its argument checks, for the VAE's own layers: the bf16 output takes a residual as well, and
+ * in_wp > 0 makes it the stride-2 3x3 convolution of a bordered image in_wp wide, rows and wp being the output's. */
+extern "C" int flux_hip_conv_image(int epilogue, const void *in, int in_wp, const void *w, const float *bias, const float *res, void *out,
+                                   int rows, int wp, int cin, int cout, int taps, float *stats, int *stats_rows) {
     GemmArgs g = {};
     g.A[0] = (const bf16 *)in;
     g.W[0] = (const bf16 *)w;
     g.C[0] = out;
     g.N = cout; g.K = taps * cin; g.lda = cin; g.ldw = taps * cin; g.ldc = cout;
     g.conv_taps = taps; g.conv_wp = wp; g.conv_rows = rows;
+    g.conv_stride = in_wp > 0 ? 2 : 1; g.conv_in_wp = in_wp > 0 ? in_wp : wp;
     g.M[0] = rows;
     if (wp > 0) {
         g.M[0] = wp > 2 && rows / wp > 2 ? (rows / wp - 2) * (wp - 2) : 0;

@@ -254,23 +254,37 @@ __global__ __launch_bounds__(256) void gn_apply_kernel(bf16 *__restrict__ out, b
     for (; r < row_end; r += rpi) one(r, load_quad(src + (size_t)r * C));
 }
 
-/* nearest-neighbour 2x upsample (flux_upsample_nearest, flux_kernels.c:1017-1036): fp32
- * [hp*wp, C] -> bf16 [(2H+2)*(2W+2), C] with a fresh zero border */
-__global__ __launch_bounds__(256) void vae_upsample_kernel(bf16 *__restrict__ out, const float *__restrict__ x, int hp, int wp, int C) {
-    const int quads = C >> 2;
-    const int H2 = 2 * (hp - 2), W2 = 2 * (wp - 2), hp2 = H2 + 2, wp2 = W2 + 2;
+/* nearest-neighbour 2x upsample (flux_upsample_nearest, flux_kernels.c:1017-1036): fp32 or bf16
+ * [hp*wp, C] -> bf16 [(2H+2)*(2W+2), C] with a fresh zero border. One thread per bordered source position and V
+ * channels, which go to the source's up to four places: interior (y, x) to rows 2y-1, 2y and columns 2x-1, 2x of the bordered output,
+ * and the border positions, as zeros, to what of that lies inside: its border. Each value is read once (a thread per
+ * output read every one four times: 512 x 512 x 256 from fp32 took 234 us). */
+template <typename T, int V>
+__global__ __launch_bounds__(256) void vae_upsample_kernel(bf16 *__restrict__ out, const T *__restrict__ x, int hp, int wp, int C) {
+    typedef __attribute__((ext_vector_type(V))) __bf16 ov;
+    const int groups = C / V, hp2 = 2 * hp - 2, wp2 = 2 * wp - 2;
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (size_t)hp2 * wp2 * quads) return;
-    const int p = (int)(idx / quads), q = (int)(idx - (size_t)p * quads);
-    const int y = p / wp2, xx = p - y * wp2;
-    bf16x4 o = {(bf16)0.0f, (bf16)0.0f, (bf16)0.0f, (bf16)0.0f};
-    if (y >= 1 && y <= H2 && xx >= 1 && xx <= W2) {
-        const int sy = 1 + ((y - 1) >> 1), sx = 1 + ((xx - 1) >> 1);
-        const f32x4 v = *(const f32x4 *)(x + ((size_t)sy * wp + sx) * C + q * 4);
+    if (idx >= (size_t)hp * wp * groups) return;
+    const int p = (int)(idx / groups), q = (int)(idx - (size_t)p * groups);
+    const int y = p / wp, xx = p - y * wp;
+    ov o;
 #pragma unroll
-        for (int e = 0; e < 4; e++) o[e] = (bf16)v[e];
+    for (int e = 0; e < V; e++) o[e] = (bf16)0.0f;
+    if (interior(p, hp, wp)) {
+#pragma unroll
+        for (int k = 0; k < V; k += 4) {
+            const f32x4 v = load_quad(x + (size_t)p * C + q * V + k);
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[k + e] = (bf16)v[e];
+        }
     }
-    *(bf16x4 *)(out + (size_t)p * C + q * 4) = o;
+#pragma unroll
+    for (int dy = -1; dy <= 0; dy++)
+#pragma unroll
+        for (int dx = -1; dx <= 0; dx++) {
+            const int oy = 2 * y + dy, ox = 2 * xx + dx;
+            if (oy >= 0 && oy < hp2 && ox >= 0 && ox < wp2) *(ov *)(out + ((size_t)oy * wp2 + ox) * C + q * V) = o;
+        }
 }
 
 /* ---- encoder side (flux_vae_encode, flux_vae.c:320-443) ---- */
@@ -537,9 +551,19 @@ extern "C" size_t flux_hip_group_norm_scratch_floats(int hp, int wp) {
 
 extern "C" int flux_hip_upsample2x(void *out_bf16, const float *x, int hp, int wp, int C) {
     if (C <= 0 || (C & 3) || hp < 3 || wp < 3) return flux_hip_fail("flux_hip_upsample2x: bad shape");
-    const size_t total = (size_t)(2 * (hp - 2) + 2) * (2 * (wp - 2) + 2) * (C / 4);
-    hipLaunchKernelGGL(vae_upsample_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, flux_hip_stream_handle(), (bf16 *)out_bf16, x, hp,
-                       wp, C);
+    const size_t total = (size_t)hp * wp * (C / 4);
+    hipLaunchKernelGGL((vae_upsample_kernel<float, 4>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, flux_hip_stream_handle(), (bf16 *)out_bf16,
+                       x, hp, wp, C);
+    LAUNCH_OK("vae_upsample_kernel");
+    return 1;
+}
+
+/* the same from a bf16 image, C a multiple of 8 */
+extern "C" int flux_hip_vae_upsample2x_bf16(void *out_bf16, const void *x_bf16, int hp, int wp, int C) {
+    if (C <= 0 || (C & 7) || hp < 3 || wp < 3) return flux_hip_fail("flux_hip_vae_upsample2x_bf16: bad shape");
+    const size_t total = (size_t)hp * wp * (C / 8);
+    hipLaunchKernelGGL((vae_upsample_kernel<bf16, 8>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, flux_hip_stream_handle(), (bf16 *)out_bf16,
+                       (const bf16 *)x_bf16, hp, wp, C);
     LAUNCH_OK("vae_upsample_kernel");
     return 1;
 }

@@ -144,7 +144,7 @@ def test_conv1x1(hip, oracle_mod):
 @pytest.mark.parametrize("H,W,cin,cout", [(1, 1, 64, 256), (1, 40, 128, 256), (301, 1, 64, 256), (17, 31, 512, 256), (16, 16, 512, 512),
                                           (280, 281, 64, 128), (200, 190, 64, 256)])
 def test_conv_tiles_and_slices(hip, H, W, cin, cout):
-    """The ring tiles (2: 256 x 256, 12: 256 x 128) against the 128 x 128 one, which test_conv3x3 ties to the oracle: the same
+    """The ring tiles (2: 256 x 256, 12: 256 x 128, 13: 128 x 128) against the 128 x 128 one, which test_conv3x3 ties to the oracle: the same
     K order, so the same bits, at images smaller than a tile, one pixel wide, with cut-off last tiles, and with more tiles
     than compute units (280 x 281: 308 tiles). K slices regroup an fp32 sum of 9 cin products: at most cin * 9 roundings
     of 2^-24 of the sum of magnitudes, in practice their root. The statistics are sums of what was written."""
@@ -180,7 +180,7 @@ def test_conv_tiles_and_slices(hip, H, W, cin, cout):
 
     for epi, r in ((hip.EPI_CONV_F32, None), (hip.EPI_CONV_F32, dres.ptr), (hip.EPI_CONV_BF16, None)):
         want = run(1, 0, epi, r) if H * W >= 4096 else run(3, 0, epi, r)
-        for tile, split in ((12, 0), (2, 0), (12, 2), (2, 2), (1, 4), (-1, 0), (-1, 8)):
+        for tile, split in ((12, 0), (13, 0), (2, 0), (12, 2), (2, 2), (13, 2), (13, 8), (1, 4), (-1, 0), (-1, 8)):
             if tile == 2 and cout % 256:
                 continue
             got = run(tile, split, epi, r)
