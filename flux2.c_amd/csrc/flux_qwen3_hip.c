@@ -332,6 +332,7 @@ float *flux_hip_qwen3_forward(flux_hip_qwen3 *q, const int *input_ids, const int
     }
     float *out = (float *)malloc((size_t)S * 3 * H * sizeof(float));
     if (!out) { flux_hip_fail("out of host memory"); return NULL; }
+    flux_hip_prefault(out, (size_t)S * 3 * H * sizeof(float));
     float *whole = NULL;    /* without a staging buffer (results under 1 MB): one download at the end */
     if (!parts) {
         whole = (float *)malloc(3 * part_bytes);

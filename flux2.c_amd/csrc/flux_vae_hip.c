@@ -31,12 +31,12 @@
 /* vae.hip */
 int flux_hip_vae_latent_in(void *out_bf16, const float *latent, const float *bn_mean, const float *bn_var,
                            const float *pq_w, const float *pq_b, int h, int w, float eps);
-int flux_hip_vae_key_bias(float *bias, int n, int hp, int wp);
+int flux_hip_vae_key_bias(float *bias, int n, int keys);
 int flux_hip_vae_image_out(uint8_t *rgb, float *rgb_f32, const float *x, int ldx, int H, int W);
 int flux_hip_vae_image_in(void *out_bf16, const float *img, int H, int W);
 int flux_hip_vae_upsample2x_bf16(void *out_bf16, const void *x_bf16, int hp, int wp, int C);
 /* gemm.hip */
-int flux_hip_conv_image(int epilogue, const void *in, int in_wp, const void *w, const float *bias, const float *res, void *out, int rows, int wp,
+int flux_hip_conv_image(int epilogue, const void *in, int in_wp, int packed, const void *w, const float *bias, const float *res, void *out, int rows, int wp,
                         int cin, int cout, int taps, float *stats, int *stats_rows);
 /* vae.hip */
 int flux_hip_vae_latent_out(float *latent, const float *x, int ldx, const float *bn_mean, const float *bn_var, int h, int w, float eps);
@@ -364,8 +364,8 @@ void flux_hip_vae_set_attention_chunk(int rows) { g_att_chunk_limit = rows > 0 ?
  * one image row + 2 positions on both sides (flux_hip_conv reads that far beyond the image). */
 static int ensure_work(flux_hip_vae *v, int h, int w) {
     const size_t hp0 = 16 * (size_t)h + 2, wp0 = 16 * (size_t)w + 2, mp0 = hp0 * wp0;
-    const size_t hpm = 2 * (size_t)h + 2, wpm = 2 * (size_t)w + 2, mpm = hpm * wpm;
-    const size_t ld = (mpm + 255) & ~(size_t)255; /* whole tiles of 256 x 256: 16900 rows of scores took 430 us in tiles of 128 x 128 */
+    const size_t mpm = 4 * (size_t)h * w; /* positions of the attention */
+    const size_t ld = (mpm + 255) & ~(size_t)255; /* whole tiles of 256 x 256: 16900 columns of scores, a multiple of 128 after padding, took 430 us in tiles of 128 x 128 */
     size_t f32_elems = mp0 * 256, guard = (wp0 + 2) * 512;
     size_t bf16_elems = mp0 * 256;
     if (bf16_elems < ld * 1536) bf16_elems = ld * 1536; /* R also holds q, k, v of the attention */
@@ -425,7 +425,7 @@ static int run_conv(vstate *s, const vconv *c, int epi, const void *in, const fl
 }
 
 static int conv_to_bf16(vstate *s, const vconv *c, const float *res, void *out_bf16) {
-    return flux_hip_conv_image(FLUX_HIP_EPI_CONV_BF16, s->A, 0, c->w, c->b, res, out_bf16, s->hp * s->wp, s->wp, c->cin_pad, c->cout_pad, c->taps, NULL, NULL);
+    return flux_hip_conv_image(FLUX_HIP_EPI_CONV_BF16, s->A, 0, 0, c->w, c->b, res, out_bf16, s->hp * s->wp, s->wp, c->cin_pad, c->cout_pad, c->taps, NULL, NULL);
 }
 
 /* resblock_forward, flux_vae.c:179-219. Every group norm takes its statistics from the epilogue of
@@ -448,15 +448,17 @@ static int run_res(vstate *s, const vres *r, void *out_bf16) {
     return run_conv(s, &r->c2, FLUX_HIP_EPI_CONV_F32, s->A, s->x, s->x, 1, v->st_x, &s->x_rows);
 }
 
-/* attnblock_forward, flux_vae.c:223-313 */
+/* attnblock_forward, flux_vae.c:223-313. Between the two 1x1 convolutions the border positions are left out: a
+ * 1024x1024 picture's 16384 positions are 128 tiles of 256 x 256 of the second product, one round of workgroups in two K slices,
+ * where the 16900 of the bordered image were 134, two rounds. */
 static int run_attn(vstate *s, const vattn *a) {
     flux_hip_vae *v = s->v;
-    const int C = 512, rows = s->hp * s->wp, ld = (rows + 255) & ~255;
+    const int C = 512, rows = (s->hp - 2) * (s->wp - 2), ld = (rows + 255) & ~255;
     if (!flux_hip_group_norm_stats(s->A, NULL, s->x, 0, a->g, a->b, v->gn, s->hp, s->wp, C, v->eps, 0, v->st_x, s->x_rows)) return 0;
     /* key rows between the image and the padded width are read by the score GEMM: zero them */
     if (ld > rows && !flux_hip_memset((char *)v->R + (size_t)rows * 3 * C * 2, 0, (size_t)(ld - rows) * 3 * C * 2)) return 0;
-    if (!run_conv(s, &a->qkv, FLUX_HIP_EPI_CONV_BF16, s->A, NULL, v->R, 0, NULL, NULL)) return 0;
-    if (!flux_hip_vae_key_bias(v->kbias, ld, s->hp, s->wp)) return 0;
+    if (!flux_hip_conv_image(FLUX_HIP_EPI_CONV_BF16, s->A, 0, 2, a->qkv.w, a->qkv.b, NULL, v->R, s->hp * s->wp, s->wp, C, 3 * C, 1, NULL, NULL)) return 0;
+    if (!flux_hip_vae_key_bias(v->kbias, ld, rows)) return 0;
     if (!flux_hip_transpose_bf16(v->VT, ld, (char *)v->R + 2 * C * 2, 3 * C, rows, C)) return 0;
     const float scale = 1.0f / sqrtf((float)C);
     int chunk = (int)v->att_chunk;
@@ -469,7 +471,7 @@ static int run_attn(vstate *s, const vattn *a) {
         flux_hip_linear_part pv = {v->P, v->VT, (char *)s->A + (size_t)r0 * C * 2, NULL, n};
         if (!flux_hip_linear(FLUX_HIP_EPI_BF16, 1, &pv, C, ld, ld, ld, C, 0, 0)) return 0;
     }
-    return run_conv(s, &a->out, FLUX_HIP_EPI_CONV_F32, s->A, s->x, s->x, 1, v->st_x, &s->x_rows);
+    return flux_hip_conv_image(FLUX_HIP_EPI_CONV_F32, s->A, 0, 1, a->out.w, a->out.b, s->x, s->x, s->hp * s->wp, s->wp, C, C, 1, v->st_x, &s->x_rows);
 }
 
 /* latent [128, h, w] on the host -> 8-bit image [16h, 16w, 3] and/or the unquantised decoder
@@ -509,6 +511,8 @@ int flux_hip_vae_decode(flux_hip_vae *v, const float *latent, int h, int w, uint
     if (!run_conv(&s, &v->conv_out, FLUX_HIP_EPI_CONV_F32, s.A, NULL, v->Hb, 1, NULL, NULL)) return 0;
     const int H = 16 * h, W = 16 * w;
     if (!flux_hip_vae_image_out(rgb ? v->img_u8 : NULL, rgb_f32 ? v->img_f32 : NULL, v->Hb, v->conv_out.cout_pad, H, W)) return 0;
+    if (rgb) flux_hip_prefault(rgb, (size_t)H * W * 3);
+    if (rgb_f32) flux_hip_prefault(rgb_f32, (size_t)H * W * 3 * 4);
     if (rgb && !flux_hip_download(rgb, v->img_u8, (size_t)H * W * 3)) return 0;
     if (rgb_f32 && !flux_hip_download(rgb_f32, v->img_f32, (size_t)H * W * 3 * 4)) return 0;
     return flux_hip_sync();
@@ -539,7 +543,7 @@ int flux_hip_vae_encode(flux_hip_vae *v, const float *img, int H, int W, float *
             s.hp = (s.hp - 2) / 2 + 2;
             s.wp = (s.wp - 2) / 2 + 2;
             /* stride 2, straight from the bordered image (gathering nine taps per position first was 250 us at 720 x 1296 x 128) */
-            if (!flux_hip_conv_image(FLUX_HIP_EPI_CONV_F32, v->R, in_wp, c->w, c->b, NULL, s.x, s.hp * s.wp, s.wp, c->cin_pad, c->cout_pad, 9, v->st_x,
+            if (!flux_hip_conv_image(FLUX_HIP_EPI_CONV_F32, v->R, in_wp, 0, c->w, c->b, NULL, s.x, s.hp * s.wp, s.wp, c->cin_pad, c->cout_pad, 9, v->st_x,
                                      &s.x_rows))
                 return 0;
         }

@@ -103,7 +103,8 @@ struct GemmArgs {
      * that what one tap fetched is still in L2 when the next asks for the neighbouring rows
      * (tap-major order re-fetched wide images 3 to 10 times from HBM). */
     int conv_taps, conv_wp, conv_rows;
-    int conv_stride, conv_in_wp; /* the operand's image: the same one, or for the downsampling steps one twice as large */
+    int conv_stride, conv_in_wp; /* the operand's image: the same one, or for the downsampling steps one twice as large; stride 0: packed rows */
+    int conv_packed_out;         /* the output holds the interior positions only, row m = GEMM row m */
     unsigned conv_magic; /* (2^32 - 1) / (conv_wp - 2) */
     const float *bias, *res;
     /* optional: per (row-tile half, 4-channel group) sums and sums of squares of what a convolution
@@ -123,7 +124,7 @@ __device__ __forceinline__ int conv_div(const GemmArgs &g, int m) {
 /* row of GEMM row m in the output: the m-th interior position of the bordered image */
 template <int EPI>
 __device__ __forceinline__ int conv_row(const GemmArgs &g, int m) {
-    if (!IsConv<EPI>::value || g.conv_wp == 0) return m;
+    if (!IsConv<EPI>::value || g.conv_wp == 0 || g.conv_packed_out) return m;
     return m + 2 * conv_div(g, m) + g.conv_wp + 1;
 }
 
@@ -132,7 +133,7 @@ __device__ __forceinline__ int conv_row(const GemmArgs &g, int m) {
  * (2 y + 2, 2 x + 2) of the bordered input; with stride 1 it is (y + 1, x + 1). */
 template <int EPI>
 __device__ __forceinline__ int conv_in_row(const GemmArgs &g, int m) {
-    if (!IsConv<EPI>::value || g.conv_wp == 0) return m;
+    if (!IsConv<EPI>::value || g.conv_wp == 0 || g.conv_stride == 0) return m;
     const int y = conv_div(g, m), x = m - y * (g.conv_wp - 2);
     return g.conv_stride * ((y + 1) * g.conv_in_wp + x + 1);
 }
@@ -173,7 +174,7 @@ __device__ __forceinline__ GemmArgs conv_args_again() {
     a.M[0] = ka->M[0]; a.C[0] = ka->C[0]; a.bias = ka->bias; a.res = ka->res; a.stats = ka->stats;
     a.N = ka->N; a.ldc = ka->ldc; a.mtiles = ka->mtiles; a.ntiles = ka->ntiles; a.total_tiles = ka->total_tiles; a.vgrid = ka->vgrid;
     a.ksplit = ka->ksplit;
-    a.conv_wp = ka->conv_wp; a.conv_rows = ka->conv_rows; a.conv_magic = ka->conv_magic;
+    a.conv_wp = ka->conv_wp; a.conv_rows = ka->conv_rows; a.conv_magic = ka->conv_magic; a.conv_packed_out = ka->conv_packed_out;
     return a;
 }
 
@@ -481,7 +482,7 @@ __device__ __forceinline__ void store_conv_tile(const GemmArgs &g, const TileId 
     if (g.res) rows(BoolC<true>{});
     else rows(BoolC<false>{});
     const int lane = lq * 16 + l15;
-    if (g.conv_wp > 0) {
+    if (g.conv_wp > 0 && !g.conv_packed_out) {
         constexpr int QPW = WN / 4, PPI = 64 / QPW; /* lanes per position, positions per instruction */
         const int wp = g.conv_wp, y0 = conv_div(g, m0), y1 = conv_div(g, min(m0 + BM, M));
         const int nside = 2 * (y1 - y0), nedge = 2 * wp + 1, per = (nedge + g.mtiles - 1) / g.mtiles;
@@ -1267,13 +1268,15 @@ __global__ __launch_bounds__(256) void conv_finish_kernel(GemmArgs g) {
                 s2 += v[e] * v[e];
             }
         }
+        if (g.conv_packed_out && !inside) continue;
+        const size_t at = (size_t)(g.conv_packed_out ? m : p) * g.ldc + n;
         if (F32) {
-            *(f32x4 *)((float *)g.C[0] + (size_t)p * g.ldc + n) = v;
+            *(f32x4 *)((float *)g.C[0] + at) = v;
         } else {
             bf16x4 o;
 #pragma unroll
             for (int e = 0; e < 4; e++) o[e] = (bf16)v[e];
-            *(bf16x4 *)((bf16 *)g.C[0] + (size_t)p * g.ldc + n) = o;
+            *(bf16x4 *)((bf16 *)g.C[0] + at) = o;
         }
     }
     if (g.stats) {
@@ -1640,6 +1643,10 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
                 double bw = 5.5e12 * (double)(resident * ahead[t] * (bm[t] + bn[t]) * 128) / 12.0e6;
                 if (bw > bw_cap) bw = bw_cap;
                 double est = t_compute > bytes / bw ? t_compute : bytes / bw;
+                /* what all tiles together fetch through the L2s: seen at 10 to 13 TB/s (14996 x 512 x 15104 on 236 tiles of 256 x 128:
+                 * 2.7 GB, 238 us; on 118 of 256 x 256 in two K slices 1.8 GB, 176 us) */
+                const double l2 = (double)tiles * (bm[t] + bn[t]) * K * 2.0 / 12.5e12;
+                if (l2 > est) est = l2;
                 if (sp > 1) est += 3.0e-6 + (sp + 2.0) * rows * N * 4.0 / 4.0e12;
                 else if (adaln) est += 3.0e-6 + rows * N * 6.0 / 4.0e12; /* the norm that the second pass would have taken along */
                 if (est < best) { best = est; tile = t; best_split = sp; }
@@ -1836,7 +1843,7 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
     static const int splits[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int M = g.M[0], N = g.N, kt_total = g.K >> 6, f = g_force_tile;
     const bool forced = f >= 0 && f < CONV_TILES && conv_bm[f] && N % conv_bn[f] == 0; /* a forced tile that this layer cannot use is ignored */
-    const bool ring_ok = g_ring && (size_t)g.conv_rows * g.conv_stride * g.conv_stride * g.lda * 2 < ((size_t)1 << 32) && (size_t)N * g.ldw * 2 < ((size_t)1 << 32) &&
+    const bool ring_ok = g_ring && (size_t)g.conv_rows * (g.conv_stride == 2 ? 4 : 1) * g.lda * 2 < ((size_t)1 << 32) && (size_t)N * g.ldw * 2 < ((size_t)1 << 32) &&
                          (size_t)g.conv_rows * N < ((size_t)1 << 32);
     int tile = -1, split = 1;
     double best = 1e30;
@@ -1882,7 +1889,7 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
     return bf ? conv_tile_launch<FLUX_HIP_EPI_CONV_BF16>(g, tile) : conv_tile_launch<FLUX_HIP_EPI_CONV_F32>(g, tile);
 }
 
-extern "C" int flux_hip_conv_image(int epilogue, const void *in, int in_wp, const void *w, const float *bias, const float *res, void *out,
+extern "C" int flux_hip_conv_image(int epilogue, const void *in, int in_wp, int packed, const void *w, const float *bias, const float *res, void *out,
                                    int rows, int wp, int cin, int cout, int taps, float *stats, int *stats_rows);
 
 /* Convolution over a zero-bordered channels-last image as one GEMM, see the header. */
@@ -1909,12 +1916,14 @@ extern "C" int flux_hip_conv_stats(int epilogue, const void *in, const void *w, 
     if ((((uintptr_t)in | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)res | (uintptr_t)out) & 15))
         return flux_hip_fail("flux_hip_conv: operands must be 16-byte aligned");
     if (res && epilogue != FLUX_HIP_EPI_CONV_F32) return flux_hip_fail("flux_hip_conv: only the fp32 epilogue adds a residual");
-    return flux_hip_conv_image(epilogue, in, 0, w, bias, res, out, rows, wp, cin, cout, taps, stats, stats_rows);
+    return flux_hip_conv_image(epilogue, in, 0, 0, w, bias, res, out, rows, wp, cin, cout, taps, stats, stats_rows);
 }
 
 /* flux_hip_conv_stats without its argument checks, for the VAE's own layers: the bf16 output takes a residual as well, and
- * in_wp > 0 makes it the stride-2 3x3 convolution of a bordered image in_wp wide, rows and wp being the output's. */
-extern "C" int flux_hip_conv_image(int epilogue, const void *in, int in_wp, const void *w, const float *bias, const float *res, void *out,
+ * in_wp > 0 makes it the stride-2 3x3 convolution of a bordered image in_wp wide, rows and wp being the output's. For 1x1
+ * convolutions without residual or statistics on that side, packed & 1: `in`, packed & 2: `out` hold the (rows / wp - 2) * (wp - 2)
+ * interior positions only. */
+extern "C" int flux_hip_conv_image(int epilogue, const void *in, int in_wp, int packed, const void *w, const float *bias, const float *res, void *out,
                                    int rows, int wp, int cin, int cout, int taps, float *stats, int *stats_rows) {
     GemmArgs g = {};
     g.A[0] = (const bf16 *)in;
@@ -1922,7 +1931,8 @@ extern "C" int flux_hip_conv_image(int epilogue, const void *in, int in_wp, cons
     g.C[0] = out;
     g.N = cout; g.K = taps * cin; g.lda = cin; g.ldw = taps * cin; g.ldc = cout;
     g.conv_taps = taps; g.conv_wp = wp; g.conv_rows = rows;
-    g.conv_stride = in_wp > 0 ? 2 : 1; g.conv_in_wp = in_wp > 0 ? in_wp : wp;
+    g.conv_packed_out = packed >> 1 & 1;
+    g.conv_stride = packed & 1 ? 0 : in_wp > 0 ? 2 : 1; g.conv_in_wp = in_wp > 0 ? in_wp : wp;
     g.M[0] = rows;
     if (wp > 0) {
         g.M[0] = wp > 2 && rows / wp > 2 ? (rows / wp - 2) * (wp - 2) : 0;

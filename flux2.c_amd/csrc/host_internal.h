@@ -85,4 +85,7 @@ float fh_tensor_value(int dtype, const void *data, int64_t i);
 int flux_hip_download_part_begin(int part, size_t stage_offset, size_t stage_total, const void *src, size_t bytes);
 const void *flux_hip_download_part_wait(int part);
 
+/* runtime.hip: touch every page of a result's destination while the device computes it */
+void flux_hip_prefault(void *dst, size_t bytes);
+
 #endif

@@ -129,6 +129,15 @@ extern "C" int flux_hip_upload(void *dst, const void *src, size_t bytes) {
     return 1;
 }
 
+/* Memory that the caller has only just allocated gets its pages one by one at the first write to each, which for a result is
+ * the copy at the end, with the device idle. Called between queueing the work and waiting for it: one write per page, while
+ * the device computes. The contents are the result's to overwrite. */
+extern "C" void flux_hip_prefault(void *dst, size_t bytes) {
+    volatile char *p = (volatile char *)dst;
+    for (size_t i = 0; i < bytes; i += 4096) p[i] = 0;
+    if (bytes) p[bytes - 1] = 0;
+}
+
 extern "C" int flux_hip_download(void *dst, const void *src, size_t bytes) {
     if (!flux_hip_available()) return 0;
     if (!bytes) return 1;

@@ -357,12 +357,12 @@ __global__ __launch_bounds__(256) void vae_latent_out_kernel(float *__restrict__
 
 /* ---- attention over all positions with one head (attnblock_forward, flux_vae.c:223-313).
  * Scores are materialised, as in the reference: S = q k^T (GEMM), P = softmax(S * scale + bias)
- * (below), O = P v (GEMM against v^T). Keys run over the bordered grid plus padding up to a
- * multiple of 128; key_bias is 0 for real pixels and -inf for border and padding columns. ---- */
-__global__ __launch_bounds__(256) void vae_key_bias_kernel(float *__restrict__ bias, int n, int rows, int hp, int wp) {
+ * (below), O = P v (GEMM against v^T). Queries and keys are the image's interior positions, packed; keys are padded up to a
+ * multiple of 256, and key_bias is 0 for real ones and -inf for the padding columns. ---- */
+__global__ __launch_bounds__(256) void vae_key_bias_kernel(float *__restrict__ bias, int n, int keys) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    bias[i] = (i < rows && interior(i, hp, wp)) ? 0.0f : -INFINITY;
+    bias[i] = i < keys ? 0.0f : -INFINITY;
 }
 
 __global__ __launch_bounds__(256) void vae_softmax_kernel(bf16 *__restrict__ P, const float *__restrict__ S, const float *__restrict__ key_bias,
@@ -593,8 +593,8 @@ extern "C" int flux_hip_vae_latent_out(float *latent, const float *x, int ldx, c
     return 1;
 }
 
-extern "C" int flux_hip_vae_key_bias(float *bias, int n, int hp, int wp) {
-    hipLaunchKernelGGL(vae_key_bias_kernel, dim3((n + 255) / 256), dim3(256), 0, flux_hip_stream_handle(), bias, n, hp * wp, hp, wp);
+extern "C" int flux_hip_vae_key_bias(float *bias, int n, int keys) {
+    hipLaunchKernelGGL(vae_key_bias_kernel, dim3((n + 255) / 256), dim3(256), 0, flux_hip_stream_handle(), bias, n, keys);
     LAUNCH_OK("vae_key_bias_kernel");
     return 1;
 }
