@@ -309,8 +309,10 @@ float *flux_hip_qwen3_forward(flux_hip_qwen3 *q, const int *input_ids, const int
     for (int li = 0; li < q->n_run; li++) {
         const qlayer *l = &q->layer[li];
         if (!normed && !flux_hip_rms_norm(q->xn, q->x, l->in_norm, S, H, c->eps)) return NULL;
-        if (!linear1(FLUX_HIP_EPI_BF16, q->xn, l->qkv, q->qkv, NULL, S, W, H, H, W, 0, 0)) return NULL;
-        if (!flux_hip_qwen3_qk_rope(q->qkv, q->vt, QW_MAX_SEQ, l->q_norm, l->k_norm, q->rope_cos, q->rope_sin, S, c->heads, c->kv_heads, c->eps)) return NULL;
+        const float *ws = NULL;
+        int slices = 0;
+        if (!flux_hip_linear_slices(q->xn, l->qkv, q->qkv, S, W, H, &ws, &slices)) return NULL;
+        if (!flux_hip_qwen3_qk_rope_slices(q->qkv, q->vt, QW_MAX_SEQ, l->q_norm, l->k_norm, q->rope_cos, q->rope_sin, S, c->heads, c->kv_heads, c->eps, ws, slices)) return NULL;
         if (!flux_hip_causal_attention(q->att, q->qkv, q->vt, QW_MAX_SEQ, mask, S, c->heads, c->kv_heads)) return NULL;
         flux_hip_linear_part po = {q->att, l->o, q->x, q->ones, S};
         flux_hip_adaln_part no = {q->xn, NULL, l->post_norm};

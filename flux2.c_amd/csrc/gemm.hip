@@ -1568,7 +1568,7 @@ static int probe_slot(int epilogue) {
 
 /* Tile and K-split choice, then the launch; `allowed` has bit t set for every tile id that may be used. */
 static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, int *tile_out = nullptr, const AdalnArgs *adaln = nullptr,
-                         int *adaln_done = nullptr, float *fixed_ws = nullptr, size_t fixed_ws_bytes = 0) {
+                         int *adaln_done = nullptr, float *fixed_ws = nullptr, size_t fixed_ws_bytes = 0, int *leave_slices = nullptr) {
     /* Choose tile and K split with a small cost model: workgroups run in rounds over
      * 256 CUs x occupancy; a workgroup's time is its FLOPs at the tile's measured rate plus a
      * fixed prologue/epilogue cost; the launch cannot beat the time to stream its operands,
@@ -1680,7 +1680,9 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
     int ok;
     const bool split = g.ksplit > 1;
     switch (epilogue) {
-        case FLUX_HIP_EPI_BF16: ok = split ? launch_split<FLUX_HIP_EPI_BF16>(g, tile) : launch_epi<FLUX_HIP_EPI_BF16>(g, tile); break;
+        case FLUX_HIP_EPI_BF16:
+            if (leave_slices) *leave_slices = split ? g.ksplit : 0;
+            ok = split && leave_slices ? launch_epi<EPI_PARTIAL>(g, tile) : split ? launch_split<FLUX_HIP_EPI_BF16>(g, tile) : launch_epi<FLUX_HIP_EPI_BF16>(g, tile); break;
         case FLUX_HIP_EPI_F32: ok = split ? launch_split<FLUX_HIP_EPI_F32>(g, tile) : launch_epi<FLUX_HIP_EPI_F32>(g, tile); break;
         case FLUX_HIP_EPI_F32_T: ok = launch_epi<FLUX_HIP_EPI_F32_T>(g, tile); break;
         case FLUX_HIP_EPI_RESID:
@@ -1750,6 +1752,22 @@ static int linear_impl(int epilogue, int nparts, const flux_hip_linear_part *par
 extern "C" int flux_hip_linear(int epilogue, int nparts, const flux_hip_linear_part *parts,
                                int N, int K, int lda, int ldw, int ldc, int w_row0, int w_row1) {
     return linear_impl(epilogue, nparts, parts, N, K, lda, ldw, ldc, w_row0, w_row1, nullptr, 0.0f, nullptr);
+}
+
+/* A bf16 projection of one row range whose reader can sum K slices itself: *slices = 0 and C is written as by flux_hip_linear, or
+ * *slices partial sums are left at *ws, fp32 [*slices][M][N], to be added in slice order (what the second pass would do), and C is
+ * untouched. The sums are valid until the next projection. */
+extern "C" int flux_hip_linear_slices(const void *A, const void *W, void *C, int M, int N, int K, const float **ws, int *slices) {
+    *slices = 0;
+    if (M <= 0) return 1;
+    if (K <= 0 || (K & 63) || N <= 0 || (N & 127)) return flux_hip_fail("flux_hip_linear_slices: N=%d must be a multiple of 128, K=%d of 64", N, K);
+    if (!A || !W || !C || ((((uintptr_t)A | (uintptr_t)W) & 15) || ((uintptr_t)C & 7))) return flux_hip_fail("flux_hip_linear_slices: NULL or unaligned operand");
+    GemmArgs g = {};
+    g.A[0] = (const bf16 *)A; g.W[0] = (const bf16 *)W; g.C[0] = C; g.M[0] = M;
+    g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = N;
+    const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_BF16, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
+    *ws = g.ws;
+    return ok;
 }
 
 /* One launch for the fused projection of a single-stream block, see the header. Never split along K. */

@@ -88,4 +88,9 @@ const void *flux_hip_download_part_wait(int part);
 /* runtime.hip: touch every page of a result's destination while the device computes it */
 void flux_hip_prefault(void *dst, size_t bytes);
 
+/* gemm.hip, qwen3.hip: a projection that may leave its K slices to the kernel that reads it */
+int flux_hip_linear_slices(const void *A, const void *W, void *C, int M, int N, int K, const float **ws, int *slices);
+int flux_hip_qwen3_qk_rope_slices(void *qkv_bf16, void *vt_bf16, int ldv, const float *q_w, const float *k_w, const float *rope_cos, const float *rope_sin,
+                                  int seq, int heads, int kv_heads, float eps, const float *ws, int slices);
+
 #endif

@@ -53,7 +53,9 @@ __global__ __launch_bounds__(256) void qwen3_rms_norm_kernel(bf16 *__restrict__ 
  * layout the attention kernel's second product reads.
  * 16 lanes share a head's row, four pairs each (8-byte accesses), 16 rows per workgroup; the v heads go through LDS in blocks of
  * 64 tokens, so that a dim's tokens leave as 16-byte stores. With one wave per row and a 2-byte store per lane and token
- * for V the launch took 10.8 us at 512 tokens x 48 heads. VEC = false: pointers or ldv that do not allow the wide accesses. */
+ * for V the launch took 10.8 us at 512 tokens x 48 heads. VEC = false: pointers or ldv that do not allow the wide accesses.
+ * SLICES: the projection ran as K slices and its partial sums are read here, summed in slice order and rounded to bf16 as its second
+ * pass would (which at 67 tokens was a launch of 4.8 us); the v columns of qkv are then not written. */
 template <bool VEC, typename V4, typename T>
 __device__ __forceinline__ V4 qw_load4(const T *p) {
     if (VEC) return *(const V4 *)p;
@@ -71,18 +73,34 @@ __device__ __forceinline__ void qw_store4(bf16 *p, bf16x4 v) {
         for (int e = 0; e < 4; e++) p[e] = v[e];
     }
 }
-template <bool VEC>
+template <bool VEC, bool SLICES>
 __global__ __launch_bounds__(256) void qwen3_qk_rope_kernel(bf16 *__restrict__ qkv, bf16 *__restrict__ vt, int ldv, const float *__restrict__ q_w,
                                                             const float *__restrict__ k_w, const float *__restrict__ rope_cos,
-                                                            const float *__restrict__ rope_sin, int seq, int heads, int kv_heads, float eps) {
+                                                            const float *__restrict__ rope_sin, int seq, int heads, int kv_heads, float eps,
+                                                            const float *__restrict__ ws, int slices) {
     __shared__ bf16 tile[64][130]; /* (rows of 65 words: a column's reads fall on different banks) */
     const int width = (heads + 2 * kv_heads) * 128, nqk = heads + kv_heads, rows = seq * nqk, qk_blocks = (rows + 15) / 16;
+    const auto load = [&](int s, int col) -> bf16x4 { /* four columns of a token's projection */
+        if (!SLICES) return qw_load4<VEC, bf16x4>(qkv + (size_t)s * width + col);
+        f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+        const float *p = ws + (size_t)s * width + col;
+#pragma unroll 4
+        for (int k = 0; k < slices; k++) {
+            const f32x4 v = *(const f32x4 *)(p + (size_t)k * seq * width);
+#pragma unroll
+            for (int e = 0; e < 4; e++) sum[e] += v[e];
+        }
+        bf16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = (bf16)sum[e];
+        return o;
+    };
     if ((int)blockIdx.x >= qk_blocks) { /* 64 tokens of a v head: transpose */
         const int vb = blockIdx.x - qk_blocks, vh = vb % kv_heads, s0 = vb / kv_heads * 64;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int idx = i * 256 + threadIdx.x, r = idx >> 5, c = (idx & 31) * 4, s = min(s0 + r, seq - 1);
-            const bf16x4 v = qw_load4<VEC, bf16x4>(qkv + (size_t)s * width + (nqk + vh) * 128 + c);
+            const bf16x4 v = load(s, (nqk + vh) * 128 + c);
 #pragma unroll
             for (int e = 0; e < 4; e++) tile[r][c + e] = v[e];
         }
@@ -109,7 +127,7 @@ __global__ __launch_bounds__(256) void qwen3_qk_rope_kernel(bf16 *__restrict__ q
     const int s = row / nqk, h = row - s * nqk;
     bf16 *p = qkv + (size_t)s * width + h * 128 + i0;
     const float *w = (h < heads ? q_w : k_w) + i0;
-    const bf16x4 lo = qw_load4<VEC, bf16x4>(p), hi = qw_load4<VEC, bf16x4>(p + 64);
+    const bf16x4 lo = load(s, h * 128 + i0), hi = load(s, h * 128 + i0 + 64);
     const f32x4 w0 = qw_load4<VEC, f32x4>(w), w1 = qw_load4<VEC, f32x4>(w + 64);
     const f32x4 cs = qw_load4<VEC, f32x4>(rope_cos + s * 64 + i0), sn = qw_load4<VEC, f32x4>(rope_sin + s * 64 + i0);
     float ss = 0.0f;
@@ -359,15 +377,24 @@ extern "C" int flux_hip_rms_norm(void *out_bf16, const float *x, const float *w,
     return 1;
 }
 
-extern "C" int flux_hip_qwen3_qk_rope(void *qkv_bf16, void *vt_bf16, int ldv, const float *q_w, const float *k_w, const float *rope_cos,
-                                      const float *rope_sin, int seq, int heads, int kv_heads, float eps) {
+/* ws, slices: what flux_hip_linear_slices left; slices = 0: qkv holds the projection */
+extern "C" int flux_hip_qwen3_qk_rope_slices(void *qkv_bf16, void *vt_bf16, int ldv, const float *q_w, const float *k_w, const float *rope_cos,
+                                             const float *rope_sin, int seq, int heads, int kv_heads, float eps, const float *ws, int slices) {
     if (seq <= 0 || heads <= 0 || kv_heads <= 0 || ldv < seq) return flux_hip_fail("flux_hip_qwen3_qk_rope: bad shape");
     const bool vec = !((((uintptr_t)qkv_bf16 | (uintptr_t)vt_bf16 | (uintptr_t)q_w | (uintptr_t)k_w | (uintptr_t)rope_cos | (uintptr_t)rope_sin) & 15) | (ldv & 7));
+    if (slices > 0 && (!vec || !ws || ((uintptr_t)ws & 15))) return flux_hip_fail("flux_hip_qwen3_qk_rope_slices: unaligned operand");
     const dim3 grid((seq * (heads + kv_heads) + 15) / 16 + (seq + 63) / 64 * kv_heads);
-    hipLaunchKernelGGL(vec ? qwen3_qk_rope_kernel<true> : qwen3_qk_rope_kernel<false>, grid, dim3(256), 0, flux_hip_stream_handle(),
-                       (bf16 *)qkv_bf16, (bf16 *)vt_bf16, ldv, q_w, k_w, rope_cos, rope_sin, seq, heads, kv_heads, eps);
+    auto kern = slices > 0 ? qwen3_qk_rope_kernel<true, true> : vec ? qwen3_qk_rope_kernel<true, false> : qwen3_qk_rope_kernel<false, false>;
+    hipLaunchKernelGGL(kern, grid,
+                       dim3(256), 0, flux_hip_stream_handle(), (bf16 *)qkv_bf16, (bf16 *)vt_bf16, ldv, q_w, k_w, rope_cos, rope_sin, seq, heads, kv_heads,
+                       eps, ws, slices);
     LAUNCH_OK("qwen3_qk_rope_kernel");
     return 1;
+}
+
+extern "C" int flux_hip_qwen3_qk_rope(void *qkv_bf16, void *vt_bf16, int ldv, const float *q_w, const float *k_w, const float *rope_cos,
+                                      const float *rope_sin, int seq, int heads, int kv_heads, float eps) {
+    return flux_hip_qwen3_qk_rope_slices(qkv_bf16, vt_bf16, ldv, q_w, k_w, rope_cos, rope_sin, seq, heads, kv_heads, eps, NULL, 0);
 }
 
 extern "C" int flux_hip_causal_attention(void *out_bf16, const void *qkv_bf16, const void *vt_bf16, int ldv, const int *mask_dev, int seq,

@@ -102,6 +102,37 @@ def test_qk_norm_rope_and_v_transpose(hip, seq, heads, kv, ldv):
     assert (vt[:, seq:] == 0x4242).all()
 
 
+@pytest.mark.parametrize("seq,split", [(1, 2), (67, 3), (67, 0), (100, 8)])
+def test_qk_rope_from_the_slices_of_the_projection(hip, seq, split):
+    """The projection as K slices that the norm + RoPE kernel sums itself: bit for bit what the second pass and the
+    kernel give one after the other (the same additions in the same order, the same rounding)."""
+    import ctypes
+    L, heads, kv, K = hip.lib(), 4, 2, 2048
+    width = (heads + 2 * kv) * 128
+    vp, ci = ctypes.c_void_p, ctypes.c_int
+    L.flux_hip_linear_slices.argtypes = [vp, vp, vp, ci, ci, ci, vp, vp]
+    L.flux_hip_qwen3_qk_rope_slices.argtypes = [vp, vp, ci, vp, vp, vp, vp, ci, ci, ci, ctypes.c_float, vp, ci]
+    d = {k: hip.DevBuf.from_array(f32_to_bf16(normal_f32(s, 76, i, 0.0, sd))) for k, s, i, sd in (("a", (seq, K), 1, 1.0), ("w", (width, K), 2, 0.05))}
+    tabs = [hip.DevBuf.from_array(normal_f32(s, 76, 3 + i, 1.0, 0.2)) for i, s in enumerate(((128,), (128,), (seq, 64), (seq, 64)))]
+    got = []
+    for leave in (False, True):
+        qkv = hip.DevBuf.from_array(np.zeros((seq, width), np.uint16))
+        vt = hip.DevBuf.from_array(np.zeros((kv * 128, 128), np.uint16))
+        ws, n = vp(0), ci(0)
+        L.flux_hip_linear_force_split(split)
+        try:
+            if leave:
+                hip.check(L.flux_hip_linear_slices(d["a"].ptr, d["w"].ptr, qkv.ptr, seq, width, K, ctypes.byref(ws), ctypes.byref(n)))
+                assert split == 0 or n.value == split
+            else:
+                hip.linear(hip.EPI_BF16, [(d["a"].ptr, d["w"].ptr, qkv.ptr, None, seq)], width, K, K, K, width, 0, 0)
+        finally:
+            L.flux_hip_linear_force_split(0)
+        hip.check(L.flux_hip_qwen3_qk_rope_slices(qkv.ptr, vt.ptr, 128, *[t.ptr for t in tabs], seq, heads, kv, 1e-6, ws if leave else None, n.value))
+        got.append((qkv.to_array(np.uint16, (seq, width))[:, :(heads + kv) * 128], vt.to_array(np.uint16, (kv * 128, 128))))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
 MID = QwenConfig(hidden=512, intermediate=1152, heads=8, kv_heads=2, layers=6, vocab=1000, out_layers=(0, 3, 5))
 
 
