@@ -51,9 +51,9 @@
  * runs (tile id 4).
  *
  * Three kernels, then: gemm_kernel (small tiles; with NS > 2 a ring of NS LDS stages for row ranges of few
- * rows, where a launch only streams weights), gemm4w_kernel (large tiles, two LDS stages; convolutions, and the
+ * rows, where a launch only streams weights), gemm4w_kernel (large tiles, two LDS stages; the
  * comparison form of the next one) and gemm4d_kernel (large tiles with an LDS ring per operand, the form the
- * transformer's projections run). What separates the last two is the barrier: __syncthreads() carries a fence
+ * transformer's projections and the VAE's convolutions run). What separates the last two is the barrier: __syncthreads() carries a fence
  * that waits for every global->LDS load in flight, so a two-stage loop can never have more than the next stage
  * on its way, requested one to two half-steps earlier; operands that come from HBM arrive later than that now and
  * then, and a wave that waits holds its three neighbours up at the barrier (measured: the same launch takes
@@ -140,7 +140,7 @@ __device__ __forceinline__ int conv_in_row(const GemmArgs &g, int m) {
 
 /* Element offset of K step kt within an activation row. Plain GEMM: kt * 64. 3x3 convolution:
  * kt = 9 * chunk + tap; the tap selects a neighbour dy*Wp + dx rows away (uniform for the whole
- * launch, because border positions are rows of the matrix too), the chunk a 64-channel slice. */
+ * launch, because border positions are rows of the operand too), the chunk a 64-channel slice. */
 template <int EPI>
 __device__ __forceinline__ int a_step_offset(const GemmArgs &g, int kt) {
     if (IsConv<EPI>::value) {
@@ -285,9 +285,9 @@ __device__ __forceinline__ void store_tile_to(const GemmArgs &g, const TileId &t
          * branches (behind a skipped store the compiler must assume that the loads in front of it are still under
          * way, and it waits for them before it reuses their registers: one row block in flight instead of two). */
         const auto cut = [&](int i) { return CutTile<BN>::value && n0 + wn * WN + i * 16 >= g.N; }; /* the same for the whole wave */
-        /* the unit that is requested ahead: a row block's TN column blocks, or half of them where the accumulators fill the
-         * AGPRs and the fragments most of the VGPRs (256 x 256) */
-        constexpr int UN = TM * TN * 4 > 224 && TN % 2 == 0 ? TN / 2 : TN, UPR = TN / UN, NU = TM * UPR;
+        /* the unit that is requested ahead: a row block's TN column blocks, or half of them with eight (256 x 256, 192 x 256), where
+         * two whole ones, the gate and the next tile's fragments are more than the VGPRs hold (192 x 256 parked seven in AGPRs) */
+        constexpr int UN = TN > 6 && TN % 2 == 0 ? TN / 2 : TN, UPR = TN / UN, NU = TM * UPR;
         constexpr int NB = 2; /* units in flight, the one being stored included (a third one measured no different: what is left is the burst itself) */
         f32x4 gt[TN], xb[NB][UN];
 #pragma unroll
@@ -1644,8 +1644,9 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
                 if (bw > bw_cap) bw = bw_cap;
                 double est = t_compute > bytes / bw ? t_compute : bytes / bw;
                 /* what all tiles together fetch through the L2s: seen at 10 to 13 TB/s (14996 x 512 x 15104 on 236 tiles of 256 x 128:
-                 * 2.7 GB, 238 us; on 118 of 256 x 256 in two K slices 1.8 GB, 176 us) */
-                const double l2 = (double)tiles * (bm[t] + bn[t]) * K * 2.0 / 12.5e12;
+                 * 2.7 GB, 238 us; on 118 of 256 x 256 in two K slices 1.8 GB, 176 us; 4608 x 3072 x 12288 on 256 tiles of 288 x 192:
+                 * 3.0 GB, 231 us, which with 12.5 TB/s here lost to 256 x 224 in the model and was 10 us faster than it) */
+                const double l2 = (double)tiles * (bm[t] + bn[t]) * K * 2.0 / 12.9e12;
                 if (l2 > est) est = l2;
                 if (sp > 1) est += 3.0e-6 + (sp + 2.0) * rows * N * 4.0 / 4.0e12;
                 else if (adaln) est += 3.0e-6 + rows * N * 6.0 / 4.0e12; /* the norm that the second pass would have taken along */
