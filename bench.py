@@ -222,7 +222,8 @@ def bench_vae(args):
         ms = np.zeros(cap, np.float32)
         n = L.flux_hip_linear_probe_read_launches(cap, tiles.ctypes.data, ms.ctypes.data)
         L.flux_hip_linear_probe(-1)
-        if n == cap:
+        assert n == min(cap, 4096), f"{n} convolutions recorded, {cap} run"
+        if n == cap:      # (the probe keeps 4096 records)
             fl = np.array([2.0 * H * W * ci * co * t for _, H, W, ci, co, t in convs] * K)
             names = {0: "gemm_kernel<64,128,2,2,CONV>", 1: "gemm_kernel<128,128,2,2,CONV>", 2: "gemm4d_kernel<8,8,CONV> (256x256 tile)",
                      3: "gemm_kernel<64,64,2,2,CONV>", 12: "gemm4d_kernel<8,4,CONV> (256x128 tile)", 13: "gemm4d_kernel<4,4,CONV> (128x128 tile)"}

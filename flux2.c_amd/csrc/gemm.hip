@@ -1888,24 +1888,30 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
     }
     if (tile < 0) tile = N % 128 == 0 ? 1 : 3; /* (a forced ring tile that cannot run) */
     g.kt_per = (kt_total + split - 1) / split;
-    g.ksplit = split;
+    g.ksplit = M == 0 ? 0 : split; /* 0: nothing but border */
     const bool bf = epilogue == FLUX_HIP_EPI_CONV_BF16;
-    int ok;
-    if (M == 0) { /* nothing but border */
-        g.ksplit = 0;
-        if (stats_rows) *stats_rows = (g.conv_rows + 31) / 32;
-        return bf ? conv_finish<FLUX_HIP_EPI_CONV_BF16>(g) : conv_finish<FLUX_HIP_EPI_CONV_F32>(g);
-    }
-    if (split > 1) {
+    if (g.ksplit > 1) {
         if (!ensure_ws((size_t)split * M * N * sizeof(float))) return 0;
         g.ws = g_ws;
         g.ws_rows = M;
-        ok = conv_tile_launch<EPI_CONV_PARTIAL>(g, tile) && (bf ? conv_finish<FLUX_HIP_EPI_CONV_BF16>(g) : conv_finish<FLUX_HIP_EPI_CONV_F32>(g));
-        if (stats_rows) *stats_rows = (g.conv_rows + 31) / 32;
-        return ok;
     }
-    if (stats_rows) *stats_rows = 2 * ((M + conv_bm[tile] - 1) / conv_bm[tile]);
-    return bf ? conv_tile_launch<FLUX_HIP_EPI_CONV_BF16>(g, tile) : conv_tile_launch<FLUX_HIP_EPI_CONV_F32>(g, tile);
+    /* one record per convolution: K slices and their second pass together */
+    const int slot = probe_slot(epilogue);
+    if (slot >= 0) {
+        g_probe_tile[slot] = (unsigned char)tile;
+        (void)hipEventRecord(g_probe_ev[slot][0], flux_hip_stream_handle());
+    }
+    int ok = 1;
+    if (g.ksplit == 1) {
+        if (stats_rows) *stats_rows = 2 * ((M + conv_bm[tile] - 1) / conv_bm[tile]);
+        ok = bf ? conv_tile_launch<FLUX_HIP_EPI_CONV_BF16>(g, tile) : conv_tile_launch<FLUX_HIP_EPI_CONV_F32>(g, tile);
+    } else {
+        if (stats_rows) *stats_rows = (g.conv_rows + 31) / 32;
+        if (g.ksplit > 1) ok = conv_tile_launch<EPI_CONV_PARTIAL>(g, tile);
+        ok = ok && (bf ? conv_finish<FLUX_HIP_EPI_CONV_BF16>(g) : conv_finish<FLUX_HIP_EPI_CONV_F32>(g));
+    }
+    if (slot >= 0) (void)hipEventRecord(g_probe_ev[slot][1], flux_hip_stream_handle());
+    return ok;
 }
 
 extern "C" int flux_hip_conv_image(int epilogue, const void *in, int in_wp, int packed, const void *w, const float *bias, const float *res, void *out,

@@ -52,7 +52,7 @@ void flux_hip_set_fused_qkv_mlp(int on);
 void flux_hip_vae_set_attention_chunk(int rows);
 
 /* Launch probe: probe(epilogue) records HIP events around every later flux_hip_linear launch with
- * that epilogue (-2: every flux_hip_conv launch; -1 stops); probe_read waits for them and returns
+ * that epilogue (-2: every convolution, K slices and their second pass as one; -1 stops); probe_read waits for them and returns
  * their count and summed duration, probe_read_tile the same for the launches that used one tile id,
  * probe_read_launches copies out, in launch order, the tile id and duration (ms) of up to `max`
  * recorded launches and returns their number (-1 on error). */

@@ -190,6 +190,48 @@ def test_conv_tiles_and_slices(hip, H, W, cin, cout):
                 assert rel_l2(got, want) < (2.0 ** -9 if epi == hip.EPI_CONV_BF16 else 2e-6)
 
 
+def test_probe_records_every_convolution(hip):
+    """Mode -2 of the launch probe: one record per convolution, in launch order, with the tile that ran; as K slices too, and
+    for the whole decoder and encoder as many as they have convolutions (the post-quant one is part of the input kernel)."""
+    import ctypes
+    from model_spec import vae_decode_convs, vae_encode_convs
+    L = hip.lib()
+    rows, wp, cin, cout = 20 * 18, 18, 64, 256
+    d, b = hip.DevBuf.from_array(np.zeros((rows + 2 * (wp + 2)) * cin, np.uint16)), hip.DevBuf.from_array(np.zeros(cout, np.float32))
+    w, out = hip.DevBuf.from_array(np.zeros((cout, 9 * cin), np.uint16)), hip.DevBuf(rows * cout * 4)
+    tiles, ms = np.full(256, -1, np.int32), np.zeros(256, np.float32)
+
+    def read():
+        return L.flux_hip_linear_probe_read_launches(256, tiles.ctypes.data, ms.ctypes.data)
+
+    try:
+        L.flux_hip_linear_probe(-2)
+        for tile, split, epi in ((1, 0, hip.EPI_CONV_F32), (2, 0, hip.EPI_CONV_BF16), (13, 2, hip.EPI_CONV_F32), (12, 0, hip.EPI_CONV_BF16), (3, 2, hip.EPI_CONV_BF16)):
+            L.flux_hip_linear_force_tile(tile)
+            L.flux_hip_linear_enable_splitk(split > 0)
+            L.flux_hip_linear_force_split(split)
+            hip.check(L.flux_hip_conv(epi, d.at((wp + 2) * cin * 2), w.ptr, b.ptr, None, out.ptr, rows, wp, cin, cout, 9))
+        assert read() == 5 and tiles[:5].tolist() == [1, 2, 13, 12, 3] and (ms[:5] > 0).all()
+        L.flux_hip_linear_force_tile(-1)
+        L.flux_hip_linear_enable_splitk(1)
+        L.flux_hip_linear_force_split(0)
+        v = hip.Vae(make_vae_weights())
+        for run, convs in ((lambda: v.decode(normal_f32((128, 4, 3), 301, 1), 4, 3), vae_decode_convs(4, 3)[1:]),
+                           (lambda: v.encode(vae_test_image(48, 64, 302)), vae_encode_convs(48, 64))):
+            L.flux_hip_linear_probe(-2)
+            run()
+            assert read() == len(convs)
+            L.flux_hip_linear_probe(hip.EPI_CONV_BF16)      # one epilogue alone
+            run()
+            assert 0 < read() < len(convs)
+        v.close()
+    finally:
+        L.flux_hip_linear_force_tile(-1)
+        L.flux_hip_linear_enable_splitk(1)
+        L.flux_hip_linear_force_split(0)
+        L.flux_hip_linear_probe(-1)
+
+
 def test_conv_of_an_image_without_interior(hip):
     """Two columns of border and nothing between them: the output is zeros."""
     d = hip.DevBuf.from_array(np.zeros(1 << 14, np.uint16))
