@@ -1851,6 +1851,20 @@ static int conv_finish(GemmArgs &g) {
     return 1;
 }
 
+/* Whether a convolution may run as K slices: they are a choice of speed, so a convolution never fails for want of their
+ * workspace, and under stream capture it takes none (the graph would keep the address of memory that a later call may
+ * free to grow it). In both cases it runs in one piece. */
+static bool conv_workspace(size_t bytes) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(flux_hip_stream_handle(), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (ensure_ws(bytes)) return true;
+    (void)hipGetLastError(); /* the next launch is not to report this one */
+    return false;
+}
+
 /* Tile and K split of a convolution by the same kind of model as gemm_dispatch's: rounds of workgroups, each a tile's time at
  * its measured rate plus the bytes of its epilogue at a compute unit's share of the memory rate (nothing overlaps those where one
  * workgroup owns the unit). K slices, which add a second pass and its partial sums, are what small images need: 32 x 32
@@ -1865,33 +1879,38 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
     const bool ring_ok = g_ring && (size_t)g.conv_rows * (g.conv_stride == 2 ? 4 : 1) * g.lda * 2 < ((size_t)1 << 32) && (size_t)N * g.ldw * 2 < ((size_t)1 << 32) &&
                          (size_t)g.conv_rows * N < ((size_t)1 << 32);
     int tile = -1, split = 1;
-    double best = 1e30;
-    for (int t = 0; t < CONV_TILES; t++) {
-        const bool ring = t == 2 || t >= 12;
-        if (!conv_bm[t] || N % conv_bn[t] || (forced && t != f)) continue;
-        if (t == 0 && !forced) continue; /* (for comparison runs) */
-        if (ring && (!ring_ok || kt_total < 4)) continue;
-        const long tiles = (long)((M + conv_bm[t] - 1) / conv_bm[t]) * (N / conv_bn[t]);
-        for (int sp : splits) {
-            const int per = (kt_total + sp - 1) / sp, used = (kt_total + per - 1) / per, last = kt_total - (used - 1) * per;
-            if (sp > 1 && (!g_splitk_enabled || per < 4 || last < 4 || used != sp || N % 64)) continue;
-            if (g_force_split && kt_total / g_force_split >= 4 && sp != g_force_split) continue;
-            const double ws = (double)sp * M * N * 4.0;
-            if (sp > 1 && ws > 256e6) continue;
-            const long blocks = tiles * sp, slots = 256L * occ[t], rounds = (blocks + slots - 1) / slots;
-            const long per_cu = (min(blocks, slots) + 255) / 256;
-            double est = rounds * (2.0 * conv_bm[t] * conv_bn[t] * 64.0 * per / (rate[t] / per_cu) + 2.5e-6 +
-                                   (double)conv_bm[t] * conv_bn[t] * (sp > 1 ? 0 : (epilogue == FLUX_HIP_EPI_CONV_BF16 ? 2 : 4) + (g.res ? 4 : 0)) / 2.0e10);
-            if (sp > 1) est += 4.0e-6 + 2.0 * ws / 4.0e12;
-            if (est < best) { best = est; tile = t; split = sp; }
+    const auto choose = [&](bool slices) {
+        double best = 1e30;
+        tile = -1;
+        split = 1;
+        for (int t = 0; t < CONV_TILES; t++) {
+            const bool ring = t == 2 || t >= 12;
+            if (!conv_bm[t] || N % conv_bn[t] || (forced && t != f)) continue;
+            if (t == 0 && !forced) continue; /* (for comparison runs) */
+            if (ring && (!ring_ok || kt_total < 4)) continue;
+            const long tiles = (long)((M + conv_bm[t] - 1) / conv_bm[t]) * (N / conv_bn[t]);
+            for (int sp : splits) {
+                const int per = (kt_total + sp - 1) / sp, used = (kt_total + per - 1) / per, last = kt_total - (used - 1) * per;
+                if (sp > 1 && (!slices || per < 4 || last < 4 || used != sp || N % 64)) continue;
+                if (slices && g_force_split && kt_total / g_force_split >= 4 && sp != g_force_split) continue;
+                const double ws = (double)sp * M * N * 4.0;
+                if (sp > 1 && ws > 256e6) continue;
+                const long blocks = tiles * sp, slots = 256L * occ[t], rounds = (blocks + slots - 1) / slots;
+                const long per_cu = (min(blocks, slots) + 255) / 256;
+                double est = rounds * (2.0 * conv_bm[t] * conv_bn[t] * 64.0 * per / (rate[t] / per_cu) + 2.5e-6 +
+                                       (double)conv_bm[t] * conv_bn[t] * (sp > 1 ? 0 : (epilogue == FLUX_HIP_EPI_CONV_BF16 ? 2 : 4) + (g.res ? 4 : 0)) / 2.0e10);
+                if (sp > 1) est += 4.0e-6 + 2.0 * ws / 4.0e12;
+                if (est < best) { best = est; tile = t; split = sp; }
+            }
         }
-    }
-    if (tile < 0) tile = N % 128 == 0 ? 1 : 3; /* (a forced ring tile that cannot run) */
+        if (tile < 0) tile = N % 128 == 0 ? 1 : 3; /* (a forced ring tile that cannot run) */
+    };
+    choose(g_splitk_enabled);
+    if (split > 1 && M > 0 && !conv_workspace((size_t)split * M * N * sizeof(float))) choose(false);
     g.kt_per = (kt_total + split - 1) / split;
     g.ksplit = M == 0 ? 0 : split; /* 0: nothing but border */
     const bool bf = epilogue == FLUX_HIP_EPI_CONV_BF16;
     if (g.ksplit > 1) {
-        if (!ensure_ws((size_t)split * M * N * sizeof(float))) return 0;
         g.ws = g_ws;
         g.ws_rows = M;
     }

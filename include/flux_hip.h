@@ -164,6 +164,9 @@ int flux_hip_linear_resid_adaln(int nparts, const flux_hip_linear_part *parts, i
  *   bias f32 [cout]; res f32 [rows, cout] or NULL (may be `out` itself); out [rows, cout]
  * Border positions of `out` are written as zeros, so it can feed the next convolution. wp = 0
  * (1x1 only) treats every row as interior. cin, cout: multiples of 64.
+ * Small images run as K slices, whose fp32 partial sums lie in flux_hip_linear's workspace (hipMalloc, kept and grown on
+ * demand). Where that cannot be had, and while the library's stream is being captured into a graph, the call runs in one
+ * piece and needs none: the same result up to fp32 summation order.
  */
 int flux_hip_conv(int epilogue, const void *in, const void *w, const float *bias, const float *res,
                   void *out, int rows, int wp, int cin, int cout, int taps);

@@ -232,6 +232,58 @@ def test_probe_records_every_convolution(hip):
         L.flux_hip_linear_probe(-1)
 
 
+def test_conv_under_graph_capture(hip):
+    """A convolution that runs as K slices otherwise (16 x 16 x 512) is captured in one piece: without a workspace of its own
+    making and without an address in the graph that a later call may free. Replayed three times between eager calls that
+    grow that workspace, each replay bit for bit the eager result in one piece, the statistics included."""
+    import ctypes
+    L = hip.lib()
+    rt = ctypes.CDLL("libamdhip64.so")
+    H, W, C = 16, 16, 512
+    rows, wp = (H + 2) * (W + 2), W + 2
+    din = Guarded(hip, to_padded(q(normal_f32((C, H, W), 59, 1))), wp)
+    dw = hip.DevBuf.from_array(conv_weight(q(normal_f32((C, C, 3, 3), 59, 2, 0.0, 0.05))))
+    db = hip.DevBuf.from_array(normal_f32((C,), 59, 3))
+    out, stats = hip.DevBuf(rows * C * 4), hip.DevBuf((rows // 32 + 2) * (C // 4) * 8)
+    n = ctypes.c_int(0)
+
+    def conv():
+        hip.check(L.flux_hip_conv_stats(hip.EPI_CONV_F32, din.ptr, dw.ptr, db.ptr, None, out.ptr, rows, wp, C, C, 9, stats.ptr, ctypes.byref(n)))
+
+    def result():
+        return out.to_array(np.float32, (rows, C)), stats.to_array(np.float32, (n.value, C // 4, 2))
+
+    conv()
+    sliced = result()
+    assert n.value == (rows + 31) // 32                      # K slices: the second pass's rows of sums
+    L.flux_hip_linear_enable_splitk(0)
+    conv()
+    L.flux_hip_linear_enable_splitk(1)
+    want = result()
+    assert n.value != (rows + 31) // 32 and rel_l2(sliced[0], want[0]) < 2e-6
+    hip.sync()
+    L.flux_hip_linear_release()                              # the capture finds no workspace
+    graph, execu, st = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p(L.flux_hip_stream())
+    assert rt.hipStreamBeginCapture(st, 2) == 0              # relaxed: only what the call itself does is looked at
+    ok = L.flux_hip_conv_stats(hip.EPI_CONV_F32, din.ptr, dw.ptr, db.ptr, None, out.ptr, rows, wp, C, C, 9, stats.ptr, ctypes.byref(n))
+    assert rt.hipStreamEndCapture(st, ctypes.byref(graph)) == 0 and ok == 1
+    assert rt.hipGraphInstantiate(ctypes.byref(execu), graph, None, None, 0) == 0
+    for slices in (3, 4, 6):
+        L.flux_hip_linear_force_split(slices)
+        conv()                                               # allocates, then grows the workspace
+        L.flux_hip_linear_force_split(0)
+        n.value = want[1].shape[0]
+        hip.check(L.flux_hip_memset(out.ptr, 0x55, rows * C * 4))
+        hip.sync()
+        assert rt.hipGraphLaunch(execu, st) == 0
+        hip.sync()
+        got = result()
+        np.testing.assert_array_equal(got[0], want[0])
+        np.testing.assert_array_equal(got[1], want[1])
+    rt.hipGraphExecDestroy(execu)
+    rt.hipGraphDestroy(graph)
+
+
 def test_conv_of_an_image_without_interior(hip):
     """Two columns of border and nothing between them: the output is zeros."""
     d = hip.DevBuf.from_array(np.zeros(1 << 14, np.uint16))
