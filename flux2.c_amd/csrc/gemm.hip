@@ -905,7 +905,7 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
         for (int i = 0; i < LB; i++) sc.voff[LA + i] = ((unsigned)weight_row<BN, WN, EPI>(g, tt.tn, lr + i * RPP) * (unsigned)g.ldw + chunk) * 2u;
     };
     /* where K step kt of an operand starts */
-    auto step_a = [&](const Src &sc, int kt) { return sc.baseA + (ptrdiff_t)a_step_offset<EPI>(g, sc.k0 + kt) * 2; };
+    auto step_a = [&](const Src &sc, int kt) { return sc.baseA + (IsConv<EPI>::value ? (ptrdiff_t)a_step_offset<EPI>(g, sc.k0 + kt) * 2 : (ptrdiff_t)kt * 128); };
     auto step_w = [&](const Src &sc, int kt) { return sc.baseW + (ptrdiff_t)kt * 128; };
     /* load i of the K step that starts at base: activation rows for i < LA (into slot sa
      * of their ring), weight rows after (slot sw). The offset passes through an empty asm statement where it is used: the
@@ -969,7 +969,13 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
                 const Src &sc = over ? nxt : cur;
                 return a ? step_a(sc, over ? ks - KT : ks) : step_w(sc, over ? ks - KT : ks);
             };
-            auto load = [&](const char *base, int ks, int sa, int sw, int i) {
+            /* A convolution's offset of a K step is a dozen scalar instructions, so the bases of the two K steps requested in
+             * this one are formed once. A projection forms the base at each load, from one byte offset for both operands:
+             * bases carried across the halves and an offset for each operand were four more scalar instructions per step. */
+            const char *first = nullptr, *second = nullptr;
+            if constexpr (IsConv<EPI>::value) first = start(kt + 2, FIRST_A), second = start(kt + NS2, !FIRST_A);
+            auto load = [&](const char *formed, int ks, int sa, int sw, int i) {
+                const char *base = IsConv<EPI>::value ? formed : start(ks, i < LA);
                 if (!TAIL) {
                     issue1(base, cur.voff[i], sa, sw, i);
                 } else {
@@ -977,7 +983,6 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
                     issue1(base, vo, sa, sw, i);
                 }
             };
-            const char *first = start(kt + 2, FIRST_A), *second = start(kt + NS2, !FIRST_A); /* the K steps requested in the two halves */
 #pragma unroll
             for (int b = 0; b < NM; b++) {
                 if (FIRST) MFMA_AGPR_NEW(accr[serp(b)][b / TN], f0[serp(b)], f0[TN + b / TN]);

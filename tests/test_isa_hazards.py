@@ -236,6 +236,26 @@ def test_gemm_kernels_fit_the_register_file(assembly):
             assert not copies, (name, copies[:4])
 
 
+def test_projection_k_loops_carry_no_second_address_chain(assembly):
+    """One K step of a projection in the ring kernel steps both operands along K by the same byte offset. Convolutions, which
+    share the loop, need a row offset of their own for the activations; when the projections' bases went through the same
+    expressions the 256-row tiles carried four scalar instructions more per step (53 instead of 49 on 256 x 256). The bound
+    is the 50 of 256 x 224, the loop's own bookkeeping included."""
+    seen = 0
+    for name, body in kernel_bodies(assembly["gemm.hip"][0]).items():
+        m = re.search(r"gemm4d_kernelILi(\d+)ELi(\d+)ELi(\d+)E", name)
+        if not m or int(m.group(3)) in (6, 7, 9):            # the convolution epilogues
+            continue
+        tm, tn = int(m.group(1)), int(m.group(2))
+        if tm != 8:
+            continue
+        loops = [(a, b) for a, b in innermost_loops(body) if sum("v_mfma" in l for l in body[a:b]) >= 2 * tm * tn]
+        scalars = min(sum(p[0].startswith("s_") for p in map(parse, body[a:b + 1]) if p) for a, b in loops)   # the steady loop; the tail's is longer
+        assert scalars <= 50, (name, scalars)
+        seen += 1
+    assert seen >= 20
+
+
 def test_the_loop_finder_sees_a_planted_copy():
     body = [".LBB0_1:", "\tv_mfma_f32_16x16x32_bf16 a[0:3], v[4:7], v[8:11], a[0:3]", ".LBB0_2:", "\tv_accvgpr_read_b32 v1, a9",
             "\tv_mfma_f32_16x16x32_bf16 a[0:3], v[4:7], v[8:11], a[0:3]", "\ts_cbranch_scc1 .LBB0_2", "\ts_cbranch_vccnz .LBB0_1", "\ts_endpgm"]
