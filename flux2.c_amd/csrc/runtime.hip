@@ -130,12 +130,17 @@ extern "C" int flux_hip_upload(void *dst, const void *src, size_t bytes) {
 }
 
 /* Memory that the caller has only just allocated gets its pages one by one at the first write to each, which for a result is
- * the copy at the end, with the device idle. Called between queueing the work and waiting for it: one write per page, while
- * the device computes. The contents are the result's to overwrite. */
+ * the copy at the end, with the device idle. Called between queueing the work and waiting for it: one write access per page, while
+ * the device computes. It replaces a zero by a zero and nothing else, so a call that fails afterwards leaves the buffer as it
+ * was (pages never written hold zeros). */
 extern "C" void flux_hip_prefault(void *dst, size_t bytes) {
-    volatile char *p = (volatile char *)dst;
-    for (size_t i = 0; i < bytes; i += 4096) p[i] = 0;
-    if (bytes) p[bytes - 1] = 0;
+    const auto touch = [](char *p) {
+        char zero = 0;
+        __atomic_compare_exchange_n(p, &zero, (char)0, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED);
+    };
+    char *p = (char *)dst;
+    for (size_t i = 0; i < bytes; i += 4096) touch(p + i);
+    if (bytes) touch(p + bytes - 1);
 }
 
 extern "C" int flux_hip_download(void *dst, const void *src, size_t bytes) {

@@ -47,6 +47,20 @@ def test_schedules_match_reference_golden(golden_dir):
         np.testing.assert_allclose(fluxhip.schedule("resolution", n, hh, ww), g[f"sched_resolution_{n}_{hh}_{ww}"], atol=6e-7)
 
 
+def test_touching_a_result_buffer_leaves_its_contents():
+    """The result's pages are touched while the device computes it; when the call fails afterwards the caller's buffer
+    holds what it held before. Sizes around a page, at offsets of every kind."""
+    f = fluxhip.lib().flux_hip_prefault
+    f.argtypes, f.restype = [ctypes.c_void_p, ctypes.c_size_t], None
+    want = np.random.default_rng(3).integers(0, 256, 1 << 17).astype(np.uint8)
+    want[::3] = 0
+    got = want.copy()
+    for offset in (0, 1, 4095, 4097):
+        for size in (0, 1, 2, 4095, 4096, 4097, 8192, 70001):
+            f(got[offset:].ctypes.data, size)
+    np.testing.assert_array_equal(got, want)
+
+
 def test_host_generator_matches_reference_golden(golden_dir):
     g = np.load(os.path.join(golden_dir, "ops.npz"))
     np.testing.assert_allclose(fluxhip.randn(64, seed=42), g["randn_42"], atol=1e-6)
