@@ -30,6 +30,17 @@ def hip():
     fluxhip.lib().flux_hip_linear_force_tile(-1)
 
 
+@pytest.fixture
+def switches(hip):
+    """The tile, slice and probe switches back at their defaults after a test that sets them."""
+    yield
+    L = hip.lib()
+    L.flux_hip_linear_force_tile(-1)
+    L.flux_hip_linear_enable_splitk(1)
+    L.flux_hip_linear_force_split(0)
+    L.flux_hip_linear_probe(-1)
+
+
 def q(x):
     return bf16_to_f32(f32_to_bf16(x))
 
@@ -70,11 +81,12 @@ def conv_weight(w):
     return f32_to_bf16(np.ascontiguousarray(w.reshape(co, ci // 64, 64, k * k).transpose(0, 1, 3, 2)).reshape(co, k * k * ci))
 
 
-@pytest.mark.parametrize("tile", [-1, 0, 1, 2, 3])
+@pytest.mark.parametrize("tile", [-1, 0, 1, 2, 3, 12, 13])
 @pytest.mark.parametrize("shape", [(9, 7, 64, 256), (5, 12, 128, 256), (20, 17, 256, 256), (6, 9, 192, 256)])
-def test_conv3x3(hip, oracle_mod, tile, shape):
+def test_conv3x3(hip, oracle_mod, switches, tile, shape):
     H, W, cin, cout = shape
     hip.lib().flux_hip_linear_force_tile(tile)
+    hip.lib().flux_hip_linear_enable_splitk(tile < 0)        # a forced tile stores its own results, not partial sums
     x = q(normal_f32((cin, H, W), 51, 1))
     w = q(normal_f32((cout, cin, 3, 3), 51, 2, 0.0, 0.05))
     b = normal_f32((cout,), 51, 3)
@@ -101,7 +113,6 @@ def test_conv3x3(hip, oracle_mod, tile, shape):
     got = bf16_to_f32(outb.to_array(np.uint16, (rows, cout)))
     assert border_is_zero(got, H, W)
     assert rel_l2(from_padded(got, H, W), want) < 4e-3
-    hip.lib().flux_hip_linear_force_tile(-1)
 
 
 def test_conv_output_widths(hip, oracle_mod):
@@ -141,13 +152,24 @@ def test_conv1x1(hip, oracle_mod):
     np.testing.assert_allclose(got[0], b, rtol=1e-6)
 
 
+CONV_BM = {0: 64, 1: 128, 2: 256, 3: 64, 12: 256, 13: 128}
+
+
+def slices_of(kt, split):
+    """Whether conv_launch cuts kt K steps into that many slices: four steps at least in each, the last one included."""
+    per = -(-kt // max(split, 1))
+    return split > 1 and kt // split >= 4 and -(-kt // per) == split and kt - (split - 1) * per >= 4
+
+
 @pytest.mark.parametrize("H,W,cin,cout", [(1, 1, 64, 256), (1, 40, 128, 256), (301, 1, 64, 256), (17, 31, 512, 256), (16, 16, 512, 512),
                                           (280, 281, 64, 128), (200, 190, 64, 256)])
-def test_conv_tiles_and_slices(hip, H, W, cin, cout):
-    """The ring tiles (2: 256 x 256, 12: 256 x 128, 13: 128 x 128) against the 128 x 128 one, which test_conv3x3 ties to the oracle: the same
-    K order, so the same bits, at images smaller than a tile, one pixel wide, with cut-off last tiles, and with more tiles
-    than compute units (280 x 281: 308 tiles). K slices regroup an fp32 sum of 9 cin products: at most cin * 9 roundings
-    of 2^-24 of the sum of magnitudes, in practice their root. The statistics are sums of what was written."""
+def test_conv_tiles_and_slices(hip, switches, H, W, cin, cout):
+    """Every tile in one piece (0: 64 x 128, 3: 64 x 64, ring tiles 2: 256 x 256, 12: 256 x 128, 13: 128 x 128) against the 128 x 128
+    one, which test_conv3x3 ties to the oracle: the same K order, so the same bits, at images smaller than a tile, one
+    pixel wide, with cut-off last tiles, and with more tiles than compute units (280 x 281: 308 tiles); with no residual,
+    one of its own and one in place, and as bf16. K slices regroup an fp32 sum of 9 cin products: at most cin * 9 roundings
+    of 2^-24 of the sum of magnitudes, in practice their root. The statistics are sums of what was written; their row count
+    tells whether slices ran."""
     import ctypes
     L = hip.lib()
     rows, wp = (H + 2) * (W + 2), W + 2
@@ -159,15 +181,17 @@ def test_conv_tiles_and_slices(hip, H, W, cin, cout):
     def run(tile, split, epi, r):
         L.flux_hip_linear_force_tile(tile)
         L.flux_hip_linear_force_split(split)
+        L.flux_hip_linear_enable_splitk(split > 0 or tile < 0)
         bf = epi == hip.EPI_CONV_BF16
-        out = hip.DevBuf.from_array(np.full((rows, cout), 3.0, np.float32))
+        out = hip.DevBuf.from_array(to_padded(res) if r == "in place" else np.full((rows, cout), 3.0, np.float32))
         stats = hip.DevBuf.from_array(np.full(((rows // 32 + 2) * (cout // 4) * 2,), np.nan, np.float32))
         n = ctypes.c_int(0)
-        try:
-            hip.check(L.flux_hip_conv_stats(epi, din.ptr, dw.ptr, db.ptr, r, out.ptr, rows, wp, cin, cout, 9, stats.ptr, ctypes.byref(n)))
-        finally:
-            L.flux_hip_linear_force_tile(-1)
-            L.flux_hip_linear_force_split(0)
+        hip.check(L.flux_hip_conv_stats(epi, din.ptr, dw.ptr, db.ptr, out.ptr if r == "in place" else r, out.ptr, rows, wp, cin, cout, 9, stats.ptr,
+                                        ctypes.byref(n)))
+        if tile >= 0 and split == 0:
+            assert n.value == 2 * -(-H * W // CONV_BM[tile])
+        elif slices_of(9 * cin // 64, split):
+            assert n.value == (rows + 31) // 32
         assert 0 < n.value <= rows // 32 + 2
         got = bf16_to_f32(out.to_array(np.uint16, (rows, cout))) if bf else out.to_array(np.float32, (rows, cout))
         assert border_is_zero(got, H, W)
@@ -178,19 +202,116 @@ def test_conv_tiles_and_slices(hip, H, W, cin, cout):
         np.testing.assert_allclose(st[:, 0], quads.sum((0, 2)), atol=tol * np.abs(quads).sum((0, 2)).max() + 1e-30)
         return got
 
-    for epi, r in ((hip.EPI_CONV_F32, None), (hip.EPI_CONV_F32, dres.ptr), (hip.EPI_CONV_BF16, None)):
-        want = run(1, 0, epi, r) if H * W >= 4096 else run(3, 0, epi, r)
-        for tile, split in ((12, 0), (13, 0), (2, 0), (12, 2), (2, 2), (13, 2), (13, 8), (1, 4), (-1, 0), (-1, 8)):
+    for epi, r in ((hip.EPI_CONV_F32, None), (hip.EPI_CONV_F32, dres.ptr), (hip.EPI_CONV_F32, "in place"), (hip.EPI_CONV_BF16, None)):
+        want = run(1, 0, epi, r)
+        for tile, split in ((0, 0), (3, 0), (12, 0), (13, 0), (2, 0), (12, 2), (2, 2), (13, 2), (13, 8), (1, 4), (3, 2), (-1, 0), (-1, 8)):
             if tile == 2 and cout % 256:
                 continue
             got = run(tile, split, epi, r)
-            if split == 0 and H * W >= 4096:
+            if split == 0 and tile >= 0:
                 np.testing.assert_array_equal(got, want)
             else:
                 assert rel_l2(got, want) < (2.0 ** -9 if epi == hip.EPI_CONV_BF16 else 2e-6)
 
 
-def test_probe_records_every_convolution(hip):
+CONV_FORMS = [(tile, split) for tile in (1, 2, 3, 12, 13) for split in (0, 2)] + [(-1, 0)]
+
+
+def conv_image(hip, tile, split, epi, in_ptr, in_wp, packed, dw, db, res, out_ptr, rows, wp, cin, cout, taps):
+    """flux_hip_conv_image on one tile, in one piece or as K slices; the probe says that this is what ran. Returns the
+    statistics unless the output is packed."""
+    import ctypes
+    L = hip.lib()
+    vp, ci = ctypes.c_void_p, ctypes.c_int
+    L.flux_hip_conv_image.argtypes = [ci, vp, ci, ci, vp, vp, vp, vp, ci, ci, ci, ci, ci, vp, vp]
+    L.flux_hip_linear_force_tile(tile)
+    L.flux_hip_linear_force_split(split)
+    L.flux_hip_linear_enable_splitk(split > 0 or tile < 0)
+    L.flux_hip_linear_probe(-2)
+    n = ci(0)
+    stats = None if packed & 2 else hip.DevBuf.from_array(np.full(((rows // 32 + 2) * (cout // 4) * 2,), np.nan, np.float32))
+    hip.check(L.flux_hip_conv_image(epi, in_ptr, in_wp, packed, dw.ptr, db.ptr, res, out_ptr, rows, wp, cin, cout, taps, stats.ptr if stats else None,
+                                    ctypes.byref(n) if stats else None))
+    ran = np.zeros(4, np.int32)
+    assert L.flux_hip_linear_probe_read_launches(4, ran.ctypes.data, None) == 1 and tile in (-1, ran[0])
+    if stats is None:
+        return None
+    interior = (rows // wp - 2) * (wp - 2)
+    assert tile < 0 or n.value == (2 * -(-interior // CONV_BM[tile]) if split == 0 else (rows + 31) // 32)
+    return stats.to_array(np.float32, (n.value, cout // 4, 2)).astype(np.float64).sum(0)
+
+
+def check_sums(stats, written):
+    quads = written.astype(np.float64).reshape(-1, stats.shape[0], 4)
+    np.testing.assert_allclose(stats[:, 1], (quads ** 2).sum((0, 2)), rtol=2.0 ** -7)     # (of the unrounded values where bf16 was written)
+    np.testing.assert_allclose(stats[:, 0], quads.sum((0, 2)), atol=2.0 ** -8 * np.abs(quads).sum((0, 2)).max() + 1e-30)
+
+
+@pytest.mark.parametrize("tile,split", CONV_FORMS)
+@pytest.mark.parametrize("C,H,W", [(64, 2, 2), (128, 8, 6), (64, 2, 74), (128, 62, 2), (128, 34, 66)])
+def test_conv_with_stride_2(hip, oracle_mod, switches, tile, split, C, H, W):
+    """The encoder's downsampling convolution from the bordered full-size image: against the oracle's, odd halves and single
+    rows and columns among them; nothing outside the bordered image is read (its buffer ends with it)."""
+    cout, H2, W2 = 256, H // 2, W // 2
+    x, w = q(normal_f32((C, H, W), 62, 1)), q(normal_f32((cout, C, 3, 3), 62, 2, 0.0, 0.05))
+    b = normal_f32((cout,), 62, 3)
+    rows, wp = (H2 + 2) * (W2 + 2), W2 + 2
+    din, dw, db = hip.DevBuf.from_array(f32_to_bf16(to_padded(x))), hip.DevBuf.from_array(conv_weight(w)), hip.DevBuf.from_array(b)
+    out = hip.DevBuf.from_array(np.full((rows + 1, cout), 3.0, np.float32))
+    st = conv_image(hip, tile, split, hip.EPI_CONV_F32, din.ptr, W + 2, 0, dw, db, None, out.ptr, rows, wp, C, cout, 9)
+    got = out.to_array(np.float32, (rows + 1, cout))
+    assert (got[rows] == 3.0).all() and border_is_zero(got[:rows], H2, W2)
+    assert rel_l2(from_padded(got[:rows], H2, W2), oracle_mod.conv2d_down(x, w, b)) < 2e-6
+    check_sums(st, got[:rows])
+
+
+@pytest.mark.parametrize("tile,split", CONV_FORMS)
+@pytest.mark.parametrize("H,W", [(1, 1), (3, 50), (19, 23)])
+def test_conv_to_bf16_with_residual(hip, oracle_mod, switches, tile, split, H, W):
+    """The last convolution of a level: fp32 residual in, bf16 out, one rounding."""
+    cin, cout = 128, 256
+    x, w = q(normal_f32((cin, H, W), 64, 1)), q(normal_f32((cout, cin, 3, 3), 64, 2, 0.0, 0.05))
+    b, res = normal_f32((cout,), 64, 3), normal_f32((cout, H, W), 64, 4)
+    rows, wp = (H + 2) * (W + 2), W + 2
+    din, dw, db = Guarded(hip, to_padded(x), wp), hip.DevBuf.from_array(conv_weight(w)), hip.DevBuf.from_array(b)
+    dres = hip.DevBuf.from_array(to_padded(res))
+    out = hip.DevBuf.from_array(np.full((rows + 1, cout), 0x4040, np.uint16))
+    st = conv_image(hip, tile, split, hip.EPI_CONV_BF16, din.ptr, 0, 0, dw, db, dres.ptr, out.ptr, rows, wp, cin, cout, 9)
+    bits = out.to_array(np.uint16, (rows + 1, cout))
+    got = bf16_to_f32(bits[:rows])
+    assert (bits[rows] == 0x4040).all() and border_is_zero(got, H, W)
+    want = oracle_mod.conv2d(x, w, b, 1) + res
+    assert rel_l2(from_padded(got, H, W), want) < 2.0 ** -8
+    assert np.abs(from_padded(got, H, W) - want).max() <= 2.0 ** -8 * np.abs(want).max()
+    check_sums(st, got)
+
+
+@pytest.mark.parametrize("tile,split", CONV_FORMS)
+@pytest.mark.parametrize("H,W", [(1, 1), (1, 70), (19, 23)])
+def test_conv1x1_with_packed_sides(hip, oracle_mod, switches, tile, split, H, W):
+    """The convolutions around the attention, between a bordered image and its H * W interior positions alone: bordered -> packed
+    bf16, and packed -> bordered fp32 with the residual in place."""
+    cin, cout = 512, 512
+    x, w = q(normal_f32((cin, H, W), 65, 1)), q(normal_f32((cout, cin, 1, 1), 65, 2, 0.0, 0.05))
+    b, res = normal_f32((cout,), 65, 3), normal_f32((cout, H, W), 65, 4)
+    rows, wp, n = (H + 2) * (W + 2), W + 2, H * W
+    want = oracle_mod.conv2d(x, w, b, 0)
+    dw, db = hip.DevBuf.from_array(conv_weight(w)), hip.DevBuf.from_array(b)
+    bordered, packed = hip.DevBuf.from_array(f32_to_bf16(to_padded(x))), hip.DevBuf.from_array(f32_to_bf16(x.transpose(1, 2, 0).reshape(n, cin)))
+    out = hip.DevBuf.from_array(np.full((n + 1, cout), 0x4040, np.uint16))
+    conv_image(hip, tile, split, hip.EPI_CONV_BF16, bordered.ptr, 0, 2, dw, db, None, out.ptr, rows, wp, cin, cout, 1)
+    bits = out.to_array(np.uint16, (n + 1, cout))
+    assert (bits[n] == 0x4040).all()
+    assert rel_l2(bf16_to_f32(bits[:n]), want.reshape(cout, n).T) < 2.0 ** -8
+    img = hip.DevBuf.from_array(np.concatenate([to_padded(res), np.full((1, cout), 3.0, np.float32)]))
+    st = conv_image(hip, tile, split, hip.EPI_CONV_F32, packed.ptr, 0, 1, dw, db, img.ptr, img.ptr, rows, wp, cin, cout, 1)
+    got = img.to_array(np.float32, (rows + 1, cout))
+    assert (got[rows] == 3.0).all() and border_is_zero(got[:rows], H, W)
+    assert rel_l2(from_padded(got[:rows], H, W), want + res) < 2e-6
+    check_sums(st, got[:rows])
+
+
+def test_probe_records_every_convolution(hip, switches):
     """Mode -2 of the launch probe: one record per convolution, in launch order, with the tile that ran; as K slices too, and
     for the whole decoder and encoder as many as they have convolutions (the post-quant one is part of the input kernel)."""
     import ctypes
@@ -204,35 +325,29 @@ def test_probe_records_every_convolution(hip):
     def read():
         return L.flux_hip_linear_probe_read_launches(256, tiles.ctypes.data, ms.ctypes.data)
 
-    try:
+    L.flux_hip_linear_probe(-2)
+    for tile, split, epi in ((1, 0, hip.EPI_CONV_F32), (2, 0, hip.EPI_CONV_BF16), (13, 2, hip.EPI_CONV_F32), (12, 0, hip.EPI_CONV_BF16), (3, 2, hip.EPI_CONV_BF16)):
+        L.flux_hip_linear_force_tile(tile)
+        L.flux_hip_linear_enable_splitk(split > 0)
+        L.flux_hip_linear_force_split(split)
+        hip.check(L.flux_hip_conv(epi, d.at((wp + 2) * cin * 2), w.ptr, b.ptr, None, out.ptr, rows, wp, cin, cout, 9))
+    assert read() == 5 and tiles[:5].tolist() == [1, 2, 13, 12, 3] and (ms[:5] > 0).all()
+    L.flux_hip_linear_force_tile(-1)
+    L.flux_hip_linear_enable_splitk(1)
+    L.flux_hip_linear_force_split(0)
+    v = hip.Vae(make_vae_weights())
+    for run, convs in ((lambda: v.decode(normal_f32((128, 4, 3), 301, 1), 4, 3), vae_decode_convs(4, 3)[1:]),
+                       (lambda: v.encode(vae_test_image(48, 64, 302)), vae_encode_convs(48, 64))):
         L.flux_hip_linear_probe(-2)
-        for tile, split, epi in ((1, 0, hip.EPI_CONV_F32), (2, 0, hip.EPI_CONV_BF16), (13, 2, hip.EPI_CONV_F32), (12, 0, hip.EPI_CONV_BF16), (3, 2, hip.EPI_CONV_BF16)):
-            L.flux_hip_linear_force_tile(tile)
-            L.flux_hip_linear_enable_splitk(split > 0)
-            L.flux_hip_linear_force_split(split)
-            hip.check(L.flux_hip_conv(epi, d.at((wp + 2) * cin * 2), w.ptr, b.ptr, None, out.ptr, rows, wp, cin, cout, 9))
-        assert read() == 5 and tiles[:5].tolist() == [1, 2, 13, 12, 3] and (ms[:5] > 0).all()
-        L.flux_hip_linear_force_tile(-1)
-        L.flux_hip_linear_enable_splitk(1)
-        L.flux_hip_linear_force_split(0)
-        v = hip.Vae(make_vae_weights())
-        for run, convs in ((lambda: v.decode(normal_f32((128, 4, 3), 301, 1), 4, 3), vae_decode_convs(4, 3)[1:]),
-                           (lambda: v.encode(vae_test_image(48, 64, 302)), vae_encode_convs(48, 64))):
-            L.flux_hip_linear_probe(-2)
-            run()
-            assert read() == len(convs)
-            L.flux_hip_linear_probe(hip.EPI_CONV_BF16)      # one epilogue alone
-            run()
-            assert 0 < read() < len(convs)
-        v.close()
-    finally:
-        L.flux_hip_linear_force_tile(-1)
-        L.flux_hip_linear_enable_splitk(1)
-        L.flux_hip_linear_force_split(0)
-        L.flux_hip_linear_probe(-1)
+        run()
+        assert read() == len(convs)
+        L.flux_hip_linear_probe(hip.EPI_CONV_BF16)      # one epilogue alone
+        run()
+        assert 0 < read() < len(convs)
+    v.close()
 
 
-def test_conv_under_graph_capture(hip):
+def test_conv_under_graph_capture(hip, switches):
     """A convolution that runs as K slices otherwise (16 x 16 x 512) is captured in one piece: without a workspace of its own
     making and without an address in the graph that a later call may free. Replayed three times between eager calls that
     grow that workspace, each replay bit for bit the eager result in one piece, the statistics included."""
@@ -328,14 +443,15 @@ def test_group_norm(hip, oracle_mod, C, swish, in_bf16):
     np.testing.assert_array_equal(raw.to_array(np.uint16, (rows, C)), f32_to_bf16(to_padded(x)))
 
 
-@pytest.mark.parametrize("tile", [-1, 0, 1, 2, 3])
+@pytest.mark.parametrize("tile", [-1, 0, 1, 2, 3, 12, 13])
 @pytest.mark.parametrize("epi_bf16", [0, 1])
-def test_group_norm_from_convolution_statistics(hip, oracle_mod, tile, epi_bf16):
+def test_group_norm_from_convolution_statistics(hip, oracle_mod, switches, tile, epi_bf16):
     """The convolution epilogue leaves the sums of what it wrote; the group norm that takes them must give
     what the group norm that computes its own sums gives, and what the oracle gives."""
     import ctypes
     H, W, cin, cout = 21, 18, 128, 256
     hip.lib().flux_hip_linear_force_tile(tile)
+    hip.lib().flux_hip_linear_enable_splitk(tile < 0)        # the sums of the tile's own epilogue, not of the K slices' second pass
     x = q(normal_f32((cin, H, W), 57, 1))
     w = q(normal_f32((cout, cin, 3, 3), 57, 2, 0.0, 0.05))
     b = normal_f32((cout,), 57, 3)
@@ -350,7 +466,8 @@ def test_group_norm_from_convolution_statistics(hip, oracle_mod, tile, epi_bf16)
     nrows = ctypes.c_int(0)
     hip.check(hip.lib().flux_hip_conv_stats(hip.EPI_CONV_BF16 if epi_bf16 else hip.EPI_CONV_F32, din.ptr, dw.ptr, db.ptr,
                                             None if epi_bf16 else out.ptr, out.ptr, rows, wp, cin, cout, 9, stats.ptr, ctypes.byref(nrows)))
-    assert 0 < nrows.value <= rows // 32 + 2
+    bm = CONV_BM.get(tile)
+    assert 0 < nrows.value <= rows // 32 + 2 and (bm is None or nrows.value == 2 * -(-H * W // bm))
     st = stats.to_array(np.float32, (nrows.value, cout // 4, 2))
     assert np.isfinite(st).all()                       # every slot was written
     scratch = hip.DevBuf(hip.lib().flux_hip_group_norm_scratch_floats(H + 2, W + 2) * 4)
@@ -365,7 +482,6 @@ def test_group_norm_from_convolution_statistics(hip, oracle_mod, tile, epi_bf16)
     conv = oracle_mod.conv2d(x, w, b, 1) + (0 if res is None else res)
     want = oracle_mod.silu(oracle_mod.group_norm(conv, gm, bt, 32, 1e-4))
     assert rel_l2(from_padded(a1, H, W), want) < 6e-3
-    hip.lib().flux_hip_linear_force_tile(-1)
 
 
 @pytest.mark.parametrize("prows,C", [(1, 128), (5, 256), (37, 512), (63, 512), (2048, 128), (2049, 128), (4100, 256)])
@@ -402,6 +518,23 @@ def test_upsample(hip, oracle_mod):
     got = bf16_to_f32(out.to_array(np.uint16, (rows2, C)))
     assert border_is_zero(got, 2 * H, 2 * W)
     np.testing.assert_array_equal(from_padded(got, 2 * H, 2 * W), q(oracle_mod.upsample_nearest(x)))
+
+
+@pytest.mark.parametrize("C,H,W", [(8, 1, 1), (512, 5, 7), (256, 16, 9)])
+def test_upsample_from_bf16(hip, C, H, W):
+    """The form that reads a bf16 image, against the fp32 one on values that bf16 holds: the same bits, nothing behind them."""
+    import ctypes
+    x = q(normal_f32((C, H, W), 55, 2))
+    rows2 = (2 * H + 2) * (2 * W + 2)
+    got = []
+    f = hip.lib().flux_hip_vae_upsample2x_bf16
+    f.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int]
+    for run, src in ((hip.lib().flux_hip_upsample2x, to_padded(x)), (f, f32_to_bf16(to_padded(x)))):
+        out, d = hip.DevBuf.from_array(np.full((rows2 + 1, C), 0x4040, np.uint16)), hip.DevBuf.from_array(src)
+        hip.check(run(out.ptr, d.ptr, H + 2, W + 2, C))
+        got.append(out.to_array(np.uint16, (rows2 + 1, C)))
+    np.testing.assert_array_equal(got[0], got[1])
+    assert (got[1][rows2] == 0x4040).all() and border_is_zero(got[1][:rows2], 2 * H, 2 * W)
 
 
 @pytest.mark.parametrize("shape", [(37, 384, 300), (3, 17024, 16900), (3, 20608, 20500)])
