@@ -355,7 +355,7 @@ void flux_hip_vae_free(flux_hip_vae *v) {
 }
 
 /* Test hook: upper bound on the query rows per attention chunk (0 = the buffer's own bound,
- * 2 GB of fp32 scores). */
+ * 1 GB of fp32 scores). */
 static int g_att_chunk_limit = 0;
 void flux_hip_vae_set_attention_chunk(int rows) { g_att_chunk_limit = rows > 0 ? rows : 0; }
 
@@ -369,7 +369,7 @@ static int ensure_work(flux_hip_vae *v, int h, int w) {
     size_t f32_elems = mp0 * 256, guard = (wp0 + 2) * 512;
     size_t bf16_elems = mp0 * 256;
     if (bf16_elems < ld * 1536) bf16_elems = ld * 1536; /* R also holds q, k, v of the attention */
-    size_t chunk = ((size_t)1 << 29) / ld;               /* at most 2 GB of fp32 scores at a time: a 1024x1024 picture's in one piece */
+    size_t chunk = ((size_t)1 << 28) / ld; /* at most 1 GB of fp32 scores at a time: a picture of 1024x1024 is one piece, 1792x1792 ten, which take what five of 2 GB do (51.1 ms a decode) */
     if (chunk < 128) chunk = 128;
     if (chunk > mpm) chunk = mpm;
     const size_t gn_floats = flux_hip_group_norm_scratch_floats((int)hp0, (int)wp0);

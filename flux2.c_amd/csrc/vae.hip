@@ -401,7 +401,7 @@ __global__ __launch_bounds__(256) void vae_softmax_kernel(bf16 *__restrict__ P, 
     }
 }
 
-/* The same for rows of up to 1024 * SOFTMAX_REG_V4 * 4 columns (1024x1024 images have 17024), with
+/* The same for rows of up to 1024 * SOFTMAX_REG_V4 * 4 columns (1024x1024 images have 16384), with
  * the row held in registers between the three steps: S is read once. */
 #define SOFTMAX_REG_V4 20
 __global__ __launch_bounds__(256) void vae_softmax_reg_kernel(bf16 *__restrict__ P, const float *__restrict__ S, const float *__restrict__ key_bias,

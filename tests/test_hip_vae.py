@@ -611,11 +611,11 @@ def test_vae_decode_smaller_after_larger(vae_pair):
 
 def test_vae_attention_in_chunks(hip, vae_pair):
     """The mid-block attention walks its queries in chunks when the score matrix would not fit its buffer
-    (1024x1024 and up); forced here at a small size: same image as in one piece."""
+    (beyond 1024x1024); forced here at a small size: same image as in one piece."""
     dev, cpu = vae_pair
     lat = normal_f32((128, 6, 5), 307, 1)
     f0, u0 = dev.decode(lat, 6, 5)
-    hip.lib().flux_hip_vae_set_attention_chunk(37)          # 12 * 14 = 168 positions -> 5 chunks, the last one ragged
+    hip.lib().flux_hip_vae_set_attention_chunk(37)          # 10 * 12 = 120 positions -> 4 chunks, the last one ragged
     try:
         f1, u1 = dev.decode(lat, 6, 5)
     finally:
@@ -628,8 +628,7 @@ def test_vae_attention_in_chunks(hip, vae_pair):
 @pytest.mark.parametrize("side", [32, pytest.param(64, marks=pytest.mark.skipif(not os.environ.get("FLUX_SLOW"), reason=(
     "the 1024x1024 decode takes the CPU oracle half a minute; the 512x512 case chooses the same kernels; set FLUX_SLOW=1")))])
 def test_vae_decode_large(vae_pair, side):
-    """Full-size decodes (512x512, 1024x1024: the 256x256 convolution tile and the chunked attention are
-    only chosen there) against the oracle."""
+    """Full-size decodes (512x512, 1024x1024: the 256x256 convolution tile is only chosen there) against the oracle."""
     dev, cpu = vae_pair
     lat = normal_f32((128, side, side), 308, 1)
     f, u = dev.decode(lat, side, side)
@@ -726,7 +725,7 @@ def test_vae_encode_after_decode(vae_pair):
 
 @pytest.mark.parametrize("side", [512, 1024])
 def test_vae_encode_large(vae_pair, side):
-    """Full-size encodes against the oracle (chunked attention at 1024; about half a minute of CPU work on 16 cores)."""
+    """Full-size encodes against the oracle (about half a minute of CPU work on 16 cores)."""
     dev, cpu = vae_pair
     img = vae_test_image(side, side, 317)
     got, want = dev.encode(img), cpu.encode(img)
@@ -735,10 +734,10 @@ def test_vae_encode_large(vae_pair, side):
     assert r <= 2e-2
 
 
-def test_vae_maximum_sizes(vae_pair):
+def test_vae_maximum_sizes(hip, vae_pair):
     """The largest images the reference accepts (1792 pixels a side, flux.h:52), where the oracle would take
-    many minutes: size-independent properties only. The row softmax takes its three-pass form here (51200
-    score columns), the attention runs in 12 chunks."""
+    many minutes: size-independent properties only. The row softmax takes its three-pass form here (48896 and 49920
+    score columns), the attention runs in 9 and 10 chunks by its own bound, and gives the same image in others."""
     dev, _ = vae_pair
     lat = normal_f32((128, 112, 109), 320, 1)
     f, u = dev.decode(lat, 112, 109)
@@ -746,6 +745,14 @@ def test_vae_maximum_sizes(vae_pair):
     assert f.shape == (3, 1792, 1744) and np.isfinite(f).all() and u.std() > 20.0
     np.testing.assert_array_equal(u, u2)
     np.testing.assert_array_equal(f, f2)
+    try:
+        hip.lib().flux_hip_linear_enable_splitk(0)           # (every tile sums K in one order, K slices depend on the chunk's height)
+        f3, _ = dev.decode(lat, 112, 109)
+        hip.lib().flux_hip_vae_set_attention_chunk(3000)
+        np.testing.assert_array_equal(dev.decode(lat, 112, 109)[0], f3)
+    finally:
+        hip.lib().flux_hip_linear_enable_splitk(1)
+        hip.lib().flux_hip_vae_set_attention_chunk(0)
     img = vae_test_image(1792, 1776, 321)
     z = dev.encode(img)
     assert z.shape == (128, 112, 111) and np.isfinite(z).all() and 0.2 < z.std() < 2.0
@@ -753,6 +760,25 @@ def test_vae_maximum_sizes(vae_pair):
     # and a small one afterwards, on the same (now large) work buffers, still agrees with the oracle
     small = normal_f32((128, 2, 3), 304, 1)
     assert rel_l2(dev.decode(small, 2, 3)[0], vae_pair[1].decode(small, 2, 3)[0]) <= 2e-2
+
+
+def test_vae_scratch_at_the_maximum(hip):
+    """What the largest decode holds on the device beside the weights: three fp32 and two bf16 images of 1794 x 1794 x 256 (9.89
+    and 3.30 GB), 1 GiB of scores and half of that of probabilities, 0.3 GB of everything else."""
+    import ctypes
+    rt = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        f, t = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert rt.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    v = hip.Vae(make_vae_weights())
+    v.decode(normal_f32((128, 2, 2), 301, 1), 2, 2)
+    before = free()
+    v.decode(normal_f32((128, 112, 112), 322, 1), 112, 112)
+    assert before - free() < (3 * 4 + 2 * 2) * 1794 ** 2 * 256 + 1.5 * 2 ** 30 + 0.5e9
+    v.close()
 
 
 def test_vae_encode_errors(hip, vae_pair):
