@@ -1648,10 +1648,16 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
                 double bw = 5.5e12 * (double)(resident * ahead[t] * (bm[t] + bn[t]) * 128) / 12.0e6;
                 if (bw > bw_cap) bw = bw_cap;
                 double est = t_compute > bytes / bw ? t_compute : bytes / bw;
-                /* what all tiles together fetch through the L2s: seen at 10 to 13 TB/s (14996 x 512 x 15104 on 236 tiles of 256 x 128:
-                 * 2.7 GB, 238 us; on 118 of 256 x 256 in two K slices 1.8 GB, 176 us; 4608 x 3072 x 12288 on 256 tiles of 288 x 192:
-                 * 3.0 GB, 231 us, which with 12.5 TB/s here lost to 256 x 224 in the model and was 10 us faster than it) */
-                const double l2 = (double)tiles * (bm[t] + bn[t]) * K * 2.0 / 12.9e12;
+                /* What all tiles together fetch through the L2s, over the rate at which that ties the tiles with fewer bytes to those with
+                 * fewer rounds (no hard limit: 128 x 128 tiles whose activations the memory-side cache held have been seen at 16 TB/s).
+                 * In the step, over 26 token counts from 219 to 10709, six prompt lengths and 20 image sizes, 12.9 TB/s
+                 * kept tiles with too few rounds' worth of them: out1 at 5993 rows 406 us on 256 x 192 in two slices, 342 on 192 x 192
+                 * (a step 1.9 % longer), 270 prompt tokens 3 % longer, P V of 5332 positions 58 us against 47. 14.5 and
+                 * none send 790 to 1300 tokens to 128 x 128 and 192 x 192, 1.2 to 3 % longer. Activations beyond the 256 MB of the
+                 * memory-side cache come from HBM and the rate is lower: P V of 14580 positions 220 us on 256 x 128, which
+                 * 13.5 chooses, and 183 on 256 x 256 in two slices. */
+                const double l2_rate = rows * K * 2.0 > 256.0e6 ? 12.9e12 : 13.5e12;
+                const double l2 = (double)tiles * (bm[t] + bn[t]) * K * 2.0 / l2_rate;
                 if (l2 > est) est = l2;
                 if (sp > 1) est += 3.0e-6 + (sp + 2.0) * rows * N * 4.0 / 4.0e12;
                 else if (adaln) est += 3.0e-6 + rows * N * 6.0 / 4.0e12; /* the norm that the second pass would have taken along */

@@ -188,6 +188,27 @@ def test_linear_small_ring_tiles(hip, oracle_mod, tile, M0, M1, N, K):
         assert rel_l2(bf16_to_f32(ref) if dtype == np.uint16 else ref, want) < (4e-3 if dtype == np.uint16 else 2e-6), epi
 
 
+@pytest.mark.parametrize("M,N,K,epi,tile", [(5993, 3072, 12288, "resid", 6), (270, 2560, 9728, "resid", 13), (5332, 512, 5376, "bf16", 12),
+                                            (14580, 512, 14592, "bf16", 2)])
+def test_linear_choice_where_the_l2_rate_decides(hip, M, N, K, epi, tile):
+    """Tiles chosen where two candidates of the cost model differ by what they fetch through the L2s, measured both ways: 5993 rows
+    on 192 x 192 342 us (256 x 192: 406), 270 rows on 128 x 128 31 (192 x 256: 35), 5332 on 256 x 128 47 (128 x 128: 58),
+    14580, whose activations come from HBM, on 256 x 256 183 (256 x 128: 220)."""
+    L = hip.lib()
+    a, w, c, g = hip.DevBuf(M * K * 2), hip.DevBuf(N * K * 2), hip.DevBuf(M * N * 4), hip.DevBuf.from_array(np.ones(N, np.float32))
+    for b in (a, w, c):
+        hip.check(L.flux_hip_memset(b.ptr, 0, b.nbytes))
+    e = hip.EPI_RESID if epi == "resid" else hip.EPI_BF16
+    ran = np.zeros(1, np.int32)
+    L.flux_hip_linear_probe(e)
+    try:
+        hip.linear(e, [(a.ptr, w.ptr, c.ptr, g.ptr, M)], N, K, K, K, N)
+        assert L.flux_hip_linear_probe_read_launches(1, ran.ctypes.data, None) == 1
+    finally:
+        L.flux_hip_linear_probe(-1)
+    assert ran[0] == tile
+
+
 @pytest.mark.parametrize("epi,N", [("resid", 3072), ("bf16", 9216)])
 def test_linear_cut_tile_at_the_double_stream_shapes(hip, epi, N):
     """256 x 224 where the model uses it: 4096 image + 512 text rows with weights of their own, K = 3072, the gated residual
