@@ -1584,8 +1584,10 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
      * many rows), 11 = 256 x 224 (4096 + 512 rows x 3072 columns are 252 such tiles, one round of workgroups on 256
      * compute units of which each does 7/8 of a 256 x 256 tile's work; 216 tiles of 256 x 256 are one round as well),
      * 12 = 256 x 128, 13 = 128 x 128 and 14 = 192 x 256 in the ring kernel, for launches of about one round: the two-stage 128 x 128
-     * tile waits for memory in every K step when it has a compute unit to itself (512 x 6144 x 2560: 31 us, in the ring 21;
-     * 1202 x 3072 x 3072: 40 and 28; 512 x 19456 x 2560 on 228 tiles of 192 x 256 51, on 152 of 256 x 256 59) */
+     * tile waits for memory in every K step when it has a compute unit to itself. With the weights coming from HBM, as in a
+     * forward: 512 x 6144 x 2560 39 us, in the ring 30; 1202 x 3072 x 3072: 49 and 34; 512 x 19456 x 2560 on 228 tiles of 192 x 256 52,
+     * on 152 of 256 x 256 60. (The rates of 12 to 14 below are those of cached operands and up to 40 % above these launches; over
+     * 133 shapes of 67 to 16384 rows with cold weights the chosen form took 0.8 % more than the best of seven on average.) */
     constexpr int NT = 15;
     static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 64, 128, 96, 256, 256, 128, 192}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 128, 128, 128, 224, 128, 128, 256};
     static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, ahead[NT] = {1, 1, 1, 1, 1, 1, 1, 1, 5, 4, 4, 1, 1, 1, 1}; /* stages a workgroup keeps in flight */
@@ -1879,7 +1881,7 @@ static bool conv_workspace(size_t bytes) {
 /* Tile and K split of a convolution by the same kind of model as gemm_dispatch's: rounds of workgroups, each a tile's time at
  * its measured rate plus the bytes of its epilogue at a compute unit's share of the memory rate (nothing overlaps those where one
  * workgroup owns the unit). K slices, which add a second pass and its partial sums, are what small images need: 32 x 32
- * positions x 512 channels are 32 tiles of 128 x 128 for 256 units, 57 us in one piece and 24 in slices; at 96 x 96 positions
+ * positions x 512 channels are 32 tiles of 128 x 128 for 256 units, 57 us in one piece and 24 in slices (27 in a decode); at 96 x 96 positions
  * one piece wins (54 us against 69). */
 static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
     static const int occ[CONV_TILES] = {3, 2, 1, 4, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1};
