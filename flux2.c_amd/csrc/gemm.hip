@@ -1661,7 +1661,11 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
                 const double l2_rate = rows * K * 2.0 > 256.0e6 ? 12.9e12 : 13.5e12;
                 const double l2 = (double)tiles * (bm[t] + bn[t]) * K * 2.0 / l2_rate;
                 if (l2 > est) est = l2;
-                if (sp > 1) est += 3.0e-6 + (sp + 2.0) * rows * N * 4.0 / 4.0e12;
+                /* Slices cost their partial sums, and beyond 128 MB of those the stores of every round as well: the K = 12288 projection at
+                 * 6148 to 6912 rows (151 to 170 MB) in two slices of 288 x 192 takes 379 + 78 us, in one piece of 256 x 192 430 and
+                 * 27 for the norm, and the step around it is 0.5 to 1.2 % longer; at 2132 to 2560 rows (52 to 63 MB) two slices
+                 * make it 1 % shorter. */
+                if (sp > 1) est += 3.0e-6 + (sp + 2.0) * rows * N * 4.0 / (sp * rows * N * 4.0 > 128.0e6 ? 2.6e12 : 4.0e12);
                 else if (adaln) est += 3.0e-6 + rows * N * 6.0 / 4.0e12; /* the norm that the second pass would have taken along */
                 if (est < best) { best = est; tile = t; best_split = sp; }
             }

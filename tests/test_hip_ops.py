@@ -209,6 +209,26 @@ def test_linear_choice_where_the_l2_rate_decides(hip, M, N, K, epi, tile):
     assert ran[0] == tile
 
 
+@pytest.mark.parametrize("M,tile,fused", [(2448, 2, 1), (6148, 7, 0), (6288, 7, 0), (6912, 7, 0)])
+def test_linear_slices_end_where_their_sums_grow_too_large(hip, M, tile, fused):
+    """The K = 12288 projection with the norm behind it: two slices of 256 x 256 at 2448 rows (the step 1.3 % shorter than with
+    one piece), one piece of 256 x 192 at 6148 to 6912 rows (0.5 to 1.2 % shorter than with two slices of 288 x 192)."""
+    L = hip.lib()
+    N, K = 3072, 12288
+    a, w, c, n = hip.DevBuf(M * K * 2), hip.DevBuf(N * K * 2), hip.DevBuf(M * N * 4), hip.DevBuf(M * N * 2)
+    for b in (a, w, c):
+        hip.check(L.flux_hip_memset(b.ptr, 0, b.nbytes))
+    v = hip.DevBuf.from_array(np.ones(N, np.float32))
+    ran = np.zeros(1, np.int32)
+    L.flux_hip_linear_probe(hip.EPI_RESID)
+    try:
+        assert hip.linear_resid_adaln([(a.ptr, w.ptr, c.ptr, v.ptr, M)], N, K, K, K, N, [(n.ptr, v.ptr, v.ptr)]) == fused
+        assert L.flux_hip_linear_probe_read_launches(1, ran.ctypes.data, None) == 1
+    finally:
+        L.flux_hip_linear_probe(-1)
+    assert ran[0] == tile
+
+
 @pytest.mark.parametrize("epi,N", [("resid", 3072), ("bf16", 9216)])
 def test_linear_cut_tile_at_the_double_stream_shapes(hip, epi, N):
     """256 x 224 where the model uses it: 4096 image + 512 text rows with weights of their own, K = 3072, the gated residual
