@@ -1496,6 +1496,21 @@ static int ensure_ws(size_t bytes) {
     return 1;
 }
 
+/* Whether K slices can have their partial sums in the growing workspace: not where the memory cannot be had, and not under stream
+ * capture (the graph would keep the address of memory that a later call may free to grow it, and growing it fails there). Slices
+ * are a choice of speed, so no call fails for that: a projection takes the static array instead, a convolution runs in
+ * one piece. */
+static bool workspace_for_slices(size_t bytes) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(flux_hip_stream_handle(), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (ensure_ws(bytes)) return true;
+    (void)hipGetLastError(); /* the next launch is not to report this one */
+    return false;
+}
+
 extern "C" void flux_hip_linear_release(void) {
     if (g_ws) (void)hipFree(g_ws);
     g_ws = nullptr;
@@ -1685,7 +1700,10 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
         if (fixed_ws) {
             g.ws = fixed_ws;
         } else {
-            if (!ensure_ws((size_t)g.ksplit * g.ws_rows * g.N * sizeof(float))) return 0;
+            if (!workspace_for_slices((size_t)g.ksplit * g.ws_rows * g.N * sizeof(float))) { /* once more, with as many slices as fit the static array */
+                float *ws = static_ws_for_current_device();
+                return ws ? gemm_dispatch(g, np, epilogue, allowed, tile_out, adaln, adaln_done, ws, STATIC_WS_BYTES, leave_slices) : 0;
+            }
             g.ws = g_ws;
         }
     }
@@ -1868,20 +1886,6 @@ static int conv_finish(GemmArgs &g) {
     return 1;
 }
 
-/* Whether a convolution may run as K slices: they are a choice of speed, so a convolution never fails for want of their
- * workspace, and under stream capture it takes none (the graph would keep the address of memory that a later call may
- * free to grow it). In both cases it runs in one piece. */
-static bool conv_workspace(size_t bytes) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(flux_hip_stream_handle(), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return false;
-    }
-    if (ensure_ws(bytes)) return true;
-    (void)hipGetLastError(); /* the next launch is not to report this one */
-    return false;
-}
-
 /* Tile and K split of a convolution by the same kind of model as gemm_dispatch's: rounds of workgroups, each a tile's time at
  * its measured rate plus the bytes of its epilogue at a compute unit's share of the memory rate (nothing overlaps those where one
  * workgroup owns the unit). K slices, which add a second pass and its partial sums, are what small images need: 32 x 32
@@ -1923,7 +1927,7 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
         if (tile < 0) tile = N % 128 == 0 ? 1 : 3; /* (a forced ring tile that cannot run) */
     };
     choose(g_splitk_enabled);
-    if (split > 1 && M > 0 && !conv_workspace((size_t)split * M * N * sizeof(float))) choose(false);
+    if (split > 1 && M > 0 && !workspace_for_slices((size_t)split * M * N * sizeof(float))) choose(false);
     g.kt_per = (kt_total + split - 1) / split;
     g.ksplit = M == 0 ? 0 : split; /* 0: nothing but border */
     const bool bf = epilogue == FLUX_HIP_EPI_CONV_BF16;

@@ -91,6 +91,9 @@ typedef struct {
  * of a double block, for one sequence or for the two sequences of a batched CFG step). K % 64 == 0 and N % 128 == 0 are required.
  * For FLUX_HIP_EPI_SWIGLU, N counts gate+up columns (2*mlp); gate rows start at W row w_row0,
  * up rows at w_row1; the output has N/2 columns. Otherwise W rows [w_row0, w_row0+N) are used.
+ * The fp32 partial sums of K slices lie in a workspace from hipMalloc, kept and grown on demand. Where that cannot be had, and
+ * while the library's stream is being captured into a graph, they go to the static array of flux_hip_linear_static (its
+ * limit and its rule on overlapping calls then hold), so that no graph keeps the address of memory that a later call frees.
  */
 int flux_hip_linear(int epilogue, int nparts, const flux_hip_linear_part *parts,
                     int N, int K, int lda, int ldw, int ldc, int w_row0, int w_row1);

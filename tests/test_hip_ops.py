@@ -229,6 +229,59 @@ def test_linear_slices_end_where_their_sums_grow_too_large(hip, M, tile, fused):
     assert ran[0] == tile
 
 
+@pytest.mark.parametrize("M", [80, 2448])
+def test_linear_under_graph_capture(hip, M):
+    """The K = 12288 projection with the norm behind it, which runs as K slices at both row counts, captured while there is no
+    workspace: its sums go to the static array, so the call succeeds and the graph keeps no address that a later call may
+    free. Replayed three times between eager calls that make and grow the workspace, each replay bit for bit the eager result."""
+    import ctypes
+    L = hip.lib()
+    rt = ctypes.CDLL("libamdhip64.so")
+    N, K = 3072, 12288
+    rng = np.random.default_rng(71)
+    a, w = (hip.DevBuf.from_array(f32_to_bf16(rng.standard_normal((r, K), np.float32) * np.float32(s))) for r, s in ((M, 1.0), (N, 0.02)))
+    res = rng.standard_normal((M, N), np.float32)
+    x, y, v = hip.DevBuf.from_array(res), hip.DevBuf(M * N * 2), hip.DevBuf.from_array(rng.standard_normal(N, np.float32))
+
+    def call():
+        return hip.linear_resid_adaln([(a.ptr, w.ptr, x.ptr, v.ptr, M)], N, K, K, K, N, [(y.ptr, v.ptr, v.ptr)])
+
+    def reset():
+        hip.check(L.flux_hip_upload(x.ptr, res.ctypes.data, res.nbytes))
+        hip.check(L.flux_hip_memset(y.ptr, 0x55, M * N * 2))
+        hip.sync()
+
+    def result():
+        hip.sync()
+        return x.to_array(np.uint32, (M, N)), y.to_array(np.uint16, (M, N))
+
+    assert call()
+    want = result()
+    reset()
+    L.flux_hip_linear_release()
+    graph, execu, st = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p(L.flux_hip_stream())
+    assert rt.hipStreamBeginCapture(st, 2) == 0              # relaxed: only what the call itself does is looked at
+    try:
+        fused = call()
+    finally:
+        ended = rt.hipStreamEndCapture(st, ctypes.byref(graph))
+    assert fused and ended == 0
+    assert rt.hipGraphInstantiate(ctypes.byref(execu), graph, None, None, 0) == 0
+    try:
+        for slices in (2, 4, 6):
+            L.flux_hip_linear_force_split(slices)
+            call()
+            L.flux_hip_linear_force_split(0)
+            reset()
+            assert rt.hipGraphLaunch(execu, st) == 0
+            for got, ref in zip(result(), want):
+                np.testing.assert_array_equal(got, ref)
+    finally:
+        L.flux_hip_linear_force_split(0)
+        rt.hipGraphExecDestroy(execu)
+        rt.hipGraphDestroy(graph)
+
+
 @pytest.mark.parametrize("epi,N", [("resid", 3072), ("bf16", 9216)])
 def test_linear_cut_tile_at_the_double_stream_shapes(hip, epi, N):
     """256 x 224 where the model uses it: 4096 image + 512 text rows with weights of their own, K = 3072, the gated residual
