@@ -1861,7 +1861,7 @@ extern "C" int flux_hip_linear_resid_adaln(int nparts, const flux_hip_linear_par
 
 
 
-/* Tiles of a convolution: ids 0 to 3 as above (64 x 128, 128 x 128, 256 x 256, 64 x 64), 12 = 256 x 128, 13 =
+/* Tiles of a convolution: 15 = conv.hip's kernel for 3x3 without stride; ids 0 to 3 as above (64 x 128, 128 x 128, 256 x 256, 64 x 64), 12 = 256 x 128, 13 =
  * 128 x 128 in the ring kernel, as is 2: 128 x 128 in two stages reached 700 to 870 TFLOP/s on 3x3 layers of 128 to 512 channels over
  * 128 x 128 to 1024 x 1024 positions, 256 x 128 reaches 920 to 1230 and 256 x 256 1200 to 1390 (bf16 output). */
 template <int EPI>
@@ -1876,8 +1876,9 @@ static int conv_tile_launch(GemmArgs &g, int tile) {
     }
 }
 
-#define CONV_TILES 14
-static const int conv_bm[CONV_TILES] = {64, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 256, 128}, conv_bn[CONV_TILES] = {128, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 128, 128};
+#define CONV_TILES 16
+static const int conv_bm[CONV_TILES] = {64, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 256, 128, 0, 256}, conv_bn[CONV_TILES] = {128, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 128, 128, 0, 128};
+#define CONV_PATCH 15 /* 16 x 16 positions x 128 channels, conv.hip */
 
 template <int EPI>
 static int conv_finish(GemmArgs &g) {
@@ -1890,15 +1891,19 @@ static int conv_finish(GemmArgs &g) {
  * its measured rate plus the bytes of its epilogue at a compute unit's share of the memory rate (nothing overlaps those where one
  * workgroup owns the unit). K slices, which add a second pass and its partial sums, are what small images need: 32 x 32
  * positions x 512 channels are 32 tiles of 128 x 128 for 256 units, 57 us in one piece and 24 in slices (27 in a decode); at 96 x 96 positions
- * one piece wins (54 us against 69). */
+ * one piece wins (54 us against 69). conv.hip's kernel is ahead from about a round of its tiles on (80 x 120 x 512: 46 us against 53 of
+ * 256 x 128) as long as the image's sides do not leave a second, nearly empty round (90 x 162 x 512: 264 of its tiles, 90 us; 228 of 256 x 128,
+ * 59 us). Over 111 forms of 37 layers the chosen tile took 1.5 % less than the best of four timed behind it, i.e. the same. */
 static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
-    static const int occ[CONV_TILES] = {3, 2, 1, 4, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1};
-    static const double rate[CONV_TILES] = {2.0e12, 3.3e12, 5.4e12, 1.5e12, 0, 0, 0, 0, 0, 0, 0, 0, 4.8e12, 4.2e12}; /* FLOP/s of one CU */
+    static const int occ[CONV_TILES] = {3, 2, 1, 4, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 0, 1};
+    static const double rate[CONV_TILES] = {2.0e12, 3.3e12, 5.4e12, 1.5e12, 0, 0, 0, 0, 0, 0, 0, 0, 4.8e12, 4.2e12, 0, 6.2e12}; /* FLOP/s of one CU */
     static const int splits[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int M = g.M[0], N = g.N, kt_total = g.K >> 6, f = g_force_tile;
     const bool forced = f >= 0 && f < CONV_TILES && conv_bm[f] && N % conv_bn[f] == 0; /* a forced tile that this layer cannot use is ignored */
     const bool ring_ok = g_ring && (size_t)g.conv_rows * (g.conv_stride == 2 ? 4 : 1) * g.lda * 2 < ((size_t)1 << 32) && (size_t)N * g.ldw * 2 < ((size_t)1 << 32) &&
                          (size_t)g.conv_rows * N < ((size_t)1 << 32);
+    const int width = g.conv_wp - 2, height = g.conv_wp > 0 ? g.conv_rows / g.conv_wp - 2 : 0;
+    const bool patch_ok = g_ring && g.conv_taps == 9 && g.conv_stride == 1 && !g.conv_packed_out && conv3_takes(height, width, g.lda, N);
     int tile = -1, split = 1;
     const auto choose = [&](bool slices) {
         double best = 1e30;
@@ -1909,10 +1914,11 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
             if (!conv_bm[t] || N % conv_bn[t] || (forced && t != f)) continue;
             if (t == 0 && !forced) continue; /* (for comparison runs) */
             if (ring && (!ring_ok || kt_total < 4)) continue;
-            const long tiles = (long)((M + conv_bm[t] - 1) / conv_bm[t]) * (N / conv_bn[t]);
+            if (t == CONV_PATCH && !patch_ok) continue;
+            const long tiles = t == CONV_PATCH ? conv3_tiles(height, width, N) : (long)((M + conv_bm[t] - 1) / conv_bm[t]) * (N / conv_bn[t]);
             for (int sp : splits) {
                 const int per = (kt_total + sp - 1) / sp, used = (kt_total + per - 1) / per, last = kt_total - (used - 1) * per;
-                if (sp > 1 && (!slices || per < 4 || last < 4 || used != sp || N % 64)) continue;
+                if (sp > 1 && (t == CONV_PATCH || !slices || per < 4 || last < 4 || used != sp || N % 64)) continue;
                 if (slices && g_force_split && kt_total / g_force_split >= 4 && sp != g_force_split) continue;
                 const double ws = (double)sp * M * N * 4.0;
                 if (sp > 1 && ws > 256e6) continue;
@@ -1920,6 +1926,8 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
                 const long per_cu = (min(blocks, slots) + 255) / 256;
                 double est = rounds * (2.0 * conv_bm[t] * conv_bn[t] * 64.0 * per / (rate[t] / per_cu) + 2.5e-6 +
                                        (double)conv_bm[t] * conv_bn[t] * (sp > 1 ? 0 : (epilogue == FLUX_HIP_EPI_CONV_BF16 ? 2 : 4) + (g.res ? 4 : 0)) / 2.0e10);
+                if (t == CONV_PATCH) /* the epilogue lies under the next tile and costs it half of its bytes' time, the last one's all */
+                    est = rounds * (2.0 * conv_bm[t] * conv_bn[t] * 64.0 * per / rate[t] + (double)conv_bm[t] * conv_bn[t] * ((epilogue == FLUX_HIP_EPI_CONV_BF16 ? 2 : 4) + (g.res ? 4 : 0)) / 4.0e10) + 6.0e-6;
                 if (sp > 1) est += 4.0e-6 + 2.0 * ws / 4.0e12;
                 if (est < best) { best = est; tile = t; split = sp; }
             }
@@ -1942,7 +1950,9 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
         (void)hipEventRecord(g_probe_ev[slot][0], flux_hip_stream_handle());
     }
     int ok = 1;
-    if (g.ksplit == 1) {
+    if (g.ksplit == 1 && tile == CONV_PATCH) {
+        ok = conv3_launch(!bf, g.A[0], g.W[0], g.bias, g.res, g.C[0], height, width, g.lda, N, g.stats, stats_rows, compute_units() & ~7);
+    } else if (g.ksplit == 1) {
         if (stats_rows) *stats_rows = 2 * ((M + conv_bm[tile] - 1) / conv_bm[tile]);
         ok = bf ? conv_tile_launch<FLUX_HIP_EPI_CONV_BF16>(g, tile) : conv_tile_launch<FLUX_HIP_EPI_CONV_F32>(g, tile);
     } else {

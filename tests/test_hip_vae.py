@@ -214,6 +214,47 @@ def test_conv_tiles_and_slices(hip, switches, H, W, cin, cout):
                 assert rel_l2(got, want) < (2.0 ** -9 if epi == hip.EPI_CONV_BF16 else 2e-6)
 
 
+@pytest.mark.parametrize("H,W,cin,cout", [(1, 1, 128, 128), (5, 15, 128, 256), (16, 16, 192, 128), (17, 33, 256, 384), (31, 48, 512, 128), (270, 260, 128, 128)])
+def test_conv_patch_tile(hip, switches, H, W, cin, cout):
+    """Tile 15 (16 x 16 positions, neighbourhood in LDS, conv.hip) against the 128 x 128 tile, which test_conv3x3 ties to the
+    oracle. The values are whole numbers whose sums fp32 holds exactly (9 * 512 products of at most 8 * 4), so that another
+    order of additions gives the same bits. Smaller than a tile, cut off on both sides, two chunks of channels (the
+    stored tile's epilogue lies under all of them), three, four and eight, three column tiles, and more tiles than compute units
+    (270 x 260: 289), so that workgroups store one tile under the next."""
+    import ctypes
+    L = hip.lib()
+    rows, wp = (H + 2) * (W + 2), W + 2
+    rng = np.random.default_rng(67)
+    x, w = rng.integers(-8, 9, (cin, H, W)).astype(np.float32), rng.integers(-4, 5, (cout, cin, 3, 3)).astype(np.float32)
+    b, res = rng.integers(-9, 10, cout).astype(np.float32), to_padded(rng.integers(-999, 1000, (cout, H, W)).astype(np.float32))
+    din = Guarded(hip, to_padded(x), wp)
+    dw, db, dres = hip.DevBuf.from_array(conv_weight(w)), hip.DevBuf.from_array(b), hip.DevBuf.from_array(res)
+
+    def run(tile, epi, r):
+        L.flux_hip_linear_force_tile(tile)
+        L.flux_hip_linear_enable_splitk(0)
+        bf = epi == hip.EPI_CONV_BF16
+        guard = np.full((1, cout), 3.0, np.float32)
+        start = np.concatenate([res if r == "in place" else np.full((rows, cout), 3.0, np.float32), guard])
+        out = hip.DevBuf.from_array(f32_to_bf16(start) if bf else start)
+        stats = hip.DevBuf.from_array(np.full(((rows // 32 + 2) * (cout // 4) * 2,), np.nan, np.float32))
+        n = ctypes.c_int(0)
+        L.flux_hip_linear_probe(-2)
+        L.flux_hip_conv_image.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_int] + [ctypes.c_void_p] * 4 + [ctypes.c_int] * 5 + [ctypes.c_void_p] * 2
+        hip.check(L.flux_hip_conv_image(epi, din.ptr, 0, 0, dw.ptr, db.ptr, out.ptr if r == "in place" else r, out.ptr, rows, wp, cin, cout, 9, stats.ptr,
+                                        ctypes.byref(n)))
+        ran = np.zeros(2, np.int32)
+        assert L.flux_hip_linear_probe_read_launches(2, ran.ctypes.data, None) == 1 and ran[0] == tile
+        assert 0 < n.value <= rows // 32 + 2
+        got = bf16_to_f32(out.to_array(np.uint16, (rows + 1, cout))) if bf else out.to_array(np.float32, (rows + 1, cout))
+        assert border_is_zero(got[:rows], H, W) and (got[rows] == 3.0).all()
+        check_sums(stats.to_array(np.float32, (n.value, cout // 4, 2)).astype(np.float64).sum(0), got[:rows])
+        return got[:rows]
+
+    for epi, r in ((hip.EPI_CONV_F32, None), (hip.EPI_CONV_F32, dres.ptr), (hip.EPI_CONV_F32, "in place"), (hip.EPI_CONV_BF16, None), (hip.EPI_CONV_BF16, dres.ptr)):
+        np.testing.assert_array_equal(run(15, epi, r), run(1, epi, r))
+
+
 CONV_FORMS = [(tile, split) for tile in (1, 2, 3, 12, 13) for split in (0, 2)] + [(-1, 0)]
 
 

@@ -55,9 +55,9 @@ MFMA_RESULT_SLOTS = 8
 
 def regs(tok):
     """'v[4:7]' -> {('v',4..7)}, 'a12' -> {('a',12)}; anything else -> empty."""
-    m = re.fullmatch(r"([va])\[(\d+):(\d+)\]", tok)
+    m = re.fullmatch(r"([va])\[(0x[0-9a-f]+|\d+)(?::(0x[0-9a-f]+|\d+))?\]", tok)      # numbers given to inline assembly print in hex beyond 64
     if m:
-        return {(m.group(1), i) for i in range(int(m.group(2)), int(m.group(3)) + 1)}
+        return {(m.group(1), i) for i in range(int(m.group(2), 0), int(m.group(3) or m.group(2), 0) + 1)}
     m = re.fullmatch(r"([va])(\d+)", tok)
     if m:
         return {(m.group(1), int(m.group(2)))}
@@ -145,14 +145,14 @@ def lint(body):
 def assembly(tmp_path_factory):
     """Assembly text and resource-usage remarks of gemm.hip and attention.hip, compiled once per test run."""
     out = {}
-    for src in ("gemm.hip", "attention.hip"):
+    for src in ("gemm.hip", "attention.hip", "conv.hip"):
         path = tmp_path_factory.mktemp("asm") / (src + ".s")
         r = compile_device(src, path, ["-S", "-Rpass-analysis=kernel-resource-usage"])
         out[src] = (path.read_text(), r.stderr)
     return out
 
 
-@pytest.mark.parametrize("src,pattern", [("attention.hip", "attention_wide_kernel"), ("gemm.hip", "gemm4w_kernel"), ("gemm.hip", "gemm4d_kernel")])
+@pytest.mark.parametrize("src,pattern", [("attention.hip", "attention_wide_kernel"), ("gemm.hip", "gemm4w_kernel"), ("gemm.hip", "gemm4d_kernel"), ("conv.hip", "conv3_kernel")])
 def test_inline_asm_mfma_hazards(src, pattern, assembly):
     kernels = {k: v for k, v in kernel_bodies(assembly[src][0]).items() if pattern in k}
     assert kernels, f"no kernel named *{pattern}* in {src}"
@@ -234,6 +234,28 @@ def test_gemm_kernels_fit_the_register_file(assembly):
         for a, b in k_loops:
             copies = [l.strip() for l in body[a:b] if "v_accvgpr" in l or "scratch_" in l]
             assert not copies, (name, copies[:4])
+
+
+def test_conv_kernel_owns_the_accumulator_registers(assembly):
+    """conv3_kernel names its 256 accumulator registers in its assembly statements: nothing that the compiler itself wrote may
+    touch one (a parked vector register would be overwritten), and nothing goes to scratch memory."""
+    usage = {k: v for k, v in resource_usage(assembly["conv.hip"][1]).items() if "conv3_kernel" in k}
+    assert len(usage) == 4
+    for name, u in sorted(usage.items()):
+        assert u["AGPRs"] == 256 and u["ScratchSize"] == 0 and u["VGPRs Spill"] == 0, (name, u)
+    for name, body in kernel_bodies(assembly["conv.hip"][0]).items():
+        if "conv3_kernel" not in name:
+            continue
+        mine, named = False, 0
+        for line in body:
+            if "#ASMSTART" in line:
+                mine = True
+            elif "#ASMEND" in line:
+                mine = False
+            elif re.search(r"\ba\[|\ba\d|accvgpr", line.split(";")[0]):
+                assert mine, (name, line)
+                named += 1
+        assert named >= 2 * 27 * 32
 
 
 def test_projection_k_loops_carry_no_second_address_chain(assembly):
