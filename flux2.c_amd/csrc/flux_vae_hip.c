@@ -34,6 +34,9 @@ int flux_hip_vae_latent_in(void *out_bf16, const float *latent, const float *bn_
 int flux_hip_vae_key_bias(float *bias, int n, int keys);
 int flux_hip_vae_image_out(uint8_t *rgb, float *rgb_f32, const float *x, int ldx, int H, int W);
 int flux_hip_vae_image_in(void *out_bf16, const float *img, int H, int W);
+size_t flux_hip_vae_attention_work_floats(int n, int ld);
+int flux_hip_vae_attention(void *out, const void *q, const void *qkv, const void *vt, void *P, float *o32, float *work, int n, int keys, int ld, float scale,
+                           int *done);
 int flux_hip_vae_upsample2x_bf16(void *out_bf16, const void *x_bf16, int hp, int wp, int C);
 /* gemm.hip */
 int flux_hip_conv_image(int epilogue, const void *in, int in_wp, int packed, const void *w, const float *bias, const float *res, void *out, int rows, int wp,
@@ -448,6 +451,9 @@ static int run_res(vstate *s, const vres *r, void *out_bf16) {
     return run_conv(s, &r->c2, FLUX_HIP_EPI_CONV_F32, s->A, s->x, s->x, 1, v->st_x, &s->x_rows);
 }
 
+/* From how many positions on the scores stay out of memory: 2048 positions take 42 us with them and 44 without (two more launches), 3072
+ * 58 and 55, 4096 81 and 66, 16384 1007 and 594 (attention alone, random operands). */
+#define ATT_EXP_ROWS 2560
 /* attnblock_forward, flux_vae.c:223-313. Between the two 1x1 convolutions the border positions are left out: a
  * 1024x1024 picture's 16384 positions are 128 tiles of 256 x 256 of the second product, one round of workgroups in two K slices,
  * where the 16900 of the bordered image were 134, two rounds. */
@@ -458,13 +464,20 @@ static int run_attn(vstate *s, const vattn *a) {
     /* key rows between the image and the padded width are read by the score GEMM: zero them */
     if (ld > rows && !flux_hip_memset((char *)v->R + (size_t)rows * 3 * C * 2, 0, (size_t)(ld - rows) * 3 * C * 2)) return 0;
     if (!flux_hip_conv_image(FLUX_HIP_EPI_CONV_BF16, s->A, 0, 2, a->qkv.w, a->qkv.b, NULL, v->R, s->hp * s->wp, s->wp, C, 3 * C, 1, NULL, NULL)) return 0;
-    if (!flux_hip_vae_key_bias(v->kbias, ld, rows)) return 0;
     if (!flux_hip_transpose_bf16(v->VT, ld, (char *)v->R + 2 * C * 2, 3 * C, rows, C)) return 0;
     const float scale = 1.0f / sqrtf((float)C);
     int chunk = (int)v->att_chunk;
     if (g_att_chunk_limit && g_att_chunk_limit < chunk) chunk = g_att_chunk_limit;
     for (int r0 = 0; r0 < rows; r0 += chunk) {
         const int n = rows - r0 < chunk ? rows - r0 : chunk;
+        if (rows >= ATT_EXP_ROWS) { /* without scores in memory; s->y and Hb are free here, and larger than that */
+            int done;
+            if (!flux_hip_vae_attention((char *)s->A + (size_t)r0 * C * 2, (char *)v->R + (size_t)r0 * 3 * C * 2, v->R, v->VT, v->P, s->y, v->Hb, n, rows, ld,
+                                        scale, &done))
+                return 0;
+            if (done) continue;
+        }
+        if (r0 == 0 && !flux_hip_vae_key_bias(v->kbias, ld, rows)) return 0;
         flux_hip_linear_part sp = {(char *)v->R + (size_t)r0 * 3 * C * 2, (char *)v->R + C * 2, v->S, NULL, n};
         if (!flux_hip_linear(FLUX_HIP_EPI_F32, 1, &sp, ld, C, 3 * C, 3 * C, ld, 0, 0)) return 0;
         if (!flux_hip_softmax_rows(v->P, v->S, v->kbias, n, ld, scale)) return 0;

@@ -110,6 +110,10 @@ struct GemmArgs {
     /* optional: per (row-tile half, 4-channel group) sums and sums of squares of what a convolution
      * epilogue writes, [prow][N/4][2], for the group norm that follows */
     float *stats;
+    /* exponentials of attention scores (EPI_EXP): 2^(exp_scale * score - bias[row]) for columns below exp_keys, 0 beyond; the sums over each
+     * wave's columns go to stats [row][2 * column tile + wave] */
+    float exp_scale;
+    int exp_keys;
 };
 
 /* internal epilogue: fp32 partial sums of one K slice of a convolution, rows = interior positions */
@@ -156,6 +160,8 @@ __device__ __forceinline__ int a_step_offset(const GemmArgs &g, int kt) {
 #define EPI_PARTIAL 5
 /* internal epilogue of flux_hip_linear_qkv_swiglu: bf16 store for the leading column tiles, SiLU(gate) * up beyond */
 #define EPI_QKV_SWIGLU 8
+/* internal epilogue of flux_hip_linear_exp, see GemmArgs */
+#define EPI_EXP 10
 
 __device__ __forceinline__ int lds_swz(int r) { return ((r >> 1) & 7) ^ ((r & 1) << 2); }
 
@@ -242,7 +248,7 @@ __device__ __forceinline__ int weight_row(const GemmArgs &g, int tn, int v) {
         return ((blk & 1) ? g.w_row1 : g.w_row0) + tn * (BN / 2) + idx;
     }
     int col;
-    if (EPI == FLUX_HIP_EPI_BF16 || EPI == EPI_QKV_SWIGLU || EPI == FLUX_HIP_EPI_CONV_BF16) col = tn * BN + wv * WN + bf16_feature<TN>(blk, r);
+    if (EPI == FLUX_HIP_EPI_BF16 || EPI == EPI_QKV_SWIGLU || EPI == FLUX_HIP_EPI_CONV_BF16 || EPI == EPI_EXP) col = tn * BN + wv * WN + bf16_feature<TN>(blk, r);
     else col = tn * BN + v;
     if (CutTile<BN>::value) col = min(col, g.N - 1);
     return g.w_row0 + col;
@@ -497,6 +503,53 @@ __device__ __forceinline__ void store_conv_tile(const GemmArgs &g, const TileId 
     }
 }
 
+/* Attention scores as unnormalised probabilities, see GemmArgs. The rows' references are requested together in front of everything, so that
+ * no row block waits for the stores of the one before; only the last column tile has columns to clear. Stores as for bf16 above. */
+template <int BN, int WM, int WN>
+__device__ __forceinline__ void store_exp_tile(const GemmArgs &g, const TileId &t, f32x4 (&acc)[WN / 16][WM / 16], int m0, int M, int wm, int wn, int l15, int lq) {
+    constexpr int TM = WM / 16, TN = WN / 16;
+    const int n = t.tn * BN + wn * WN + 8 * lq, first = m0 + wm * WM + l15;
+    float r[TM];
+#pragma unroll
+    for (int j = 0; j < TM; j++) r[j] = g.bias[min(first + 16 * j, M - 1)];
+    const auto rows = [&](auto cut_c) {
+#pragma unroll
+        for (int j = 0; j < TM; j++) {
+            const int m = min(first + 16 * j, M - 1); /* rows beyond the last one are copies of it, operand and reference: they store the same */
+            bf16 *C = (bf16 *)g.C[0] + (size_t)m * g.ldc + n;
+            float sum = 0.0f;
+            int keys = g.exp_keys - n;
+            asm volatile("" : "+v"(keys)); /* compared anew for each row: 32 kept lane masks are spilled */
+#pragma unroll
+            for (int p = 0; p < TN / 2; p++) {
+                float v[8];
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    f32x4 a = acc[2 * p + k][j];
+                    asm volatile("" : "+v"(a)); /* out of its AGPRs here, one block at a time */
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        v[4 * k + e] = fast_exp2(fmaf(a[e], g.exp_scale, -r[j]));
+                        if (decltype(cut_c)::value && 32 * p + 4 * k + e >= keys) v[4 * k + e] = 0.0f;
+                    }
+                }
+                bf16x4 lo, hi;
+#pragma unroll
+                for (int e = 0; e < 4; e++) { lo[e] = (bf16)v[e]; hi[e] = (bf16)v[4 + e]; }
+                store_bf16x8(C + 32 * p, lo, hi, true);
+                /* of what is stored: a row's largest probability then carries no rounding of its own into the quotient */
+#pragma unroll
+                for (int e = 0; e < 4; e++) sum += (float)lo[e] + (float)hi[e];
+            }
+            sum += __shfl_xor(sum, 16);
+            sum += __shfl_xor(sum, 32);
+            if (lq == 0) g.stats[(size_t)m * (2 * g.ntiles) + 2 * t.tn + wn] = sum;
+        }
+    };
+    if (t.tn * BN + BN > g.exp_keys) rows(BoolC<true>{});
+    else rows(BoolC<false>{});
+}
+
 /* Cp, ldc, tn: where the tile goes - the part's output, or for the fused [Q|K|V|gate|up] projection the output of the
  * side of the boundary the tile lies on (the tile width divides nq_cols, so a tile is wholly on one side) */
 template <int BN, int WM, int WN, int EPI, int WGM, bool PINNED = false>
@@ -504,6 +557,8 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, const TileId &t, f
                                            int wm, int wn, int l15, int lq, int prow) {
     if constexpr (EPI == FLUX_HIP_EPI_CONV_BF16 || EPI == FLUX_HIP_EPI_CONV_F32) {
         store_conv_tile<BN, WM, WN, EPI, WGM, PINNED>(g, t, acc, m0, M, wm, wn, l15, lq, prow);
+    } else if constexpr (EPI == EPI_EXP) {
+        store_exp_tile<BN, WM, WN>(g, t, acc, m0, M, wm, wn, l15, lq);
     } else if constexpr (EPI == EPI_QKV_SWIGLU) {
         /* HERE = true: each side reads the accumulators through an empty asm statement, row by row. The conversions
          * are then work of that side; left to itself the compiler converted the whole tile to bf16 in front of the
@@ -840,7 +895,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm4w_kernel(GemmArgs g) {
 template <int EPI, int TM, int TN>
 struct EpilogueOps { /* vector memory instructions a wave issues in the epilogue of a tile whose rows are all valid */
     static constexpr int value = EPI == FLUX_HIP_EPI_SWIGLU || EPI == EPI_QKV_SWIGLU ? TM * (TN / 4 + TN / 2 % 2) /* 16-byte stores + a last 8-byte one */
-                                 : EPI == FLUX_HIP_EPI_BF16 || EPI == FLUX_HIP_EPI_CONV_BF16 ? TM * (TN / 2 + TN % 2) : EPI == FLUX_HIP_EPI_F32_T ? 4 * TM * TN : TM * TN;
+                                 : EPI == FLUX_HIP_EPI_BF16 || EPI == FLUX_HIP_EPI_CONV_BF16 || EPI == EPI_EXP ? TM * (TN / 2 + TN % 2) : EPI == FLUX_HIP_EPI_F32_T ? 4 * TM * TN : TM * TN;
 };
 
 template <int TM, int TN, int EPI, int NSA, int NSW>
@@ -1141,7 +1196,7 @@ static int launch_4d(GemmArgs &g) {
     g.total_tiles = g.mtiles * g.ntiles;
     size_t span = ((size_t)max(max(g.w_row0, g.w_row1), g.w_row2) + g.N) * g.ldw * 2;
     for (int i = 0; i < GEMM_MAX_PARTS; i++) span = max(span, (size_t)g.M[i] * g.lda * 2);
-    if constexpr (!IsConv<EPI>::value) /* (conv_launch has looked) */
+    if constexpr (!IsConv<EPI>::value && EPI != EPI_EXP) /* (conv_launch and flux_hip_linear_exp have looked) */
         if (span >= ((size_t)1 << 32)) return g.N % 128 == 0 ? launch_cfg<128, 128, 2, 2, EPI>(g) : launch_cfg<64, 64, 2, 2, EPI>(g);
     g.vgrid = (g.total_tiles * g.ksplit + 7) & ~7;
     const int grid = min(g.vgrid, compute_units() & ~7);
@@ -1435,6 +1490,14 @@ __global__ __launch_bounds__(256) void splitk_finish_adaln_kernel(GemmArgs g, Ad
     }
 }
 
+static int launch_exp(GemmArgs &g, int tile) {
+    switch (tile) {
+        case 2: return launch_4d<8, 8, EPI_EXP, 2, 3>(g);
+        case 12: return launch_4d<8, 4, EPI_EXP, 3, 3>(g);
+        default: return launch_4d<4, 4, EPI_EXP, 3, 3>(g);
+    }
+}
+
 template <int EPI>
 static int launch_split(GemmArgs &g, int tile) {
     if (!launch_epi<EPI_PARTIAL>(g, tile)) return 0;
@@ -1719,7 +1782,10 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
         case FLUX_HIP_EPI_BF16:
             if (leave_slices) *leave_slices = split ? g.ksplit : 0;
             ok = split && leave_slices ? launch_epi<EPI_PARTIAL>(g, tile) : split ? launch_split<FLUX_HIP_EPI_BF16>(g, tile) : launch_epi<FLUX_HIP_EPI_BF16>(g, tile); break;
-        case FLUX_HIP_EPI_F32: ok = split ? launch_split<FLUX_HIP_EPI_F32>(g, tile) : launch_epi<FLUX_HIP_EPI_F32>(g, tile); break;
+        case EPI_EXP: ok = launch_exp(g, tile); break;
+        case FLUX_HIP_EPI_F32:
+            if (leave_slices) *leave_slices = split ? g.ksplit : 0;
+            ok = split && leave_slices ? launch_epi<EPI_PARTIAL>(g, tile) : split ? launch_split<FLUX_HIP_EPI_F32>(g, tile) : launch_epi<FLUX_HIP_EPI_F32>(g, tile); break;
         case FLUX_HIP_EPI_F32_T: ok = launch_epi<FLUX_HIP_EPI_F32_T>(g, tile); break;
         case FLUX_HIP_EPI_RESID:
             if (split && adaln) {
@@ -1802,6 +1868,37 @@ extern "C" int flux_hip_linear_slices(const void *A, const void *W, void *C, int
     g.A[0] = (const bf16 *)A; g.W[0] = (const bf16 *)W; g.C[0] = C; g.M[0] = M;
     g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = N;
     const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_BF16, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
+    *ws = g.ws;
+    return ok;
+}
+
+/* Attention scores as unnormalised probabilities, P[m][n] = 2^(scale * A[m] . W[n] - ref[m]) in bf16 for n < keys and 0 for keys <= n < N, and
+ * their fp32 sums over pieces of each row, sums [M][*pieces] (at most N / 64 of them). N a multiple of 256, K of 64 and at least 256. In the
+ * ring kernel's epilogue, where they cost a multiply-add, an exponential and half a store of 16 bytes per eight: 16384 x 16384 scores
+ * written as fp32 and read by a softmax took 395 + 348 us. Returns 0 without an error where that kernel is switched off. */
+extern "C" int flux_hip_linear_exp(const void *A, const void *W, void *P, int M, int N, int K, int lda, int ldw, const float *ref, float scale, int keys,
+                                   float *sums, int *pieces) {
+    if (!g_ring || !g_persistent || M <= 0 || N <= 0 || (N & 255) || K < 256 || (K & 63) || lda < K || ldw < K || (lda & 7) || (ldw & 7) ||
+        ((((uintptr_t)A | (uintptr_t)W | (uintptr_t)P) & 15) != 0) || ((size_t)M * lda | (size_t)N * ldw) >= ((size_t)1 << 31))
+        return 0;
+    GemmArgs g = {};
+    g.A[0] = (const bf16 *)A; g.W[0] = (const bf16 *)W; g.C[0] = P; g.M[0] = M;
+    g.N = N; g.K = K; g.lda = lda; g.ldw = ldw; g.ldc = N;
+    g.bias = ref; g.stats = sums; g.exp_scale = scale; g.exp_keys = keys;
+    const int ok = gemm_dispatch(g, 1, EPI_EXP, 1u << 2 | 1u << 12 | 1u << 13);
+    *pieces = 2 * g.ntiles;
+    return ok;
+}
+
+/* C = A W^T in fp32 for a reader that sums K slices itself, as flux_hip_linear_slices: *slices = 0 and C is written, or *slices partial sums
+ * are left at *ws. */
+extern "C" int flux_hip_linear_f32_slices(const void *A, const void *W, float *C, int M, int N, int K, const float **ws, int *slices) {
+    *slices = 0;
+    if (M <= 0) return 1;
+    GemmArgs g = {};
+    g.A[0] = (const bf16 *)A; g.W[0] = (const bf16 *)W; g.C[0] = C; g.M[0] = M;
+    g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = N;
+    const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_F32, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
     *ws = g.ws;
     return ok;
 }

@@ -449,6 +449,84 @@ __global__ __launch_bounds__(256) void vae_softmax_reg_kernel(bf16 *__restrict__
     }
 }
 
+/* ---- the same attention for many positions, without the scores: P leaves the first product as 2^(scale score - reference)
+ * (flux_hip_linear_exp), the second product is divided by the row sums. A softmax does not care about its reference as long as
+ * nothing overflows: here it is the row's largest score over 256 keys spread over the image (2 to 3 % of the first product's work). A row
+ * with a score more than 2^100 above that - its sums show it - is computed once more by its wave, key by key. In a decode
+ * of 1024 x 1024 (16384 positions): 394 us of scores + 347 of softmax + 222 of P v with the scores in memory; now 18 + 295 + 244, of which
+ * the exponentials, which nothing overlaps, are about 80. (In chunks whose P the memory-side cache would hold it is no faster.) ---- */
+#define ATT_C 512          /* channels of the one head */
+#define ATT_SAMPLE 256     /* keys that give the reference */
+#define ATT_SUM_MAX 0x1p100f
+
+/* ref[row] = scale * the largest of the row's ATT_SAMPLE scores; one wave per row */
+__global__ __launch_bounds__(256) void vae_attention_ref_kernel(float *__restrict__ ref, const float *__restrict__ s, int n, float scale) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= n) return;
+    const f32x4 v = *(const f32x4 *)(s + (size_t)row * ATT_SAMPLE + lane * 4);
+    float m = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if (lane == 0) ref[row] = m * scale;
+}
+
+__device__ __forceinline__ float wave_sum(float v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
+
+/* out[row] = (sum of the slices) / (sum of the row's sums), one wave per row, eight channels per lane */
+__global__ __launch_bounds__(256) void vae_attention_out_kernel(bf16 *__restrict__ out, const float *__restrict__ o, int slices, const float *__restrict__ sums,
+                                                                int pieces, const bf16 *__restrict__ q, const bf16 *__restrict__ qkv, int n, int keys,
+                                                                float scale) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane * 8;
+    if (row >= n) return;
+    const size_t slice = (size_t)n * ATT_C;
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[e] = 0.0f;
+    for (int k = 0; k < slices; k++) {
+        const f32x4 *p = (const f32x4 *)(o + k * slice + (size_t)row * ATT_C + c);
+        const f32x4 a = p[0], b = p[1];
+#pragma unroll
+        for (int e = 0; e < 4; e++) { acc[e] += a[e]; acc[4 + e] += b[e]; }
+    }
+    float sum = 0.0f;
+    bool beyond = false;
+    for (int i = lane; i < pieces; i += 64) {
+        const float v = sums[(size_t)row * pieces + i];
+        sum += v;
+        beyond = beyond || v > ATT_SUM_MAX;
+    }
+    sum = wave_sum(sum);
+    if (__any(beyond)) {
+        const bf16x8 qr = *(const bf16x8 *)(q + (size_t)row * 3 * ATT_C + c);
+        const auto score = [&](int key) {
+            const bf16x8 kr = *(const bf16x8 *)(qkv + (size_t)key * 3 * ATT_C + ATT_C + c);
+            float d = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) d += (float)qr[e] * (float)kr[e];
+            return wave_sum(d) * scale;
+        };
+        float m = -INFINITY;
+        for (int key = 0; key < keys; key++) m = fmaxf(m, score(key));
+        sum = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] = 0.0f;
+        for (int key = 0; key < keys; key++) {
+            const float p = fast_exp2(score(key) - m);
+            const bf16x8 vr = *(const bf16x8 *)(qkv + (size_t)key * 3 * ATT_C + 2 * ATT_C + c);
+            sum += p;
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc[e] += p * (float)vr[e];
+        }
+    }
+    const float inv = 1.0f / sum;
+    bf16x8 r;
+#pragma unroll
+    for (int e = 0; e < 8; e++) r[e] = (bf16)(acc[e] * inv);
+    *(bf16x8 *)(out + (size_t)row * ATT_C + c) = r;
+}
+
 /* vt[c][j] = v[j][c] for j < rows, 0 for rows <= j < ld: the value matrix as the "weight" operand
  * of the second attention GEMM. 64 x 64 tiles through LDS. */
 __global__ __launch_bounds__(256) void vae_transpose_kernel(bf16 *__restrict__ vt, int ld, const bf16 *__restrict__ v, int ldv, int rows) {
@@ -606,6 +684,38 @@ extern "C" int flux_hip_softmax_rows(void *p_bf16, const float *s, const float *
     else
         hipLaunchKernelGGL(vae_softmax_kernel, dim3(rows), dim3(256), 0, flux_hip_stream_handle(), (bf16 *)p_bf16, s, key_bias, ld, scale);
     LAUNCH_OK("vae_softmax_kernel");
+    return 1;
+}
+
+extern "C" int flux_hip_linear_exp(const void *A, const void *W, void *P, int M, int N, int K, int lda, int ldw, const float *ref, float scale, int keys,
+                                   float *sums, int *pieces);
+extern "C" int flux_hip_linear_f32_slices(const void *A, const void *W, float *C, int M, int N, int K, const float **ws, int *slices);
+
+extern "C" size_t flux_hip_vae_attention_work_floats(int n, int ld) { return (size_t)n * (ATT_SAMPLE + 1 + ld / 64) + 4; }
+
+/* Attention of n queries (rows of qkv from q on, 3 * 512 wide) over `keys` positions: out [n][512]. qkv: every position's [q | k | v], ld rows of
+ * them (zeros beyond keys); vt: v transposed, [512][ld]; P: n x ld bf16; o32: n x 512; work: flux_hip_vae_attention_work_floats. At least
+ * 256 keys, ld a multiple of 256. *done = 0 where the scores' kernel is not to be had: nothing is computed. */
+extern "C" int flux_hip_vae_attention(void *out, const void *q, const void *qkv, const void *vt, void *P, float *o32, float *work, int n, int keys, int ld,
+                                      float scale, int *done) {
+    *done = 0;
+    if (n <= 0 || keys < ATT_SAMPLE || ld < keys || (ld & 255)) return flux_hip_fail("flux_hip_vae_attention: bad shape (%d queries, %d keys, %d columns)", n, keys, ld);
+    const float scale2 = scale * 1.44269504088896341f;
+    float *sample = work, *ref = work + (size_t)n * ATT_SAMPLE, *sums = ref + ((n + 3) & ~3);
+    hipStream_t st = flux_hip_stream_handle();
+    const bf16 *k = (const bf16 *)qkv + ATT_C;
+    flux_hip_linear_part sp = {q, k, sample, nullptr, n};
+    if (!flux_hip_linear(FLUX_HIP_EPI_F32, 1, &sp, ATT_SAMPLE, ATT_C, 3 * ATT_C, keys / ATT_SAMPLE * 3 * ATT_C, ATT_SAMPLE, 0, 0)) return 0;
+    hipLaunchKernelGGL(vae_attention_ref_kernel, dim3((n + 3) / 4), dim3(256), 0, st, ref, sample, n, scale2);
+    LAUNCH_OK("vae_attention_ref_kernel");
+    int pieces = 0, slices = 0;
+    if (!flux_hip_linear_exp(q, k, P, n, ld, ATT_C, 3 * ATT_C, 3 * ATT_C, ref, scale2, keys, sums, &pieces)) return 1;
+    const float *ws = nullptr;
+    if (!flux_hip_linear_f32_slices(P, vt, o32, n, ATT_C, ld, &ws, &slices)) return 0;
+    hipLaunchKernelGGL(vae_attention_out_kernel, dim3((n + 3) / 4), dim3(256), 0, st, (bf16 *)out, slices ? ws : o32, slices ? slices : 1, sums, pieces,
+                       (const bf16 *)q, (const bf16 *)qkv, n, keys, scale2);
+    LAUNCH_OK("vae_attention_out_kernel");
+    *done = 1;
     return 1;
 }
 

@@ -578,6 +578,53 @@ def test_upsample_from_bf16(hip, C, H, W):
     assert (got[1][rows2] == 0x4040).all() and border_is_zero(got[1][:rows2], 2 * H, 2 * W)
 
 
+@pytest.mark.parametrize("keys,n", [(256, 256), (260, 9), (1300, 1300), (2048, 300), (3004, 3004)])
+@pytest.mark.parametrize("planted", [False, True])
+def test_attention_without_scores(hip, switches, keys, n, planted):
+    """One head of 512 channels over all positions with unnormalised probabilities, against float64: padded columns, few queries,
+    cut tiles. Scores of order one; planted: for some queries one key that the reference's sample does not hold lies 2^150 above
+    the sample's largest, so that those rows are computed anew, another 2^90 above (within the range), and a third row's sample holds
+    its largest. Two roundings to bf16 (probability, output) and fp32 sums: 2^-8."""
+    import ctypes
+    C, ld = 512, (keys + 255) & ~255
+    rng = np.random.default_rng(keys + n)
+    qkv = np.zeros((ld, 3, C), np.float32)
+    qkv[:keys] = q(rng.standard_normal((keys, 3, C)).astype(np.float32))
+    scale = 1.0 / np.sqrt(C)
+    if planted:
+        step, ln2 = keys // 256, float(np.log(2.0))
+        qkv[:keys, 1, 0] = 0.0
+        unsampled = 1 if step > 1 else min(256, keys - 1)
+        for row, key, height in ((0, unsampled, 150.0), (3, 0, 150.0), (5, unsampled, 90.0)):
+            qkv[row, 0, 0] = height * ln2 / scale / 64.0
+        qkv[unsampled, 1, 0] = 64.0
+        if keys > 256:
+            qkv[3, 0, 0] *= -1.0                    # that row's large scores are negative: nothing special
+        qkv = q(qkv)
+    dq = hip.DevBuf.from_array(f32_to_bf16(qkv.reshape(ld, 3 * C)))
+    vt = np.zeros((C, ld), np.float32)
+    vt[:] = qkv[:, 2].T
+    dv, P = hip.DevBuf.from_array(f32_to_bf16(vt)), hip.DevBuf(n * ld * 2)
+    L = hip.lib()
+    L.flux_hip_vae_attention_work_floats.restype = ctypes.c_size_t
+    work, o32 = hip.DevBuf(L.flux_hip_vae_attention_work_floats(n, ld) * 4 + 64), hip.DevBuf(n * C * 4)
+    out = hip.DevBuf.from_array(np.full((n + 1, C), 0x4040, np.uint16))
+    L.flux_hip_vae_attention.argtypes = [ctypes.c_void_p] * 7 + [ctypes.c_int] * 3 + [ctypes.c_float, ctypes.c_void_p]
+    done = ctypes.c_int(0)
+    first = keys - n if not planted else 0
+    hip.check(L.flux_hip_vae_attention(out.ptr, dq.at(first * 3 * C * 2), dq.ptr, dv.ptr, P.ptr, o32.ptr, work.ptr, n, keys, ld, scale, ctypes.byref(done)))
+    assert done.value == 1
+    bits = out.to_array(np.uint16, (n + 1, C))
+    assert (bits[n] == 0x4040).all()
+    x = qkv[:keys].astype(np.float64)
+    s = x[first:first + n, 0] @ x[:, 1].T * scale
+    p = np.exp(s - s.max(1, keepdims=True))
+    want = p @ x[:, 2] / p.sum(1, keepdims=True)
+    got = bf16_to_f32(bits[:n])
+    assert rel_l2(got, want) < 2.0 ** -8
+    np.testing.assert_array_less(np.abs(got - want).max(1), 2.0 ** -6 * np.abs(want).max(1) + 1e-6)
+
+
 @pytest.mark.parametrize("shape", [(37, 384, 300), (3, 17024, 16900), (3, 20608, 20500)])
 def test_softmax_rows_and_transpose(hip, oracle_mod, shape):
     """Rows of up to 20480 columns go through the kernel that keeps the row in registers, longer ones
