@@ -225,7 +225,7 @@ __device__ __forceinline__ int bf16_pair_feature(int blk, int r) { return 32 * (
 /* the same for a wave that owns TN blocks: with TN odd the last block has no neighbour and keeps the plain numbering */
 template <int TN>
 __device__ __forceinline__ int bf16_feature(int blk, int r) { return blk < (TN & ~1) ? bf16_pair_feature(blk, r) : 16 * blk + r; }
-/* Tile widths that divide none of the model's matrix widths (224: 3072 = 13 x 224 + 160, 9216 = 41 x 224 + 32): the
+/* Tile widths that do not divide all of the models' matrix widths (224: 3072 = 13 x 224 + 160, 9216 = 41 x 224 + 32; 96: 19456 = 202 x 96 + 64): the
  * last column tile is cut off. Its missing weight rows are read from the matrix's last row and its missing columns are
  * not stored (whole 16-column blocks for fp32 outputs, whole pairs of blocks for bf16: N is a multiple of 32). */
 template <int BN> struct CutTile { static constexpr bool value = BN % 64 != 0; };
@@ -243,7 +243,8 @@ __device__ __forceinline__ int weight_row(const GemmArgs &g, int tn, int v) {
     constexpr int TN = WN / 16;
     const int wv = v / WN, blk = (v % WN) >> 4, r = v & 15;
     if (EPI == FLUX_HIP_EPI_SWIGLU || (EPI == EPI_QKV_SWIGLU && tn >= g.nq_tiles)) {
-        const int idx = wv * (WN / 2) + swiglu_feature<TN>(blk, r);
+        int idx = wv * (WN / 2) + swiglu_feature<TN>(blk, r);
+        if (CutTile<BN>::value && EPI == FLUX_HIP_EPI_SWIGLU) idx = min(idx, g.N / 2 - 1 - tn * (BN / 2));
         if (EPI == EPI_QKV_SWIGLU) return ((blk & 1) ? g.w_row2 : g.w_row1) + (tn - g.nq_tiles) * (BN / 2) + idx;
         return ((blk & 1) ? g.w_row1 : g.w_row0) + tn * (BN / 2) + idx;
     }
@@ -343,6 +344,7 @@ __device__ __forceinline__ void store_tile_to(const GemmArgs &g, const TileId &t
             }
         }
         if (EPI == FLUX_HIP_EPI_SWIGLU) {
+            if (CutTile<BN>::value && tn * BN + wn * WN >= g.N) continue; /* the same for the whole wave (N counts gate and up columns) */
             /* see swiglu_feature: two (gate, up) pairs give eight consecutive features, a last odd pair four */
             bf16 *C = (bf16 *)Cp + (size_t)m * ldc + tn * (BN / 2) + wn * (WN / 2);
             bf16x4 o[TN / 2];
@@ -1142,7 +1144,7 @@ static int launch_cfg(GemmArgs &g) {
         attr_done = true;
     }
     set_row_tiles(g, BM);
-    g.ntiles = g.N / BN;
+    g.ntiles = (g.N + BN - 1) / BN; /* (a last tile that is cut off: CutTile) */
     g.nq_tiles = g.nq_cols / BN;
     g.total_tiles = g.mtiles * g.ntiles;
     int grid = (g.total_tiles * g.ksplit + 7) & ~7;
@@ -1228,7 +1230,7 @@ static int launch_epi(GemmArgs &g, int tile) {
             default: break;
         }
     }
-    if (tile >= 11) tile = g.N % 256 == 0 ? 2 : 1; /* (the dispatch offers these only where the ring kernel takes them) */
+    if (tile >= 11 && tile < 15) tile = g.N % 256 == 0 ? 2 : 1; /* (the dispatch offers these only where the ring kernel takes them) */
     switch (tile) {
         case 2: return launch_4w<8, 8, EPI>(g);
         case 5: return launch_4w<9, 6, EPI>(g);
@@ -1240,6 +1242,7 @@ static int launch_epi(GemmArgs &g, int tile) {
         case 8: return launch_cfg<64, 128, 2, 2, EPI, 6>(g);  /* few rows: the same tiles with a ring that fills the LDS */
         case 9: return launch_cfg<128, 128, 2, 2, EPI, 5>(g);
         case 10: return launch_cfg<96, 128, 2, 2, EPI, 5>(g);
+        case 16: return launch_cfg<96, 96, 2, 3, EPI, 6>(g);
         default: return launch_cfg<64, 128, 2, 2, EPI>(g);
     }
 }
@@ -1581,7 +1584,7 @@ extern "C" void flux_hip_linear_release(void) {
 }
 
 static int g_force_tile = -1;
-#define TILE_MASK_ALL 0x7FEFu /* tiles the automatic choice may use: all but the 8-wave form of 256 x 256 */
+#define TILE_MASK_ALL 0x17FEFu /* tiles the automatic choice may use: all but the 8-wave form of 256 x 256 */
 static unsigned g_tile_mask = TILE_MASK_ALL;
 static int g_splitk_enabled = 1;
 extern "C" void flux_hip_linear_force_tile(int tile) { g_force_tile = tile; }
@@ -1659,17 +1662,20 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
     /* tile ids: 0..3 the small tiles and 256 x 256, 4 = the 8-wave form of 256 x 256 (only when
      * forced, for comparison runs), 5 = 288 x 192, 6 = 192 x 192, 7 = 256 x 192, 8, 9 and 10 = 64 x 128, 128 x 128 and
      * 96 x 128 with a ring of 6, 5 and 5 stages instead of 2 (one workgroup per compute unit; for parts of at most that
-     * many rows), 11 = 256 x 224 (4096 + 512 rows x 3072 columns are 252 such tiles, one round of workgroups on 256
+     * many rows), 16 = 96 x 96 with a ring of 6 and six waves: a compute unit takes in 50 to 55 KB of cold operands a microsecond whatever its
+     * ring and its waves (0.56 us per K step of 96 + 128 rows with 20 workgroups on the chip as with 152), so the width that
+     * leaves fewest units idle is the fastest: 67 x 19456 x 2560 32.7 us on 152 units and 28.6 on 203, 80 x 3072 x 12288 in slices 28.9 on
+     * 192 and 26.8 on 256, 11 = 256 x 224 (4096 + 512 rows x 3072 columns are 252 such tiles, one round of workgroups on 256
      * compute units of which each does 7/8 of a 256 x 256 tile's work; 216 tiles of 256 x 256 are one round as well),
      * 12 = 256 x 128, 13 = 128 x 128 and 14 = 192 x 256 in the ring kernel, for launches of about one round: the two-stage 128 x 128
      * tile waits for memory in every K step when it has a compute unit to itself. With the weights coming from HBM, as in a
      * forward: 512 x 6144 x 2560 39 us, in the ring 30; 1202 x 3072 x 3072: 49 and 34; 512 x 19456 x 2560 on 228 tiles of 192 x 256 52,
      * on 152 of 256 x 256 60. (The rates of 12 to 14 below are those of cached operands and up to 40 % above these launches; over
      * 133 shapes of 67 to 16384 rows with cold weights the chosen form took 0.8 % more than the best of seven on average.) */
-    constexpr int NT = 15;
-    static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 64, 128, 96, 256, 256, 128, 192}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 128, 128, 128, 224, 128, 128, 256};
-    static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, ahead[NT] = {1, 1, 1, 1, 1, 1, 1, 1, 5, 4, 4, 1, 1, 1, 1}; /* stages a workgroup keeps in flight */
-    static const double rate[NT] = {2.0e12, 2.9e12, 6.05e12, 1.5e12, 4.6e12, 6.0e12, 5.7e12, 5.75e12, 1.6e12, 3.0e12, 2.4e12, 5.9e12, 5.3e12, 4.4e12, 5.5e12}; /* FLOP/s of one CU running this tile */
+    constexpr int NT = 17;
+    static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 64, 128, 96, 256, 256, 128, 192, 0, 96}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 128, 128, 128, 224, 128, 128, 256, 1, 96};
+    static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, ahead[NT] = {1, 1, 1, 1, 1, 1, 1, 1, 5, 4, 4, 1, 1, 1, 1, 1, 5}; /* stages a workgroup keeps in flight */
+    static const double rate[NT] = {2.0e12, 2.9e12, 6.05e12, 1.5e12, 4.6e12, 6.0e12, 5.7e12, 5.75e12, 1.6e12, 3.0e12, 2.4e12, 5.9e12, 5.3e12, 4.4e12, 5.5e12, 1.0, 2.3e12}; /* FLOP/s of one CU running this tile */
     const int kt_total = g.K >> 6;
     int tile = -1, best_split = 1;
     {
@@ -1690,9 +1696,10 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
             if (cut && !((epilogue == FLUX_HIP_EPI_RESID || epilogue == FLUX_HIP_EPI_BF16) && g_ring && g_persistent && kt_total >= 4)) continue;
             /* bf16 outputs leave in pairs of 16-column blocks: the cut must fall between two pairs of a wave's 112 columns */
             if (cut && epilogue == FLUX_HIP_EPI_BF16 && (N % 224) % 112 % 32 != 0) continue;
-            if (!cut && (N % bn[t] || g.nq_cols % bn[t])) continue;
+            /* 96 x 96 (tile 16) cuts its last column tile off as well, at a multiple of 32, i.e. between two waves' columns */
+            if (!cut && ((N % bn[t] && (t != 16 || epilogue == EPI_QKV_SWIGLU)) || g.nq_cols % bn[t])) continue;
             if (!((allowed >> t) & 1)) continue;
-            if (t >= 12 && !(g_ring && g_persistent && kt_total >= 4)) continue;
+            if (t >= 12 && t < 15 && !(g_ring && g_persistent && kt_total >= 4)) continue;
             if (ahead[t] > 1) { /* the deep rings stream the weights once: every part in one row tile */
                 bool fits = true;
                 for (int i = 0; i < np; i++) fits = fits && g.M[i] <= bm[t];
@@ -1739,6 +1746,7 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
                 const double l2_rate = rows * K * 2.0 > 256.0e6 ? 12.9e12 : 13.5e12;
                 const double l2 = (double)tiles * (bm[t] + bn[t]) * K * 2.0 / l2_rate;
                 if (l2 > est) est = l2;
+                if (ahead[t] > 1) est += 0.03 * t_compute; /* of two that stream their weights at the same rate the one with less to do */
                 /* Slices cost their partial sums, and beyond 128 MB of those the stores of every round as well: the K = 12288 projection at
                  * 6148 to 6912 rows (151 to 170 MB) in two slices of 288 x 192 takes 379 + 78 us, in one piece of 256 x 192 430 and
                  * 27 for the norm, and the step around it is 0.5 to 1.2 % longer; at 2132 to 2560 rows (52 to 63 MB) two slices
@@ -1847,7 +1855,7 @@ static int linear_impl(int epilogue, int nparts, const flux_hip_linear_part *par
     g.N = N; g.K = K; g.lda = lda; g.ldw = ldw; g.ldc = ldc; g.w_row0 = w_row0; g.w_row1 = w_row1;
     a.ldo = N;
     a.eps = eps;
-    return gemm_dispatch(g, np, epilogue, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7FFFu, nullptr, norm ? &a : nullptr, fused,
+    return gemm_dispatch(g, np, epilogue, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x17FFFu, nullptr, norm ? &a : nullptr, fused,
                          fixed_ws, fixed_ws_bytes);
 }
 
@@ -1867,7 +1875,7 @@ extern "C" int flux_hip_linear_slices(const void *A, const void *W, void *C, int
     GemmArgs g = {};
     g.A[0] = (const bf16 *)A; g.W[0] = (const bf16 *)W; g.C[0] = C; g.M[0] = M;
     g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = N;
-    const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_BF16, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
+    const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_BF16, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x17FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
     *ws = g.ws;
     return ok;
 }
@@ -1898,7 +1906,7 @@ extern "C" int flux_hip_linear_f32_slices(const void *A, const void *W, float *C
     GemmArgs g = {};
     g.A[0] = (const bf16 *)A; g.W[0] = (const bf16 *)W; g.C[0] = C; g.M[0] = M;
     g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = N;
-    const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_F32, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
+    const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_F32, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x17FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
     *ws = g.ws;
     return ok;
 }
@@ -1922,7 +1930,7 @@ extern "C" int flux_hip_linear_qkv_swiglu(const void *A, const void *W, void *qk
     int tile = -1;
     const int saved = g_splitk_enabled;
     g_splitk_enabled = 0;
-    const int ok = gemm_dispatch(g, 1, EPI_QKV_SWIGLU, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7FFFu, &tile);
+    const int ok = gemm_dispatch(g, 1, EPI_QKV_SWIGLU, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x17FFFu, &tile);
     g_splitk_enabled = saved;
     return ok;
 }

@@ -616,6 +616,59 @@ def test_linear_deep_ring_tiles(hip, oracle_mod, tile, M, K):
     np.testing.assert_array_equal(fm, sw)
 
 
+@pytest.mark.parametrize("M,K", [(1, 64), (67, 192), (80, 448), (96, 1024)])
+@pytest.mark.parametrize("N", [384, 512, 640])
+def test_linear_96_wide_ring_tile(hip, oracle_mod, M, K, N):
+    """Tile 16 (96 x 96, six waves) whose last column tile is cut off after one wave's columns (512), two (640) or not at all (384): bit
+    for bit what the two-stage 128 x 128 tile gives, as bf16, fp32, gated residual, SwiGLU (whose cut lies within gate and up), the fused
+    launch where 96 divides both sides, and as K slices; columns beyond N stay as they were."""
+    import ctypes
+    L = hip.lib()
+    L.flux_hip_linear_qkv_swiglu.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 8
+    x, W = q(normal_f32((M, K), 72, 1)), q(normal_f32((2 * N, K), 72, 2, 0.0, 0.1))
+    gate, res = normal_f32((N,), 72, 3), normal_f32((M, N), 72, 4)
+    dx, dW, dg = dev_bf16(hip, x), dev_bf16(hip, W), hip.DevBuf.from_array(gate)
+    ld, mlp, outs = N + 64, N // 2, {}
+    try:
+        for t in (16, 1):
+            L.flux_hip_linear_force_tile(t)
+            L.flux_hip_linear_enable_splitk(0)
+            L.flux_hip_linear_probe(hip.EPI_BF16)
+            o16, o32, r = hip.DevBuf.from_array(np.full((M, ld), 7, np.uint16)), hip.DevBuf.from_array(np.full((M, ld), 7.0, np.float32)), hip.DevBuf.from_array(res)
+            hip.linear(hip.EPI_BF16, [(dx.ptr, dW.ptr, o16.ptr, None, M)], N, K, K, K, ld)
+            tiles = np.zeros(4, np.int32)
+            assert L.flux_hip_linear_probe_read_launches(4, tiles.ctypes.data, None) == 1 and tiles[0] == t
+            L.flux_hip_linear_probe(-1)
+            hip.linear(hip.EPI_F32, [(dx.ptr, dW.ptr, o32.ptr, None, M)], N, K, K, K, ld)
+            hip.linear(hip.EPI_RESID, [(dx.ptr, dW.ptr, r.ptr, dg.ptr, M)], N, K, K, K, N)
+            sw = hip.DevBuf.from_array(np.full((M, mlp + 64), 7, np.uint16))
+            hip.linear(hip.EPI_SWIGLU, [(dx.ptr, dW.ptr, sw.ptr, None, M)], N, K, K, K, mlp + 64, 0, mlp)
+            got = [o16.to_array(np.uint16, (M, ld)), o32.to_array(np.float32, (M, ld)), r.to_array(np.float32, (M, N)), sw.to_array(np.uint16, (M, mlp + 64))]
+            if N == 384:
+                fq, fm = hip.DevBuf(M * N * 2), hip.DevBuf(M * 192 * 2)
+                hip.check(L.flux_hip_linear_qkv_swiglu(dx.ptr, dW.ptr, fq.ptr, fm.ptr, M, N, 192, K, K, K, N, 192), "flux_hip_linear_qkv_swiglu")
+                got += [fq.to_array(np.uint16, (M, N)), fm.to_array(np.uint16, (M, 192))]
+            if K >= 512:
+                L.flux_hip_linear_enable_splitk(1)
+                L.flux_hip_linear_force_split(4)
+                s32 = hip.DevBuf(M * N * 4)
+                hip.linear(hip.EPI_F32, [(dx.ptr, dW.ptr, s32.ptr, None, M)], N, K, K, K, N)
+                L.flux_hip_linear_force_split(0)
+                got.append(s32.to_array(np.float32, (M, N)))
+            outs[t] = got
+    finally:
+        L.flux_hip_linear_enable_splitk(1)
+        L.flux_hip_linear_force_split(0)
+        L.flux_hip_linear_force_tile(-1)
+        L.flux_hip_linear_probe(-1)
+    for a, b in zip(outs[16], outs[1]):
+        np.testing.assert_array_equal(a, b)
+    assert (outs[16][0][:, N:] == 7).all() and (outs[16][1][:, N:] == 7.0).all() and (outs[16][3][:, mlp:] == 7).all()
+    lin = oracle_mod.linear(x, W)
+    assert rel_l2(outs[16][1][:, :N], lin[:, :N]) < 2e-6
+    assert rel_l2(bf16_to_f32(outs[16][3][:, :mlp]), oracle_mod.silu(lin[:, :mlp]) * lin[:, mlp:N]) < 4e-3
+
+
 def test_linear_rejects_bad_shapes(hip):
     d = hip.DevBuf(1024)
     with pytest.raises(hip.FluxHipError):
