@@ -431,7 +431,157 @@ int launch(const Args &g, int grid) {
     return 1;
 }
 
+/* ---- the first and the last convolution, which have three channels on one side ---- */
+
+/* 128 -> 3 channels and the picture itself. As a GEMM with its outputs padded to 64 columns and fp32 rows for a second kernel to read this was
+ * 288 + 56 us at 1024 x 1024, and is 75; HBM: 268 MB in. A workgroup makes 16 x 32 pixels: every position of
+ * their 18 x 34 neighbourhood is read once and multiplied with the weights of all nine taps, 27 outputs (two MFMA blocks, K = 128), which go
+ * to LDS; a pixel is the sum of nine of its neighbours' numbers. */
+#define OUT_PH 16
+#define OUT_PW 32
+#define OUT_LD 28 /* floats per position: 9 taps x 3 channels, and one to keep 16-byte alignment */
+__global__ __launch_bounds__(256) void conv_out_kernel(uint8_t *__restrict__ rgb, float *__restrict__ rgb_f32, const bf16 *__restrict__ in, const bf16 *__restrict__ w,
+                                                       const float *__restrict__ bias, int H, int W) {
+    __shared__ __attribute__((aligned(16))) float part[(OUT_PH + 2) * (OUT_PW + 2) * OUT_LD];
+    constexpr int POS = (OUT_PH + 2) * (OUT_PW + 2), BLOCKS = (POS + 15) / 16, PER = (BLOCKS + 3) / 4;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l15 = lane & 15, lq = lane >> 4;
+    const int x0 = blockIdx.x * OUT_PW, y0 = blockIdx.y * OUT_PH, wp = W + 2;
+    bf16x8 fw[2][4]; /* row r = 3 tap + output channel */
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+        const int r = min(16 * b + l15, 26), tap = r / 3, o = r - 3 * tap;
+#pragma unroll
+        for (int k = 0; k < 4; k++) fw[b][k] = *(const bf16x8 *)(w + (size_t)o * 9 * 128 + (k >> 1) * 9 * 64 + tap * 64 + (k & 1) * 32 + lq * 8);
+    }
+    const auto row = [&](int blk) { /* this lane's position of a block; those beyond the image repeat its last row and column */
+        const int p = min(blk * 16 + l15, POS - 1), py = p / (OUT_PW + 2), px = p - py * (OUT_PW + 2);
+        return in + ((size_t)min(y0 + py, H + 1) * wp + min(x0 + px, W + 1)) * 128 + lq * 8;
+    };
+#pragma unroll
+    for (int i = 0; i < PER; i += 2) { /* two blocks' loads on their way together */
+        bf16x8 f[2][4];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const bf16 *src = row(min((i + u) * 4 + wave, BLOCKS - 1));
+#pragma unroll
+            for (int k = 0; k < 4; k++) f[u][k] = *(const bf16x8 *)(src + k * 32);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            f32x4 a[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int b = 0; b < 2; b++) a[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[b][k], f[u][k], a[b], 0, 0, 0);
+            const int p = ((i + u) * 4 + wave) * 16 + l15;
+            if (p < POS) {
+                *(f32x4 *)(part + p * OUT_LD + 4 * lq) = a[0];
+                if (lq < 3) *(f32x4 *)(part + p * OUT_LD + 16 + 4 * lq) = a[1];
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < OUT_PH * OUT_PW / 256; i++) {
+        const int n = i * 256 + threadIdx.x, py = n / OUT_PW, px = n % OUT_PW, y = y0 + py, x = x0 + px;
+        if (y >= H || x >= W) continue;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            float v = 0.0f;
+#pragma unroll
+            for (int tap = 0; tap < 9; tap++) v += part[((py + tap / 3) * (OUT_PW + 2) + px + tap % 3) * OUT_LD + 3 * tap + c];
+            v += bias[c];
+            float val = (v + 1.0f) * 0.5f * 255.0f; /* flux_vae.c:820-833 */
+            val = val < 0.0f ? 0.0f : val > 255.0f ? 255.0f : val;
+            if (rgb) rgb[((size_t)y * W + x) * 3 + c] = (uint8_t)val;
+            if (rgb_f32) rgb_f32[((size_t)c * H + y) * W + x] = v;
+        }
+    }
+}
+
+/* 3 -> 128 channels (flux_vae.c:336-338): the 27 values under a position's window are one MFMA's K, gathered from the fp32 picture
+ * as the operand. As rows of 64 bf16 written by one kernel and multiplied by the next it was 69 + 146 us at 720 x 1296, and is 129; HBM: 478 MB out. A wave
+ * makes IN_BLOCKS blocks of 16 bordered positions (zeros on the border) and leaves one row of sums for the group norm. */
+#define IN_BLOCKS 8
+__global__ __launch_bounds__(256) void conv_in_kernel(float *__restrict__ out, const float *__restrict__ img, const bf16 *__restrict__ w, const float *__restrict__ bias,
+                                                      float *__restrict__ stats, int H, int W) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l15 = lane & 15, lq = lane >> 4;
+    const int wp = W + 2, rows = (H + 2) * wp, first = (blockIdx.x * 4 + wave) * IN_BLOCKS * 16;
+    bf16x8 fw[8]; /* w: [128][64], element 3 tap + channel, zeros from 27 on */
+    f32x4 bv[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        fw[i] = *(const bf16x8 *)(w + (16 * i + l15) * 64 + lq * 8);
+        bv[i] = *(const f32x4 *)(bias + 16 * i + 4 * lq);
+    }
+    float s[8], q[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) s[i] = q[i] = 0.0f;
+    float g[8]; /* a block's values, requested one block ahead */
+    bool inside_next;
+    const auto gather = [&](int blk) {
+        const int p = first + blk * 16 + l15, py = p / wp, px = p - py * wp;
+        inside_next = p < rows && py >= 1 && py <= H && px >= 1 && px <= W;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int k = lq * 8 + e, tap = k / 3, c = k - 3 * tap, y = py - 2 + tap / 3, x = px - 2 + tap % 3;
+            g[e] = inside_next && k < 27 && y >= 0 && y < H && x >= 0 && x < W ? img[((size_t)c * H + y) * W + x] : 0.0f;
+        }
+    };
+    gather(0);
+    for (int blk = 0; blk < IN_BLOCKS; blk++) {
+        const int p = first + blk * 16 + l15;
+        const bool inside = inside_next;
+        bf16x8 f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) f[e] = (bf16)g[e];
+        gather(blk + 1);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            f32x4 v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[i], f, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                v[e] = inside ? v[e] + bv[i][e] : 0.0f;
+                s[i] += v[e];
+                q[i] += v[e] * v[e];
+            }
+            if (p < rows) *(f32x4 *)(out + (size_t)p * 128 + 16 * i + 4 * lq) = v;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const f32x2 t = {row_sum(s[i]), row_sum(q[i])};
+        if (l15 == 0) *(f32x2 *)(stats + ((size_t)(blockIdx.x * 4 + wave) * 32 + 4 * i + lq) * 2) = t;
+    }
+}
+
 } // namespace
+
+int conv_probe_begin(int epilogue, int tile);
+void conv_probe_end(int slot);
+
+/* in: bf16 [(H + 2) * (W + 2)][128]; w: the first three rows of flux_hip_conv's weights; rgb 8-bit [H][W][3] and/or rgb_f32 [3][H][W] */
+extern "C" int flux_hip_vae_conv_out(uint8_t *rgb, float *rgb_f32, const void *in, const void *w, const float *bias, int H, int W) {
+    if (H <= 0 || W <= 0 || !in || !w || !bias) return flux_hip_fail("flux_hip_vae_conv_out: bad argument");
+    const int slot = conv_probe_begin(FLUX_HIP_EPI_CONV_F32, 17);
+    hipLaunchKernelGGL(conv_out_kernel, dim3((W + OUT_PW - 1) / OUT_PW, (H + OUT_PH - 1) / OUT_PH), dim3(256), 0, flux_hip_stream_handle(), rgb, rgb_f32, (const bf16 *)in,
+                       (const bf16 *)w, bias, H, W);
+    conv_probe_end(slot);
+    HIP_OK(hipGetLastError());
+    return 1;
+}
+
+/* img: fp32 [3][H][W]; w: bf16 [128][64]; out: fp32 [(H + 2) * (W + 2)][128], its border zeros; stats: as flux_hip_conv_stats */
+extern "C" int flux_hip_vae_conv_in(float *out, const float *img, const void *w, const float *bias, int H, int W, float *stats, int *stats_rows) {
+    if (H <= 0 || W <= 0 || !out || !img || !w || !bias || !stats || !stats_rows) return flux_hip_fail("flux_hip_vae_conv_in: bad argument");
+    const int rows = (H + 2) * (W + 2), wg = (rows + 64 * IN_BLOCKS - 1) / (64 * IN_BLOCKS);
+    const int slot = conv_probe_begin(FLUX_HIP_EPI_CONV_F32, 18);
+    hipLaunchKernelGGL(conv_in_kernel, dim3(wg), dim3(256), 0, flux_hip_stream_handle(), out, img, (const bf16 *)w, bias, stats, H, W);
+    conv_probe_end(slot);
+    HIP_OK(hipGetLastError());
+    *stats_rows = 4 * wg;
+    return 1;
+}
 
 /* Whether the kernel takes this convolution: two chunks of input channels at least, the image in 32-bit byte offsets below OUTSIDE, tile
  * numbers below 2^16, and no more rows of statistics than one per 32 positions of the bordered image + 2. */

@@ -32,12 +32,13 @@
 int flux_hip_vae_latent_in(void *out_bf16, const float *latent, const float *bn_mean, const float *bn_var,
                            const float *pq_w, const float *pq_b, int h, int w, float eps);
 int flux_hip_vae_key_bias(float *bias, int n, int keys);
-int flux_hip_vae_image_out(uint8_t *rgb, float *rgb_f32, const float *x, int ldx, int H, int W);
-int flux_hip_vae_image_in(void *out_bf16, const float *img, int H, int W);
 size_t flux_hip_vae_attention_work_floats(int n, int ld);
 int flux_hip_vae_attention(void *out, const void *q, const void *qkv, const void *vt, void *P, float *o32, float *work, int n, int keys, int ld, float scale,
                            int *done);
 int flux_hip_vae_upsample2x_bf16(void *out_bf16, const void *x_bf16, int hp, int wp, int C);
+/* conv.hip */
+int flux_hip_vae_conv_out(uint8_t *rgb, float *rgb_f32, const void *in, const void *w, const float *bias, int H, int W);
+int flux_hip_vae_conv_in(float *out, const float *img, const void *w, const float *bias, int H, int W, float *stats, int *stats_rows);
 /* gemm.hip */
 int flux_hip_conv_image(int epilogue, const void *in, int in_wp, int packed, const void *w, const float *bias, const float *res, void *out, int rows, int wp,
                         int cin, int cout, int taps, float *stats, int *stats_rows);
@@ -82,7 +83,7 @@ struct flux_hip_vae {
     vattn attn;
     float *out_g, *out_b;
     /* encoder */
-    vconv enc_conv_in; /* K = 27 in one row of 64, see vae_image_in_kernel */
+    vconv enc_conv_in; /* K = 27 in one row of 64, see conv_in_kernel */
     vconv enc_down_conv[3], enc_conv_out, quant;
     vres enc_down[8], enc_mid[2];
     vattn enc_attn;
@@ -521,9 +522,8 @@ int flux_hip_vae_decode(flux_hip_vae *v, const float *latent, int h, int w, uint
         }
     }
     if (!flux_hip_group_norm_stats(s.A, NULL, s.x, 0, v->out_g, v->out_b, v->gn, s.hp, s.wp, 128, v->eps, 1, v->st_x, s.x_rows)) return 0;
-    if (!run_conv(&s, &v->conv_out, FLUX_HIP_EPI_CONV_F32, s.A, NULL, v->Hb, 1, NULL, NULL)) return 0;
     const int H = 16 * h, W = 16 * w;
-    if (!flux_hip_vae_image_out(rgb ? v->img_u8 : NULL, rgb_f32 ? v->img_f32 : NULL, v->Hb, v->conv_out.cout_pad, H, W)) return 0;
+    if (!flux_hip_vae_conv_out(rgb ? v->img_u8 : NULL, rgb_f32 ? v->img_f32 : NULL, s.A, v->conv_out.w, v->conv_out.b, H, W)) return 0;
     if (rgb) flux_hip_prefault(rgb, (size_t)H * W * 3);
     if (rgb_f32) flux_hip_prefault(rgb_f32, (size_t)H * W * 3 * 4);
     if (rgb && !flux_hip_download(rgb, v->img_u8, (size_t)H * W * 3)) return 0;
@@ -541,8 +541,7 @@ int flux_hip_vae_encode(flux_hip_vae *v, const float *img, int H, int W, float *
     if (!vae_complete(v, SIDE_ENCODER) || !ensure_work(v, h, w)) return 0;
     vstate s = {v, v->X, v->Y, (char *)v->A_base + v->guard * 2, H + 2, W + 2, 0, 0};
     if (!flux_hip_upload(v->img_f32, img, (size_t)3 * H * W * 4)) return 0;
-    if (!flux_hip_vae_image_in(s.A, v->img_f32, H, W)) return 0;
-    if (!run_conv(&s, &v->enc_conv_in, FLUX_HIP_EPI_CONV_F32, s.A, NULL, s.x, 1, v->st_x, &s.x_rows)) return 0;
+    if (!flux_hip_vae_conv_in(s.x, v->img_f32, v->enc_conv_in.w, v->enc_conv_in.b, H, W, v->st_x, &s.x_rows)) return 0;
     int done = 0, bi = 0;
     const int total = 11; /* 8 down + 3 mid, the reference's count (flux_vae.c:343) */
     for (int level = 0; level < 4; level++) {

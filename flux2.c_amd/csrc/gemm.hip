@@ -1652,6 +1652,19 @@ static int probe_slot(int epilogue) {
     return g_probe_n++;
 }
 
+/* for the convolutions of conv.hip that are not launched from here */
+int conv_probe_begin(int epilogue, int tile) {
+    const int slot = probe_slot(epilogue);
+    if (slot >= 0) {
+        g_probe_tile[slot] = (unsigned char)tile;
+        (void)hipEventRecord(g_probe_ev[slot][0], flux_hip_stream_handle());
+    }
+    return slot;
+}
+void conv_probe_end(int slot) {
+    if (slot >= 0) (void)hipEventRecord(g_probe_ev[slot][1], flux_hip_stream_handle());
+}
+
 /* Tile and K-split choice, then the launch; `allowed` has bit t set for every tile id that may be used. */
 static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, int *tile_out = nullptr, const AdalnArgs *adaln = nullptr,
                          int *adaln_done = nullptr, float *fixed_ws = nullptr, size_t fixed_ws_bytes = 0, int *leave_slices = nullptr) {
@@ -2049,11 +2062,7 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
         g.ws_rows = M;
     }
     /* one record per convolution: K slices and their second pass together */
-    const int slot = probe_slot(epilogue);
-    if (slot >= 0) {
-        g_probe_tile[slot] = (unsigned char)tile;
-        (void)hipEventRecord(g_probe_ev[slot][0], flux_hip_stream_handle());
-    }
+    const int slot = conv_probe_begin(epilogue, tile);
     int ok = 1;
     if (g.ksplit == 1 && tile == CONV_PATCH) {
         ok = conv3_launch(!bf, g.A[0], g.W[0], g.bias, g.res, g.C[0], height, width, g.lda, N, g.stats, stats_rows, compute_units() & ~7);
@@ -2065,7 +2074,7 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
         if (g.ksplit > 1) ok = conv_tile_launch<EPI_CONV_PARTIAL>(g, tile);
         ok = ok && (bf ? conv_finish<FLUX_HIP_EPI_CONV_BF16>(g) : conv_finish<FLUX_HIP_EPI_CONV_F32>(g));
     }
-    if (slot >= 0) (void)hipEventRecord(g_probe_ev[slot][1], flux_hip_stream_handle());
+    conv_probe_end(slot);
     return ok;
 }
 

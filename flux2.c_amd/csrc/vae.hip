@@ -543,25 +543,6 @@ __global__ __launch_bounds__(256) void vae_transpose_kernel(bf16 *__restrict__ v
     }
 }
 
-/* decoder output fp32 [hp*wp, ldx] (channels 0..2 used) -> image: 8-bit [H, W, 3] with the
- * reference's conversion (v + 1) * 0.5 * 255, clamped, truncated (flux_vae.c:820-833), and
- * optionally the unquantised values as [3, H, W] */
-__global__ __launch_bounds__(256) void vae_image_kernel(uint8_t *__restrict__ rgb, float *__restrict__ rgb_f32, const float *__restrict__ x,
-                                                        int ldx, int H, int W) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= H * W) return;
-    const int y = i / W, xx = i - y * W;
-    const float *src = x + ((size_t)(y + 1) * (W + 2) + xx + 1) * ldx;
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        const float v = src[c];
-        float val = (v + 1.0f) * 0.5f * 255.0f;
-        val = val < 0.0f ? 0.0f : val > 255.0f ? 255.0f : val;
-        if (rgb) rgb[(size_t)i * 3 + c] = (uint8_t)val;
-        if (rgb_f32) rgb_f32[(size_t)c * H * W + i] = v;
-    }
-}
-
 /* ------------------------------------------------------------------ host entry points */
 
 extern "C" int flux_hip_vae_latent_in(void *out_bf16, const float *latent, const float *bn_mean, const float *bn_var,
@@ -724,11 +705,5 @@ extern "C" int flux_hip_transpose_bf16(void *vt, int ld, const void *v, int ldv,
     hipLaunchKernelGGL(vae_transpose_kernel, dim3((ld + 63) / 64, cols / 64), dim3(256), 0, flux_hip_stream_handle(), (bf16 *)vt, ld, (const bf16 *)v,
                        ldv, rows);
     LAUNCH_OK("vae_transpose_kernel");
-    return 1;
-}
-
-extern "C" int flux_hip_vae_image_out(uint8_t *rgb, float *rgb_f32, const float *x, int ldx, int H, int W) {
-    hipLaunchKernelGGL(vae_image_kernel, dim3((H * W + 255) / 256), dim3(256), 0, flux_hip_stream_handle(), rgb, rgb_f32, x, ldx, H, W);
-    LAUNCH_OK("vae_image_kernel");
     return 1;
 }

@@ -115,6 +115,50 @@ def test_conv3x3(hip, oracle_mod, switches, tile, shape):
     assert rel_l2(from_padded(got, H, W), want) < 4e-3
 
 
+@pytest.mark.parametrize("H,W", [(1, 1), (16, 32), (17, 33), (5, 70), (48, 16)])
+def test_conv_out_to_picture(hip, oracle_mod, H, W):
+    """128 -> 3 channels straight to the picture: against the oracle's convolution, and the bytes from the floats; tiles cut
+    on both sides, one whole one. Weights as the VAE holds them, padded to 64 rows of which three are read."""
+    import ctypes
+    x, w = q(normal_f32((128, H, W), 68, 1)), q(normal_f32((3, 128, 3, 3), 68, 2, 0.0, 0.02))
+    b = normal_f32((3,), 68, 3, 0.0, 0.1)
+    din, dw, db = hip.DevBuf.from_array(f32_to_bf16(to_padded(x))), hip.DevBuf.from_array(conv_weight(w)), hip.DevBuf.from_array(b)
+    rgb, f32 = hip.DevBuf.from_array(np.full(H * W * 3 + 1, 77, np.uint8)), hip.DevBuf.from_array(np.full(3 * H * W + 1, 7.0, np.float32))
+    L = hip.lib()
+    L.flux_hip_vae_conv_out.argtypes = [ctypes.c_void_p] * 5 + [ctypes.c_int] * 2
+    hip.check(L.flux_hip_vae_conv_out(rgb.ptr, f32.ptr, din.ptr, dw.ptr, db.ptr, H, W))
+    got, bytes_ = f32.to_array(np.float32, (3 * H * W + 1,)), rgb.to_array(np.uint8, (H * W * 3 + 1,))
+    assert got[-1] == 7.0 and bytes_[-1] == 77
+    got = got[:-1].reshape(3, H, W)
+    assert rel_l2(got, oracle_mod.conv2d(x, w, b, 1)) < 2e-6
+    want = np.clip((got + np.float32(1.0)) * np.float32(0.5) * np.float32(255.0), 0, 255).astype(np.uint8).transpose(1, 2, 0)
+    np.testing.assert_array_equal(bytes_[:-1].reshape(H, W, 3), want)
+
+
+@pytest.mark.parametrize("H,W", [(1, 1), (16, 16), (5, 70), (33, 47)])
+def test_conv_in_from_picture(hip, H, W):
+    """3 -> 128 channels from the fp32 picture: bit for bit the 1x1 convolution of flux_hip_vae_image_in's rows (the same 27
+    products in one MFMA and a second one of zeros), with zeros on the border, nothing behind it, and the sums of what was written."""
+    import ctypes
+    img = vae_test_image(16 * -(-H // 16), 16 * -(-W // 16), 69)[:, :H, :W].copy()
+    w64 = np.zeros((128, 64), np.float32)
+    w64[:, :27] = q(normal_f32((128, 27), 69, 2, 0.0, 0.2))
+    b, rows, wp = normal_f32((128,), 69, 3), (H + 2) * (W + 2), W + 2
+    dimg, dw, db = hip.DevBuf.from_array(img), hip.DevBuf.from_array(f32_to_bf16(w64)), hip.DevBuf.from_array(b)
+    cols, want = hip.DevBuf(rows * 64 * 2), hip.DevBuf(rows * 128 * 4)
+    L = hip.lib()
+    hip.check(L.flux_hip_vae_image_in(cols.ptr, dimg.ptr, H, W))
+    hip.check(L.flux_hip_conv(hip.EPI_CONV_F32, cols.ptr, dw.ptr, db.ptr, None, want.ptr, rows, wp, 64, 128, 1))
+    out, n = hip.DevBuf.from_array(np.full((rows + 1, 128), 3.0, np.float32)), ctypes.c_int(0)
+    stats = hip.DevBuf.from_array(np.full(((rows // 32 + 2) * 32 * 2 + 256,), np.nan, np.float32))
+    L.flux_hip_vae_conv_in.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 2 + [ctypes.c_void_p] * 2
+    hip.check(L.flux_hip_vae_conv_in(out.ptr, dimg.ptr, dw.ptr, db.ptr, H, W, stats.ptr, ctypes.byref(n)))
+    got = out.to_array(np.float32, (rows + 1, 128))
+    np.testing.assert_array_equal(got[:rows], want.to_array(np.float32, (rows, 128)))
+    assert (got[rows] == 3.0).all() and border_is_zero(got[:rows], H, W)
+    check_sums(stats.to_array(np.float32, (n.value, 32, 2)).astype(np.float64).sum(0), got[:rows])
+
+
 def test_conv_output_widths(hip, oracle_mod):
     """64 output channels (the padded conv_out) and 512 (mid block), automatic tile."""
     for cin, cout, H, W in ((128, 64, 11, 6), (512, 512, 6, 6)):
