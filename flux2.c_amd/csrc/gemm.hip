@@ -229,13 +229,19 @@ __device__ __forceinline__ int bf16_feature(int blk, int r) { return blk < (TN &
  * last column tile is cut off. Its missing weight rows are read from the matrix's last row and its missing columns are
  * not stored (whole 16-column blocks for fp32 outputs, whole pairs of blocks for bf16: N is a multiple of 32). */
 template <int BN> struct CutTile { static constexpr bool value = BN % 64 != 0; };
+/* the tiles of gemm4x_kernel */
+template <int BN, int WM> struct IsWide { static constexpr bool value = 2 * WM * BN > 256 * 256; };
 /* SiLU(gate) * up: blocks alternate gate, up, so that a lane holds matching pairs; the (gate, up) pairs interleave
- * two by two in the same way, and a last odd pair keeps the plain numbering (features 16 k + r). */
+ * two by two in the same way, and a last odd pair keeps the plain numbering (features 16 k + r). With an odd number of
+ * blocks the last one holds gate rows and up rows, two and two: a lane's four results are gate, gate, up, up of two features. */
 template <int TN>
 __device__ __forceinline__ int swiglu_feature(int blk, int r) {
     const int k = blk >> 1;
+    if (TN % 2 && blk == TN - 1) return 16 * k + 2 * (r >> 2) + (r & 1);
     return k < 2 * (TN / 4) ? bf16_pair_feature(k, r) : 16 * k + r;
 }
+template <int TN>
+__device__ __forceinline__ bool swiglu_up(int blk, int r) { return TN % 2 && blk == TN - 1 ? r & 2 : blk & 1; }
 
 /* Weight row that feeds column v of the tile. */
 template <int BN, int WN, int EPI>
@@ -245,13 +251,14 @@ __device__ __forceinline__ int weight_row(const GemmArgs &g, int tn, int v) {
     if (EPI == FLUX_HIP_EPI_SWIGLU || (EPI == EPI_QKV_SWIGLU && tn >= g.nq_tiles)) {
         int idx = wv * (WN / 2) + swiglu_feature<TN>(blk, r);
         if (CutTile<BN>::value && EPI == FLUX_HIP_EPI_SWIGLU) idx = min(idx, g.N / 2 - 1 - tn * (BN / 2));
-        if (EPI == EPI_QKV_SWIGLU) return ((blk & 1) ? g.w_row2 : g.w_row1) + (tn - g.nq_tiles) * (BN / 2) + idx;
-        return ((blk & 1) ? g.w_row1 : g.w_row0) + tn * (BN / 2) + idx;
+        if (CutTile<BN>::value && EPI == EPI_QKV_SWIGLU) idx = min(idx, g.w_row2 - g.w_row1 - 1 - (tn - g.nq_tiles) * (BN / 2));
+        if (EPI == EPI_QKV_SWIGLU) return (swiglu_up<TN>(blk, r) ? g.w_row2 : g.w_row1) + (tn - g.nq_tiles) * (BN / 2) + idx;
+        return (swiglu_up<TN>(blk, r) ? g.w_row1 : g.w_row0) + tn * (BN / 2) + idx;
     }
     int col;
     if (EPI == FLUX_HIP_EPI_BF16 || EPI == EPI_QKV_SWIGLU || EPI == FLUX_HIP_EPI_CONV_BF16 || EPI == EPI_EXP) col = tn * BN + wv * WN + bf16_feature<TN>(blk, r);
     else col = tn * BN + v;
-    if (CutTile<BN>::value) col = min(col, g.N - 1);
+    if (CutTile<BN>::value) col = min(col, (EPI == EPI_QKV_SWIGLU ? g.nq_cols : g.N) - 1);
     return g.w_row0 + col;
 }
 
@@ -275,9 +282,10 @@ template <int V> struct IntC { static constexpr int value = V; };
  * token m = lane%16 of the 16-row block. */
 template <int BN, int WM, int WN, int EPI, bool HERE = false>
 __device__ __forceinline__ void store_tile_to(const GemmArgs &g, const TileId &t, f32x4 (&acc_in)[WN / 16][WM / 16], int m0, int M,
-                                              int wm, int wn, int l15, int lq, int prow, void *Cp, const int ldc, const int tn) {
+                                              int wm, int wn, int l15, int lq, int prow, void *Cp, const int ldc, const int tn, const int cols) {
     constexpr int TM = WM / 16, TN = WN / 16;
     const int prob = t.prob, n0 = tn * BN, ks = t.ks;
+    constexpr bool LANE_CUT = CutTile<BN>::value && IsWide<BN, WM>::value; /* a last column tile is cut at any multiple of eight columns, lane by lane */
     const bool aligned16 = (((uintptr_t)Cp | ((uintptr_t)ldc << 1)) & 15) == 0; /* every 8-feature group of the output starts on 16 bytes */
     f32x4 acc_here[HERE ? TN : 1][HERE ? TM : 1];
     auto &acc = [&]() -> auto & { if constexpr (HERE) return acc_here; else return acc_in; }();
@@ -344,8 +352,9 @@ __device__ __forceinline__ void store_tile_to(const GemmArgs &g, const TileId &t
             }
         }
         if (EPI == FLUX_HIP_EPI_SWIGLU) {
-            if (CutTile<BN>::value && tn * BN + wn * WN >= g.N) continue; /* the same for the whole wave (N counts gate and up columns) */
-            /* see swiglu_feature: two (gate, up) pairs give eight consecutive features, a last odd pair four */
+            if (CutTile<BN>::value && tn * BN + wn * WN >= cols) continue; /* the same for the whole wave (gate and up columns count) */
+            /* see swiglu_feature: two (gate, up) pairs give eight consecutive features, a last odd pair four, a last odd block two */
+            const int left = LANE_CUT ? cols / 2 - tn * (BN / 2) - wn * (WN / 2) : 0; /* features of the wave's that exist */
             bf16 *C = (bf16 *)Cp + (size_t)m * ldc + tn * (BN / 2) + wn * (WN / 2);
             bf16x4 o[TN / 2];
 #pragma unroll
@@ -353,20 +362,25 @@ __device__ __forceinline__ void store_tile_to(const GemmArgs &g, const TileId &t
 #pragma unroll
                 for (int e = 0; e < 4; e++) o[k][e] = (bf16)(silu_f(acc[2 * k][j][e]) * acc[2 * k + 1][j][e]);
 #pragma unroll
-            for (int p = 0; p < TN / 4; p++) store_bf16x8(C + 32 * p + 8 * lq, o[2 * p], o[2 * p + 1], aligned16);
-            if (TN / 2 % 2) *(bf16x4 *)(C + 16 * (TN / 2 - 1) + 4 * lq) = o[TN / 2 - 1];
+            for (int p = 0; p < TN / 4; p++)
+                if (!LANE_CUT || 32 * p + 8 * lq < left) store_bf16x8(C + 32 * p + 8 * lq, o[2 * p], o[2 * p + 1], aligned16);
+            if (TN / 2 % 2 && (!LANE_CUT || 16 * (TN / 2 - 1) + 4 * lq < left)) *(bf16x4 *)(C + 16 * (TN / 2 - 1) + 4 * lq) = o[TN / 2 - 1];
+            if (TN % 2 && (!LANE_CUT || 16 * (TN / 2) + 2 * lq < left)) {
+                const f32x4 a = acc[TN - 1][j];
+                *(bf16x2 *)(C + 16 * (TN / 2) + 2 * lq) = bf16x2{(bf16)(silu_f(a[0]) * a[2]), (bf16)(silu_f(a[1]) * a[3])};
+            }
         } else if (EPI == FLUX_HIP_EPI_BF16) {
             /* see bf16_pair_feature: blocks 2p and 2p + 1 give eight consecutive features */
             bf16 *C = (bf16 *)Cp + (size_t)m * ldc + n0 + wn * WN + 8 * lq;
 #pragma unroll
             for (int p = 0; p < TN / 2; p++) {
-                if (CutTile<BN>::value && n0 + wn * WN + 32 * p >= g.N) continue; /* the same for the whole wave */
+                if (CutTile<BN>::value && n0 + wn * WN + 32 * p + (LANE_CUT ? 8 * lq : 0) >= cols) continue; /* (without LANE_CUT the same for the whole wave) */
                 bf16x4 lo, hi;
 #pragma unroll
                 for (int e = 0; e < 4; e++) { lo[e] = (bf16)acc[2 * p][j][e]; hi[e] = (bf16)acc[2 * p + 1][j][e]; }
                 store_bf16x8(C + 32 * p, lo, hi, aligned16);
             }
-            if (TN % 2 && !(CutTile<BN>::value && n0 + wn * WN + 16 * (TN - 1) >= g.N)) { /* a last block without a neighbour */
+            if (TN % 2 && !(CutTile<BN>::value && n0 + wn * WN + 16 * (TN - 1) + (LANE_CUT ? 4 * lq : 0) >= cols)) { /* a last block without a neighbour */
                 bf16x4 o;
 #pragma unroll
                 for (int e = 0; e < 4; e++) o[e] = (bf16)acc[TN - 1][j][e];
@@ -566,12 +580,12 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, const TileId &t, f
          * are then work of that side; left to itself the compiler converted the whole tile to bf16 in front of the
          * branch, for both sides, and kept the hundred results in registers next to the other side's work, past
          * what the register file holds beside the fragments. */
-        if (t.tn < g.nq_tiles) store_tile_to<BN, WM, WN, FLUX_HIP_EPI_BF16, true>(g, t, acc, m0, M, wm, wn, l15, lq, prow, g.C[0], g.ldc, t.tn);
-        else store_tile_to<BN, WM, WN, FLUX_HIP_EPI_SWIGLU, true>(g, t, acc, m0, M, wm, wn, l15, lq, prow, g.C2, g.ldc2, t.tn - g.nq_tiles);
+        if (t.tn < g.nq_tiles) store_tile_to<BN, WM, WN, FLUX_HIP_EPI_BF16, true>(g, t, acc, m0, M, wm, wn, l15, lq, prow, g.C[0], g.ldc, t.tn, g.nq_cols);
+        else store_tile_to<BN, WM, WN, FLUX_HIP_EPI_SWIGLU, true>(g, t, acc, m0, M, wm, wn, l15, lq, prow, g.C2, g.ldc2, t.tn - g.nq_tiles, g.N - g.nq_cols);
     } else {
         /* PINNED: the kernels whose accumulators live in AGPRs take them out row by row as well (the 16-byte / 8-byte
          * choice of the bf16 stores is a branch with the same conversions on both sides) */
-        store_tile_to<BN, WM, WN, EPI, PINNED>(g, t, acc, m0, M, wm, wn, l15, lq, prow, g.C[t.prob], g.ldc, t.tn);
+        store_tile_to<BN, WM, WN, EPI, PINNED>(g, t, acc, m0, M, wm, wn, l15, lq, prow, g.C[t.prob], g.ldc, t.tn, g.N);
     }
 }
 
@@ -693,6 +707,10 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_kernel(GemmArgs g) {
 #define MFMA_AGPR(acc, a, b) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b))
 /* the first MFMA of an accumulator block: adds to zero instead of to the register's old contents */
 #define MFMA_AGPR_NEW(acc, a, b) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b))
+
+/* accumulators in VGPRs (gemm4x_kernel) */
+#define MFMA_VGPR(acc, a, b) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b))
+#define MFMA_VGPR_NEW(acc, a, b) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b))
 
 /* The compiler neither sees those MFMAs' register hazards nor keeps plain register moves in order
  * around them. acc_fence passes every accumulator through an empty asm statement that is ordered
@@ -1110,6 +1128,189 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+/* Tiles with more accumulators than the 256 AGPRs hold (288 x 288, 384 x 224, 320 x 256 and the like; 16 x 16 blocks beyond the 64th
+ * accumulate in VGPRs), for the fused projection of a single-stream block. What bounds the 4-wave tiles beside the matrix
+ * pipes is LDS traffic and the issue of loads, both a matter of a wave tile's circumference: 144 x 144 takes 0.222 fragment reads and
+ * 0.111 global->LDS loads per MFMA, 144 x 96 0.278 and 0.139; and more sizes leave fewer units idle in the last round (768 x 27648 is 432 tiles
+ * of 256 x 192, two rounds, and 250 of 384 x 224, one). K = 3072 and N = 27648 with the weights from HBM, us, the best tile of up to 256
+ * registers and this kernel's: 600 rows 108 -> 83, 768 109 -> 94, 1202 168 -> 159, 1536 194 -> 175, 2304 273 -> 260, 2560 324 -> 299,
+ * 4608 544 -> 518 (1512 TFLOP/s), 5120 601 -> 576, 10000 1179 -> 1133, 13056 1525 -> 1497. What pays for the registers and the LDS (two slots
+ * of one K step per operand):
+ * activation fragments of the next half-step are read into the registers that this one has done with, a row of blocks behind the
+ * MFMAs (the last SP rows, whose reads the barrier would have to wait for, have spare ones; the weights are double-buffered);
+ * and with two slots for both operands the loads of a tile's last two steps all belong to the next tile, so that one set of source
+ * offsets is enough.
+ *
+ * Step kt: half 0 multiplies (kt, first 32 of K) and reads (kt, second 32), weights first. Once all waves have read the weights (a
+ * barrier behind LW MFMAs) their slot takes those of step kt + 2. At the barrier between the halves the same holds for the
+ * activations, which follow in half 1, and step kt + 1 has landed: everything but the weights of step kt + 2. Reading the weights
+ * two, three or four MFMAs apart and the barrier six or twelve behind them measured the same within 1 %. */
+template <int TM, int TN, int SP, int RW, int RA>
+struct WideReads { /* which fragment is read behind MFMA b of a half-step: of[b], or -1 */
+    static constexpr int NF = TM + TN;
+    signed char of[TM * TN];
+    static constexpr int at(int q) {
+        const int b = q < TN ? RW * q : RW * TN + RA * (q - TN), row = q - TN - SP;
+        return row < 0 || b >= (row + 1) * TN ? b : (row + 1) * TN;
+    }
+    constexpr WideReads() : of() {
+        for (int b = 0; b < TM * TN; b++) of[b] = -1;
+        for (int q = 0; q < NF; q++) of[at(q)] = (signed char)q;
+    }
+    static constexpr int issued(int first, int b) {
+        int n = 0;
+        for (int q = first; q < NF; q++) n += at(q) <= b;
+        return n;
+    }
+    static constexpr bool in_order() {
+        for (int q = 1; q < NF; q++)
+            if (at(q) <= at(q - 1)) return false;
+        return true;
+    }
+};
+
+template <int TM, int TN, int EPI>
+__global__ __launch_bounds__(256) void gemm4x_kernel(GemmArgs g) {
+    constexpr int WGM = 2, WGN = 2;
+    constexpr int WM = 16 * TM, WN = 16 * TN, BM = WGM * WM, BN = WGN * WN;
+    constexpr int RPP = 32;
+    constexpr int LA = BM / RPP, LB = BN / RPP, NL = LA + LB;
+    constexpr int NF = TM + TN, NM = TM * TN;
+    constexpr int ASZ = BM * 128, WSZ = BN * 128;
+    static_assert(2 * (ASZ + WSZ) <= 160 * 1024 && NM > 64 && IsWide<BN, WM>::value, "two slots per operand");
+    constexpr int SP = 2;                       /* activation rows with spare registers */
+    constexpr int AGPR_BLOCKS = 64;
+    /* the MFMA behind which fragment q is read: weights, the last SP activation rows, the other activation rows, each when its MFMAs of
+     * this half have been issued */
+    constexpr int RW = 2, RA = (NM - 8 - RW * TN) / TM;
+    constexpr int LW = RW * (TN - 1) + 6;   /* MFMAs in front of the barrier that frees the weights' slot */
+    constexpr WideReads<TM, TN, SP, RW, RA> reads;
+    constexpr int LATE = reads.issued(TN, LW - 1); /* reads behind the weights' by then */
+    static_assert(RA >= 2 && reads.at(NF - 1) + 6 <= NM && reads.in_order(), "reads in order between the MFMAs, done before the barrier");
+    constexpr int SW = (NM - LW) / LB, SA = NM / LA;
+    static_assert(SW >= 2 && SA >= 2, "the loads of a half fit between its MFMAs");
+    constexpr int E = EpilogueOps<EPI, TM, TN>::value;
+    constexpr int AHEAD = LB, AHEAD_STORES = LB + E < 63 ? LB + E : 63;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+    const int wm = wave / WGN, wn = wave % WGN;
+    const int lrow = tid >> 3, lchunk = tid & 7;
+    const int l15 = lane & 15, lq = lane >> 4;
+    const int swzl = lds_swz(l15);
+    const unsigned coff0 = (lq ^ swzl) << 4, coff1 = ((4 + lq) ^ swzl) << 4;
+    const unsigned a_frag = (wm * WM + l15) * 128, w_frag = 2 * ASZ + (wn * WN + l15) * 128;
+
+    int vb = blockIdx.x;
+    TileId t;
+    if (!decode_tile<false>(g, vb, t)) return;
+
+    unsigned voff[NL];
+    const char *baseA, *baseW;
+    auto set_sources = [&](const TileId &tt) {
+        const int M = g.M[tt.prob], m0 = tt.tml * BM;
+        int lr = lrow;
+        asm volatile("" : "+v"(lr));
+        const int chunk = (lchunk ^ lds_swz(lr)) << 3;
+        baseA = (const char *)g.A[tt.prob];
+        baseW = (const char *)g.W[tt.prob];
+#pragma unroll
+        for (int i = 0; i < LA; i++) voff[i] = ((unsigned)min(m0 + lr + i * RPP, M - 1) * (unsigned)g.lda + chunk) * 2u;
+#pragma unroll
+        for (int i = 0; i < LB; i++) voff[LA + i] = ((unsigned)weight_row<BN, WN, EPI>(g, tt.tn, lr + i * RPP) * (unsigned)g.ldw + chunk) * 2u;
+    };
+    auto issue1 = [&](int ks, int slot, int i) { /* load i of K step ks: activation rows, then weight rows */
+        const char *base = (i < LA ? baseA : baseW) + (ptrdiff_t)ks * 128;
+        const int dst = i < LA ? slot * ASZ + (wave * 8 + i * RPP) * 128 : 2 * ASZ + slot * WSZ + (wave * 8 + (i - LA) * RPP) * 128;
+        asm volatile("" : "+v"(voff[i]));
+        __builtin_amdgcn_global_load_lds(GLOBAL_PTR(base + voff[i]), LDS_PTR(smem + dst), 16, 0, 0);
+    };
+    const int KT = g.K >> 6; /* at least 4 */
+
+    bf16x8 w0[TN], w1[TN], fa[TM];
+    f32x4 acc[TN][TM];
+    int slot = 0;
+    set_sources(t);
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int i = 0; i < NL; i++) issue1(s, s, i);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < TN; i++) w0[i] = *(const bf16x8 *)(smem + w_frag + coff0 + i * 2048);
+#pragma unroll
+    for (int j = 0; j < TM; j++) fa[j] = *(const bf16x8 *)(smem + a_frag + coff0 + j * 2048);
+    bool strict = false;
+
+    for (;;) {
+        auto serp = [](int b) { return ((b / TN) & 1) ? TN - 1 - b % TN : b % TN; };
+        /* a half-step: MFMAs of the fragments held, reads of the next half's from the rows at xa, xw, and `between` at every MFMA */
+        auto half = [&](bf16x8 (&w)[TN], bf16x8 (&wn_)[TN], unsigned xa, unsigned xw, auto new_c, auto between) {
+            bf16x8 sp[SP];
+#pragma unroll
+            for (int b = 0; b < NM; b++) {
+                const int j = b / TN, i = serp(b);
+                if (decltype(new_c)::value) {
+                    if (b < AGPR_BLOCKS) MFMA_AGPR_NEW(acc[i][j], w[i], fa[j]);
+                    else MFMA_VGPR_NEW(acc[i][j], w[i], fa[j]);
+                } else {
+                    if (b < AGPR_BLOCKS) MFMA_AGPR(acc[i][j], w[i], fa[j]);
+                    else MFMA_VGPR(acc[i][j], w[i], fa[j]);
+                }
+                const int q = reads.of[b];
+                if (q >= 0) {
+                    if (q < TN) wn_[q] = *(const bf16x8 *)(smem + xw + q * 2048);
+                    else if (q < TN + SP) sp[q - TN] = *(const bf16x8 *)(smem + xa + (TM - SP + q - TN) * 2048);
+                    else fa[q - TN - SP] = *(const bf16x8 *)(smem + xa + (q - TN - SP) * 2048);
+                }
+                between(b);
+            }
+#pragma unroll
+            for (int k = 0; k < SP; k++) fa[TM - SP + k] = sp[k];
+        };
+        /* ks: the K step that is requested, of the tile that voff and the bases belong to */
+        auto step = [&](int ks, auto wait_c, auto first_c) {
+            constexpr int WAIT = decltype(wait_c)::value;
+            constexpr bool FIRST = decltype(first_c)::value;
+            half(w0, w1, a_frag + slot * ASZ + coff1, w_frag + slot * WSZ + coff1, first_c, [&](int b) {
+                if (b == LW - 1) asm volatile("s_waitcnt lgkmcnt(%0)\n\ts_barrier" ::"n"(LATE) : "memory"); /* all have their weights of this step */
+                if (b >= LW && (b - LW) % SW == 0 && (b - LW) / SW < LB) issue1(ks, slot, LA + (b - LW) / SW);
+            });
+            if (FIRST && strict) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD) : "memory");
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(WAIT) : "memory");
+            const int ns = slot ^ 1;
+            half(w1, w0, a_frag + ns * ASZ + coff0, w_frag + ns * WSZ + coff0, BoolC<false>{}, [&](int b) {
+                if (b % SA == 1 && b / SA < LA) issue1(ks, slot, b / SA);
+            });
+            slot = ns;
+        };
+        step(2, IntC<AHEAD_STORES>{}, BoolC<true>{});
+        for (int kt = 1; kt < KT - 2; kt++) step(kt + 2, IntC<AHEAD>{}, BoolC<false>{});
+        /* the last two steps request the first two of the workgroup's next tile; after the last tile this tile's once more,
+         * into slots that nobody reads again */
+        const TileId done = t;
+        vb += gridDim.x;
+        const bool again = vb < g.vgrid && decode_tile<false>(g, vb, t);
+        if (again) set_sources(t);
+#pragma clang loop unroll(disable)
+        for (int kt = 0; kt < 2; kt++) step(kt, IntC<AHEAD>{}, BoolC<false>{});
+
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); /* the last MFMA results retire before they are read */
+#pragma unroll
+        for (int b = 0; b < NM; b++) {
+            if (b < AGPR_BLOCKS) asm volatile("" : "+a"(acc[serp(b)][b / TN]));
+            else asm volatile("" : "+v"(acc[serp(b)][b / TN]));
+        }
+        int l15e = l15, lqe = lq;
+        asm volatile("" : "+v"(l15e), "+v"(lqe));
+        store_tile<BN, WM, WN, EPI, WGM, true>(g, done, acc, done.tml * BM, g.M[done.prob], wm, wn, l15e, lqe, done.tm * WGM + wm);
+        if (!again) break;
+        strict = done.tml * BM + wm * WM + WM > g.M[done.prob] || (CutTile<BN>::value && (done.tn == g.ntiles - 1 || done.tn == g.nq_tiles - 1));
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 /* ------------------------------------------------------------------ host side */
 
 static int g_persistent = 1;
@@ -1207,6 +1408,29 @@ static int launch_4d(GemmArgs &g) {
     return 1;
 }
 
+template <int TM, int TN, int EPI>
+static int launch_4x(GemmArgs &g) {
+    constexpr int BM = 32 * TM, BN = 32 * TN, LDS = 2 * (BM + BN) * 128;
+    static bool attr_done = false;
+    auto kern = gemm4x_kernel<TM, TN, EPI>;
+    if (!attr_done) {
+        HIP_OK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        attr_done = true;
+    }
+    set_row_tiles(g, BM);
+    g.nq_tiles = (g.nq_cols + BN - 1) / BN; /* both sides of the fused projection end in a tile that may be cut off */
+    g.ntiles = g.nq_tiles + (g.N - g.nq_cols + BN - 1) / BN;
+    g.total_tiles = g.mtiles * g.ntiles;
+    size_t span = ((size_t)max(max(g.w_row0, g.w_row1), g.w_row2) + g.N) * g.ldw * 2;
+    for (int i = 0; i < GEMM_MAX_PARTS; i++) span = max(span, (size_t)g.M[i] * g.lda * 2);
+    if (span >= ((size_t)1 << 32)) return g.N % 128 == 0 ? launch_cfg<128, 128, 2, 2, EPI>(g) : launch_cfg<64, 64, 2, 2, EPI>(g);
+    g.vgrid = (g.total_tiles + 7) & ~7;
+    const int grid = min(g.vgrid, compute_units() & ~7);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), LDS, flux_hip_stream_handle(), g);
+    HIP_OK(hipGetLastError());
+    return 1;
+}
+
 template <int EPI>
 static int launch_epi(GemmArgs &g, int tile) {
     /* the ring kernel runs its tiles as one pipeline and wants at least four K steps in every K slice (the last slice
@@ -1224,13 +1448,19 @@ static int launch_epi(GemmArgs &g, int tile) {
             case 12: return launch_4d<8, 4, EPI, 3, 3>(g);
             case 13: return launch_4d<4, 4, EPI, 3, 3>(g);
             case 14: return launch_4d<6, 8, EPI, 2, 3>(g);
+            case 17: if constexpr (EPI == EPI_QKV_SWIGLU) return launch_4x<9, 9, EPI>(g); break;
+            case 18: if constexpr (EPI == EPI_QKV_SWIGLU) return launch_4x<12, 7, EPI>(g); break;
+            case 19: if constexpr (EPI == EPI_QKV_SWIGLU) return launch_4x<10, 7, EPI>(g); break;
+            case 20: if constexpr (EPI == EPI_QKV_SWIGLU) return launch_4x<10, 8, EPI>(g); break;
+            case 21: if constexpr (EPI == EPI_QKV_SWIGLU) return launch_4x<9, 8, EPI>(g); break;
+            case 22: if constexpr (EPI == EPI_QKV_SWIGLU) return launch_4x<11, 7, EPI>(g); break;
             case 11:
                 if constexpr (EPI == FLUX_HIP_EPI_RESID || EPI == FLUX_HIP_EPI_BF16) return launch_4d<8, 7, EPI, 2, 3>(g);
                 break;
             default: break;
         }
     }
-    if (tile >= 11 && tile < 15) tile = g.N % 256 == 0 ? 2 : 1; /* (the dispatch offers these only where the ring kernel takes them) */
+    if ((tile >= 11 && tile < 15) || tile > 16) tile = g.N % 256 == 0 ? 2 : 1; /* (the dispatch offers these only where the ring kernel takes them) */
     switch (tile) {
         case 2: return launch_4w<8, 8, EPI>(g);
         case 5: return launch_4w<9, 6, EPI>(g);
@@ -1584,7 +1814,7 @@ extern "C" void flux_hip_linear_release(void) {
 }
 
 static int g_force_tile = -1;
-#define TILE_MASK_ALL 0x17FEFu /* tiles the automatic choice may use: all but the 8-wave form of 256 x 256 */
+#define TILE_MASK_ALL 0x7F7FEFu /* tiles the automatic choice may use: all but the 8-wave form of 256 x 256 */
 static unsigned g_tile_mask = TILE_MASK_ALL;
 static int g_splitk_enabled = 1;
 extern "C" void flux_hip_linear_force_tile(int tile) { g_force_tile = tile; }
@@ -1684,11 +1914,14 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
      * tile waits for memory in every K step when it has a compute unit to itself. With the weights coming from HBM, as in a
      * forward: 512 x 6144 x 2560 39 us, in the ring 30; 1202 x 3072 x 3072: 49 and 34; 512 x 19456 x 2560 on 228 tiles of 192 x 256 52,
      * on 152 of 256 x 256 60. (The rates of 12 to 14 below are those of cached operands and up to 40 % above these launches; over
-     * 133 shapes of 67 to 16384 rows with cold weights the chosen form took 0.8 % more than the best of seven on average.) */
-    constexpr int NT = 17;
-    static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 64, 128, 96, 256, 256, 128, 192, 0, 96}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 128, 128, 128, 224, 128, 128, 256, 1, 96};
-    static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, ahead[NT] = {1, 1, 1, 1, 1, 1, 1, 1, 5, 4, 4, 1, 1, 1, 1, 1, 5}; /* stages a workgroup keeps in flight */
-    static const double rate[NT] = {2.0e12, 2.9e12, 6.05e12, 1.5e12, 4.6e12, 6.0e12, 5.7e12, 5.75e12, 1.6e12, 3.0e12, 2.4e12, 5.9e12, 5.3e12, 4.4e12, 5.5e12, 1.0, 2.3e12}; /* FLOP/s of one CU running this tile */
+     * 133 shapes of 67 to 16384 rows with cold weights the chosen form took 0.8 % more than the best of seven on average.)
+     * 17 to 22 = gemm4x_kernel's, for the fused projection: 288 x 288, 384 x 224, 320 x 224, 320 x 256, 288 x 256, 352 x 224. Over 29 row counts
+     * from 300 to 13056 the chosen tile takes 0.3 % more than the best on average; 256 x 288 was never the best, 352 x 256 (two row
+     * counts, 3 %) spills. */
+    constexpr int NT = 23;
+    static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 64, 128, 96, 256, 256, 128, 192, 0, 96, 288, 384, 320, 320, 288, 352}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 128, 128, 128, 224, 128, 128, 256, 1, 96, 288, 224, 224, 256, 256, 224};
+    static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, ahead[NT] = {1, 1, 1, 1, 1, 1, 1, 1, 5, 4, 4, 1, 1, 1, 1, 1, 5, 1, 1, 1, 1, 1, 1}; /* stages a workgroup keeps in flight */
+    static const double rate[NT] = {2.0e12, 2.9e12, 6.05e12, 1.5e12, 4.6e12, 6.0e12, 5.7e12, 5.75e12, 1.6e12, 3.0e12, 2.4e12, 5.9e12, 5.3e12, 4.4e12, 5.5e12, 1.0, 2.3e12, 6.3e12, 6.1e12, 6.15e12, 6.4e12, 6.3e12, 6.15e12}; /* FLOP/s of one CU running this tile */
     const int kt_total = g.K >> 6;
     int tile = -1, best_split = 1;
     {
@@ -1710,7 +1943,10 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
             /* bf16 outputs leave in pairs of 16-column blocks: the cut must fall between two pairs of a wave's 112 columns */
             if (cut && epilogue == FLUX_HIP_EPI_BF16 && (N % 224) % 112 % 32 != 0) continue;
             /* 96 x 96 (tile 16) cuts its last column tile off as well, at a multiple of 32, i.e. between two waves' columns */
-            if (!cut && ((N % bn[t] && (t != 16 || epilogue == EPI_QKV_SWIGLU)) || g.nq_cols % bn[t])) continue;
+            const bool wide = t >= 17;
+            if (wide && !(epilogue == EPI_QKV_SWIGLU && g_ring && g_persistent && kt_total >= 4)) continue;
+            if (wide && bn[t] == 256 && (g.nq_cols & 255 || N & 255)) continue; /* (CutTile) */
+            if (!cut && !wide && ((N % bn[t] && (t != 16 || epilogue == EPI_QKV_SWIGLU)) || g.nq_cols % bn[t])) continue;
             if (!((allowed >> t) & 1)) continue;
             if (t >= 12 && t < 15 && !(g_ring && g_persistent && kt_total >= 4)) continue;
             if (ahead[t] > 1) { /* the deep rings stream the weights once: every part in one row tile */
@@ -1720,10 +1956,10 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
             }
             long tiles = 0;
             for (int i = 0; i < np; i++) tiles += (g.M[i] + bm[t] - 1) / bm[t];
-            tiles *= (N + bn[t] - 1) / bn[t];
+            tiles *= (g.nq_cols + bn[t] - 1) / bn[t] + (N - g.nq_cols + bn[t] - 1) / bn[t];
             for (int si = 0; si < 10; si++) {
                 const int sp = splits[si];
-                if (sp > 1 && (cut || !can_split || kt_total / sp < 4)) break;
+                if (sp > 1 && (cut || wide || !can_split || kt_total / sp < 4)) break;
                 if (g_force_split && can_split && sp != g_force_split && kt_total / g_force_split >= 4) continue;
                 if (sp > 1 && fixed_ws && (double)sp * rows * N * sizeof(float) > (double)fixed_ws_bytes) {
                     /* the slices must fit the given workspace: fewer slices then, down to none - unless this number
@@ -1943,7 +2179,7 @@ extern "C" int flux_hip_linear_qkv_swiglu(const void *A, const void *W, void *qk
     int tile = -1;
     const int saved = g_splitk_enabled;
     g_splitk_enabled = 0;
-    const int ok = gemm_dispatch(g, 1, EPI_QKV_SWIGLU, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x17FFFu, &tile);
+    const int ok = gemm_dispatch(g, 1, EPI_QKV_SWIGLU, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7F7FFFu, &tile);
     g_splitk_enabled = saved;
     return ok;
 }

@@ -561,6 +561,50 @@ def test_linear_qkv_swiglu_one_launch(hip, oracle_mod, tile, M):
     assert not got_q[:, qc:].any() and not got_m[:, :64].any() and not got_m[:, 64 + mlp:].any()
 
 
+@pytest.mark.parametrize("tile,bm", [(17, 288), (18, 384), (19, 320), (20, 320), (21, 288), (22, 352)])
+@pytest.mark.parametrize("qc,mlp,K,rows", [(128, 64, 256, (1, 17)), (384, 320, 320, (-1, 0, 1)), (1152, 768, 576, (-40, 33)), (9216, 9216, 256, (500,))])
+def test_linear_qkv_swiglu_wide_tiles(hip, oracle_mod, tile, bm, qc, mlp, K, rows):
+    """The tiles with more accumulators than AGPRs. Both sides of the projection narrower than a tile, cut off in either wave's
+    columns and whole; K from the least the kernel takes (four steps) to odd step counts; rows from one to a row more than a
+    tile; and enough tiles that a workgroup walks several, valid rows and columns of one tile and the next differing. Bit for bit what the
+    128 x 128 tile gives (the order of K does not depend on the tile), right against the oracle where that is quick, nothing written
+    outside the outputs; the launch probe confirms which tile ran."""
+    import ctypes
+    L = hip.lib()
+    L.flux_hip_linear_qkv_swiglu.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 8
+    if tile in (20, 21):                                # the 256-wide ones are taken where they divide both sides
+        qc, mlp = -(-qc // 256) * 256, -(-mlp // 128) * 128
+    W = q(normal_f32((qc + 2 * mlp, K), 73, 2, 0.0, 0.1))
+    dW = dev_bf16(hip, W)
+    for r in rows:
+        M = r if mlp <= 128 else bm + r
+        ldq, ldm = qc + 8, mlp + 72
+        x = q(normal_f32((M, K), 73, 1))
+        dx, outs = dev_bf16(hip, x), {}
+        try:
+            for t in (tile, 1):
+                fq = hip.DevBuf.from_array(np.full((M + 1, ldq), 7, np.uint16))
+                fm = hip.DevBuf.from_array(np.full((M + 1, ldm), 7, np.uint16))
+                L.flux_hip_linear_force_tile(t)
+                L.flux_hip_linear_probe(8)
+                hip.check(L.flux_hip_linear_qkv_swiglu(dx.ptr, dW.ptr, fq.ptr, fm.at(64 * 2), M, qc, mlp, K, K, K, ldq, ldm), "flux_hip_linear_qkv_swiglu")
+                ran = np.zeros(4, np.int32)
+                assert L.flux_hip_linear_probe_read_launches(4, ran.ctypes.data, None) == 1 and ran[0] == t
+                L.flux_hip_linear_probe(-1)
+                outs[t] = fq.to_array(np.uint16, (M + 1, ldq)), fm.to_array(np.uint16, (M + 1, ldm))
+        finally:
+            L.flux_hip_linear_force_tile(-1)
+            L.flux_hip_linear_probe(-1)
+        for a, b in zip(outs[tile], outs[1]):
+            np.testing.assert_array_equal(a, b)
+        got_q, got_m = outs[tile]
+        assert (got_q[:, qc:] == 7).all() and (got_q[M] == 7).all() and (got_m[:, :64] == 7).all() and (got_m[:, 64 + mlp:] == 7).all() and (got_m[M] == 7).all()
+        if qc < 9216:
+            lin = oracle_mod.linear(x, W)
+            assert rel_l2(bf16_to_f32(got_q[:M, :qc]), lin[:, :qc]) < 4e-3
+            assert rel_l2(bf16_to_f32(got_m[:M, 64:64 + mlp]), oracle_mod.silu(lin[:, qc:qc + mlp]) * lin[:, qc + mlp:]) < 4e-3
+
+
 @pytest.mark.parametrize("tile,M", [(8, 1), (8, 37), (8, 64), (9, 80), (9, 128), (10, 80), (10, 96)])
 @pytest.mark.parametrize("K", [64, 192, 320, 448, 1024])
 def test_linear_deep_ring_tiles(hip, oracle_mod, tile, M, K):

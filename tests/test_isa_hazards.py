@@ -236,6 +236,24 @@ def test_gemm_kernels_fit_the_register_file(assembly):
             assert not copies, (name, copies[:4])
 
 
+def test_wide_gemm_tiles_keep_their_accumulators_in_place(assembly):
+    """gemm4x_kernel: 64 accumulator blocks in AGPRs and the others in VGPRs, no MFMA near a hazard, and a K loop that holds its MFMAs, reads
+    and loads without a register copy or scratch access among them."""
+    usage = resource_usage(assembly["gemm.hip"][1])
+    kernels = {k: v for k, v in kernel_bodies(assembly["gemm.hip"][0]).items() if "gemm4x_kernel" in k}
+    assert len(kernels) >= 6
+    for name, body in sorted(kernels.items()):
+        tm, tn = map(int, re.search(r"kernelILi(\d+)ELi(\d+)E", name).groups())
+        assert lint(body) == [] and usage[name]["AGPRs"] == 256, (name, lint(body)[:4], usage[name])
+        loops = [(a, b) for a, b in innermost_loops(body) if sum("v_mfma" in l for l in body[a:b]) >= 2 * tm * tn]
+        assert len(loops) == 2, name
+        for a, b in loops:
+            ops = [p[0] for p in map(parse, body[a:b]) if p]
+            assert ops.count("ds_read_b128") == 2 * (tm + tn) and ops.count("global_load_lds_dwordx4") == tm + tn and ops.count("s_barrier") == 2, name
+            copies = [o for o in ops if o.startswith(("v_accvgpr", "v_mov", "scratch_"))]
+            assert not copies, (name, copies[:4])
+
+
 def test_conv_kernel_owns_the_accumulator_registers(assembly):
     """conv3_kernel names its 256 accumulator registers in its assembly statements: nothing that the compiler itself wrote may
     touch one (a parked vector register would be overwritten), and nothing goes to scratch memory."""
