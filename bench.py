@@ -46,9 +46,9 @@ PEAK_BF16_TFLOPS = 2500.0   # MI355X dense bf16 MFMA peak (datasheet)
 # Bytes per launch that the dominant kernel moves beyond its L2s: not measured in this run (it takes hardware counters) but
 # taken from profiles/gemm_qkv_swiglu_c4_traffic.txt, i.e. from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of
 # `bench.py --calibrate` on the kernel as it is in this tree, scaled by the same counters on a streaming kernel of known size.
-# The figure follows from the tile walk (1189 MB of operand rows per launch by construction) and has not moved with the loop.
+# (288 x 288 tiles: 1197 MB; the 288 x 192 tiles that ran before moved 1365.)
 PEAK_HBM_GBPS = 8000.0      # MI355X HBM3E peak (datasheet)
-TRAFFIC_BYTES = {("c4", True): 1_365_000_000}   # keyed by (workload, fused [Q|K|V|gate|up] launch); null where no profile covers the launch
+TRAFFIC_BYTES = {("c4", True): 1_197_000_000}   # keyed by (workload, fused [Q|K|V|gate|up] launch); null where no profile covers the launch
 
 # (latent h, w, text tokens, reference-image latents [(h, w, t_offset)], cfg, schedule steps)
 WORKLOADS = {
@@ -666,7 +666,11 @@ def measure_workload(model, cfg, name, K, Wm, fused, args, headline):
                   3: f"gemm_kernel<64,64,2,2,{epi_name}>", 4: f"gemm_kernel<256,256,2,4,{epi_name}>", 5: f"gemm4d_kernel<9,6,{epi_name}> (288x192 tile)",
                   6: f"gemm4d_kernel<6,6,{epi_name}> (192x192 tile)", 7: f"gemm4d_kernel<8,6,{epi_name}> (256x192 tile)",
                   8: f"gemm_kernel<64,128,2,2,{epi_name},6> (ring of 6 stages)", 9: f"gemm_kernel<128,128,2,2,{epi_name},5> (ring of 5 stages)",
-                  10: f"gemm_kernel<96,128,2,2,{epi_name},5> (ring of 5 stages)"}
+                  10: f"gemm_kernel<96,128,2,2,{epi_name},5> (ring of 5 stages)", 12: f"gemm4d_kernel<8,4,{epi_name}> (256x128 tile)",
+                  13: f"gemm4d_kernel<4,4,{epi_name}> (128x128 tile)", 14: f"gemm4d_kernel<6,8,{epi_name}> (192x256 tile)",
+                  16: f"gemm_kernel<96,96,2,2,{epi_name},6> (ring of 6 stages)",
+                  **{17 + i: f"gemm4x_kernel<{tm},{tn},{epi_name}> ({32 * tm}x{32 * tn} tile)"
+                     for i, (tm, tn) in enumerate([(9, 9), (12, 7), (10, 7), (10, 8), (9, 8), (11, 7)])}}
     k_tile = -1
     for tile in TILE_NAMES:
         n_t, ms_t = ctypes.c_int(0), ctypes.c_float(0.0)
