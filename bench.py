@@ -669,6 +669,7 @@ def measure_workload(model, cfg, name, K, Wm, fused, args, headline):
                   10: f"gemm_kernel<96,128,2,2,{epi_name},5> (ring of 5 stages)", 12: f"gemm4d_kernel<8,4,{epi_name}> (256x128 tile)",
                   13: f"gemm4d_kernel<4,4,{epi_name}> (128x128 tile)", 14: f"gemm4d_kernel<6,8,{epi_name}> (192x256 tile)",
                   16: f"gemm_kernel<96,96,2,2,{epi_name},6> (ring of 6 stages)",
+                  23: f"gemm4d_kernel<8,5,{epi_name}> (256x160 tile)",
                   **{17 + i: f"gemm4x_kernel<{tm},{tn},{epi_name}> ({32 * tm}x{32 * tn} tile)"
                      for i, (tm, tn) in enumerate([(9, 9), (12, 7), (10, 7), (10, 8), (9, 8), (11, 7)])}}
     k_tile = -1

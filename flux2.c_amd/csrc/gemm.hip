@@ -231,6 +231,8 @@ __device__ __forceinline__ int bf16_feature(int blk, int r) { return blk < (TN &
 template <int BN> struct CutTile { static constexpr bool value = BN % 64 != 0; };
 /* the tiles of gemm4x_kernel */
 template <int BN, int WM> struct IsWide { static constexpr bool value = 2 * WM * BN > 256 * 256; };
+/* tiles whose last column tile is cut at any multiple of eight columns, lane by lane: those, and 256 x 160 */
+template <int BN, int WM> struct LaneCut { static constexpr bool value = CutTile<BN>::value && (IsWide<BN, WM>::value || BN == 160); };
 /* SiLU(gate) * up: blocks alternate gate, up, so that a lane holds matching pairs; the (gate, up) pairs interleave
  * two by two in the same way, and a last odd pair keeps the plain numbering (features 16 k + r). With an odd number of
  * blocks the last one holds gate rows and up rows, two and two: a lane's four results are gate, gate, up, up of two features. */
@@ -285,7 +287,7 @@ __device__ __forceinline__ void store_tile_to(const GemmArgs &g, const TileId &t
                                               int wm, int wn, int l15, int lq, int prow, void *Cp, const int ldc, const int tn, const int cols) {
     constexpr int TM = WM / 16, TN = WN / 16;
     const int prob = t.prob, n0 = tn * BN, ks = t.ks;
-    constexpr bool LANE_CUT = CutTile<BN>::value && IsWide<BN, WM>::value; /* a last column tile is cut at any multiple of eight columns, lane by lane */
+    constexpr bool LANE_CUT = LaneCut<BN, WM>::value;
     const bool aligned16 = (((uintptr_t)Cp | ((uintptr_t)ldc << 1)) & 15) == 0; /* every 8-feature group of the output starts on 16 bytes */
     f32x4 acc_here[HERE ? TN : 1][HERE ? TM : 1];
     auto &acc = [&]() -> auto & { if constexpr (HERE) return acc_here; else return acc_in; }();
@@ -718,7 +720,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_kernel(GemmArgs g) {
  * Idle cycles for the hazards are placed explicitly next to it. */
 template <int TM, int TN>
 __device__ __forceinline__ void acc_fence(f32x4 (&acc)[TN][TM]) {
-    static_assert(TN == 8 || TN == 7 || TN == 6 || TN == 4, "one asm statement per accumulator column");
+    static_assert(TN == 8 || TN == 7 || TN == 6 || TN == 5 || TN == 4, "one asm statement per accumulator column");
 #pragma unroll
     for (int j = 0; j < TM; j++) {
         if constexpr (TN == 7)
@@ -730,6 +732,8 @@ __device__ __forceinline__ void acc_fence(f32x4 (&acc)[TN][TM]) {
         else if constexpr (TN == 6)
             asm volatile("" : "+a"(acc[0][j]), "+a"(acc[1][j]), "+a"(acc[2][j]), "+a"(acc[3][j]),
                               "+a"(acc[4][j]), "+a"(acc[5][j]));
+        else if constexpr (TN == 5)
+            asm volatile("" : "+a"(acc[0][j]), "+a"(acc[1][j]), "+a"(acc[2][j]), "+a"(acc[3][j]), "+a"(acc[4][j]));
         else
             asm volatile("" : "+a"(acc[0][j]), "+a"(acc[1][j]), "+a"(acc[2][j]), "+a"(acc[3][j]));
     }
@@ -914,7 +918,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm4w_kernel(GemmArgs g) {
  * requested only then, with the matrix pipes idle: 12 % of a 288 x 192 x 3072 tile's time. */
 template <int EPI, int TM, int TN>
 struct EpilogueOps { /* vector memory instructions a wave issues in the epilogue of a tile whose rows are all valid */
-    static constexpr int value = EPI == FLUX_HIP_EPI_SWIGLU || EPI == EPI_QKV_SWIGLU ? TM * (TN / 4 + TN / 2 % 2) /* 16-byte stores + a last 8-byte one */
+    static constexpr int value = EPI == FLUX_HIP_EPI_SWIGLU ? TM * (TN / 4 + TN / 2 % 2 + TN % 2) /* 16-byte stores + a last 8-byte and 4-byte one */
+                                 : EPI == EPI_QKV_SWIGLU ? TM * (TN / 4 + TN / 2 % 2)
                                  : EPI == FLUX_HIP_EPI_BF16 || EPI == FLUX_HIP_EPI_CONV_BF16 || EPI == EPI_EXP ? TM * (TN / 2 + TN % 2) : EPI == FLUX_HIP_EPI_F32_T ? 4 * TM * TN : TM * TN;
 };
 
@@ -929,7 +934,8 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
     constexpr int ASZ = BM * 128, WSZ = BN * 128;
     static_assert((NSA == 2 || NSA == 3) && (NSW == 2 || NSW == 3) && (NSA == 3 || NSW == 3) && NSA * ASZ + NSW * WSZ <= 160 * 1024,
                   "rings of two or three slots within the LDS, one of them with three");
-    static_assert((EPI != FLUX_HIP_EPI_SWIGLU && EPI != EPI_QKV_SWIGLU) || (TN % 2 == 0), "swiglu pairs 16-column blocks");
+    static_assert((EPI != FLUX_HIP_EPI_SWIGLU && EPI != EPI_QKV_SWIGLU) || TN % 2 == 0 || (EPI == FLUX_HIP_EPI_SWIGLU && LaneCut<BN, WM>::value),
+                  "swiglu pairs 16-column blocks");
     static_assert(RD >= 2 && RD * (NF - 1) + 1 < NM, "reads must fit between the MFMAs");
     constexpr bool FIRST_A = NSA == 3;
     constexpr int LF = FIRST_A ? LA : LB, LS = FIRST_A ? LB : LA, NS2 = FIRST_A ? NSW : NSA;
@@ -1454,6 +1460,7 @@ static int launch_epi(GemmArgs &g, int tile) {
             case 20: if constexpr (EPI == EPI_QKV_SWIGLU) return launch_4x<10, 8, EPI>(g); break;
             case 21: if constexpr (EPI == EPI_QKV_SWIGLU) return launch_4x<9, 8, EPI>(g); break;
             case 22: if constexpr (EPI == EPI_QKV_SWIGLU) return launch_4x<11, 7, EPI>(g); break;
+            case 23: if constexpr (EPI == FLUX_HIP_EPI_SWIGLU) return launch_4d<8, 5, EPI, 3, 3>(g); break;
             case 11:
                 if constexpr (EPI == FLUX_HIP_EPI_RESID || EPI == FLUX_HIP_EPI_BF16) return launch_4d<8, 7, EPI, 2, 3>(g);
                 break;
@@ -1814,7 +1821,7 @@ extern "C" void flux_hip_linear_release(void) {
 }
 
 static int g_force_tile = -1;
-#define TILE_MASK_ALL 0x7F7FEFu /* tiles the automatic choice may use: all but the 8-wave form of 256 x 256 */
+#define TILE_MASK_ALL 0xFF7FEFu /* tiles the automatic choice may use: all but the 8-wave form of 256 x 256 */
 static unsigned g_tile_mask = TILE_MASK_ALL;
 static int g_splitk_enabled = 1;
 extern "C" void flux_hip_linear_force_tile(int tile) { g_force_tile = tile; }
@@ -1918,10 +1925,10 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
      * 17 to 22 = gemm4x_kernel's, for the fused projection: 288 x 288, 384 x 224, 320 x 224, 320 x 256, 288 x 256, 352 x 224. Over 29 row counts
      * from 300 to 13056 the chosen tile takes 0.3 % more than the best on average; 256 x 288 was never the best, 352 x 256 (two row
      * counts, 3 %) spills. */
-    constexpr int NT = 23;
-    static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 64, 128, 96, 256, 256, 128, 192, 0, 96, 288, 384, 320, 320, 288, 352}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 128, 128, 128, 224, 128, 128, 256, 1, 96, 288, 224, 224, 256, 256, 224};
-    static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, ahead[NT] = {1, 1, 1, 1, 1, 1, 1, 1, 5, 4, 4, 1, 1, 1, 1, 1, 5, 1, 1, 1, 1, 1, 1}; /* stages a workgroup keeps in flight */
-    static const double rate[NT] = {2.0e12, 2.9e12, 6.05e12, 1.5e12, 4.6e12, 6.0e12, 5.7e12, 5.75e12, 1.6e12, 3.0e12, 2.4e12, 5.9e12, 5.3e12, 4.4e12, 5.5e12, 1.0, 2.3e12, 6.3e12, 6.1e12, 6.15e12, 6.4e12, 6.3e12, 6.15e12}; /* FLOP/s of one CU running this tile */
+    constexpr int NT = 24;
+    static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 64, 128, 96, 256, 256, 128, 192, 0, 96, 288, 384, 320, 320, 288, 352, 256}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 128, 128, 128, 224, 128, 128, 256, 1, 96, 288, 224, 224, 256, 256, 224, 160};
+    static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, ahead[NT] = {1, 1, 1, 1, 1, 1, 1, 1, 5, 4, 4, 1, 1, 1, 1, 1, 5, 1, 1, 1, 1, 1, 1, 1}; /* stages a workgroup keeps in flight */
+    static const double rate[NT] = {2.0e12, 2.9e12, 6.05e12, 1.5e12, 4.6e12, 6.0e12, 5.7e12, 5.75e12, 1.6e12, 3.0e12, 2.4e12, 5.9e12, 5.3e12, 4.4e12, 5.5e12, 1.0, 2.3e12, 6.3e12, 6.1e12, 6.15e12, 6.4e12, 6.3e12, 6.15e12, 5.4e12}; /* FLOP/s of one CU running this tile */
     const int kt_total = g.K >> 6;
     int tile = -1, best_split = 1;
     {
@@ -1943,10 +1950,16 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
             /* bf16 outputs leave in pairs of 16-column blocks: the cut must fall between two pairs of a wave's 112 columns */
             if (cut && epilogue == FLUX_HIP_EPI_BF16 && (N % 224) % 112 % 32 != 0) continue;
             /* 96 x 96 (tile 16) cuts its last column tile off as well, at a multiple of 32, i.e. between two waves' columns */
-            const bool wide = t >= 17;
+            const bool wide = t >= 17 && t < 23;
+            /* 256 x 160 (tile 23) likewise, at a multiple of eight features: for SwiGLU alone. The text encoder's gate and up rows (19456 x
+             * 2560) are 244 tiles of it at 512 rows, of which 256 units run all at once; with the weights from HBM, us, 23 / the best other: 260 rows
+             * 43.8 / 45.8, 300 44.7 / 46.0, 384 47.0 / 46.8, 400 47.2 / 52.4, 512 47.4 / 53.8; 200 45.2 / 40.4 and 256 44.5 / 40.3,
+             * where the model takes 256 x 128. */
+            const bool cut160 = t == 23;
+            if (cut160 && !(epilogue == FLUX_HIP_EPI_SWIGLU && N % 64 == 0 && g_ring && g_persistent && kt_total >= 4)) continue;
             if (wide && !(epilogue == EPI_QKV_SWIGLU && g_ring && g_persistent && kt_total >= 4)) continue;
             if (wide && bn[t] == 256 && (g.nq_cols & 255 || N & 255)) continue; /* (CutTile) */
-            if (!cut && !wide && ((N % bn[t] && (t != 16 || epilogue == EPI_QKV_SWIGLU)) || g.nq_cols % bn[t])) continue;
+            if (!cut && !cut160 && !wide && ((N % bn[t] && (t != 16 || epilogue == EPI_QKV_SWIGLU)) || g.nq_cols % bn[t])) continue;
             if (!((allowed >> t) & 1)) continue;
             if (t >= 12 && t < 15 && !(g_ring && g_persistent && kt_total >= 4)) continue;
             if (ahead[t] > 1) { /* the deep rings stream the weights once: every part in one row tile */
@@ -1959,7 +1972,7 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
             tiles *= (g.nq_cols + bn[t] - 1) / bn[t] + (N - g.nq_cols + bn[t] - 1) / bn[t];
             for (int si = 0; si < 10; si++) {
                 const int sp = splits[si];
-                if (sp > 1 && (cut || wide || !can_split || kt_total / sp < 4)) break;
+                if (sp > 1 && (cut || cut160 || wide || !can_split || kt_total / sp < 4)) break;
                 if (g_force_split && can_split && sp != g_force_split && kt_total / g_force_split >= 4) continue;
                 if (sp > 1 && fixed_ws && (double)sp * rows * N * sizeof(float) > (double)fixed_ws_bytes) {
                     /* the slices must fit the given workspace: fewer slices then, down to none - unless this number
@@ -2104,7 +2117,7 @@ static int linear_impl(int epilogue, int nparts, const flux_hip_linear_part *par
     g.N = N; g.K = K; g.lda = lda; g.ldw = ldw; g.ldc = ldc; g.w_row0 = w_row0; g.w_row1 = w_row1;
     a.ldo = N;
     a.eps = eps;
-    return gemm_dispatch(g, np, epilogue, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x17FFFu, nullptr, norm ? &a : nullptr, fused,
+    return gemm_dispatch(g, np, epilogue, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x817FFFu, nullptr, norm ? &a : nullptr, fused,
                          fixed_ws, fixed_ws_bytes);
 }
 

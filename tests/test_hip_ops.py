@@ -660,6 +660,36 @@ def test_linear_deep_ring_tiles(hip, oracle_mod, tile, M, K):
     np.testing.assert_array_equal(fm, sw)
 
 
+@pytest.mark.parametrize("M,K", [(1, 256), (255, 320), (257, 448), (512, 2560)])
+@pytest.mark.parametrize("mlp", [64, 128, 192, 320, 9728])
+def test_linear_swiglu_160_wide_tile(hip, M, K, mlp):
+    """Tile 23 (256 x 160), 80 features a tile, whose last column tile is cut off within the first wave's 40 features (192), within the
+    second's (64, 128, 9728) or not at all (320): bit for bit what the two-stage tiles give; rows and
+    columns beyond the output stay as they were, also in rows that are not a multiple of 16 bytes."""
+    L = hip.lib()
+    x, W = q(normal_f32((M, K), 73, 1)), q(normal_f32((2 * mlp, K), 73, 2, 0.0, 0.1))
+    dx, dW = dev_bf16(hip, x), dev_bf16(hip, W)
+    try:
+        L.flux_hip_linear_enable_splitk(0)
+        for ld in (mlp + 8, mlp + 12):
+            outs = []
+            for t in (23, 3):
+                L.flux_hip_linear_force_tile(t)
+                L.flux_hip_linear_probe(hip.EPI_SWIGLU)
+                o = hip.DevBuf.from_array(np.full((M + 1, ld), 7, np.uint16))
+                hip.linear(hip.EPI_SWIGLU, [(dx.ptr, dW.ptr, o.ptr, None, M)], 2 * mlp, K, K, K, ld, 0, mlp)
+                tiles = np.zeros(4, np.int32)
+                assert L.flux_hip_linear_probe_read_launches(4, tiles.ctypes.data, None) == 1 and tiles[0] == t
+                L.flux_hip_linear_probe(-1)
+                outs.append(o.to_array(np.uint16, (M + 1, ld)))
+            assert np.array_equal(outs[0], outs[1])
+            assert (outs[0][M] == 7).all() and (outs[0][:, mlp:] == 7).all()
+    finally:
+        L.flux_hip_linear_force_tile(-1)
+        L.flux_hip_linear_enable_splitk(1)
+        L.flux_hip_linear_probe(-1)
+
+
 @pytest.mark.parametrize("M,K", [(1, 64), (67, 192), (80, 448), (96, 1024)])
 @pytest.mark.parametrize("N", [384, 512, 640])
 def test_linear_96_wide_ring_tile(hip, oracle_mod, M, K, N):
