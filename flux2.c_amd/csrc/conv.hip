@@ -49,7 +49,9 @@ struct Args {
 
 constexpr int TM = 8, TN = 4, NM = TM * TN, NF = TM + TN, RD = 2; /* blocks of a wave, MFMAs and fragments of a half-step, MFMAs per fragment read */
 constexpr int PITCH = 20, PATCH = 384 * 128, SLOT = 128 * 128, W0 = 2 * PATCH, LDS_BYTES = 2 * PATCH + 4 * SLOT;
-constexpr unsigned OUTSIDE = 0xF0000000u; /* beyond every buffer: the host admits images of less than 3.7e9 bytes */
+/* Beyond every buffer: the host admits images of less than 3.7e9 bytes, and seven image rows of results of less than 2^28, so that a column
+ * beyond the image stays there with a row's offset added (and 2 * OUTSIDE mod 2^32 = 3.76e9, a column and a row beyond it, as well). */
+constexpr unsigned OUTSIDE = 0xF0000000u;
 static_assert(LDS_BYTES <= 160 * 1024, "LDS");
 
 #define LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
@@ -584,11 +586,13 @@ extern "C" int flux_hip_vae_conv_in(float *out, const float *img, const void *w,
 }
 
 /* Whether the kernel takes this convolution: two chunks of input channels at least, the image in 32-bit byte offsets below OUTSIDE, tile
- * numbers below 2^16, and no more rows of statistics than one per 32 positions of the bordered image + 2. */
+ * numbers below 2^16, no more rows of statistics than one per 32 positions of the bordered image + 2, and rows short enough for OUTSIDE
+ * (16 x 20001 positions x 512 channels came round to the start of the image). */
 bool conv3_takes(int H, int W, int cin, int cout) {
     const long long pos = (long long)(H + 2) * (W + 2), tiles = (long long)((H + 15) / 16) * ((W + 15) / 16);
     return H > 0 && W > 0 && cin >= 128 && cin % 64 == 0 && cout % 128 == 0 && pos * max(cin * 2, cout * 4) < 3700000000LL &&
-           (long long)cout * cin * 18 < 2000000000LL && tiles * (cout / 128) < 65536 && 2 * tiles <= pos / 32 + 2;
+           (long long)cout * cin * 18 < 2000000000LL && tiles * (cout / 128) < 65536 && 2 * tiles <= pos / 32 + 2 &&
+           7LL * (W + 2) * cout * 4 + 65536 <= 1LL << 28;
 }
 long conv3_tiles(int H, int W, int cout) { return (long)((H + 15) / 16) * ((W + 15) / 16) * (cout / 128); }
 

@@ -47,6 +47,26 @@ def test_schedules_match_reference_golden(golden_dir):
         np.testing.assert_allclose(fluxhip.schedule("resolution", n, hh, ww), g[f"sched_resolution_{n}_{hh}_{ww}"], atol=6e-7)
 
 
+def test_patch_convolution_keeps_skipped_positions_outside():
+    """The 3x3 convolution that holds a tile's neighbourhood in LDS gives positions beyond the image an offset of 0xF0000000
+    and adds up to seven image rows of fp32 results to it: the sum must not come round to the buffer's start. Images too wide for that are
+    refused (the other tiles take them); everything the VAE has is taken."""
+    f = fluxhip.lib()._Z11conv3_takesiiii
+    f.argtypes, f.restype = [ctypes.c_int] * 4, ctypes.c_bool
+    taken = 0
+    for cout in (128, 256, 512, 4096):
+        for W in [1, 1792] + [int(1000 * 1.05 ** i) for i in range(140)]:
+            for H in (1, 16, 500):
+                if f(H, W, 128, cout):
+                    taken += 1
+                    last = 0xF0000000 + 7 * (W + 2) * cout * 4 + 128 + 64 + 16      # (bytes of the last access behind its lane's row)
+                    assert last <= 1 << 32, (H, W, cout)
+    assert taken > 100
+    assert not f(16, 20001, 128, 512) and f(16, 18000, 128, 512)
+    for H, W, cin, cout in ((1, 1, 128, 128), (1792, 1792, 256, 128), (1792, 1792, 128, 128), (896, 896, 512, 256), (448, 448, 512, 512), (16, 1792, 256, 256)):
+        assert f(H, W, cin, cout), (H, W, cin, cout)
+
+
 def test_touching_a_result_buffer_leaves_its_contents():
     """The result's pages are touched while the device computes it; when the call fails afterwards the caller's buffer
     holds what it held before. Sizes around a page, at offsets of every kind."""
