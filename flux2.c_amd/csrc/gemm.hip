@@ -2145,12 +2145,17 @@ extern "C" int flux_hip_linear_slices(const void *A, const void *W, void *C, int
 /* Attention scores as unnormalised probabilities, P[m][n] = 2^(scale * A[m] . W[n] - ref[m]) in bf16 for n < keys and 0 for keys <= n < N, and
  * their fp32 sums over pieces of each row, sums [M][*pieces] (at most N / 64 of them). N a multiple of 256, K of 64 and at least 256. In the
  * ring kernel's epilogue, where they cost a multiply-add, an exponential and half a store of 16 bytes per eight: 16384 x 16384 scores
- * written as fp32 and read by a softmax took 395 + 348 us. Returns 0 without an error where that kernel is switched off. */
+ * written as fp32 and read by a softmax took 395 + 348 us. Not to be had where that kernel is switched off, which its caller asks first:
+ * everything that fails here is an error. */
+extern "C" int flux_hip_linear_exp_available(void) { return g_ring && g_persistent; }
 extern "C" int flux_hip_linear_exp(const void *A, const void *W, void *P, int M, int N, int K, int lda, int ldw, const float *ref, float scale, int keys,
                                    float *sums, int *pieces) {
-    if (!g_ring || !g_persistent || M <= 0 || N <= 0 || (N & 255) || K < 256 || (K & 63) || lda < K || ldw < K || (lda & 7) || (ldw & 7) ||
-        ((((uintptr_t)A | (uintptr_t)W | (uintptr_t)P) & 15) != 0) || ((size_t)M * lda | (size_t)N * ldw) >= ((size_t)1 << 31))
-        return 0;
+    *pieces = 0;
+    if (!flux_hip_linear_exp_available()) return flux_hip_fail("flux_hip_linear_exp: the ring kernel is switched off");
+    if (M <= 0 || N <= 0 || (N & 255) || K < 256 || (K & 63) || lda < K || ldw < K || (lda & 7) || (ldw & 7) || ((size_t)M * lda | (size_t)N * ldw) >= ((size_t)1 << 31))
+        return flux_hip_fail("flux_hip_linear_exp: bad shape (M=%d, N=%d, K=%d, lda=%d, ldw=%d)", M, N, K, lda, ldw);
+    if (!A || !W || !P || !ref || !sums || (((uintptr_t)A | (uintptr_t)W | (uintptr_t)P) & 15))
+        return flux_hip_fail("flux_hip_linear_exp: NULL or unaligned operand");
     GemmArgs g = {};
     g.A[0] = (const bf16 *)A; g.W[0] = (const bf16 *)W; g.C[0] = P; g.M[0] = M;
     g.N = N; g.K = K; g.lda = lda; g.ldw = ldw; g.ldc = N;

@@ -668,6 +668,7 @@ extern "C" int flux_hip_softmax_rows(void *p_bf16, const float *s, const float *
     return 1;
 }
 
+extern "C" int flux_hip_linear_exp_available(void);
 extern "C" int flux_hip_linear_exp(const void *A, const void *W, void *P, int M, int N, int K, int lda, int ldw, const float *ref, float scale, int keys,
                                    float *sums, int *pieces);
 extern "C" int flux_hip_linear_f32_slices(const void *A, const void *W, float *C, int M, int N, int K, const float **ws, int *slices);
@@ -676,11 +677,12 @@ extern "C" size_t flux_hip_vae_attention_work_floats(int n, int ld) { return (si
 
 /* Attention of n queries (rows of qkv from q on, 3 * 512 wide) over `keys` positions: out [n][512]. qkv: every position's [q | k | v], ld rows of
  * them (zeros beyond keys); vt: v transposed, [512][ld]; P: n x ld bf16; o32: n x 512; work: flux_hip_vae_attention_work_floats. At least
- * 256 keys, ld a multiple of 256. *done = 0 where the scores' kernel is not to be had: nothing is computed. */
+ * 256 keys, ld a multiple of 256. *done = 0 where the scores' kernel is switched off: nothing is launched. */
 extern "C" int flux_hip_vae_attention(void *out, const void *q, const void *qkv, const void *vt, void *P, float *o32, float *work, int n, int keys, int ld,
                                       float scale, int *done) {
     *done = 0;
     if (n <= 0 || keys < ATT_SAMPLE || ld < keys || (ld & 255)) return flux_hip_fail("flux_hip_vae_attention: bad shape (%d queries, %d keys, %d columns)", n, keys, ld);
+    if (!flux_hip_linear_exp_available()) return 1;
     const float scale2 = scale * 1.44269504088896341f;
     float *sample = work, *ref = work + (size_t)n * ATT_SAMPLE, *sums = ref + ((n + 3) & ~3);
     hipStream_t st = flux_hip_stream_handle();
@@ -690,7 +692,7 @@ extern "C" int flux_hip_vae_attention(void *out, const void *q, const void *qkv,
     hipLaunchKernelGGL(vae_attention_ref_kernel, dim3((n + 3) / 4), dim3(256), 0, st, ref, sample, n, scale2);
     LAUNCH_OK("vae_attention_ref_kernel");
     int pieces = 0, slices = 0;
-    if (!flux_hip_linear_exp(q, k, P, n, ld, ATT_C, 3 * ATT_C, 3 * ATT_C, ref, scale2, keys, sums, &pieces)) return 1;
+    if (!flux_hip_linear_exp(q, k, P, n, ld, ATT_C, 3 * ATT_C, 3 * ATT_C, ref, scale2, keys, sums, &pieces)) return 0;
     const float *ws = nullptr;
     if (!flux_hip_linear_f32_slices(P, vt, o32, n, ATT_C, ld, &ws, &slices)) return 0;
     hipLaunchKernelGGL(vae_attention_out_kernel, dim3((n + 3) / 4), dim3(256), 0, st, (bf16 *)out, slices ? ws : o32, slices ? slices : 1, sums, pieces,

@@ -67,6 +67,32 @@ def test_patch_convolution_keeps_skipped_positions_outside():
         assert f(H, W, cin, cout), (H, W, cin, cout)
 
 
+def test_exponential_scores_tell_switched_off_from_failed():
+    """With the ring kernel switched off the VAE's attention without scores is not to be had: that is no error, nothing is
+    launched, and its caller goes on with the scores in memory. What the product itself refuses is an error with its own text."""
+    L = fluxhip.lib()
+    vp, ci, cf = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    L.flux_hip_linear_exp.argtypes = [vp] * 3 + [ci] * 5 + [vp, cf, ci, vp, vp]
+    L.flux_hip_vae_attention.argtypes = [vp] * 7 + [ci] * 3 + [cf, vp]
+    buf = np.zeros(4096, np.uint8)
+    p = (buf.ctypes.data + 15) & ~15
+    done, pieces = ci(7), ci(7)
+
+    def exp(P=p, M=256, N=256, K=512):
+        L.flux_hip_vae_attention(p, p, p, p, p, p, p, 0, 0, 0, 1.0, ctypes.byref(ci(0)))       # an error of another function
+        assert b"flux_hip_vae_attention" in L.flux_hip_last_error()
+        return L.flux_hip_linear_exp(p, p, P, M, N, K, 512, 512, p, 1.0, 256, p, ctypes.byref(pieces))
+
+    for bad in (dict(P=p + 8), dict(P=None), dict(M=0), dict(N=384), dict(K=192)):
+        assert exp(**bad) == 0 and b"flux_hip_linear_exp" in L.flux_hip_last_error(), bad
+    L.flux_hip_linear_ring(0)
+    try:
+        assert exp() == 0 and b"switched off" in L.flux_hip_last_error()
+        assert L.flux_hip_vae_attention(p, p, p, p, p, p, p, 256, 256, 256, 1.0, ctypes.byref(done)) == 1 and done.value == 0
+    finally:
+        L.flux_hip_linear_ring(1)
+
+
 def test_touching_a_result_buffer_leaves_its_contents():
     """The result's pages are touched while the device computes it; when the call fails afterwards the caller's buffer
     holds what it held before. Sizes around a page, at offsets of every kind."""

@@ -669,6 +669,21 @@ def test_attention_without_scores(hip, switches, keys, n, planted):
     np.testing.assert_array_less(np.abs(got - want).max(1), 2.0 ** -6 * np.abs(want).max(1) + 1e-6)
 
 
+def test_attention_without_scores_reports_a_refused_product(hip):
+    """What the score product refuses (here probabilities that do not start on 16 bytes, looked at on the host) is the caller's
+    error, not a reason to go on with the scores in memory."""
+    import ctypes
+    keys, C, L = 256, 512, hip.lib()
+    L.flux_hip_vae_attention_work_floats.restype = ctypes.c_size_t
+    L.flux_hip_vae_attention.argtypes = [ctypes.c_void_p] * 7 + [ctypes.c_int] * 3 + [ctypes.c_float, ctypes.c_void_p]
+    dq, dv = hip.DevBuf.from_array(np.zeros((keys, 3 * C), np.uint16)), hip.DevBuf.from_array(np.zeros((C, keys), np.uint16))
+    P, o32, out = hip.DevBuf(keys * keys * 2 + 16), hip.DevBuf(keys * C * 4), hip.DevBuf(keys * C * 2)
+    work, done = hip.DevBuf(L.flux_hip_vae_attention_work_floats(keys, keys) * 4), ctypes.c_int(7)
+    assert L.flux_hip_vae_attention(out.ptr, dq.ptr, dq.ptr, dv.ptr, P.at(8), o32.ptr, work.ptr, keys, keys, keys, 1.0, ctypes.byref(done)) == 0
+    assert b"flux_hip_linear_exp" in L.flux_hip_last_error() and done.value == 0
+    hip.sync()
+
+
 @pytest.mark.parametrize("shape", [(37, 384, 300), (3, 17024, 16900), (3, 20608, 20500)])
 def test_softmax_rows_and_transpose(hip, oracle_mod, shape):
     """Rows of up to 20480 columns go through the kernel that keeps the row in registers, longer ones
