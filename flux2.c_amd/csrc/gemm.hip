@@ -2170,6 +2170,8 @@ extern "C" int flux_hip_linear_exp(const void *A, const void *W, void *P, int M,
 extern "C" int flux_hip_linear_f32_slices(const void *A, const void *W, float *C, int M, int N, int K, const float **ws, int *slices) {
     *slices = 0;
     if (M <= 0) return 1;
+    if (K <= 0 || (K & 63) || N <= 0 || (N & 127)) return flux_hip_fail("flux_hip_linear_f32_slices: N=%d must be a multiple of 128, K=%d of 64", N, K);
+    if (!A || !W || !C || (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) & 15)) return flux_hip_fail("flux_hip_linear_f32_slices: NULL or unaligned operand");
     GemmArgs g = {};
     g.A[0] = (const bf16 *)A; g.W[0] = (const bf16 *)W; g.C[0] = C; g.M[0] = M;
     g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = N;

@@ -93,6 +93,20 @@ def test_exponential_scores_tell_switched_off_from_failed():
         L.flux_hip_linear_ring(1)
 
 
+@pytest.mark.parametrize("name", ["flux_hip_linear_slices", "flux_hip_linear_f32_slices"])
+def test_projections_that_leave_slices_check_their_arguments(name):
+    """Widths and K that no tile takes, missing and unaligned operands are refused on the host, by name."""
+    f, vp, ci = getattr(fluxhip.lib(), name), ctypes.c_void_p, ctypes.c_int
+    f.argtypes = [vp] * 3 + [ci] * 3 + [vp] * 2
+    buf = np.zeros(64, np.uint8)
+    p, ws, n = (buf.ctypes.data + 15) & ~15, vp(0), ci(7)
+    for A, W, C, N, K in ((p, p, p, 192, 512), (p, p, p, 0, 512), (p, p, p, 256, 96), (p, p, p, 256, 0), (None, p, p, 256, 512), (p, None, p, 256, 512),
+                          (p, p, None, 256, 512), (p + 8, p, p, 256, 512), (p, p + 2, p, 256, 512), (p, p, p + 4, 256, 512)):
+        assert f(A, W, C, 256, N, K, ctypes.byref(ws), ctypes.byref(n)) == 0
+        assert name.encode() in fluxhip.lib().flux_hip_last_error() and n.value == 0
+    assert f(None, None, None, 0, 256, 512, ctypes.byref(ws), ctypes.byref(n)) == 1      # no rows: nothing to do
+
+
 def test_touching_a_result_buffer_leaves_its_contents():
     """The result's pages are touched while the device computes it; when the call fails afterwards the caller's buffer
     holds what it held before. Sizes around a page, at offsets of every kind."""
