@@ -503,7 +503,8 @@ __global__ __launch_bounds__(256) void conv_out_kernel(uint8_t *__restrict__ rgb
 
 /* 3 -> 128 channels (flux_vae.c:336-338): the 27 values under a position's window are one MFMA's K, gathered from the fp32 picture
  * as the operand. As rows of 64 bf16 written by one kernel and multiplied by the next it was 69 + 146 us at 720 x 1296, and is 129; HBM: 478 MB out. A wave
- * makes IN_BLOCKS blocks of 16 bordered positions (zeros on the border) and leaves one row of sums for the group norm. */
+ * makes IN_BLOCKS blocks of 16 bordered positions (zeros on the border) and leaves one row of sums for the group norm (none if all its
+ * positions lie behind the last one). */
 #define IN_BLOCKS 8
 __global__ __launch_bounds__(256) void conv_in_kernel(float *__restrict__ out, const float *__restrict__ img, const bf16 *__restrict__ w, const float *__restrict__ bias,
                                                       float *__restrict__ stats, int H, int W) {
@@ -550,6 +551,7 @@ __global__ __launch_bounds__(256) void conv_in_kernel(float *__restrict__ out, c
             if (p < rows) *(f32x4 *)(out + (size_t)p * 128 + 16 * i + 4 * lq) = v;
         }
     }
+    if (first >= rows) return; /* a wave behind the last position has no sums */
 #pragma unroll
     for (int i = 0; i < 8; i++) {
         const f32x2 t = {row_sum(s[i]), row_sum(q[i])};
@@ -581,7 +583,7 @@ extern "C" int flux_hip_vae_conv_in(float *out, const float *img, const void *w,
     hipLaunchKernelGGL(conv_in_kernel, dim3(wg), dim3(256), 0, flux_hip_stream_handle(), out, img, (const bf16 *)w, bias, stats, H, W);
     conv_probe_end(slot);
     HIP_OK(hipGetLastError());
-    *stats_rows = 4 * wg;
+    *stats_rows = (rows + 16 * IN_BLOCKS - 1) / (16 * IN_BLOCKS); /* one per wave that has positions, within the rows / 32 + 2 that a caller provides */
     return 1;
 }
 

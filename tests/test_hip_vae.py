@@ -135,10 +135,11 @@ def test_conv_out_to_picture(hip, oracle_mod, H, W):
     np.testing.assert_array_equal(bytes_[:-1].reshape(H, W, 3), want)
 
 
-@pytest.mark.parametrize("H,W", [(1, 1), (16, 16), (5, 70), (33, 47)])
+@pytest.mark.parametrize("H,W", [(1, 1), (3, 2), (16, 16), (5, 70), (33, 47)])
 def test_conv_in_from_picture(hip, H, W):
     """3 -> 128 channels from the fp32 picture: bit for bit the 1x1 convolution of flux_hip_vae_image_in's rows (the same 27
-    products in one MFMA and a second one of zeros), with zeros on the border, nothing behind it, and the sums of what was written."""
+    products in one MFMA and a second one of zeros), with zeros on the border, nothing behind it, and the sums of what was written, in
+    no more rows than a caller provides."""
     import ctypes
     img = vae_test_image(16 * -(-H // 16), 16 * -(-W // 16), 69)[:, :H, :W].copy()
     w64 = np.zeros((128, 64), np.float32)
@@ -150,13 +151,17 @@ def test_conv_in_from_picture(hip, H, W):
     hip.check(L.flux_hip_vae_image_in(cols.ptr, dimg.ptr, H, W))
     hip.check(L.flux_hip_conv(hip.EPI_CONV_F32, cols.ptr, dw.ptr, db.ptr, None, want.ptr, rows, wp, 64, 128, 1))
     out, n = hip.DevBuf.from_array(np.full((rows + 1, 128), 3.0, np.float32)), ctypes.c_int(0)
-    stats = hip.DevBuf.from_array(np.full(((rows // 32 + 2) * 32 * 2 + 256,), np.nan, np.float32))
+    room = (rows // 32 + 2) * 32 * 2            # what flux_hip_conv_stats asks for, and the rows of one more workgroup behind it
+    stats = hip.DevBuf.from_array(np.full((room + 256,), 7.0, np.float32))
     L.flux_hip_vae_conv_in.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 2 + [ctypes.c_void_p] * 2
     hip.check(L.flux_hip_vae_conv_in(out.ptr, dimg.ptr, dw.ptr, db.ptr, H, W, stats.ptr, ctypes.byref(n)))
     got = out.to_array(np.float32, (rows + 1, 128))
     np.testing.assert_array_equal(got[:rows], want.to_array(np.float32, (rows, 128)))
     assert (got[rows] == 3.0).all() and border_is_zero(got[:rows], H, W)
-    check_sums(stats.to_array(np.float32, (n.value, 32, 2)).astype(np.float64).sum(0), got[:rows])
+    assert 0 < n.value <= rows // 32 + 2
+    sums = stats.to_array(np.float32, (room + 256,))
+    assert (sums[n.value * 64:] == 7.0).all()
+    check_sums(sums[:n.value * 64].reshape(n.value, 32, 2).astype(np.float64).sum(0), got[:rows])
 
 
 def test_conv_output_widths(hip, oracle_mod):
