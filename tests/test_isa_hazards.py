@@ -276,6 +276,65 @@ def test_conv_kernel_owns_the_accumulator_registers(assembly):
         assert named >= 2 * 27 * 32
 
 
+def conv_barriers(body):
+    """[(what a wave issues between the barrier before and this one, vmcnt of the wait in front of this one)] of conv3_kernel, from the
+    first barrier (behind the preloads) on. W: a weight load into LDS (it has a scalar offset; a step has four), P: a patch load into LDS, V: any other
+    vector memory operation. What stands in front of a label may be skipped and is not counted."""
+    out, issued, wait = [], "", None
+    for line in body:
+        if re.match(r"^\.LBB\d+_\d+:", line):
+            issued = ""
+        p = parse(line)
+        if not p:
+            continue
+        text = line.split(";")[0]
+        if p[0].startswith(("buffer_", "global_", "flat_")):
+            issued += "V" if " lds" not in text else "P" if ", 0 offen lds" in text else "W"
+        elif p[0] == "s_waitcnt" and "lgkmcnt(0)" in text and "vmcnt" in text:
+            wait = int(re.search(r"vmcnt\((\d+)\)", text).group(1))
+        elif p[0] == "s_barrier":
+            out.append((issued, wait))
+            issued = ""
+    return out[1:]
+
+
+def early_barriers(steps):
+    """The steps whose barrier lets the next step's weights be on their way still: the wait's count is larger than the number of
+    operations behind their requests, which stand two steps earlier. Steps 0 to 17 follow each other and 18 to 26 do; of the step in front of
+    a sequence its four weight loads are certain."""
+    bad = []
+    for first, last in ((0, 18), (18, 27)):
+        for s in range(first, last):
+            behind = "".join(issued for issued, _ in steps[max(first, s - 2):s + 1])
+            if s - 2 >= first:
+                behind = behind.split("W", 4)[4]
+            elif s == first:
+                behind = "WWWW" + behind
+            if steps[s][1] > len(behind):
+                bad.append((s, steps[s][1], behind))
+    return bad
+
+
+def test_conv_kernel_waits_for_its_weights(assembly):
+    """conv3_kernel's barriers wait with a count, the number of vector memory operations behind the loads that must have landed. The
+    compiler may merge operations that the count holds as two (it did that to two 8-byte stores of sums: the wait then let the last weight loads
+    through, and one bf16 launch in about ten thousand multiplied with the weights that the slot held before) or move one, so they are counted in its
+    output."""
+    kernels = {k: v for k, v in kernel_bodies(assembly["conv.hip"][0]).items() if "conv3_kernel" in k}
+    assert len(kernels) == 4
+    for name, body in sorted(kernels.items()):
+        steps = conv_barriers(body)
+        assert len(steps) == 27 and all(issued.count("W") == 4 for issued, _ in steps), (name, steps)
+        assert not early_barriers(steps), (name, early_barriers(steps))
+
+
+def test_the_barrier_count_sees_a_merged_store():
+    steps = [("WWWWVV", 10), ("PPWWWWV", 13), ("PPWWWWV", 15)] + [("PPWWWWV", 15)] * 15 + [("WWWW", 8)] * 9
+    assert early_barriers(steps) == [] and early_barriers(steps[:18] + [("WWWW", 9)] + steps[19:]) == [(18, 9, "WWWWWWWW")]
+    merged = steps[:9] + [("PPWWWW", 15)] + steps[10:]                  # one operation fewer than three waits count
+    assert [s for s, _, _ in early_barriers(merged)] == [9, 10, 11]
+
+
 def test_projection_k_loops_carry_no_second_address_chain(assembly):
     """One K step of a projection in the ring kernel steps both operands along K by the same byte offset. Convolutions, which
     share the loop, need a row offset of their own for the activations; when the projections' bases went through the same
