@@ -675,6 +675,20 @@ extern "C" int flux_hip_linear_f32_slices(const void *A, const void *W, float *C
 
 extern "C" size_t flux_hip_vae_attention_work_floats(int n, int ld) { return (size_t)n * (ATT_SAMPLE + 1 + ld / 64) + 4; }
 
+/* The reference's keys are 0, step, 2 step, ...: the largest step that stays within the image and has no factor in common with
+ * its positions, hence none with its width. Multiples of it then fall on as many columns as there are samples (every 64th of 128 x 128
+ * positions are two columns, one of them at the border). From 2560 positions on that is at most 13 below the largest that stays within, and the
+ * samples span 46 % of the image at least. */
+extern "C" int flux_hip_vae_attention_sample_step(int keys) {
+    const auto common = [](int a, int b) {
+        while (b) { const int r = a % b; a = b; b = r; }
+        return a;
+    };
+    int step = keys / ATT_SAMPLE;
+    while (step > 1 && common(keys, step) != 1) step--;
+    return step;
+}
+
 /* Attention of n queries (rows of qkv from q on, 3 * 512 wide) over `keys` positions: out [n][512]. qkv: every position's [q | k | v], ld rows of
  * them (zeros beyond keys); vt: v transposed, [512][ld]; P: n x ld bf16; o32: n x 512; work: flux_hip_vae_attention_work_floats. At least
  * 256 keys, ld a multiple of 256. *done = 0 where the scores' kernel is switched off: nothing is launched. */
@@ -688,7 +702,7 @@ extern "C" int flux_hip_vae_attention(void *out, const void *q, const void *qkv,
     hipStream_t st = flux_hip_stream_handle();
     const bf16 *k = (const bf16 *)qkv + ATT_C;
     flux_hip_linear_part sp = {q, k, sample, nullptr, n};
-    if (!flux_hip_linear(FLUX_HIP_EPI_F32, 1, &sp, ATT_SAMPLE, ATT_C, 3 * ATT_C, keys / ATT_SAMPLE * 3 * ATT_C, ATT_SAMPLE, 0, 0)) return 0;
+    if (!flux_hip_linear(FLUX_HIP_EPI_F32, 1, &sp, ATT_SAMPLE, ATT_C, 3 * ATT_C, flux_hip_vae_attention_sample_step(keys) * 3 * ATT_C, ATT_SAMPLE, 0, 0)) return 0;
     hipLaunchKernelGGL(vae_attention_ref_kernel, dim3((n + 3) / 4), dim3(256), 0, st, ref, sample, n, scale2);
     LAUNCH_OK("vae_attention_ref_kernel");
     int pieces = 0, slices = 0;

@@ -107,6 +107,25 @@ def test_projections_that_leave_slices_check_their_arguments(name):
     assert f(None, None, None, 0, 256, 512, ctypes.byref(ws), ctypes.byref(n)) == 1      # no rows: nothing to do
 
 
+def test_attention_reference_samples_every_column():
+    """The 256 keys that give the VAE attention's reference are spread over the image: over its columns - all of them, or as many as there
+    are keys - and over at least two fifths of its rows; for every image from 2560 positions on that a picture or a latent can have. (The position
+    count alone decides, so the step has no factor in common with it.)"""
+    f = fluxhip.lib().flux_hip_vae_attention_sample_step
+    f.argtypes = [ctypes.c_int]
+    for h in range(2, 225, 2):
+        for w in range(2, 225, 2):
+            keys = h * w
+            if keys < 2560:
+                continue
+            step = f(keys)
+            assert 1 <= step <= keys // 256, (h, w)
+            sample = np.arange(256) * step
+            assert len(np.unique(sample % w)) >= min(w, 256), (h, w, step)
+            assert sample[-1] >= 0.4 * keys, (h, w, step)
+    assert f(256) == 1 and f(511) == 1
+
+
 def test_touching_a_result_buffer_leaves_its_contents():
     """The result's pages are touched while the device computes it; when the call fails afterwards the caller's buffer
     holds what it held before. Sizes around a page, at offsets of every kind."""
