@@ -452,7 +452,7 @@ __global__ __launch_bounds__(256) void vae_softmax_reg_kernel(bf16 *__restrict__
 /* ---- the same attention for many positions, without the scores: P leaves the first product as 2^(scale score - reference)
  * (flux_hip_linear_exp), the second product is divided by the row sums. A softmax does not care about its reference as long as
  * nothing overflows: here it is the row's largest score over 256 keys spread over the image (2 to 3 % of the first product's work). A row
- * with a score more than 2^100 above that - its sums show it - is computed once more by its wave, key by key. In a decode
+ * with a score more than 2^100 above that - its sums show it - is computed once more by a kernel of its own. In a decode
  * of 1024 x 1024 (16384 positions): 394 us of scores + 347 of softmax + 222 of P v with the scores in memory; now 18 + 295 + 244, of which
  * the exponentials, which nothing overlaps, are about 80. (In chunks whose P the memory-side cache would hold it is no faster.) ---- */
 #define ATT_C 512          /* channels of the one head */
@@ -474,10 +474,10 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-/* out[row] = (sum of the slices) / (sum of the row's sums), one wave per row, eight channels per lane */
-__global__ __launch_bounds__(256) void vae_attention_out_kernel(bf16 *__restrict__ out, const float *__restrict__ o, int slices, const float *__restrict__ sums,
-                                                                int pieces, const bf16 *__restrict__ q, const bf16 *__restrict__ qkv, int n, int keys,
-                                                                float scale) {
+/* out[row] = (sum of the slices) / (sum of the row's sums), one wave per row, eight channels per lane; missed[row] = 1 where a sum says that
+ * the reference was too low, else 0 */
+__global__ __launch_bounds__(256) void vae_attention_out_kernel(bf16 *__restrict__ out, float *__restrict__ missed, const float *__restrict__ o, int slices,
+                                                                const float *__restrict__ sums, int pieces, int n) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, c = lane * 8;
     if (row >= n) return;
     const size_t slice = (size_t)n * ATT_C;
@@ -498,33 +498,125 @@ __global__ __launch_bounds__(256) void vae_attention_out_kernel(bf16 *__restrict
         beyond = beyond || v > ATT_SUM_MAX;
     }
     sum = wave_sum(sum);
-    if (__any(beyond)) {
-        const bf16x8 qr = *(const bf16x8 *)(q + (size_t)row * 3 * ATT_C + c);
-        const auto score = [&](int key) {
-            const bf16x8 kr = *(const bf16x8 *)(qkv + (size_t)key * 3 * ATT_C + ATT_C + c);
-            float d = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 8; e++) d += (float)qr[e] * (float)kr[e];
-            return wave_sum(d) * scale;
-        };
-        float m = -INFINITY;
-        for (int key = 0; key < keys; key++) m = fmaxf(m, score(key));
-        sum = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 8; e++) acc[e] = 0.0f;
-        for (int key = 0; key < keys; key++) {
-            const float p = fast_exp2(score(key) - m);
-            const bf16x8 vr = *(const bf16x8 *)(qkv + (size_t)key * 3 * ATT_C + 2 * ATT_C + c);
-            sum += p;
-#pragma unroll
-            for (int e = 0; e < 8; e++) acc[e] += p * (float)vr[e];
-        }
-    }
+    beyond = __any(beyond);
+    if (lane == 0) missed[row] = beyond ? 1.0f : 0.0f;
     const float inv = 1.0f / sum;
     bf16x8 r;
 #pragma unroll
     for (int e = 0; e < 8; e++) r[e] = (bf16)(acc[e] * inv);
     *(bf16x8 *)(out + (size_t)row * ATT_C + c) = r;
+}
+
+/* The rows that missed, anew. A workgroup looks at 16 rows at a time (usually none of them missed), each of its waves takes every fourth run of 32
+ * keys with a running maximum, and the four results are joined. S^T = K Q^T leaves a lane four scores of one row and block; the second block's keys lie
+ * between the first one's, so that the lane's eight are those it holds of the second product's operand. Probabilities stay fp32 as far as
+ * two bf16 operands carry them (2^-17). What bounds it is how long the loads of a run take: one wave per SIMD, whose 32 of K and then of V are requested
+ * together. Attention over 16384 positions, us: 590 with no row missed, 1740 with one, 4250 with all (4096: 64, 311, 304); key by key in one wave, with a
+ * reduction for each score, one row took 19900 (3790). The launch itself is 2 us. */
+#define REDO_ROWS 16
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void vae_attention_redo_kernel(
+    bf16 *__restrict__ out, const float *__restrict__ missed, const bf16 *__restrict__ q, const bf16 *__restrict__ qkv, const bf16 *__restrict__ vt, int n, int keys,
+    int ld, float scale) {
+    __shared__ __attribute__((aligned(16))) float so[REDO_ROWS][ATT_C + 4];
+    __shared__ float sm[4][REDO_ROWS], sl[4][REDO_ROWS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l15 = lane & 15, lq = lane >> 4;
+    constexpr int KS = ATT_C / 32, CB = ATT_C / 16;
+    constexpr float LOW = -3.402823466e38f; /* finite: no difference of two of them is NaN */
+    const __amdgpu_buffer_rsrc_t kbuf = __builtin_amdgcn_make_buffer_rsrc((void *)qkv, 0, (int)((unsigned)ld * 3 * ATT_C * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t vbuf = __builtin_amdgcn_make_buffer_rsrc((void *)vt, 0, (int)((unsigned)ld * ATT_C * 2), 0x00020000);
+    const auto load = [](__amdgpu_buffer_rsrc_t b, unsigned off, int soff) { return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(b, off, soff, 0)); };
+    for (int r0 = blockIdx.x * REDO_ROWS; r0 < n; r0 += gridDim.x * REDO_ROWS) {
+        if (!__any(r0 + l15 < n && missed[min(r0 + l15, n - 1)] != 0.0f)) continue; /* the same in all four waves */
+        bf16x8 fq[KS], f[KS];
+#pragma unroll
+        for (int k = 0; k < KS; k++) fq[k] = *(const bf16x8 *)(q + (size_t)min(r0 + l15, n - 1) * 3 * ATT_C + 32 * k + 8 * lq);
+        f32x4 o[CB];
+#pragma unroll
+        for (int i = 0; i < CB; i++) o[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        float m = LOW, l = 0.0f;
+        for (int k0 = 32 * wave; k0 < ld; k0 += 128) { /* ld is a multiple of 256, and every wave's first run has keys */
+            float p[8], mx = m;
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                const unsigned at = (unsigned)((k0 + 8 * (l15 >> 2) + 4 * b + (l15 & 3)) * 3 * ATT_C + ATT_C + 8 * lq) * 2u;
+                f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int k = 0; k < KS; k++) f[k] = load(kbuf, at + 64 * k, 0);
+#pragma unroll
+                for (int k = 0; k < KS; k++) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[k], fq[k], s, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    p[4 * b + e] = k0 + 8 * lq + 4 * b + e < keys ? s[e] * scale : LOW;
+                    mx = fmaxf(mx, p[4 * b + e]);
+                }
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            if (__any(mx > m)) {
+                const float a = fast_exp2(m - mx);
+                l *= a;
+#pragma unroll
+                for (int i = 0; i < CB; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[i][e] *= a;
+                m = mx;
+            }
+            bf16x8 hi, lo;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float v = k0 + 8 * lq + e < keys ? fast_exp2(p[e] - m) : 0.0f;
+                l += v;
+                hi[e] = (bf16)v;
+                lo[e] = (bf16)(v - (float)hi[e]);
+            }
+#pragma unroll
+            for (int h = 0; h < CB; h += KS) {
+#pragma unroll
+                for (int i = 0; i < KS; i++) f[i] = load(vbuf, (unsigned)(l15 * ld + k0 + 8 * lq) * 2u, 32 * (h + i) * ld);
+#pragma unroll
+                for (int i = 0; i < KS; i++) {
+                    o[h + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[i], hi, o[h + i], 0, 0, 0);
+                    o[h + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[i], lo, o[h + i], 0, 0, 0);
+                }
+            }
+        }
+        l += __shfl_xor(l, 16);
+        l += __shfl_xor(l, 32);
+        if (lq == 0) {
+            sm[wave][l15] = m;
+            sl[wave][l15] = l;
+        }
+        __syncthreads();
+        const float share = fast_exp2(m - fmaxf(fmaxf(sm[0][l15], sm[1][l15]), fmaxf(sm[2][l15], sm[3][l15])));
+        for (int w = 0; w < 4; w++) {
+            if (wave == w)
+#pragma unroll
+                for (int i = 0; i < CB; i++) {
+                    f32x4 *d = (f32x4 *)&so[l15][16 * i + 4 * lq];
+                    f32x4 v = w ? *d : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] += o[i][e] * share;
+                    *d = v;
+                }
+            __syncthreads();
+        }
+        const int r = threadIdx.x >> 4, c0 = (threadIdx.x & 15) * 8, row = r0 + r;
+        if (row < n && missed[row] != 0.0f) {
+            const float top = fmaxf(fmaxf(sm[0][r], sm[1][r]), fmaxf(sm[2][r], sm[3][r]));
+            float sum = 0.0f;
+#pragma unroll
+            for (int w = 0; w < 4; w++) sum += sl[w][r] * fast_exp2(sm[w][r] - top);
+            const float inv = 1.0f / sum;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                bf16x8 v;
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] = (bf16)(so[r][c0 + 128 * k + e] * inv);
+                *(bf16x8 *)(out + (size_t)row * ATT_C + c0 + 128 * k) = v;
+            }
+        }
+        __syncthreads(); /* the next 16 rows write the same LDS */
+    }
 }
 
 /* vt[c][j] = v[j][c] for j < rows, 0 for rows <= j < ld: the value matrix as the "weight" operand
@@ -709,9 +801,11 @@ extern "C" int flux_hip_vae_attention(void *out, const void *q, const void *qkv,
     if (!flux_hip_linear_exp(q, k, P, n, ld, ATT_C, 3 * ATT_C, 3 * ATT_C, ref, scale2, keys, sums, &pieces)) return 0;
     const float *ws = nullptr;
     if (!flux_hip_linear_f32_slices(P, vt, o32, n, ATT_C, ld, &ws, &slices)) return 0;
-    hipLaunchKernelGGL(vae_attention_out_kernel, dim3((n + 3) / 4), dim3(256), 0, st, (bf16 *)out, slices ? ws : o32, slices ? slices : 1, sums, pieces,
-                       (const bf16 *)q, (const bf16 *)qkv, n, keys, scale2);
+    hipLaunchKernelGGL(vae_attention_out_kernel, dim3((n + 3) / 4), dim3(256), 0, st, (bf16 *)out, ref, slices ? ws : o32, slices ? slices : 1, sums, pieces, n);
     LAUNCH_OK("vae_attention_out_kernel");
+    hipLaunchKernelGGL(vae_attention_redo_kernel, dim3(min((n + REDO_ROWS - 1) / REDO_ROWS, 256)), dim3(256), 0, st, (bf16 *)out, ref, (const bf16 *)q, (const bf16 *)qkv,
+                       (const bf16 *)vt, n, keys, ld, scale2);
+    LAUNCH_OK("vae_attention_redo_kernel");
     *done = 1;
     return 1;
 }

@@ -674,6 +674,51 @@ def test_attention_without_scores(hip, switches, keys, n, planted):
     np.testing.assert_array_less(np.abs(got - want).max(1), 2.0 ** -6 * np.abs(want).max(1) + 1e-6)
 
 
+@pytest.mark.parametrize("keys,n", [(256, 17), (300, 300), (1300, 1023), (4096, 4096)])
+def test_attention_without_scores_rows_anew(hip, switches, keys, n):
+    """Rows whose largest scores lie 2^150 above the reference - here three keys outside the sample, within a factor of 2^2.4 of each
+    other, so that the result mixes them - against float64: every row, and every third one, between rows that did not miss. They cost
+    no more than a small multiple of the others (key by key in one wave they took 60 times as long at 4096 positions)."""
+    import ctypes
+    C, ld, L = 512, (keys + 255) & ~255, hip.lib()
+    rng = np.random.default_rng(keys + n)
+    qkv = np.zeros((ld, 3, C), np.float32)
+    qkv[:keys] = q(rng.standard_normal((keys, 3, C)).astype(np.float32))
+    scale, first = 1.0 / np.sqrt(C), keys - n
+    sample = np.arange(256) * L.flux_hip_vae_attention_sample_step(keys)
+    outside = np.setdiff1d(np.arange(keys), sample)
+    planted = outside[[0, len(outside) // 2, -1]] if len(outside) else np.array([0, 100, 255])      # 256 keys: all are in the sample, no row misses
+    qkv[:keys, 1, 0] = 0.0
+    qkv[planted, 1, 0] = 64.0, 63.5, 63.0
+    L.flux_hip_vae_attention_work_floats.restype = ctypes.c_size_t
+    L.flux_hip_vae_attention.argtypes = [ctypes.c_void_p] * 7 + [ctypes.c_int] * 3 + [ctypes.c_float, ctypes.c_void_p]
+    P, work, o32 = hip.DevBuf(n * ld * 2), hip.DevBuf(L.flux_hip_vae_attention_work_floats(n, ld) * 4), hip.DevBuf(n * C * 4)
+    dv, done = hip.DevBuf.from_array(f32_to_bf16(np.ascontiguousarray(qkv[:, 2].T))), ctypes.c_int(0)
+    us = {}
+    for every in (1, 3, 0):
+        qkv[:, 0, 0] = 0.0
+        if every:
+            qkv[:keys:every, 0, 0] = 150.0 * np.log(2.0) / scale / 64.0
+        x = q(qkv)
+        dq = hip.DevBuf.from_array(f32_to_bf16(x.reshape(ld, 3 * C)))
+        out = hip.DevBuf.from_array(np.full((n + 1, C), 0x4040, np.uint16))
+        for _ in range(3):
+            hip.sync()
+            L.flux_hip_timer_start()
+            hip.check(L.flux_hip_vae_attention(out.ptr, dq.at(first * 3 * C * 2), dq.ptr, dv.ptr, P.ptr, o32.ptr, work.ptr, n, keys, ld, scale, ctypes.byref(done)))
+            us[every] = min(us.get(every, 1e9), 1e3 * L.flux_hip_timer_stop())
+        assert done.value == 1
+        bits = out.to_array(np.uint16, (n + 1, C))
+        assert (bits[n] == 0x4040).all()
+        x = x[:keys].astype(np.float64)
+        s = x[first:, 0] @ x[:, 1].T * scale
+        p = np.exp(s - s.max(1, keepdims=True))
+        want, got = p @ x[:, 2] / p.sum(1, keepdims=True), bf16_to_f32(bits[:n])
+        assert rel_l2(got, want) < 2.0 ** -8
+        np.testing.assert_array_less(np.abs(got - want).max(1), 2.0 ** -6 * np.abs(want).max(1) + 1e-6)
+    assert max(us[1], us[3]) < 20.0 * us[0], us
+
+
 def test_attention_without_scores_reports_a_refused_product(hip):
     """What the score product refuses (here probabilities that do not start on 16 bytes, looked at on the host) is the caller's
     error, not a reason to go on with the scores in memory."""
