@@ -91,7 +91,7 @@ struct flux_hip_vae {
     vslot *slots;
     int nslots, cap_slots, adding_side;
     /* work buffers, grown on demand */
-    size_t f32_elems, bf16_elems, guard, att_ld, att_chunk, gn_floats, lat_elems, img_pixels, st_floats;
+    size_t f32_elems, bf16_elems, guard, att_ld, att_chunk, s_elems, gn_floats, lat_elems, img_pixels, st_floats;
     float *X, *Y, *Hb, *S, *kbias, *gn, *lat, *img_f32, *st_x, *st_h;
     void *A_base, *R, *P, *VT;
     uint8_t *img_u8;
@@ -336,7 +336,7 @@ static void free_work(flux_hip_vae *v) {
     v->X = v->Y = v->Hb = v->S = v->kbias = v->gn = v->lat = v->img_f32 = v->st_x = v->st_h = NULL;
     v->A_base = v->R = v->P = v->VT = NULL;
     v->img_u8 = NULL;
-    v->f32_elems = v->bf16_elems = v->guard = v->att_ld = v->att_chunk = v->gn_floats = v->lat_elems = v->img_pixels = v->st_floats = 0;
+    v->f32_elems = v->bf16_elems = v->guard = v->att_ld = v->att_chunk = v->s_elems = v->gn_floats = v->lat_elems = v->img_pixels = v->st_floats = 0;
 }
 
 void flux_hip_vae_free(flux_hip_vae *v) {
@@ -358,8 +358,12 @@ void flux_hip_vae_free(flux_hip_vae *v) {
     free(v);
 }
 
+/* From how many positions on the attention's scores stay out of memory: 2048 positions take 42 us with them and 44 without (two more launches), 3072
+ * 58 and 55, 4096 81 and 66, 16384 1007 and 594 (attention alone, random operands). */
+#define ATT_EXP_ROWS 2560
+
 /* Test hook: upper bound on the query rows per attention chunk (0 = the buffer's own bound,
- * 1 GB of fp32 scores). */
+ * 512 MB of probabilities). */
 static int g_att_chunk_limit = 0;
 void flux_hip_vae_set_attention_chunk(int rows) { g_att_chunk_limit = rows > 0 ? rows : 0; }
 
@@ -373,12 +377,15 @@ static int ensure_work(flux_hip_vae *v, int h, int w) {
     size_t f32_elems = mp0 * 256, guard = (wp0 + 2) * 512;
     size_t bf16_elems = mp0 * 256;
     if (bf16_elems < ld * 1536) bf16_elems = ld * 1536; /* R also holds q, k, v of the attention */
-    size_t chunk = ((size_t)1 << 28) / ld; /* at most 1 GB of fp32 scores at a time: a picture of 1024x1024 is one piece, 1792x1792 ten, which take what five of 2 GB do (51.1 ms a decode) */
+    size_t chunk = ((size_t)1 << 28) / ld; /* at most 512 MB of probabilities at a time: a picture of 1024x1024 is one piece, 1792x1792 ten, which take what five do (51.1 ms a decode) */
     if (chunk < 128) chunk = 128;
     if (chunk > mpm) chunk = mpm;
+    /* scores: only below ATT_EXP_ROWS positions (26 MB; beyond, 1 GB of them stood here unused), and for runs with the ring kernel switched off, in
+     * as many more pieces as that takes */
+    const size_t s_elems = mpm < ATT_EXP_ROWS ? mpm * ld : (size_t)ATT_EXP_ROWS * ATT_EXP_ROWS;
     const size_t gn_floats = flux_hip_group_norm_scratch_floats((int)hp0, (int)wp0);
     const size_t st_floats = (mp0 / 32 + 2) * (256 / 4) * 2; /* convolution statistics: at most rows/32 + 2 partial rows of cout/4 quads */
-    if (f32_elems <= v->f32_elems && bf16_elems <= v->bf16_elems && guard <= v->guard && ld <= v->att_ld && chunk <= v->att_chunk &&
+    if (f32_elems <= v->f32_elems && bf16_elems <= v->bf16_elems && guard <= v->guard && ld <= v->att_ld && chunk <= v->att_chunk && s_elems <= v->s_elems &&
         gn_floats <= v->gn_floats && st_floats <= v->st_floats && (size_t)128 * h * w <= v->lat_elems && (size_t)256 * h * w <= v->img_pixels)
         return 1;
     flux_hip_sync();
@@ -388,7 +395,7 @@ static int ensure_work(flux_hip_vae *v, int h, int w) {
     v->Hb = (float *)flux_hip_malloc(f32_elems * 4);
     v->A_base = flux_hip_malloc((bf16_elems + 2 * guard) * 2);
     v->R = flux_hip_malloc(bf16_elems * 2);
-    v->S = (float *)flux_hip_malloc(chunk * ld * 4);
+    v->S = (float *)flux_hip_malloc(s_elems * 4);
     v->P = flux_hip_malloc(chunk * ld * 2);
     v->VT = flux_hip_malloc(512 * ld * 2);
     v->kbias = (float *)flux_hip_malloc(ld * 4);
@@ -405,7 +412,7 @@ static int ensure_work(flux_hip_vae *v, int h, int w) {
     }
     /* guards are read (their contents never reach an output that is kept), so give them defined values */
     if (!flux_hip_memset(v->A_base, 0, (bf16_elems + 2 * guard) * 2)) return 0;
-    v->f32_elems = f32_elems; v->bf16_elems = bf16_elems; v->guard = guard; v->att_ld = ld; v->att_chunk = chunk;
+    v->f32_elems = f32_elems; v->bf16_elems = bf16_elems; v->guard = guard; v->att_ld = ld; v->att_chunk = chunk; v->s_elems = s_elems;
     v->gn_floats = gn_floats; v->st_floats = st_floats; v->lat_elems = (size_t)128 * h * w; v->img_pixels = (size_t)256 * h * w;
     return 1;
 }
@@ -452,9 +459,6 @@ static int run_res(vstate *s, const vres *r, void *out_bf16) {
     return run_conv(s, &r->c2, FLUX_HIP_EPI_CONV_F32, s->A, s->x, s->x, 1, v->st_x, &s->x_rows);
 }
 
-/* From how many positions on the scores stay out of memory: 2048 positions take 42 us with them and 44 without (two more launches), 3072
- * 58 and 55, 4096 81 and 66, 16384 1007 and 594 (attention alone, random operands). */
-#define ATT_EXP_ROWS 2560
 /* attnblock_forward, flux_vae.c:223-313. Between the two 1x1 convolutions the border positions are left out: a
  * 1024x1024 picture's 16384 positions are 128 tiles of 256 x 256 of the second product, one round of workgroups in two K slices,
  * where the 16900 of the bordered image were 134, two rounds. */
@@ -469,8 +473,9 @@ static int run_attn(vstate *s, const vattn *a) {
     const float scale = 1.0f / sqrtf((float)C);
     int chunk = (int)v->att_chunk;
     if (g_att_chunk_limit && g_att_chunk_limit < chunk) chunk = g_att_chunk_limit;
-    for (int r0 = 0; r0 < rows; r0 += chunk) {
-        const int n = rows - r0 < chunk ? rows - r0 : chunk;
+    int n, masked = 0;
+    for (int r0 = 0; r0 < rows; r0 += n) {
+        n = rows - r0 < chunk ? rows - r0 : chunk;
         if (rows >= ATT_EXP_ROWS) { /* without scores in memory; s->y and Hb are free here, and larger than that */
             int done;
             if (!flux_hip_vae_attention((char *)s->A + (size_t)r0 * C * 2, (char *)v->R + (size_t)r0 * 3 * C * 2, v->R, v->VT, v->P, s->y, v->Hb, n, rows, ld,
@@ -478,7 +483,9 @@ static int run_attn(vstate *s, const vattn *a) {
                 return 0;
             if (done) continue;
         }
-        if (r0 == 0 && !flux_hip_vae_key_bias(v->kbias, ld, rows)) return 0;
+        if ((size_t)n * ld > v->s_elems) n = (int)(v->s_elems / ld); /* (the switched-off case) */
+        if (!masked && !flux_hip_vae_key_bias(v->kbias, ld, rows)) return 0;
+        masked = 1;
         flux_hip_linear_part sp = {(char *)v->R + (size_t)r0 * 3 * C * 2, (char *)v->R + C * 2, v->S, NULL, n};
         if (!flux_hip_linear(FLUX_HIP_EPI_F32, 1, &sp, ld, C, 3 * C, 3 * C, ld, 0, 0)) return 0;
         if (!flux_hip_softmax_rows(v->P, v->S, v->kbias, n, ld, scale)) return 0;

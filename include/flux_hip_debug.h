@@ -53,7 +53,7 @@ void flux_hip_set_batched_cfg(int on);
 /* The fused projection of a single-stream block: 1 (default) = one launch (flux_hip_linear_qkv_swiglu), 0 = two
  * (QKV, then gate/up). */
 void flux_hip_set_fused_qkv_mlp(int on);
-/* VAE attention: at most `rows` query rows per chunk (0 = default: 1 GB of fp32 scores per chunk). */
+/* VAE attention: at most `rows` query rows per chunk (0 = default: 512 MB of bf16 probabilities per chunk). */
 void flux_hip_vae_set_attention_chunk(int rows);
 
 /* Launch probe: probe(epilogue) records HIP events around every later flux_hip_linear launch with
