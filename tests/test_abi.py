@@ -126,6 +126,22 @@ def test_attention_reference_samples_every_column():
     assert f(256) == 1 and f(511) == 1
 
 
+def test_bench_names_the_kernels_that_tiles_launch():
+    """bench.py's names of the tiles, which are looked up in kernel traces, have the template arguments of the launches."""
+    source, bench = (open(os.path.join(ROOT, *p)).read() for p in (("flux2.c_amd", "csrc", "gemm.hip"), ("bench.py",)))
+    body = source[source.index("static int launch_epi("):]
+    body = body[:body.index("\n}\n")]
+    launched = {int(i): (kind, [a for a in args.replace(" ", "").split(",") if a != "EPI"])
+                for i, kind, args in re.findall(r"case (\d+):.*?return launch_(cfg|4d|4w|4x)<([^>]*)>", body)}
+    named = {int(i): args.split(",") for i, args in re.findall(r'(\d+): f"gemm\w*_kernel<([^>]*)>', bench)}
+    assert len(named) >= 13 and len(launched) >= 20
+    for tile, args in named.items():
+        if tile in launched:                                     # (0 is the default)
+            kind, want = launched[tile]
+            got = [a for a in args if a != "{epi_name}"]
+            assert got == (want[:2] if len(got) == 2 and kind != "cfg" else want), (tile, args, want)      # (a ring's depths are left out)
+
+
 def test_touching_a_result_buffer_leaves_its_contents():
     """The result's pages are touched while the device computes it; when the call fails afterwards the caller's buffer
     holds what it held before. Sizes around a page, at offsets of every kind."""
