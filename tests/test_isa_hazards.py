@@ -254,6 +254,71 @@ def test_wide_gemm_tiles_keep_their_accumulators_in_place(assembly):
             assert not copies, (name, copies[:4])
 
 
+def reads_before_first_barrier(body, a, b):
+    """Of the loop body[a:b]: the address registers of its LDS reads in front of the first barrier, and how many the wait there lets through."""
+    addresses, late = [], None
+    for p in map(parse, body[a:b]):
+        if p and p[0].startswith("ds_read"):
+            addresses.append(p[1][1])
+        elif p and p[0] == "s_waitcnt":
+            late = int(re.search(r"lgkmcnt\((\d+)\)", " ".join(p[1])).group(1))
+        elif p and p[0] == "s_barrier":
+            return addresses, late
+
+
+def test_wide_gemm_tiles_read_their_weights_before_the_barrier(assembly):
+    """gemm4x_kernel's first barrier of a step gives the weights' slot to the loads of the step after next: every weight read of the step must have
+    come back. The wait in front of it lets the last reads through, which have to be activation reads, and as many as it counts; they are ordinary
+    reads that the compiler could move, hence this look at its output."""
+    kernels = {k: v for k, v in kernel_bodies(assembly["gemm.hip"][0]).items() if "gemm4x_kernel" in k}
+    assert len(kernels) >= 6
+    for name, body in sorted(kernels.items()):
+        tm, tn = map(int, re.search(r"kernelILi(\d+)ELi(\d+)E", name).groups())
+        loops = [(a, b) for a, b in innermost_loops(body) if sum("v_mfma" in l for l in body[a:b]) >= 2 * tm * tn]
+        assert len(loops) == 2, name
+        for a, b in loops:
+            addresses, late = reads_before_first_barrier(body, a, b)
+            assert len(set(addresses[:tn])) == 1 and addresses[0] not in addresses[tn:], (name, addresses)
+            assert late is not None and late <= len(addresses) - tn, (name, late, addresses)
+
+
+def test_the_read_order_sees_a_late_weight_read():
+    read = "\tds_read_b128 v[%d:%d], %s offset:%d"
+    body = [".LBB0_1:", read % (0, 3, "v90", 0), read % (4, 7, "v90", 2048), read % (8, 11, "v91", 0), "\ts_waitcnt lgkmcnt(1)", "\ts_barrier", "\ts_cbranch_scc1 .LBB0_1"]
+    assert reads_before_first_barrier(body, 0, 6) == (["v90", "v90", "v91"], 1)
+    assert reads_before_first_barrier([body[0], body[1], body[3], body[2]] + body[4:], 0, 6) == (["v90", "v91", "v90"], 1)
+
+
+def test_counted_epilogue_stores_are_there(assembly):
+    """The first step of a tile in the ring kernels waits with the stores of the tile before counted in (at least one per row and group of columns, see
+    EpilogueOps): two that the compiler made into one would let it through early. Epilogues with one path hold exactly that many; of those
+    with two (whole and cut tiles, or 16- and 8-byte stores) the two may share the last one."""
+    seen = 0
+    for name, body in kernel_bodies(assembly["gemm.hip"][0]).items():
+        m = re.search(r"gemm4[dx]_kernelILi(\d+)ELi(\d+)ELi(\d+)E", name)
+        if not m:
+            continue
+        tm, tn, epi = map(int, m.groups())
+        stores = sum(bool(p) and p[0].startswith(("global_store", "buffer_store", "flat_store")) for p in map(parse, body))
+        pairs = tm * (tn // 2 + tn % 2)
+        if epi in (1, 2, 5, 9):                          # fp32, its transpose, partial sums
+            assert stores == tm * tn * (4 if epi == 2 else 1), (name, stores)
+        elif epi == 0:                                   # bf16 in 16-byte or 8-byte stores
+            assert stores >= 2 * tm * (tn // 2) + tm * (tn % 2), (name, stores)
+        elif epi == 3:                                   # residual: whole tiles and cut ones
+            assert stores >= 2 * tm * tn - 1, (name, stores)
+        elif epi == 4:                                   # SiLU(gate) * up
+            assert stores >= tm * (2 * (tn // 4) + tn // 2 % 2 + tn % 2), (name, stores)
+        elif epi == 8:                                   # bf16 on one side, SiLU(gate) * up on the other
+            assert stores >= 2 * tm * (tn // 2) + tm * (tn % 2) + tm * (2 * (tn // 4) + tn // 2 % 2 + tn % 2), (name, stores)
+        elif epi == 10:                                  # exponentials: with columns to clear and without, and a sum per row
+            assert stores >= 2 * (pairs + tm) - 1, (name, stores)
+        else:
+            continue
+        seen += 1
+    assert seen >= 50
+
+
 def test_conv_kernel_owns_the_accumulator_registers(assembly):
     """conv3_kernel names its 256 accumulator registers in its assembly statements: nothing that the compiler itself wrote may
     touch one (a parked vector register would be overwritten), and nothing goes to scratch memory."""
