@@ -16,8 +16,9 @@
  * runs (buffer offsets at flux_vae.c:203, loop order at flux_kernels.c:441-470), its BLAS path in
  * one tile does not.
  *
- * Convolutions run as MFMA GEMMs over bordered channels-last images (flux_hip_conv), the
- * attention as two GEMMs around a row softmax; everything else is in vae.hip.
+ * Convolutions run as MFMA GEMMs over bordered channels-last images (flux_hip_conv; conv.hip for the
+ * large 3x3 ones and those of three channels), the attention as two GEMMs around a row softmax, or, from
+ * ATT_EXP_ROWS positions on, without scores in memory (flux_hip_vae_attention); everything else is in vae.hip.
  */
 #include "../../include/flux_hip.h"
 #include "../../include/flux_hip_debug.h"
