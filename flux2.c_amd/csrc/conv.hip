@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256) void conv3_kernel(Args g) {
             for (int i = 0; i < 4; i++) load_w(t.n0 * ldw * 2 + k * 128, k, i);
     }
     int woff = t.n0 * ldw * 2 + 3 * 128; /* the weights of the step three ahead */
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory"); /* the patch and the first tap's weights have landed */
 #pragma unroll
     for (int q = 0; q < NF; q++) f0[q] = frag(0, 0, 0, q);
 

@@ -1021,13 +1021,14 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
     auto frag = [&](unsigned xa, unsigned xw, int coff, int q) -> bf16x8 {
         return q < TN ? *(const bf16x8 *)(smem + xw + coff + q * 2048) : *(const bf16x8 *)(smem + xa + coff + (q - TN) * 2048);
     };
-    /* the first tile: its first steps are requested here, and everything has landed before its step 0 */
+    /* the first tile: its first steps are requested here, and its step 0 starts when that one has landed (a compute unit takes in 50 KB of cold
+     * operands a microsecond: the other steps of the rings, 64 to 100 KB, are 1.3 to 2 us of every launch) */
     set_sources(cur, t);
     prime(cur, k_steps(t));
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NL + (NS2 == 3 ? LS : 0)) : "memory");
 #pragma unroll
     for (int q = 0; q < NF; q++) f0[q] = frag(va, vw, coff0, q);
-    bool strict = false; /* the first barrier of the tile must not count on the stored tile's operations */
+    bool strict = true; /* the first barrier of the tile must not count on the operations of a stored tile */
 
     for (;;) {
         const int KT = k_steps(t); /* at least 4: the host sends shorter K ranges to gemm4w_kernel */
@@ -1088,8 +1089,7 @@ __global__ __launch_bounds__(256) void gemm4d_kernel(GemmArgs g) {
             va = van;
             vw = vwn;
         };
-        /* step 0: the stored tile's memory operations are older than anything its barrier needs (for the first tile
-         * everything has landed already) */
+        /* step 0: the stored tile's memory operations are older than anything its barrier needs */
         step(0, BoolC<false>{}, IntC<AHEAD_STORES>{}, BoolC<true>{});
         int kt = 1;
         for (; kt < KT - 3; kt++) step(kt, BoolC<false>{}, IntC<AHEAD>{}, BoolC<false>{});
@@ -1242,12 +1242,12 @@ __global__ __launch_bounds__(256) void gemm4x_kernel(GemmArgs g) {
     for (int s = 0; s < 2; s++)
 #pragma unroll
         for (int i = 0; i < NL; i++) issue1(s, s, i);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NL) : "memory"); /* step 0 has landed, as in gemm4d_kernel */
 #pragma unroll
     for (int i = 0; i < TN; i++) w0[i] = *(const bf16x8 *)(smem + w_frag + coff0 + i * 2048);
 #pragma unroll
     for (int j = 0; j < TM; j++) fa[j] = *(const bf16x8 *)(smem + a_frag + coff0 + j * 2048);
-    bool strict = false;
+    bool strict = true;
 
     for (;;) {
         auto serp = [](int b) { return ((b / TN) & 1) ? TN - 1 - b % TN : b % TN; };
