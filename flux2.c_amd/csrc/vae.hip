@@ -254,6 +254,84 @@ __global__ __launch_bounds__(256) void gn_apply_kernel(bf16 *__restrict__ out, b
     for (; r < row_end; r += rpi) one(r, load_quad(src + (size_t)r * C));
 }
 
+/* gn_stats_kernel and gn_apply_kernel in one launch, for images whose convolutions leave few partial rows: a workgroup owns 64 channels of
+ * `span` positions and sums those channels' partial rows itself, with its first positions already requested. What bounds the small images'
+ * norms is the launches, not the bytes. Back to back, one launch against two, us: 16 x 16 x 512 (11 rows of sums) 3.3 / 5.4, 32 x 32 x 512 (37) 3.7 / 5.6,
+ * 64 x 64 x 512 (137) 6.0 / 6.9, 84 x 84 x 512 (72) 6.9 / 7.7, 128 x 128 x 512 (128) 12.7 / 13.0. Every workgroup reads the rows anew: with 232
+ * to 256 of them it is no gain (8.2 / 8.1, 9.0 / 8.5), with 512 a loss (18 / 13). */
+#define GN_FUSED_ROWS 160
+template <typename T>
+__global__ __launch_bounds__(256) void gn_fused_kernel(bf16 *__restrict__ out, bf16 *__restrict__ raw, const T *__restrict__ x, const float *__restrict__ conv,
+                                                       int prows, double count, float eps, const float *__restrict__ gamma, const float *__restrict__ beta,
+                                                       int rows, int C, int hp, int wp, unsigned long long magic, int swish, int span) {
+    __shared__ double part[16][16][2];
+    __shared__ float norm[16][2];
+    const int q = threadIdx.x & 15, r0 = threadIdx.x >> 4, quads = C >> 2, qpg = quads >> 5; /* quads of a group: 1, 2 or 4 */
+    const int quad = blockIdx.y * 16 + q;
+    const int row_begin = blockIdx.x * span, row_end = min(rows, row_begin + span);
+    const T *src = x + quad * 4;
+    f32x4 v[4];
+    const auto request = [&](int r) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = load_quad(src + (size_t)min(r + 16 * k, row_end - 1) * C);
+    };
+    request(row_begin + r0);
+    const f32x4 gm = *(const f32x4 *)(gamma + quad * 4), bt = *(const f32x4 *)(beta + quad * 4);
+    double a = 0.0, b = 0.0;
+#pragma unroll 8
+    for (int r = r0; r < prows; r += 16) {
+        const f32x2 t = *(const f32x2 *)(conv + ((size_t)r * quads + quad) * 2);
+        a += (double)t[0];
+        b += (double)t[1];
+    }
+    part[r0][q][0] = a;
+    part[r0][q][1] = b;
+    __syncthreads();
+    if (threadIdx.x < 64) { /* four lanes a quad, then the quads of a group */
+        const int p = threadIdx.x & 15, k = threadIdx.x >> 4;
+        a = (part[k][p][0] + part[k + 4][p][0]) + (part[k + 8][p][0] + part[k + 12][p][0]);
+        b = (part[k][p][1] + part[k + 4][p][1]) + (part[k + 8][p][1] + part[k + 12][p][1]);
+        a += __shfl_xor(a, 16); b += __shfl_xor(b, 16);
+        a += __shfl_xor(a, 32); b += __shfl_xor(b, 32);
+        for (int o = 1; o < qpg; o <<= 1) { a += __shfl_xor(a, o); b += __shfl_xor(b, o); }
+        const double mean = a / count;
+        double var = b / count - mean * mean;
+        if (var < 0.0) var = 0.0;
+        if (k == 0) {
+            norm[p][0] = (float)mean;
+            norm[p][1] = (float)(1.0 / sqrt(var + (double)eps));
+        }
+    }
+    __syncthreads();
+    const float mean = norm[q][0], rstd = norm[q][1];
+    f32x4 sc, sh;
+#pragma unroll
+    for (int e = 0; e < 4; e++) { sc[e] = gm[e] * rstd; sh[e] = bt[e] - mean * sc[e]; }
+    for (int r = row_begin + r0; r < row_end; r += 64) {
+        f32x4 w[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) w[k] = v[k];
+        if (r + 64 < row_end) request(r + 64);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int rk = r + 16 * k;
+            if (rk >= row_end) break;
+            const int y = div_wp(rk, magic), xx = rk - y * wp;
+            const bool in = y >= 1 && y < hp - 1 && xx >= 1 && xx < wp - 1;
+            bf16x4 o, rw;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float t = w[k][e] * sc[e] + sh[e];
+                if (swish) t = silu_f(t);
+                o[e] = (bf16)(in ? t : 0.0f);
+                rw[e] = (bf16)w[k][e];
+            }
+            *(bf16x4 *)(out + (size_t)rk * C + quad * 4) = o;
+            if (raw) *(bf16x4 *)(raw + (size_t)rk * C + quad * 4) = rw;
+        }
+    }
+}
+
 /* nearest-neighbour 2x upsample (flux_upsample_nearest, flux_kernels.c:1017-1036): fp32 or bf16
  * [hp*wp, C] -> bf16 [(2H+2)*(2W+2), C] with a fresh zero border. One thread per bordered source position and V
  * channels, which go to the source's up to four places: interior (y, x) to rows 2y-1, 2y and columns 2x-1, 2x of the bordered output,
@@ -654,6 +732,14 @@ static int group_norm_run(void *out_bf16, void *raw_bf16, const T *x, const floa
     float *partial = scratch + 64, *stats = scratch;
     hipStream_t st = flux_hip_stream_handle();
     const double count = (double)(hp - 2) * (wp - 2) * (C / 32);
+    const unsigned long long magic = ((1ull << 40) + (unsigned)wp - 1) / (unsigned)wp;
+    if (conv_stats && conv_stats_rows <= GN_FUSED_ROWS) {
+        const int span = (rows + 63) / 64 * (C / 64) > 1024 ? 128 : 64;
+        hipLaunchKernelGGL(gn_fused_kernel<T>, dim3((rows + span - 1) / span, C / 64), dim3(256), 0, st, (bf16 *)out_bf16, (bf16 *)raw_bf16, x, conv_stats,
+                           conv_stats_rows, count, eps, gamma, beta, rows, C, hp, wp, magic, swish, span);
+        LAUNCH_OK("gn_fused_kernel");
+        return 1;
+    }
     if (conv_stats && conv_stats_rows <= GN_ONE_PASS_ROWS) {
         hipLaunchKernelGGL(gn_stats_kernel, dim3(32), dim3(256), 0, st, stats, conv_stats, conv_stats_rows, C, count, eps);
         LAUNCH_OK("gn_stats_kernel");
@@ -671,7 +757,6 @@ static int group_norm_run(void *out_bf16, void *raw_bf16, const T *x, const floa
         hipLaunchKernelGGL(gn_finalize_kernel, dim3(32), dim3(256), 0, st, stats, partial, nblocks, count, eps);
         LAUNCH_OK("gn_finalize_kernel");
     }
-    const unsigned long long magic = ((1ull << 40) + (unsigned)wp - 1) / (unsigned)wp;
     /* as many positions per workgroup as leave 2048 workgroups, at least four per thread */
     int span = GN_ROWS;
     while (span > 4 * (256 / (C / 4)) && (rows + span - 1) / span < 2048) span >>= 1;

@@ -598,6 +598,31 @@ def test_group_norm_statistics_in_one_or_two_launches(hip, prows, C):
     assert rel_l2(from_padded(got, H, W), want) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("H,W,C", [(3, 5, 128), (34, 31, 256), (9, 8, 512), (92, 91, 512)])
+@pytest.mark.parametrize("prows", [1, 17, 160])
+@pytest.mark.parametrize("in_bf16", [0, 1])
+def test_group_norm_in_one_launch(hip, H, W, C, prows, in_bf16):
+    """Up to 160 rows of sums the norm is one launch. Rows of zeros behind them send the same sums to two: the same doubles but for the
+    order of their additions, so at most one bf16 rounding (2^-8 relative) apart; the raw copy is the same."""
+    rows = (H + 2) * (W + 2)
+    x = to_padded(normal_f32((C, H, W), 61, 1, 0.3, 1.0))
+    part = np.abs(normal_f32((prows, C // 4, 2), 61, 2))
+    part *= np.array([0.3, 1.09], np.float32) * 4 * H * W / part.sum(0, keepdims=True)
+    dx = hip.DevBuf.from_array(f32_to_bf16(x) if in_bf16 else x)
+    dg, dbt = hip.DevBuf.from_array(normal_f32((C,), 61, 3, 1.0, 0.2)), hip.DevBuf.from_array(normal_f32((C,), 61, 4))
+    scratch = hip.DevBuf(hip.lib().flux_hip_group_norm_scratch_floats(H + 2, W + 2) * 4)
+    got = []
+    for n in (prows, 161):
+        dp = hip.DevBuf.from_array(np.concatenate([part, np.zeros((n - prows, C // 4, 2), np.float32)]))
+        out, raw = (hip.DevBuf.from_array(np.full((rows + 1, C), 0x4040, np.uint16)) for _ in range(2))
+        hip.check(hip.lib().flux_hip_group_norm_stats(out.ptr, raw.ptr, dx.ptr, in_bf16, dg.ptr, dbt.ptr, scratch.ptr, H + 2, W + 2, C, 1e-4, 1, dp.ptr, n))
+        got.append((bf16_to_f32(out.to_array(np.uint16, (rows + 1, C))), raw.to_array(np.uint16, (rows + 1, C))))
+    assert border_is_zero(got[0][0][:rows], H, W)
+    np.testing.assert_allclose(got[0][0], got[1][0], rtol=2.0 ** -7, atol=1e-6)
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+    assert (got[0][0][rows] == got[0][0][rows, 0]).all() and (got[0][1][rows] == 0x4040).all()
+
+
 def test_upsample(hip, oracle_mod):
     C, H, W = 128, 5, 7
     x = normal_f32((C, H, W), 55, 1)
