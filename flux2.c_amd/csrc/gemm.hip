@@ -1317,6 +1317,191 @@ __global__ __launch_bounds__(256) void gemm4x_kernel(GemmArgs g) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+/* 3x3 convolutions of images with too few 16 x 16 tiles for conv.hip's kernel: 128 positions x 64 channels per workgroup.
+ * As a GEMM (the ring kernel's 128 x 128 tile) every K step fetches its 128 positions x 64 channels again, nine times what a chunk of channels
+ * holds, and images this small then need K slices with a second pass to give every compute unit work. Here the positions that a tile's nine taps touch
+ * lie in LDS for a whole chunk (those of the next chunk arrive meanwhile), and the ring holds the weights alone: 11 to 14 KB a step.
+ *
+ * GEMM rows are interior positions in row-major order, so a tile is a run of positions whatever the image's sides. Its neighbourhood is one run
+ * of the bordered image, from a row above the first position to a row below the last one, as long as that is at most 448 positions, and
+ * otherwise (images wider than 155) three runs, one per tap row, CONVP_BAND apart in LDS: the LDS row of position p's tap (dy, dx) is
+ * p - (the tile's first position) + dy * pitch + dx either way, pitch being the image's or CONVP_BAND. NPL: loads of eight LDS rows per wave
+ * and chunk, 28, 40 or 56 KB twice; the weights have the rest.
+ *
+ * Four waves of 64 x 32 would read 1.5 times as many bytes of fragments as the LDS delivers during their MFMAs. So two waves share 64 x 64 and split
+ * the K step, 32 channels each (32 KB of fragments for 256 cycles); their sums meet in LDS at the end. A step is one phase: its fragments are in
+ * registers when it begins, those of the next one are read behind its first MFMAs, and the barrier in front of it waits for the weights of the next
+ * step and leaves the slot of its own to those of SLOTS steps on.
+ *
+ * Alone, operands from the memory-side cache, bf16, us, against the best of the other tiles: 16 x 16 x 512 -> 512 15.9 -> 13.6 (four slices), 32 x 32 x 512 22.4 -> 16.3
+ * (two), 42 x 42 x 512 24.2 -> 16.4, 64 x 64 x 512 29.3 -> 20.2 (two slices before), 84 x 84 x 512 -> 256 29.3 -> 18.4, 64 x 64 x 256 20.6 -> 11.2,
+ * 128 x 128 x 128 13.8 -> 9.9. What bounds it: a unit takes in 12 KB of a step in 0.175 us, 70 KB a microsecond, which is 256 lines on their way
+ * (loads return in order) at the memory-side cache's latency; the MFMAs are 0.11 us of it. 128 channels a tile (with and without the split of K) was 5 %
+ * faster than the ring kernel's 128 x 128 where that has a round of tiles, which was not worth a second kernel. */
+#define CONVP_BAND 144
+template <int NPL> struct ConvP {
+    static constexpr int PP = 3, LW = 2; /* a step's patch loads at most, and weight loads, of a wave */
+    static constexpr int PATCH = NPL * 4096, WSZ = 64 * 128, LAST_TAP = (NPL + PP - 1) / PP - 1, ROOM = (160 * 1024 - 2 * PATCH) / WSZ;
+    static constexpr int SLOTS = ROOM < 9 - LAST_TAP ? ROOM : 9 - LAST_TAP; /* the last patch load of a chunk is older than the weights that the next chunk waits for */
+    static constexpr int LDS = 2 * PATCH + SLOTS * WSZ;
+    static constexpr int patch_loads(int tap) { return tap < 0 || PP * tap >= NPL ? 0 : NPL - PP * tap < PP ? NPL - PP * tap : PP; }
+    /* memory operations that a wave has issued, when it reaches the barrier in front of a tap, behind the weights of the tap after it: what
+     * the steps since have requested, patch loads first (a chunk's last steps request none) */
+    static constexpr int pending(int tap, bool last) {
+        int n = LW * (last && 7 - tap < SLOTS - 2 ? 7 - tap : SLOTS - 2);
+        for (int k = 1; k <= SLOTS - 2; k++) n += last ? 0 : patch_loads(tap - k);
+        return n;
+    }
+    static_assert(SLOTS >= 3 && LDS <= 160 * 1024, "rings");
+};
+
+template <int NPL, int EPI>
+__global__ __launch_bounds__(256) void convp_kernel(GemmArgs g) {
+    using C = ConvP<NPL>;
+    constexpr int BN = 64, TM = 4, TN = 4, NM = TM * TN, NF = TM + TN, SLOTS = C::SLOTS, W0 = 2 * C::PATCH;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, kh = wave >> 1, half = wave & 1; /* half of the K step, half of the positions */
+    const int l15 = lane & 15, lq = lane >> 4;
+    TileId t;
+    if (!decode_tile<true>(g, blockIdx.x, t)) return;
+    const int M = g.M[0], m0 = t.tm * 128, wp = g.conv_wp;
+    const int first = conv_row<FLUX_HIP_EPI_CONV_F32>(g, m0), last_pos = conv_row<FLUX_HIP_EPI_CONV_F32>(g, min(m0 + 127, M - 1));
+    const int span = last_pos - first + 3;                      /* of a tap row's run */
+    const bool bands = span + 2 * wp > NPL * 32;                /* (the host has made sure of 3 * CONVP_BAND <= 32 NPL then) */
+    const int pitch = bands ? CONVP_BAND : wp;
+    const int c0 = t.ks * (g.kt_per / 9), c1 = min(g.lda >> 6, c0 + g.kt_per / 9);
+
+    unsigned prel[NPL], wrel[C::LW]; /* byte offsets of this lane's loads: positions (LDS row r), weights */
+#pragma unroll
+    for (int j = 0; j < NPL; j++) {
+        const int r = 8 * (4 * j + wave) + (lane >> 3);
+        const int b = r >= 2 * CONVP_BAND ? 2 : r >= CONVP_BAND ? 1 : 0;
+        const int p = bands ? first + (b - 1) * wp - 1 + min(r - b * CONVP_BAND, span - 1) : first - wp - 1 + min(r, span + 2 * wp - 1);
+        prel[j] = ((unsigned)p * (unsigned)g.lda + (((lane & 7) ^ lds_swz(r)) << 3)) * 2u;
+    }
+#pragma unroll
+    for (int i = 0; i < C::LW; i++) {
+        const int v = 8 * (4 * i + wave) + (lane >> 3);
+        wrel[i] = ((unsigned)weight_row<BN, BN / 2, EPI>(g, t.tn, v) * (unsigned)g.ldw + (((lane & 7) ^ lds_swz(v)) << 3)) * 2u;
+    }
+    auto load_patch = [&](int chunk, int to, int j) {
+        asm volatile("" : "+v"(prel[j]));
+        __builtin_amdgcn_global_load_lds(GLOBAL_PTR((const char *)g.A[0] + chunk * 128 + prel[j]), LDS_PTR(smem + to + (4 * j + wave) * 1024), 16, 0, 0);
+    };
+    auto load_w = [&](int kt, int slot, int i) {
+        asm volatile("" : "+v"(wrel[i]));
+        __builtin_amdgcn_global_load_lds(GLOBAL_PTR((const char *)g.W[0] + (ptrdiff_t)kt * 128 + wrel[i]), LDS_PTR(smem + W0 + slot * C::WSZ + (4 * i + wave) * 1024), 16, 0, 0);
+    };
+    int kt = 9 * c0, slot = 0, to = C::PATCH; /* K step at work, its slot; where the next chunk's patch goes */
+#pragma unroll
+    for (int j = 0; j < NPL; j++) load_patch(c0, 0, j);
+#pragma unroll
+    for (int s = 0; s < SLOTS; s++)
+#pragma unroll
+        for (int i = 0; i < C::LW; i++) load_w(kt + s, s, i);
+
+    unsigned pa[9][TM]; /* this lane's fragment addresses in the patch at work: a block's positions under each tap */
+#pragma unroll
+    for (int j = 0; j < TM; j++) {
+        const int rel = conv_row<FLUX_HIP_EPI_CONV_F32>(g, min(m0 + half * 64 + j * 16 + l15, M - 1)) - first;
+#pragma unroll
+        for (int tap = 0; tap < 9; tap++) {
+            const int r = rel + tap / 3 * pitch + tap % 3;
+            pa[tap][j] = r * 128 + (((kh * 4 + lq) ^ lds_swz(r)) << 4);
+        }
+    }
+    const unsigned wa = W0 + l15 * 128 + (((kh * 4 + lq) ^ lds_swz(l15)) << 4);
+    auto frag = [&](int tap, int ws, int q) -> bf16x8 {
+        return q < TN ? *(const bf16x8 *)(smem + wa + ws * C::WSZ + q * 2048) : *(const bf16x8 *)(smem + pa[tap][q - TN]);
+    };
+
+    /* Block (i, j) accumulates in a[4 (i TM + j)], by name (left to allocate them the compiler moves all accumulators at the joins of the paths
+     * below); the compiler uses no AGPR (the tests look at its output for that) */
+    asm volatile("" ::: "a255");
+#pragma unroll
+    for (int n = 0; n < 4 * NM; n++) asm volatile("v_accvgpr_write_b32 a[%0], 0" ::"i"(n));
+    asm volatile("s_nop 7" ::: "memory");
+
+    bf16x8 f[2][NF];
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::LW * (SLOTS - 1)) : "memory"); /* the patch and the first tap's weights */
+#pragma unroll
+    for (int q = 0; q < NF; q++) f[0][q] = frag(0, 0, q);
+
+    auto serp = [](int b) { return ((b / TN) & 1) ? TN - 1 - b % TN : b % TN; };
+    auto step = [&](int chunk, auto tap_c, auto last_c, auto set_c) {
+        constexpr int TAP = decltype(tap_c)::value, SET = decltype(set_c)::value; /* the fragments' register set */
+        constexpr bool LAST = decltype(last_c)::value, END = LAST && TAP == 8;    /* the slice's last chunk, and its last step */
+        const int next = slot == SLOTS - 1 ? 0 : slot + 1;
+        if (!END) { /* the next step's weights (and patch) have landed, and this step's have been read */
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(C::pending(TAP, LAST)) : "memory");
+            if (TAP == 8) {
+                const unsigned d = to - (C::PATCH - to);
+#pragma unroll
+                for (int k = 0; k < 9 * TM; k++) pa[k / TM][k % TM] += d;
+                to = C::PATCH - to;
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < NM; b++) {
+            asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(f[SET][serp(b)]), "v"(f[SET][TN + b / TN]),
+                         "i"(4 * (serp(b) * TM + b / TN)), "i"(4 * (serp(b) * TM + b / TN) + 3));
+            if (!END && b < NF) f[SET ^ 1][b] = frag((TAP + 1) % 9, next, b);
+            if (!LAST && b >= NF && b - NF < C::patch_loads(TAP)) load_patch(chunk + 1, to, C::PP * TAP + b - NF);
+            if ((!LAST || TAP + SLOTS <= 8) && b >= 12 && b % 2 == 0 && (b - 12) / 2 < C::LW) load_w(kt + SLOTS, slot, (b - 12) / 2);
+        }
+        slot = next;
+        kt++;
+    };
+    auto taps = [&](int chunk, auto last_c, auto set_c) {
+        constexpr int S = decltype(set_c)::value;
+        step(chunk, IntC<0>{}, last_c, IntC<S>{}); step(chunk, IntC<1>{}, last_c, IntC<S ^ 1>{}); step(chunk, IntC<2>{}, last_c, IntC<S>{});
+        step(chunk, IntC<3>{}, last_c, IntC<S ^ 1>{}); step(chunk, IntC<4>{}, last_c, IntC<S>{}); step(chunk, IntC<5>{}, last_c, IntC<S ^ 1>{});
+        step(chunk, IntC<6>{}, last_c, IntC<S>{}); step(chunk, IntC<7>{}, last_c, IntC<S ^ 1>{}); step(chunk, IntC<8>{}, last_c, IntC<S>{});
+    };
+    for (int c = c0;; c += 2) {
+        if (c == c1 - 1) { taps(c, BoolC<true>{}, IntC<0>{}); break; }
+        taps(c, BoolC<false>{}, IntC<0>{});
+        if (c + 1 == c1 - 1) { taps(c + 1, BoolC<true>{}, IntC<1>{}); break; }
+        taps(c + 1, BoolC<false>{}, IntC<1>{});
+    }
+
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); /* the last MFMA results retire before they are read */
+    /* The two halves of K: a wave keeps half of the channels of its 64 x 64 and hands the others to its partner */
+    constexpr int KN = TN / 2;
+    f32x4 sum[KN][TM];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); /* nobody reads patches or weights any more */
+    const auto hand = [&](auto kh_c) {
+        constexpr int K = decltype(kh_c)::value;
+        const auto block = [&](int keep, int i, int j) {
+            const int n = (keep * KN + i) * TM + j;
+            f32x4 a;
+            asm volatile("v_accvgpr_read_b32 %0, a[%4]\n\tv_accvgpr_read_b32 %1, a[%5]\n\tv_accvgpr_read_b32 %2, a[%6]\n\tv_accvgpr_read_b32 %3, a[%7]"
+                         : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]) : "i"(4 * n), "i"(4 * n + 1), "i"(4 * n + 2), "i"(4 * n + 3));
+            return a;
+        };
+#pragma unroll
+        for (int i = 0; i < KN; i++)
+#pragma unroll
+            for (int j = 0; j < TM; j++) {
+                *(f32x4 *)(smem + ((wave * KN + i) * TM + j) * 1024 + lane * 16) = block(K ^ 1, i, j);
+                sum[i][j] = block(K, i, j);
+            }
+    };
+    if (kh) hand(IntC<1>{});
+    else hand(IntC<0>{});
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < KN; i++)
+#pragma unroll
+        for (int j = 0; j < TM; j++) sum[i][j] += *(const f32x4 *)(smem + (((wave ^ 2) * KN + i) * TM + j) * 1024 + lane * 16);
+    int l15e = l15, lqe = lq;
+    asm volatile("" : "+v"(l15e), "+v"(lqe));
+    const GemmArgs ge = conv_args_again();
+    if constexpr (EPI == EPI_CONV_PARTIAL) store_tile<BN, 64, BN / 2, EPI, 2, true>(g, t, sum, m0, M, half, kh, l15e, lqe, t.tm * 2 + half);
+    else store_tile<BN, 64, BN / 2, EPI, 2, true>(ge, t, sum, m0, ge.M[0], half, kh, l15e, lqe, t.tm * 2 + half);
+}
+
 /* ------------------------------------------------------------------ host side */
 
 static int g_persistent = 1;
@@ -2238,8 +2423,37 @@ extern "C" int flux_hip_linear_resid_adaln(int nparts, const flux_hip_linear_par
 /* Tiles of a convolution: 15 = conv.hip's kernel for 3x3 without stride; ids 0 to 3 as above (64 x 128, 128 x 128, 256 x 256, 64 x 64), 12 = 256 x 128, 13 =
  * 128 x 128 in the ring kernel, as is 2: 128 x 128 in two stages reached 700 to 870 TFLOP/s on 3x3 layers of 128 to 512 channels over
  * 128 x 128 to 1024 x 1024 positions, 256 x 128 reaches 920 to 1230 and 256 x 256 1200 to 1390 (bf16 output). */
+#define CONV_PATCH 15 /* 16 x 16 positions x 128 channels, conv.hip */
+#define CONV_RUN 14   /* 128 consecutive positions x 64 channels, convp_kernel */
+/* LDS rows that the largest neighbourhood of 128 consecutive positions takes, see convp_kernel */
+static int convp_rows(int width) {
+    const int run = 128 + 2 * ((127 + width - 1) / width) + 2, one = run + 2 * (width + 2);
+    return one <= 448 ? one : run <= CONVP_BAND ? 3 * CONVP_BAND : 1 << 30;
+}
+template <int NPL, int EPI>
+static int launch_convp(GemmArgs &g) {
+    constexpr int LDS = ConvP<NPL>::LDS;
+    static bool attr_done = false;
+    auto kern = convp_kernel<NPL, EPI>;
+    if (!attr_done) {
+        HIP_OK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        attr_done = true;
+    }
+    set_row_tiles(g, 128);
+    g.ntiles = g.N / 64;
+    g.total_tiles = g.mtiles * g.ntiles;
+    g.vgrid = (g.total_tiles * g.ksplit + 7) & ~7;
+    hipLaunchKernelGGL(kern, dim3(g.vgrid), dim3(256), LDS, flux_hip_stream_handle(), g);
+    HIP_OK(hipGetLastError());
+    return 1;
+}
+
 template <int EPI>
 static int conv_tile_launch(GemmArgs &g, int tile) {
+    if (tile == CONV_RUN) {
+        const int rows = convp_rows(g.conv_wp - 2);
+        return rows <= 224 ? launch_convp<7, EPI>(g) : rows <= 320 ? launch_convp<10, EPI>(g) : launch_convp<14, EPI>(g);
+    }
     switch (tile) {
         case 2: return launch_4d<8, 8, EPI, 2, 3>(g);
         case 12: return launch_4d<8, 4, EPI, 3, 3>(g);
@@ -2251,8 +2465,7 @@ static int conv_tile_launch(GemmArgs &g, int tile) {
 }
 
 #define CONV_TILES 16
-static const int conv_bm[CONV_TILES] = {64, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 256, 128, 0, 256}, conv_bn[CONV_TILES] = {128, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 128, 128, 0, 128};
-#define CONV_PATCH 15 /* 16 x 16 positions x 128 channels, conv.hip */
+static const int conv_bm[CONV_TILES] = {64, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 256, 128, 128, 256}, conv_bn[CONV_TILES] = {128, 128, 256, 64, 0, 0, 0, 0, 0, 0, 0, 0, 128, 128, 64, 128};
 
 template <int EPI>
 static int conv_finish(GemmArgs &g) {
@@ -2269,8 +2482,8 @@ static int conv_finish(GemmArgs &g) {
  * 256 x 128) as long as the image's sides do not leave a second, nearly empty round (90 x 162 x 512: 264 of its tiles, 90 us; 228 of 256 x 128,
  * 59 us). Over 111 forms of 37 layers the chosen tile took 1.5 % less than the best of four timed behind it, i.e. the same. */
 static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
-    static const int occ[CONV_TILES] = {3, 2, 1, 4, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 0, 1};
-    static const double rate[CONV_TILES] = {2.0e12, 3.3e12, 5.4e12, 1.5e12, 0, 0, 0, 0, 0, 0, 0, 0, 4.8e12, 4.2e12, 0, 6.2e12}; /* FLOP/s of one CU */
+    static const int occ[CONV_TILES] = {3, 2, 1, 4, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1};
+    static const double rate[CONV_TILES] = {2.0e12, 3.3e12, 5.4e12, 1.5e12, 0, 0, 0, 0, 0, 0, 0, 0, 4.8e12, 4.2e12, 5.0e12, 6.2e12}; /* FLOP/s of one CU */
     static const int splits[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int M = g.M[0], N = g.N, kt_total = g.K >> 6, f = g_force_tile;
     const bool forced = f >= 0 && f < CONV_TILES && conv_bm[f] && N % conv_bn[f] == 0; /* a forced tile that this layer cannot use is ignored */
@@ -2278,6 +2491,7 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
                          (size_t)g.conv_rows * N < ((size_t)1 << 32);
     const int width = g.conv_wp - 2, height = g.conv_wp > 0 ? g.conv_rows / g.conv_wp - 2 : 0;
     const bool patch_ok = g_ring && g.conv_taps == 9 && g.conv_stride == 1 && !g.conv_packed_out && conv3_takes(height, width, g.lda, N);
+    const bool run_ok = ring_ok && g.conv_taps == 9 && g.conv_stride == 1 && !g.conv_packed_out && M > 0 && convp_rows(width) <= 448;
     int tile = -1, split = 1;
     const auto choose = [&](bool slices) {
         double best = 1e30;
@@ -2289,20 +2503,26 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
             if (t == 0 && !forced) continue; /* (for comparison runs) */
             if (ring && (!ring_ok || kt_total < 4)) continue;
             if (t == CONV_PATCH && !patch_ok) continue;
+            const bool run = t == CONV_RUN;
+            if (run && !run_ok) continue;
             const long tiles = t == CONV_PATCH ? conv3_tiles(height, width, N) : (long)((M + conv_bm[t] - 1) / conv_bm[t]) * (N / conv_bn[t]);
             for (int sp : splits) {
-                const int per = (kt_total + sp - 1) / sp, used = (kt_total + per - 1) / per, last = kt_total - (used - 1) * per;
-                if (sp > 1 && (t == CONV_PATCH || !slices || per < 4 || last < 4 || used != sp || N % 64)) continue;
+                const int unit = run ? 9 : 1; /* a slice is whole chunks of channels there, two at least (of one it is mostly its first loads: 15.2 us against 13.6 at 16 x 16 x 512) */
+                const int per = (kt_total / unit + sp - 1) / sp * unit, used = (kt_total + per - 1) / per, last = kt_total - (used - 1) * per;
+                if (sp > 1 && (t == CONV_PATCH || !slices || per < 4 || last < 4 || used != sp || N % 64 || (run && per < 18 && !forced))) continue;
                 if (slices && g_force_split && kt_total / g_force_split >= 4 && sp != g_force_split) continue;
                 const double ws = (double)sp * M * N * 4.0;
                 if (sp > 1 && ws > 256e6) continue;
                 const long blocks = tiles * sp, slots = 256L * occ[t], rounds = (blocks + slots - 1) / slots;
+                if (run && rounds > 2 && !forced) continue; /* (72 x 276 x 512 in five rounds: 98 us, in conv.hip's 16 x 16 tiles 90) */
                 const long per_cu = (min(blocks, slots) + 255) / 256;
                 double est = rounds * (2.0 * conv_bm[t] * conv_bn[t] * 64.0 * per / (rate[t] / per_cu) + 2.5e-6 +
                                        (double)conv_bm[t] * conv_bn[t] * (sp > 1 ? 0 : (epilogue == FLUX_HIP_EPI_CONV_BF16 ? 2 : 4) + (g.res ? 4 : 0)) / 2.0e10);
                 if (t == CONV_PATCH) /* the epilogue lies under the next tile and costs it half of its bytes' time, the last one's all */
                     est = rounds * (2.0 * conv_bm[t] * conv_bn[t] * 64.0 * per / rate[t] + (double)conv_bm[t] * conv_bn[t] * ((epilogue == FLUX_HIP_EPI_CONV_BF16 ? 2 : 4) + (g.res ? 4 : 0)) / 4.0e10) + 6.0e-6;
+                if (run) est += 0.5e-6 + (rounds - 1) * 3.5e-6;           /* (a second round's first loads meet the first one's stores) */
                 if (sp > 1) est += 4.0e-6 + 2.0 * ws / 4.0e12;
+                if (sp > 1 && run_ok) est += run ? 1.5e-6 : 3.0e-6; /* against CONV_RUN in one piece, which the images that want slices mostly take */
                 if (est < best) { best = est; tile = t; split = sp; }
             }
         }
@@ -2310,7 +2530,7 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
     };
     choose(g_splitk_enabled);
     if (split > 1 && M > 0 && !workspace_for_slices((size_t)split * M * N * sizeof(float))) choose(false);
-    g.kt_per = (kt_total + split - 1) / split;
+    g.kt_per = tile == CONV_RUN ? (kt_total / 9 + split - 1) / split * 9 : (kt_total + split - 1) / split;
     g.ksplit = M == 0 ? 0 : split; /* 0: nothing but border */
     const bool bf = epilogue == FLUX_HIP_EPI_CONV_BF16;
     if (g.ksplit > 1) {

@@ -201,7 +201,7 @@ def test_conv1x1(hip, oracle_mod):
     np.testing.assert_allclose(got[0], b, rtol=1e-6)
 
 
-CONV_BM = {0: 64, 1: 128, 2: 256, 3: 64, 12: 256, 13: 128}
+CONV_BM = {0: 64, 1: 128, 2: 256, 3: 64, 12: 256, 13: 128, 14: 128}
 
 
 def slices_of(kt, split):
@@ -302,6 +302,38 @@ def test_conv_patch_tile(hip, switches, H, W, cin, cout):
 
     for epi, r in ((hip.EPI_CONV_F32, None), (hip.EPI_CONV_F32, dres.ptr), (hip.EPI_CONV_F32, "in place"), (hip.EPI_CONV_BF16, None), (hip.EPI_CONV_BF16, dres.ptr)):
         np.testing.assert_array_equal(run(15, epi, r), run(1, epi, r))
+
+
+@pytest.mark.parametrize("H,W,cin,cout", [(1, 1, 64, 128), (1, 40, 128, 128), (130, 1, 128, 128), (70, 2, 64, 128), (7, 5, 64, 256), (21, 18, 128, 256), (9, 42, 192, 128),
+                                          (13, 63, 512, 128), (4, 90, 128, 384), (5, 127, 128, 128), (3, 155, 128, 128), (3, 157, 256, 128), (2, 300, 64, 64)])
+def test_conv_run_tile(hip, switches, H, W, cin, cout):
+    """Tile 14 (a run of 128 positions x 64 channels, its neighbourhood in LDS) against the 64 x 64 tile, on whole numbers whose sums fp32
+    holds exactly (9 * 512 products of at most 8 * 4). One to eight chunks of channels; the neighbourhood as one run of up to 224, 320 and 448
+    positions (from width 156 on as three); images one pixel wide and high, cut-off tiles; in one piece and in slices of whole chunks."""
+    import ctypes
+    L = hip.lib()
+    rows, wp = (H + 2) * (W + 2), W + 2
+    rng = np.random.default_rng(71)
+    x, w = rng.integers(-8, 9, (cin, H, W)).astype(np.float32), rng.integers(-4, 5, (cout, cin, 3, 3)).astype(np.float32)
+    b, res = rng.integers(-9, 10, cout).astype(np.float32), to_padded(rng.integers(-999, 1000, (cout, H, W)).astype(np.float32))
+    din = Guarded(hip, to_padded(x), wp)
+    dw, db, dres = hip.DevBuf.from_array(conv_weight(w)), hip.DevBuf.from_array(b), hip.DevBuf.from_array(res)
+
+    def run(tile, split, epi, r):
+        bf = epi == hip.EPI_CONV_BF16
+        start = np.concatenate([res if r == "in place" else np.full((rows, cout), 3.0, np.float32), np.full((1, cout), 3.0, np.float32)])
+        out = hip.DevBuf.from_array(f32_to_bf16(start) if bf else start)
+        sums = conv_image(hip, tile, split, epi, din.ptr, 0, 0, dw, db, out.ptr if r == "in place" else r, out.ptr, rows, wp, cin, cout, 9)
+        got = bf16_to_f32(out.to_array(np.uint16, (rows + 1, cout))) if bf else out.to_array(np.float32, (rows + 1, cout))
+        assert border_is_zero(got[:rows], H, W) and (got[rows] == 3.0).all()
+        check_sums(sums, got[:rows])
+        return got[:rows]
+
+    for epi, r in ((hip.EPI_CONV_F32, None), (hip.EPI_CONV_F32, "in place"), (hip.EPI_CONV_BF16, None), (hip.EPI_CONV_BF16, dres.ptr)):
+        want = run(3, 0, epi, r)
+        for split in (0, 2, 4, 8):
+            if split <= 1 or (cin // 64) % split == 0:
+                np.testing.assert_array_equal(run(14, split, epi, r), want)
 
 
 CONV_FORMS = [(tile, split) for tile in (1, 2, 3, 12, 13) for split in (0, 2)] + [(-1, 0)]

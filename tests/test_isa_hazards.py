@@ -152,7 +152,7 @@ def assembly(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("src,pattern", [("attention.hip", "attention_wide_kernel"), ("gemm.hip", "gemm4w_kernel"), ("gemm.hip", "gemm4d_kernel"), ("conv.hip", "conv3_kernel")])
+@pytest.mark.parametrize("src,pattern", [("attention.hip", "attention_wide_kernel"), ("gemm.hip", "gemm4w_kernel"), ("gemm.hip", "gemm4d_kernel"), ("gemm.hip", "convp_kernel"), ("conv.hip", "conv3_kernel")])
 def test_inline_asm_mfma_hazards(src, pattern, assembly):
     kernels = {k: v for k, v in kernel_bodies(assembly[src][0]).items() if pattern in k}
     assert kernels, f"no kernel named *{pattern}* in {src}"
@@ -398,6 +398,70 @@ def test_the_barrier_count_sees_a_merged_store():
     assert early_barriers(steps) == [] and early_barriers(steps[:18] + [("WWWW", 9)] + steps[19:]) == [(18, 9, "WWWWWWWW")]
     merged = steps[:9] + [("PPWWWW", 15)] + steps[10:]                  # one operation fewer than three waits count
     assert [s for s, _, _ in early_barriers(merged)] == [9, 10, 11]
+
+
+def test_run_convolution_owns_the_accumulator_registers(assembly):
+    """convp_kernel names its accumulator registers as conv3_kernel does."""
+    kernels = {k: v for k, v in kernel_bodies(assembly["gemm.hip"][0]).items() if "convp_kernel" in k}
+    assert len(kernels) == 9
+    for name, body in sorted(kernels.items()):
+        mine, named = False, 0
+        for line in body:
+            if "#ASMSTART" in line:
+                mine = True
+            elif "#ASMEND" in line:
+                mine = False
+            elif re.search(r"\ba\[|\ba\d|accvgpr", line.split(";")[0]):
+                assert mine, (name, line)
+                named += 1
+        assert named >= 4 * 9 * 16 + 64, (name, named)
+
+
+def run_barriers(body):
+    """[(loads into LDS and other vector memory operations since the barrier before, vmcnt of the wait)] of convp_kernel's barriers"""
+    out, lds, other, wait = [], 0, 0, None
+    for line in body:
+        p = parse(line)
+        if not p:
+            continue
+        text = line.split(";")[0]
+        if p[0].startswith(("buffer_", "global_", "flat_", "scratch_")):
+            lds, other = lds + (" lds" in text or "lds_" in p[0]), other + (" lds" not in text and "lds_" not in p[0])
+        elif p[0] == "s_waitcnt" and "lgkmcnt(0)" in text:
+            m = re.search(r"vmcnt\((\d+)\)", text)
+            wait = int(m.group(1)) if m else None
+        elif p[0] == "s_barrier":
+            out.append((lds, other, wait))
+            lds, other, wait = 0, 0, None
+    return out
+
+
+def test_run_convolution_waits_for_its_weights(assembly):
+    """What convp_kernel's barriers let be on its way is at most what a wave has requested behind the weights of the next step (and, in
+    front of a chunk's first step, behind its last patch load): counted in the compiler's output, step by step, from each barrier's own loads."""
+    kernels = {k: v for k, v in kernel_bodies(assembly["gemm.hip"][0]).items() if "convp_kernel" in k}
+    for name, body in sorted(kernels.items()):
+        npl = int(re.search(r"convp_kernelILi(\d+)E", name).group(1))
+        last_tap = (npl + 2) // 3 - 1
+        slots = min((160 * 1024 - 2 * npl * 4096) // 8192, 9 - last_tap)
+        patch = [max(0, min(3, npl - 3 * t)) for t in range(9)]
+        steps = run_barriers(body)
+        assert steps[0][0] == npl + 2 * slots and steps[0][2] == 2 * (slots - 1), (name, steps[0])
+        assert steps[-2][2] is None and steps[-1][2] is None, name            # the two around the exchange of sums
+        steps = steps[1:-2]
+        assert len(steps) == 2 * 9 + 2 * 8 and all(other == 0 for _, other, _ in steps), (name, steps)
+        for first, taps, last in ((0, 9, False), (9, 9, False), (18, 8, True), (26, 8, True)):
+            block = steps[first:first + taps]
+            issued = [0 if last else p for p in patch]                       # patch loads come first in a step, two weight loads behind them
+            weights = [2 if not last or t + slots <= 8 else 0 for t in range(9)]
+            assert [lds for lds, _, _ in block[1:]] == [issued[t] + weights[t] for t in range(taps - 1)], (name, block)
+            for t, (_, _, wait) in enumerate(block):
+                behind = 0                                                     # the weights of step t + 1 were requested in step t + 1 - slots
+                for k in range(t + 2 - slots, t):
+                    behind += issued[k] + weights[k] if k >= 0 else 2        # (a chunk's last steps request weights alone)
+                assert wait <= behind, (name, t, wait, behind)
+                if t == 8:
+                    assert wait <= 2 * (8 - last_tap) - 2 * (patch[last_tap] == 0), (name, wait)
 
 
 def test_projection_k_loops_carry_no_second_address_chain(assembly):
