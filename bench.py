@@ -226,7 +226,7 @@ def bench_vae(args):
         if n == cap:      # (the probe keeps 4096 records)
             fl = np.array([2.0 * H * W * ci * co * t for _, H, W, ci, co, t in convs] * K)
             names = {0: "gemm_kernel<64,128,2,2,CONV>", 1: "gemm_kernel<128,128,2,2,CONV>", 2: "gemm4d_kernel<8,8,CONV> (256x256 tile)",
-                     3: "gemm_kernel<64,64,2,2,CONV>", 12: "gemm4d_kernel<8,4,CONV> (256x128 tile)", 13: "gemm4d_kernel<4,4,CONV> (128x128 tile)",
+                     3: "gemm_kernel<64,64,2,2,CONV>", 12: "gemm4d_kernel<8,4,CONV> (256x128 tile)", 13: "gemm4d_kernel<4,4,CONV> (128x128 tile)", 14: "convp_kernel (128 positions x 64 channels)",
                      15: "conv3_kernel (16x16 positions x 128 channels)", 17: "conv_out_kernel", 18: "conv_in_kernel"}
             per_tile = {int(t): (float(ms[tiles == t].sum()), float(fl[tiles == t].sum()), int((tiles == t).sum())) for t in np.unique(tiles)}
             dom = max(per_tile, key=lambda t: per_tile[t][0])
@@ -665,10 +665,9 @@ def measure_workload(model, cfg, name, K, Wm, fused, args, headline):
     TILE_NAMES = {0: f"gemm_kernel<64,128,2,2,{epi_name}>", 1: f"gemm_kernel<128,128,2,2,{epi_name}>", 2: f"gemm4d_kernel<8,8,{epi_name}> (256x256 tile)",
                   3: f"gemm_kernel<64,64,2,2,{epi_name}>", 4: f"gemm4w_kernel<8,4,{epi_name},2,4> (256x256 tile, 8 waves)", 5: f"gemm4d_kernel<9,6,{epi_name}> (288x192 tile)",
                   6: f"gemm4d_kernel<6,6,{epi_name}> (192x192 tile)", 7: f"gemm4d_kernel<8,6,{epi_name}> (256x192 tile)",
-                  8: f"gemm_kernel<64,128,2,2,{epi_name},6> (ring of 6 stages)", 9: f"gemm_kernel<128,128,2,2,{epi_name},5> (ring of 5 stages)",
-                  10: f"gemm_kernel<96,128,2,2,{epi_name},5> (ring of 5 stages)", 12: f"gemm4d_kernel<8,4,{epi_name}> (256x128 tile)",
+                  **{t: f"gemm_few_kernel<{bn},{epi_name}> ({bn} columns)" for t, bn in ((8, 80), (16, 96), (10, 112), (9, 128), (24, 144))},
+                  12: f"gemm4d_kernel<8,4,{epi_name}> (256x128 tile)",
                   13: f"gemm4d_kernel<4,4,{epi_name}> (128x128 tile)", 14: f"gemm4d_kernel<6,8,{epi_name}> (192x256 tile)",
-                  16: f"gemm_kernel<96,96,2,3,{epi_name},6> (ring of 6 stages)",
                   23: f"gemm4d_kernel<8,5,{epi_name}> (256x160 tile)",
                   **{17 + i: f"gemm4x_kernel<{tm},{tn},{epi_name}> ({32 * tm}x{32 * tn} tile)"
                      for i, (tm, tn) in enumerate([(9, 9), (12, 7), (10, 7), (10, 8), (9, 8), (11, 7)])}}

@@ -50,8 +50,8 @@
  * per SIMD) on the 256 x 256 tile it runs at the speed of the 4-wave form and is kept for comparison
  * runs (tile id 4).
  *
- * Three kernels, then: gemm_kernel (small tiles; with NS > 2 a ring of NS LDS stages for row ranges of few
- * rows, where a launch only streams weights), gemm4w_kernel (large tiles, two LDS stages; the
+ * Four kernels, then: gemm_kernel (small tiles), gemm_few_kernel (row ranges of at most 128 rows, where a
+ * launch only streams weights), gemm4w_kernel (large tiles, two LDS stages; the
  * comparison form of the next one) and gemm4d_kernel (large tiles with an LDS ring per operand, the form the
  * transformer's projections and the VAE's convolutions run). What separates the last two is the barrier: __syncthreads() carries a fence
  * that waits for every global->LDS load in flight, so a two-stage loop can never have more than the next stage
@@ -231,8 +231,8 @@ __device__ __forceinline__ int bf16_feature(int blk, int r) { return blk < (TN &
 template <int BN> struct CutTile { static constexpr bool value = BN % 64 != 0; };
 /* the tiles of gemm4x_kernel */
 template <int BN, int WM> struct IsWide { static constexpr bool value = 2 * WM * BN > 256 * 256; };
-/* tiles whose last column tile is cut at any multiple of eight columns, lane by lane: those, and 256 x 160 */
-template <int BN, int WM> struct LaneCut { static constexpr bool value = CutTile<BN>::value && (IsWide<BN, WM>::value || BN == 160); };
+/* tiles whose last column tile is cut at any multiple of eight columns, lane by lane: those, 256 x 160 and gemm_few_kernel's */
+template <int BN, int WM> struct LaneCut { static constexpr bool value = CutTile<BN>::value && (IsWide<BN, WM>::value || BN == 160 || WM == 16); };
 /* SiLU(gate) * up: blocks alternate gate, up, so that a lane holds matching pairs; the (gate, up) pairs interleave
  * two by two in the same way, and a last odd pair keeps the plain numbering (features 16 k + r). With an odd number of
  * blocks the last one holds gate rows and up rows, two and two: a lane's four results are gate, gate, up, up of two features. */
@@ -591,7 +591,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs &g, const TileId &t, f
     }
 }
 
-template <int BM, int BN, int WGM, int WGN, int EPI, int NS = 2>
+template <int BM, int BN, int WGM, int WGN, int EPI>
 __global__ __launch_bounds__(WGM *WGN * 64) void gemm_kernel(GemmArgs g) {
     constexpr int T = WGM * WGN * 64;
     constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;
@@ -645,11 +645,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_kernel(GemmArgs g) {
     };
     const int kt_begin = ks * g.kt_per;
     const int KT = min(g.K >> 6, kt_begin + g.kt_per) - kt_begin;
-    /* NS - 1 stages are requested ahead: with few rows (M <= BM, weights streamed once, hardly any arithmetic) a
-     * workgroup is only as fast as the bytes it keeps in flight, and the ring then takes the whole LDS */
-#pragma unroll
-    for (int s = 0; s < NS - 1; s++)
-        if (s < KT) issue(kt_begin + s, s);
+    if (KT > 0) issue(kt_begin, 0);
 
     f32x4 acc[TN][TM];
 #pragma unroll
@@ -664,21 +660,12 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_kernel(GemmArgs g) {
     const int a_frag = (wm * WM + l15) * 128;
     const int b_frag = BM * 128 + (wn * WN + l15) * 128;
 
-    int cur = 0;
     for (int kt = 0; kt < KT; kt++) {
-        /* stage `cur` has landed for this wave (the NS - 2 stages requested after it may still be on their way);
-         * after the barrier it has for all, and everyone is done reading the stage before it, which is refilled */
-        if constexpr (NS > 2) {
-            /* __syncthreads() would wait for every load in flight (its fence counts the global->LDS loads); here the
-             * wait names what must have landed, and this wave's own LDS reads of the stage that is refilled next */
-            if (kt + NS - 2 < KT) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * (PA + PB)) : "memory");
-            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        } else {
-            WAIT_VMCNT0();
-            __syncthreads();
-        }
-        const int refill = cur == 0 ? NS - 1 : cur - 1;
-        if (kt + NS - 1 < KT) issue(kt_begin + kt + NS - 1, refill);
+        /* the stage has landed for this wave; after the barrier it has for all, and everyone is done reading the other one, which is refilled */
+        WAIT_VMCNT0();
+        __syncthreads();
+        const int cur = kt & 1;
+        if (kt + 1 < KT) issue(kt_begin + kt + 1, cur ^ 1);
         const char *st = smem + cur * STAGE;
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
@@ -694,10 +681,88 @@ __global__ __launch_bounds__(WGM *WGN * 64) void gemm_kernel(GemmArgs g) {
                 for (int j = 0; j < TM; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[i], fa[j], acc[i][j], 0, 0, 0);
         }
-        cur = cur == NS - 1 ? 0 : cur + 1;
     }
 
     store_tile<BN, WM, WN, EPI, WGM>(g, t, acc, m0, M, wm, wn, l15, lq, t.tm * WGM + wm);
+}
+
+/* Projections of few rows (at most 128 per part): weights streamed once, hardly any arithmetic. What bounds them is how fast a compute unit takes in
+ * cold lines, 50 to 55 KB a microsecond however many it has requested beyond 32 KB (loads return in order, so activations from the L2 wait
+ * behind weights from HBM), and then HBM itself. Hence: as many columns per workgroup as leave every unit one tile (BN = 80 to 144 in steps
+ * of 16, the last column tile cut off), and no loads for rows that do not exist: the loads of a K step, eight rows each, are dealt out to
+ * the eight waves, those of ceil(M / 8) activation groups and BN / 8 weight groups. A wave owns 16 rows and all columns; waves beyond the last row only
+ * load. One ring of 4 to 6 stages fills the LDS. The order of additions is that of the other tiles.
+ * Against a ring of 96 x 96 and 128 x 96 tiles in which every wave loaded its share of all 96 or 128 rows, weights from HBM: 80 rows (64 + 16)
+ * of the fused 27648 x 3072 37.7 -> 35.8 us, 9216 x 3072 with two weight matrices 29.6 -> 25.4, their SwiGLU 18432 49.5 -> 44.5, 3072 x 9216 34.6 ->
+ * 29.8, 3072 x 3072 18.1 -> 16.6; 19456 x 2560 at 16 rows 24.8 -> 21.4 (4.7 TB/s), at 128 rows 34.4 -> 30.2. */
+template <int BN, int EPI>
+__global__ __launch_bounds__(512) void gemm_few_kernel(GemmArgs g) {
+    constexpr int BM = 128, TN = BN / 16, STAGE = (BM + BN) * 128, NS = 160 * 1024 / STAGE < 6 ? 160 * 1024 / STAGE : 6;
+    constexpr int CM = (BM / 8 + BN / 8 + 7) / 8; /* a wave's loads per K step, at most */
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    TileId t;
+    if (!decode_tile<false>(g, blockIdx.x, t)) return;
+    const int M = g.M[t.prob], lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int na = (M + 7) >> 3, own = (na + BN / 8 - wave + 7) >> 3; /* this wave's loads */
+    const bf16 *src[CM];
+    int dst[CM];
+#pragma unroll
+    for (int k = 0; k < CM; k++) {
+        const int i = wave + 8 * k;
+        const bool act = i < na;
+        const int r = 8 * (act ? i : min(i - na, BN / 8 - 1)) + (lane >> 3), chunk = ((lane & 7) ^ lds_swz(r)) << 3;
+        src[k] = act ? g.A[t.prob] + (size_t)min(r, M - 1) * g.lda + chunk : g.W[t.prob] + (size_t)weight_row<BN, BN, EPI>(g, t.tn, r) * g.ldw + chunk;
+        dst[k] = act ? i * 1024 : BM * 128 + (i - na) * 1024;
+    }
+    const int kt_begin = t.ks * g.kt_per, KT = min(g.K >> 6, kt_begin + g.kt_per) - kt_begin;
+    auto issue = [&](int kt, int stage) {
+#pragma unroll
+        for (int k = 0; k < CM; k++)
+            if (k < own) __builtin_amdgcn_global_load_lds(GLOBAL_PTR(src[k] + (kt_begin + kt) * 64), LDS_PTR(smem + stage * STAGE + dst[k]), 16, 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < NS - 1; s++)
+        if (s < KT) issue(s, s);
+    f32x4 acc[TN][1];
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[i][0][e] = 0.0f;
+    const int l15 = lane & 15, lq = lane >> 4, swzl = lds_swz(l15);
+    const bool works = wave * 16 < M;
+    int cur = 0;
+    for (int kt = 0; kt < KT; kt++) {
+        /* stage `cur` has landed for this wave (the NS - 2 stages requested after it may still be on their way); after the barrier it has for all, and
+         * everyone is done reading the stage before it, which is refilled */
+        if (kt + NS - 2 < KT) {
+            if (own == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NS - 2) : "memory");
+            else if (own == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (NS - 2)) : "memory");
+            else if (own == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * (NS - 2)) : "memory");
+            else if (own == 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * (NS - 2)) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(5 * (NS - 2)) : "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const int refill = cur == 0 ? NS - 1 : cur - 1;
+        if (kt + NS - 1 < KT) issue(kt + NS - 1, refill);
+        if (works) {
+            const char *st = smem + cur * STAGE;
+#pragma unroll
+            for (int kk = 0; kk < 2; kk++) {
+                const int coff = ((kk * 4 + lq) ^ swzl) << 4;
+                const bf16x8 fa = *(const bf16x8 *)(st + (wave * 16 + l15) * 128 + coff);
+                bf16x8 fb[TN];
+#pragma unroll
+                for (int i = 0; i < TN; i++) fb[i] = *(const bf16x8 *)(st + (BM + i * 16 + l15) * 128 + coff);
+#pragma unroll
+                for (int i = 0; i < TN; i++) acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[i], fa, acc[i][0], 0, 0, 0);
+            }
+        }
+        cur = cur == NS - 1 ? 0 : cur + 1;
+    }
+    static_assert(CM <= 5 && NS >= 4, "a case for every count");
+    if (works) store_tile<BN, 16, BN, EPI, 8>(g, t, acc, 0, M, wave, 0, l15, lq, t.tm * 8 + wave);
 }
 
 /* The large tiles: 4 waves (2 x 2), one per SIMD, each owning a (16 TM) x (16 TN) part of a
@@ -1524,24 +1589,42 @@ static void set_row_tiles(GemmArgs &g, int BM) {
     g.mtiles = end;
 }
 
-template <int BM, int BN, int WGM, int WGN, int EPI, int NS = 2>
+template <int BM, int BN, int WGM, int WGN, int EPI>
 static int launch_cfg(GemmArgs &g) {
     constexpr int T = WGM * WGN * 64;
-    constexpr int LDS = NS * (BM + BN) * 128;
-    static_assert(LDS <= 160 * 1024 && (NS - 2) * ((BM + BN) * 8 / T) < 64, "the ring fits the LDS, the loads in flight the wait counter");
+    constexpr int LDS = 2 * (BM + BN) * 128;
     static bool attr_done = false;
-    auto kern = gemm_kernel<BM, BN, WGM, WGN, EPI, NS>;
+    auto kern = gemm_kernel<BM, BN, WGM, WGN, EPI>;
     if (!attr_done) {
         HIP_OK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
         attr_done = true;
     }
     set_row_tiles(g, BM);
-    g.ntiles = (g.N + BN - 1) / BN; /* (a last tile that is cut off: CutTile) */
+    g.ntiles = g.N / BN;
     g.nq_tiles = g.nq_cols / BN;
     g.total_tiles = g.mtiles * g.ntiles;
     int grid = (g.total_tiles * g.ksplit + 7) & ~7;
     g.vgrid = grid;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(T), LDS, flux_hip_stream_handle(), g);
+    HIP_OK(hipGetLastError());
+    return 1;
+}
+
+template <int BN, int EPI>
+static int launch_few(GemmArgs &g) {
+    constexpr int STAGE = (128 + BN) * 128, LDS = (160 * 1024 / STAGE < 6 ? 160 * 1024 / STAGE : 6) * STAGE;
+    static bool attr_done = false;
+    auto kern = gemm_few_kernel<BN, EPI>;
+    if (!attr_done) {
+        HIP_OK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        attr_done = true;
+    }
+    set_row_tiles(g, 128);
+    g.nq_tiles = (g.nq_cols + BN - 1) / BN; /* both sides of the fused projection end in a tile that may be cut off */
+    g.ntiles = g.nq_tiles + (g.N - g.nq_cols + BN - 1) / BN;
+    g.total_tiles = g.mtiles * g.ntiles;
+    g.vgrid = (g.total_tiles * g.ksplit + 7) & ~7;
+    hipLaunchKernelGGL(kern, dim3(g.vgrid), dim3(512), LDS, flux_hip_stream_handle(), g);
     HIP_OK(hipGetLastError());
     return 1;
 }
@@ -1652,7 +1735,7 @@ static int launch_epi(GemmArgs &g, int tile) {
             default: break;
         }
     }
-    if ((tile >= 11 && tile < 15) || tile > 16) tile = g.N % 256 == 0 ? 2 : 1; /* (the dispatch offers these only where the ring kernel takes them) */
+    if ((tile >= 11 && tile < 15) || (tile > 16 && tile < 24)) tile = g.N % 256 == 0 ? 2 : 1; /* (the dispatch offers these only where the ring kernel takes them) */
     switch (tile) {
         case 2: return launch_4w<8, 8, EPI>(g);
         case 5: return launch_4w<9, 6, EPI>(g);
@@ -1661,10 +1744,11 @@ static int launch_epi(GemmArgs &g, int tile) {
         case 4: return launch_4w<8, 4, EPI, 2, 4>(g); /* 8 waves, two per SIMD, on the 256x256 tile */
         case 1: return launch_cfg<128, 128, 2, 2, EPI>(g);
         case 3: return launch_cfg<64, 64, 2, 2, EPI>(g);
-        case 8: return launch_cfg<64, 128, 2, 2, EPI, 6>(g);  /* few rows: the same tiles with a ring that fills the LDS */
-        case 9: return launch_cfg<128, 128, 2, 2, EPI, 5>(g);
-        case 10: return launch_cfg<96, 128, 2, 2, EPI, 5>(g);
-        case 16: return launch_cfg<96, 96, 2, 3, EPI, 6>(g);
+        case 8: return launch_few<80, EPI>(g);
+        case 9: return launch_few<128, EPI>(g);
+        case 10: return launch_few<112, EPI>(g);
+        case 16: return launch_few<96, EPI>(g);
+        case 24: return launch_few<144, EPI>(g);
         default: return launch_cfg<64, 128, 2, 2, EPI>(g);
     }
 }
@@ -2006,7 +2090,7 @@ extern "C" void flux_hip_linear_release(void) {
 }
 
 static int g_force_tile = -1;
-#define TILE_MASK_ALL 0xFF7FEFu /* tiles the automatic choice may use: all but the 8-wave form of 256 x 256 */
+#define TILE_MASK_ALL 0x1FF7FEFu /* tiles the automatic choice may use: all but the 8-wave form of 256 x 256 */
 static unsigned g_tile_mask = TILE_MASK_ALL;
 static int g_splitk_enabled = 1;
 extern "C" void flux_hip_linear_force_tile(int tile) { g_force_tile = tile; }
@@ -2095,12 +2179,8 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
      * fixed prologue/epilogue cost; the launch cannot beat the time to stream its operands,
      * which depends on how many bytes the resident workgroups keep in flight. */
     /* tile ids: 0..3 the small tiles and 256 x 256, 4 = the 8-wave form of 256 x 256 (only when
-     * forced, for comparison runs), 5 = 288 x 192, 6 = 192 x 192, 7 = 256 x 192, 8, 9 and 10 = 64 x 128, 128 x 128 and
-     * 96 x 128 with a ring of 6, 5 and 5 stages instead of 2 (one workgroup per compute unit; for parts of at most that
-     * many rows), 16 = 96 x 96 with a ring of 6 and six waves: a compute unit takes in 50 to 55 KB of cold operands a microsecond whatever its
-     * ring and its waves (0.56 us per K step of 96 + 128 rows with 20 workgroups on the chip as with 152), so the width that
-     * leaves fewest units idle is the fastest: 67 x 19456 x 2560 32.7 us on 152 units and 28.6 on 203, 80 x 3072 x 12288 in slices 28.9 on
-     * 192 and 26.8 on 256, 11 = 256 x 224 (4096 + 512 rows x 3072 columns are 252 such tiles, one round of workgroups on 256
+     * forced, for comparison runs), 5 = 288 x 192, 6 = 192 x 192, 7 = 256 x 192, 8, 16, 10, 9 and 24 = gemm_few_kernel's, 80, 96, 112, 128 and 144
+     * columns wide, for parts of at most 128 rows, 11 = 256 x 224 (4096 + 512 rows x 3072 columns are 252 such tiles, one round of workgroups on 256
      * compute units of which each does 7/8 of a 256 x 256 tile's work; 216 tiles of 256 x 256 are one round as well),
      * 12 = 256 x 128, 13 = 128 x 128 and 14 = 192 x 256 in the ring kernel, for launches of about one round: the two-stage 128 x 128
      * tile waits for memory in every K step when it has a compute unit to itself. With the weights coming from HBM, as in a
@@ -2110,10 +2190,10 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
      * 17 to 22 = gemm4x_kernel's, for the fused projection: 288 x 288, 384 x 224, 320 x 224, 320 x 256, 288 x 256, 352 x 224. Over 29 row counts
      * from 300 to 13056 the chosen tile takes 0.3 % more than the best on average; 256 x 288 was never the best, 352 x 256 (two row
      * counts, 3 %) spills. */
-    constexpr int NT = 24;
-    static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 64, 128, 96, 256, 256, 128, 192, 0, 96, 288, 384, 320, 320, 288, 352, 256}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 128, 128, 128, 224, 128, 128, 256, 1, 96, 288, 224, 224, 256, 256, 224, 160};
-    static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, ahead[NT] = {1, 1, 1, 1, 1, 1, 1, 1, 5, 4, 4, 1, 1, 1, 1, 1, 5, 1, 1, 1, 1, 1, 1, 1}; /* stages a workgroup keeps in flight */
-    static const double rate[NT] = {2.0e12, 2.9e12, 6.05e12, 1.5e12, 4.6e12, 6.0e12, 5.7e12, 5.75e12, 1.6e12, 3.0e12, 2.4e12, 5.9e12, 5.3e12, 4.4e12, 5.5e12, 1.0, 2.3e12, 6.3e12, 6.1e12, 6.15e12, 6.4e12, 6.3e12, 6.15e12, 5.4e12}; /* FLOP/s of one CU running this tile */
+    constexpr int NT = 25;
+    static const int bm[NT] = {64, 128, 256, 64, 256, 288, 192, 256, 128, 128, 128, 256, 256, 128, 192, 0, 128, 288, 384, 320, 320, 288, 352, 256, 128}, bn[NT] = {128, 128, 256, 64, 256, 192, 192, 192, 80, 128, 112, 224, 128, 128, 256, 1, 96, 288, 224, 224, 256, 256, 224, 160, 144};
+    static const int occ[NT] = {3, 2, 1, 4, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1};
+    static const double rate[NT] = {2.0e12, 2.9e12, 6.05e12, 1.5e12, 4.6e12, 6.0e12, 5.7e12, 5.75e12, 0, 0, 0, 5.9e12, 5.3e12, 4.4e12, 5.5e12, 1.0, 0, 6.3e12, 6.1e12, 6.15e12, 6.4e12, 6.3e12, 6.15e12, 5.4e12, 0}; /* FLOP/s of one CU running this tile; 0: gemm_few_kernel */
     const int kt_total = g.K >> 6;
     int tile = -1, best_split = 1;
     {
@@ -2126,15 +2206,23 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
                                (epilogue == FLUX_HIP_EPI_RESID || epilogue == FLUX_HIP_EPI_BF16 || epilogue == FLUX_HIP_EPI_F32 ||
                                 (epilogue == FLUX_HIP_EPI_SWIGLU && w_row1 == w_row0 + N / 2));
         double rows = 0.0;
-        for (int i = 0; i < np; i++) rows += g.M[i];
+        int most = 0;
+        for (int i = 0; i < np; i++) rows += g.M[i], most = max(most, g.M[i]);
+        int weights = 0; /* matrices of weights: sequences share them, streams do not */
+        for (int i = 0; i < np; i++) {
+            weights++;
+            for (int j = 0; j < i; j++)
+                if (g.W[j] == g.W[i]) { weights--; break; }
+        }
         for (int t = 0; t < NT; t++) {
+            const bool few = rate[t] == 0;
+            if (few && most > 128) continue; /* they stream the weights once: every part in one row tile */
             /* 256 x 224 (tile 11) divides no width and cuts its last column tile off: for the outputs whose stores can do
              * that, through the ring kernel only, never in K slices */
             const bool cut = t == 11;
             if (cut && !((epilogue == FLUX_HIP_EPI_RESID || epilogue == FLUX_HIP_EPI_BF16) && g_ring && g_persistent && kt_total >= 4)) continue;
             /* bf16 outputs leave in pairs of 16-column blocks: the cut must fall between two pairs of a wave's 112 columns */
             if (cut && epilogue == FLUX_HIP_EPI_BF16 && (N % 224) % 112 % 32 != 0) continue;
-            /* 96 x 96 (tile 16) cuts its last column tile off as well, at a multiple of 32, i.e. between two waves' columns */
             const bool wide = t >= 17 && t < 23;
             /* 256 x 160 (tile 23) likewise, at a multiple of eight features: for SwiGLU alone. The text encoder's gate and up rows (19456 x
              * 2560) are 244 tiles of it at 512 rows, of which 256 units run all at once; with the weights from HBM, us, 23 / the best other: 260 rows
@@ -2144,14 +2232,9 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
             if (cut160 && !(epilogue == FLUX_HIP_EPI_SWIGLU && N % 64 == 0 && g_ring && g_persistent && kt_total >= 4)) continue;
             if (wide && !(epilogue == EPI_QKV_SWIGLU && g_ring && g_persistent && kt_total >= 4)) continue;
             if (wide && bn[t] == 256 && (g.nq_cols & 255 || N & 255)) continue; /* (CutTile) */
-            if (!cut && !cut160 && !wide && ((N % bn[t] && (t != 16 || epilogue == EPI_QKV_SWIGLU)) || g.nq_cols % bn[t])) continue;
+            if (!cut && !cut160 && !wide && !few && (N % bn[t] || g.nq_cols % bn[t])) continue;
             if (!((allowed >> t) & 1)) continue;
             if (t >= 12 && t < 15 && !(g_ring && g_persistent && kt_total >= 4)) continue;
-            if (ahead[t] > 1) { /* the deep rings stream the weights once: every part in one row tile */
-                bool fits = true;
-                for (int i = 0; i < np; i++) fits = fits && g.M[i] <= bm[t];
-                if (!fits) continue;
-            }
             long tiles = 0;
             for (int i = 0; i < np; i++) tiles += (g.M[i] + bm[t] - 1) / bm[t];
             tiles *= (g.nq_cols + bn[t] - 1) / bn[t] + (N - g.nq_cols + bn[t] - 1) / bn[t];
@@ -2175,11 +2258,11 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
                 const long per_cu = (resident + 255) / 256;          /* workgroups sharing one CU */
                 const double t_block = 2.0 * bm[t] * bn[t] * 64.0 * per / (rate[t] / per_cu) + 2.5e-6;
                 double t_compute = rounds * t_block;
-                const double bytes = (rows + N) * (double)K * 2.0;
-                /* what a launch that only streams its operands has been seen to reach: 3.2-3.5 TB/s with two LDS stages
-                 * (every step waits for the loads it has just requested), 4.3-5.2 TB/s with a deep ring */
-                const double bw_cap = ahead[t] > 1 ? 4.6e12 : 3.4e12;
-                double bw = 5.5e12 * (double)(resident * ahead[t] * (bm[t] + bn[t]) * 128) / 12.0e6;
+                const double bytes = (rows + (most <= 128 ? weights : 1) * (double)N) * K * 2.0;
+                /* what a launch that only streams its operands has been seen to reach with two LDS stages (every step waits for the loads it
+                 * has just requested): 3.2-3.5 TB/s */
+                const double bw_cap = 3.4e12;
+                double bw = 5.5e12 * (double)(resident * (bm[t] + bn[t]) * 128) / 12.0e6;
                 if (bw > bw_cap) bw = bw_cap;
                 double est = t_compute > bytes / bw ? t_compute : bytes / bw;
                 /* What all tiles together fetch through the L2s, over the rate at which that ties the tiles with fewer bytes to those with
@@ -2193,12 +2276,24 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
                 const double l2_rate = rows * K * 2.0 > 256.0e6 ? 12.9e12 : 13.5e12;
                 const double l2 = (double)tiles * (bm[t] + bn[t]) * K * 2.0 / l2_rate;
                 if (l2 > est) est = l2;
-                if (ahead[t] > 1) est += 0.03 * t_compute; /* of two that stream their weights at the same rate the one with less to do */
+                if (few) {
+                    /* See gemm_few_kernel: round by round a workgroup's intake (or its LDS reads), or the round's weights from HBM. 62 launches of 16 to
+                     * 128 rows: the chosen width and slices take 1 % more than the best of up to 20 on average. */
+                    const double intake = ((most + 7) / 8 * 8 + bn[t]) * 128 / 54.0e9, lds = (most + 15) / 16 * (1 + bn[t] / 16) * 2048 / (128 * 2.1e9);
+                    const double wg = per * (intake > lds ? intake : lds), hbm = (rows + (double)weights * N) * K * 2.0 / 6.0e12;
+                    est = 3.5e-6 + 0.2 * rounds * wg;
+                    for (long left = blocks; left > 0; left -= 256) {
+                        const double part = hbm * (left < 256 ? left : 256) / blocks;
+                        est += (wg > part ? wg : part) + 2.0e-6;
+                    }
+                } else if (most <= 128) {
+                    est += 4.0e-6; /* their launches of few rows take that much longer than this model has them */
+                }
                 /* Slices cost their partial sums, and beyond 128 MB of those the stores of every round as well: the K = 12288 projection at
                  * 6148 to 6912 rows (151 to 170 MB) in two slices of 288 x 192 takes 379 + 78 us, in one piece of 256 x 192 430 and
                  * 27 for the norm, and the step around it is 0.5 to 1.2 % longer; at 2132 to 2560 rows (52 to 63 MB) two slices
                  * make it 1 % shorter. */
-                if (sp > 1) est += 3.0e-6 + (sp + 2.0) * rows * N * 4.0 / (sp * rows * N * 4.0 > 128.0e6 ? 2.6e12 : 4.0e12);
+                if (sp > 1) est += 3.0e-6 + (sp + 2.0) * rows * N * 4.0 / (few ? 8.0e12 : sp * rows * N * 4.0 > 128.0e6 ? 2.6e12 : 4.0e12);
                 else if (adaln) est += 3.0e-6 + rows * N * 6.0 / 4.0e12; /* the norm that the second pass would have taken along */
                 if (est < best) { best = est; tile = t; best_split = sp; }
             }
@@ -2302,7 +2397,7 @@ static int linear_impl(int epilogue, int nparts, const flux_hip_linear_part *par
     g.N = N; g.K = K; g.lda = lda; g.ldw = ldw; g.ldc = ldc; g.w_row0 = w_row0; g.w_row1 = w_row1;
     a.ldo = N;
     a.eps = eps;
-    return gemm_dispatch(g, np, epilogue, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x817FFFu, nullptr, norm ? &a : nullptr, fused,
+    return gemm_dispatch(g, np, epilogue, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x1817FFFu, nullptr, norm ? &a : nullptr, fused,
                          fixed_ws, fixed_ws_bytes);
 }
 
@@ -2322,7 +2417,7 @@ extern "C" int flux_hip_linear_slices(const void *A, const void *W, void *C, int
     GemmArgs g = {};
     g.A[0] = (const bf16 *)A; g.W[0] = (const bf16 *)W; g.C[0] = C; g.M[0] = M;
     g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = N;
-    const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_BF16, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x17FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
+    const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_BF16, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x1017FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
     *ws = g.ws;
     return ok;
 }
@@ -2360,7 +2455,7 @@ extern "C" int flux_hip_linear_f32_slices(const void *A, const void *W, float *C
     GemmArgs g = {};
     g.A[0] = (const bf16 *)A; g.W[0] = (const bf16 *)W; g.C[0] = C; g.M[0] = M;
     g.N = N; g.K = K; g.lda = K; g.ldw = K; g.ldc = N;
-    const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_F32, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x17FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
+    const int ok = gemm_dispatch(g, 1, FLUX_HIP_EPI_F32, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x1017FFFu, nullptr, nullptr, nullptr, nullptr, 0, slices);
     *ws = g.ws;
     return ok;
 }
@@ -2384,7 +2479,7 @@ extern "C" int flux_hip_linear_qkv_swiglu(const void *A, const void *W, void *qk
     int tile = -1;
     const int saved = g_splitk_enabled;
     g_splitk_enabled = 0;
-    const int ok = gemm_dispatch(g, 1, EPI_QKV_SWIGLU, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x7F7FFFu, &tile);
+    const int ok = gemm_dispatch(g, 1, EPI_QKV_SWIGLU, (g_force_tile >= 0 ? 1u << g_force_tile : g_tile_mask) & 0x17F7FFFu, &tile);
     g_splitk_enabled = saved;
     return ok;
 }

@@ -660,6 +660,53 @@ def test_linear_deep_ring_tiles(hip, oracle_mod, tile, M, K):
     np.testing.assert_array_equal(fm, sw)
 
 
+@pytest.mark.parametrize("tile", [8, 16, 10, 9, 24])
+@pytest.mark.parametrize("M,K", [(1, 64), (8, 576), (9, 256), (67, 320), (128, 448)])
+@pytest.mark.parametrize("N", [128, 256, 640])
+def test_linear_few_row_tiles(hip, tile, M, K, N):
+    """gemm_few_kernel, 80 to 144 columns wide: loads of whole and of cut-off groups of eight rows dealt out to eight waves (one row to 128), rings
+    longer and shorter than K, last column tiles cut off anywhere or wider than the matrix, parts of different row counts with weights of
+    their own: bit for bit what the two-stage 64 x 64 tile gives; rows and columns beyond the output stay as they were."""
+    import ctypes
+    L = hip.lib()
+    L.flux_hip_linear_qkv_swiglu.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 8
+    M2, mlp, ld = M // 2 + 1, N // 2, N + 64
+    x, x2, W = q(normal_f32((M, K), 74, 1)), q(normal_f32((M2, K), 74, 2)), q(normal_f32((3 * N, K), 74, 3, 0.0, 0.1))
+    dx, dx2, dW, dg = dev_bf16(hip, x), dev_bf16(hip, x2), dev_bf16(hip, W), hip.DevBuf.from_array(normal_f32((N,), 74, 4))
+    res = normal_f32((M + 1, N), 74, 5), normal_f32((M2 + 1, N), 74, 6)
+    full16, full32 = (lambda r, c: np.full((r, c), 7, np.uint16)), (lambda r, c: np.full((r, c), 7.0, np.float32))
+    outs = []
+    try:
+        L.flux_hip_linear_enable_splitk(0)
+        for t in (tile, 3):
+            L.flux_hip_linear_force_tile(t)
+            L.flux_hip_linear_probe(hip.EPI_BF16)
+            o16, o32, ot, sw = hip.DevBuf.from_array(full16(M + 1, ld)), hip.DevBuf.from_array(full32(M + 1, ld)), hip.DevBuf(N * (M + 3) * 4), hip.DevBuf.from_array(full16(M + 1, mlp + 12))
+            fq, fm = hip.DevBuf.from_array(full16(M + 1, N + 4)), hip.DevBuf.from_array(full16(M + 1, N + 8))
+            r = [hip.DevBuf.from_array(a) for a in res]
+            hip.linear(hip.EPI_BF16, [(dx.ptr, dW.ptr, o16.ptr, None, M)], N, K, K, K, ld)
+            tiles = np.zeros(4, np.int32)
+            assert L.flux_hip_linear_probe_read_launches(4, tiles.ctypes.data, None) == 1 and tiles[0] == t
+            L.flux_hip_linear_probe(-1)
+            hip.linear(hip.EPI_F32, [(dx.ptr, dW.ptr, o32.ptr, None, M)], N, K, K, K, ld)
+            hip.check(L.flux_hip_memset(ot.ptr, 0, N * (M + 3) * 4))
+            hip.linear(hip.EPI_F32_T, [(dx.ptr, dW.ptr, ot.ptr, None, M)], N, K, K, K, M + 3)
+            hip.linear(hip.EPI_RESID, [(dx.ptr, dW.ptr, r[0].ptr, dg.ptr, M), (dx2.ptr, dW.at(N * K * 2), r[1].ptr, dg.ptr, M2)], N, K, K, K, N)
+            hip.linear(hip.EPI_SWIGLU, [(dx.ptr, dW.ptr, sw.ptr, None, M)], N, K, K, K, mlp + 12, 0, mlp)
+            hip.check(L.flux_hip_linear_qkv_swiglu(dx.ptr, dW.ptr, fq.ptr, fm.ptr, M, N, N, K, K, K, N + 4, N + 8), "flux_hip_linear_qkv_swiglu")
+            outs.append([o16.to_array(np.uint16, (M + 1, ld)), o32.to_array(np.float32, (M + 1, ld)), ot.to_array(np.float32, (N, M + 3)), r[0].to_array(np.float32, (M + 1, N)),
+                         r[1].to_array(np.float32, (M2 + 1, N)), sw.to_array(np.uint16, (M + 1, mlp + 12)), fq.to_array(np.uint16, (M + 1, N + 4)), fm.to_array(np.uint16, (M + 1, N + 8))])
+    finally:
+        L.flux_hip_linear_force_tile(-1)
+        L.flux_hip_linear_enable_splitk(1)
+        L.flux_hip_linear_probe(-1)
+    for a, b in zip(*outs):
+        np.testing.assert_array_equal(a, b)
+    o16, o32, _, r0, r1, sw, fq, fm = outs[0]
+    assert all((o[M:] == 7).all() and (o[:, w:] == 7).all() for o, w in ((o16, N), (o32, N), (sw, mlp), (fq, N), (fm, N)))
+    assert (r0[M] == res[0][M]).all() and (r1[M2] == res[1][M2]).all()
+
+
 @pytest.mark.parametrize("M,K", [(1, 256), (255, 320), (257, 448), (512, 2560)])
 @pytest.mark.parametrize("mlp", [64, 128, 192, 320, 9728])
 def test_linear_swiglu_160_wide_tile(hip, M, K, mlp):
