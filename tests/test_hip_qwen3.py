@@ -72,6 +72,32 @@ def test_causal_attention(hip, oracle_mod, seq, heads, kv, masked):
         assert rel_l2(got[0, :128], vv[:, :128].mean(axis=0)) < 6e-3     # uniform over ALL columns
 
 
+@pytest.mark.parametrize("seq,used,holes", [(512, 1, ()), (512, 31, (5, 30)), (512, 32, ()), (512, 33, (1, 2, 3)), (200, 64, ()), (512, 65, ()), (512, 128, (127,)),
+                                            (512, 129, ()), (512, 257, tuple(range(32, 256))), (399, 385, ()), (512, 511, ()), (512, 67, (0,))])
+def test_causal_attention_of_padded_prompts(hip, oracle_mod, seq, used, holes):
+    """Keys behind the last admissible one are left out: last tokens around the 32 keys of a step and the step counts of the
+    compiled bodies, holes before them, and a masked first key, with which nothing may be left out. Where no row is without an
+    admissible key, the tokens' own rows are bit for bit those of the prompt without its padding (the padding's probabilities are exactly 0)."""
+    heads, kv = 4, 2
+    mask = (np.arange(seq) < used).astype(np.int32)
+    mask[list(holes)] = 0
+    x = [q(normal_f32((seq, n * 128), 77, 1 + i)) for i, n in enumerate((heads, kv, kv))]
+
+    def run(n):
+        ldv = (n + 31) // 32 * 32
+        vt = np.zeros((kv * 128, ldv), np.float32)
+        vt[:, :n] = x[2][:n].T
+        d = [hip.DevBuf.from_array(f32_to_bf16(a)) for a in (np.concatenate([a[:n] for a in x], axis=1), vt)]
+        dm, out = hip.DevBuf.from_array(mask[:n].copy()), hip.DevBuf(n * heads * 128 * 2)
+        hip.check(hip.lib().flux_hip_causal_attention(out.ptr, d[0].ptr, d[1].ptr, ldv, dm.ptr, n, heads, kv))
+        return out.to_array(np.uint16, (n, heads * 128))
+
+    got = run(seq)
+    assert rel_l2(bf16_to_f32(got), oracle_mod.qwen3_attention(*x, mask, heads, kv)) < 6e-3
+    if mask[0]:
+        assert np.array_equal(got[:used], run(used))
+
+
 @pytest.mark.parametrize("seq,heads,kv,ldv", [(1, 2, 1, 32), (7, 4, 2, 512), (64, 8, 2, 64), (65, 3, 1, 96), (135, 4, 2, 137)])
 def test_qk_norm_rope_and_v_transpose(hip, seq, heads, kv, ldv):
     """Rows that fill no workgroup, token counts around the 64 of a V block and the 8 of a store, a row stride of V^T that
