@@ -23,7 +23,7 @@ hipStream_t flux_hip_stream_handle(void);
 /* conv.hip, for gemm.hip's choice among the convolution kernels */
 bool conv3_takes(int H, int W, int cin, int cout);
 long conv3_tiles(int H, int W, int cout);
-int conv3_launch(bool f32, const void *in, const void *w, const float *bias, const float *res, void *out, int H, int W, int cin, int cout, float *stats,
+int conv3_launch(bool f32, bool up, const void *in, const void *w, const float *bias, const float *res, void *out, int H, int W, int cin, int cout, float *stats,
                  int *stats_rows, int units);
 
 #define HIP_OK(call)                                                                   \

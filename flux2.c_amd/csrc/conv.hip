@@ -31,6 +31,10 @@
  * Fragment addresses: patch row r = 20 (row) + column; a row's 16-byte chunks are swizzled by lds_swz(r mod 16) as in gemm.hip.
  * A step down by one image row moves r by 20, which changes the swizzle by 2 (r / 2 mod 8), two rows by 4, i.e. one XOR: twelve
  * addresses per lane (3 dx x row parity x half) and immediates cover all taps and rows.
+ *
+ * up = 1: the operand is the nearest-neighbour 2x enlargement of the image that is given. Bordered position (y, x) of the enlargement holds position
+ * ((y + 1) / 2, (x + 1) / 2) of the bordered source, border included, and a tile starts at multiples of 16, so that only the patch's source
+ * offsets differ.
  */
 #include "common.h"
 #include "../../include/flux_hip.h"
@@ -44,6 +48,7 @@ struct Args {
     float *stats;
     int H, W, cin, cout;
     int tiles_x, ntiles, total, vgrid; /* total = tiles of positions x tiles of channels */
+    int up; /* fp32 results without residual alone */
     unsigned magic_x, magic_n;         /* ceil(2^32 / tiles_x), ceil(2^32 / ntiles): exact for numbers below 2^16 */
 };
 
@@ -255,7 +260,7 @@ __global__ __launch_bounds__(256) void conv3_kernel(Args g) {
     using O = Ops<F32, RES>;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, wm = wave >> 1, wn = wave & 1;
     const int l15 = lane & 15, lq = lane >> 4;
-    const int wp = g.W + 2, nch = g.cin >> 6, ldw = 9 * g.cin;
+    const int up = F32 && !RES ? g.up : 0, wp = (g.W >> up) + 2, nch = g.cin >> 6, ldw = 9 * g.cin; /* wp: the source's */
 
     Tile t, nx;
     int vb = blockIdx.x;
@@ -267,17 +272,17 @@ __global__ __launch_bounds__(256) void conv3_kernel(Args g) {
 #pragma unroll
     for (int q = 0; q < 12; q++) {
         const int r = 8 * (4 * q + wave) + (lane >> 3), py = min(r / PITCH, 17), px = min(r % PITCH, 17);
-        prel[q] = (unsigned)((py * wp + px) * g.cin + (((lane & 7) ^ lds_swz(r)) << 3)) * 2u;
+        prel[q] = (unsigned)((((py + up) >> up) * wp + ((px + up) >> up)) * g.cin + (((lane & 7) ^ lds_swz(r)) << 3)) * 2u;
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int v = 32 * i + 8 * wave + (lane >> 3), n = F32 ? v : (v & 64) + bf16_pair_feature((v & 63) >> 4, v & 15);
         wrel[i] = (unsigned)(n * ldw + (((lane & 7) ^ lds_swz(v)) << 3)) * 2u;
     }
-    const long long in_elems = (long long)(g.H + 2) * wp * g.cin;
+    const long long in_elems = (long long)((g.H >> up) + 2) * wp * g.cin;
     const __amdgpu_buffer_rsrc_t wbuf = buffer(g.w, (long long)g.cout * ldw * 2);
     auto patch_buffer = [&](const Tile &tt, int chunk) {
-        const long long o = ((long long)tt.y0 * wp + tt.x0) * g.cin + chunk * 64;
+        const long long o = ((long long)(tt.y0 >> up) * wp + (tt.x0 >> up)) * g.cin + chunk * 64;
         return buffer(g.in + o, (in_elems - o) * 2);
     };
     auto load_patch = [&](__amdgpu_buffer_rsrc_t b, int to, int q) {
@@ -602,11 +607,12 @@ bool conv3_takes(int H, int W, int cin, int cout) {
 }
 long conv3_tiles(int H, int W, int cout) { return (long)((H + 15) / 16) * ((W + 15) / 16) * (cout / 128); }
 
-int conv3_launch(bool f32, const void *in, const void *w, const float *bias, const float *res, void *out, int H, int W, int cin, int cout, float *stats,
+/* up: H x W is the 2x enlargement of the image at `in`; fp32 without residual alone */
+int conv3_launch(bool f32, bool up, const void *in, const void *w, const float *bias, const float *res, void *out, int H, int W, int cin, int cout, float *stats,
                  int *stats_rows, int units) {
     Args g = {};
     g.in = (const bf16 *)in; g.w = (const bf16 *)w; g.bias = bias; g.res = res; g.out = out; g.stats = stats;
-    g.H = H; g.W = W; g.cin = cin; g.cout = cout;
+    g.H = H; g.W = W; g.cin = cin; g.cout = cout; g.up = up;
     g.tiles_x = (W + 15) / 16;
     g.ntiles = cout / 128;
     g.total = (int)conv3_tiles(H, W, cout);
@@ -615,6 +621,7 @@ int conv3_launch(bool f32, const void *in, const void *w, const float *bias, con
     g.magic_n = (unsigned)(((1ull << 32) + g.ntiles - 1) / g.ntiles);
     if (stats_rows) *stats_rows = 2 * (g.total / g.ntiles);
     const int grid = min(g.vgrid, units);
+    if (up && (!f32 || res || ((H | W) & 1))) return flux_hip_fail("conv3_launch: an enlargement has even sides, fp32 results and no residual");
     if (f32) return res ? launch<true, true>(g, grid) : launch<true, false>(g, grid);
     return res ? launch<false, true>(g, grid) : launch<false, false>(g, grid);
 }

@@ -36,11 +36,12 @@ int flux_hip_vae_key_bias(float *bias, int n, int keys);
 size_t flux_hip_vae_attention_work_floats(int n, int ld);
 int flux_hip_vae_attention(void *out, const void *q, const void *qkv, const void *vt, void *P, float *o32, float *work, int n, int keys, int ld, float scale,
                            int *done);
-int flux_hip_vae_upsample2x_bf16(void *out_bf16, const void *x_bf16, int hp, int wp, int C);
 /* conv.hip */
 int flux_hip_vae_conv_out(uint8_t *rgb, float *rgb_f32, const void *in, const void *w, const float *bias, int H, int W);
 int flux_hip_vae_conv_in(float *out, const float *img, const void *w, const float *bias, int H, int W, float *stats, int *stats_rows);
 /* gemm.hip */
+int flux_hip_conv_enlarged(const void *in, void *enlarged, const void *w, const float *bias, float *out, int rows, int wp, int cin, int cout, float *stats,
+                           int *stats_rows);
 int flux_hip_conv_image(int epilogue, const void *in, int in_wp, int packed, const void *w, const float *bias, const float *res, void *out, int rows, int wp,
                         int cin, int cout, int taps, float *stats, int *stats_rows);
 /* vae.hip */
@@ -523,10 +524,9 @@ int flux_hip_vae_decode(flux_hip_vae *v, const float *latent, int h, int w, uint
         }
         if (level > 0) {
             const vconv *c = &v->up_conv[3 - level];
-            if (!flux_hip_vae_upsample2x_bf16(s.A, v->R, s.hp, s.wp, c->cin)) return 0;
             s.hp = 2 * (s.hp - 2) + 2;
             s.wp = 2 * (s.wp - 2) + 2;
-            if (!run_conv(&s, c, FLUX_HIP_EPI_CONV_F32, s.A, NULL, s.x, 1, v->st_x, &s.x_rows)) return 0;
+            if (!flux_hip_conv_enlarged(v->R, s.A, c->w, c->b, s.x, s.hp * s.wp, s.wp, c->cin_pad, c->cout_pad, v->st_x, &s.x_rows)) return 0;
         }
     }
     if (!flux_hip_group_norm_stats(s.A, NULL, s.x, 0, v->out_g, v->out_b, v->gn, s.hp, s.wp, 128, v->eps, 1, v->st_x, s.x_rows)) return 0;

@@ -2569,6 +2569,8 @@ static int conv_finish(GemmArgs &g) {
     return 1;
 }
 
+extern "C" int flux_hip_vae_upsample2x_bf16(void *out_bf16, const void *x_bf16, int hp, int wp, int C); /* vae.hip */
+
 /* Tile and K split of a convolution by the same kind of model as gemm_dispatch's: rounds of workgroups, each a tile's time at
  * its measured rate plus the bytes of its epilogue at a compute unit's share of the memory rate (nothing overlaps those where one
  * workgroup owns the unit). K slices, which add a second pass and its partial sums, are what small images need: 32 x 32
@@ -2576,7 +2578,7 @@ static int conv_finish(GemmArgs &g) {
  * one piece wins (54 us against 69). conv.hip's kernel is ahead from about a round of its tiles on (80 x 120 x 512: 46 us against 53 of
  * 256 x 128) as long as the image's sides do not leave a second, nearly empty round (90 x 162 x 512: 264 of its tiles, 90 us; 228 of 256 x 128,
  * 59 us). Over 111 forms of 37 layers the chosen tile took 1.5 % less than the best of four timed behind it, i.e. the same. */
-static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
+static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows, void *enlarged = nullptr) {
     static const int occ[CONV_TILES] = {3, 2, 1, 4, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1};
     static const double rate[CONV_TILES] = {2.0e12, 3.3e12, 5.4e12, 1.5e12, 0, 0, 0, 0, 0, 0, 0, 0, 4.8e12, 4.2e12, 5.0e12, 6.2e12}; /* FLOP/s of one CU */
     static const int splits[] = {1, 2, 3, 4, 6, 8, 12, 16};
@@ -2632,11 +2634,16 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows) {
         g.ws = g_ws;
         g.ws_rows = M;
     }
+    const bool direct = g.ksplit == 1 && tile == CONV_PATCH;
+    if (enlarged && !direct) {
+        if (!flux_hip_vae_upsample2x_bf16(enlarged, g.A[0], height / 2 + 2, width / 2 + 2, g.lda)) return 0;
+        g.A[0] = (const bf16 *)enlarged;
+    }
     /* one record per convolution: K slices and their second pass together */
     const int slot = conv_probe_begin(epilogue, tile);
     int ok = 1;
-    if (g.ksplit == 1 && tile == CONV_PATCH) {
-        ok = conv3_launch(!bf, g.A[0], g.W[0], g.bias, g.res, g.C[0], height, width, g.lda, N, g.stats, stats_rows, compute_units() & ~7);
+    if (direct) {
+        ok = conv3_launch(!bf, enlarged != nullptr, g.A[0], g.W[0], g.bias, g.res, g.C[0], height, width, g.lda, N, g.stats, stats_rows, compute_units() & ~7);
     } else if (g.ksplit == 1) {
         if (stats_rows) *stats_rows = 2 * ((M + conv_bm[tile] - 1) / conv_bm[tile]);
         ok = bf ? conv_tile_launch<FLUX_HIP_EPI_CONV_BF16>(g, tile) : conv_tile_launch<FLUX_HIP_EPI_CONV_F32>(g, tile);
@@ -2661,6 +2668,21 @@ extern "C" int flux_hip_conv(int epilogue, const void *in, const void *w, const 
     return flux_hip_conv_stats(epilogue, in, w, bias, res, out, rows, wp, cin, cout, taps, nullptr, nullptr);
 }
 
+static GemmArgs conv_args(const void *in, const void *w, void *out, int rows, int wp, int cin, int cout, int taps) {
+    GemmArgs g = {};
+    g.A[0] = (const bf16 *)in;
+    g.W[0] = (const bf16 *)w;
+    g.C[0] = out;
+    g.N = cout; g.K = taps * cin; g.lda = cin; g.ldw = taps * cin; g.ldc = cout;
+    g.conv_taps = taps; g.conv_wp = wp; g.conv_rows = rows;
+    g.M[0] = rows;
+    if (wp > 0) {
+        g.M[0] = wp > 2 && rows / wp > 2 ? (rows / wp - 2) * (wp - 2) : 0;
+        g.conv_magic = wp > 2 ? 0xFFFFFFFFu / (unsigned)(wp - 2) : 0;
+    }
+    return g;
+}
+
 /* The same, and (stats != NULL) the sums for the group norm that follows, see the header. */
 extern "C" int flux_hip_conv_stats(int epilogue, const void *in, const void *w, const float *bias, const float *res, void *out, int rows,
                                    int wp, int cin, int cout, int taps, float *stats, int *stats_rows) {
@@ -2679,25 +2701,30 @@ extern "C" int flux_hip_conv_stats(int epilogue, const void *in, const void *w, 
     return flux_hip_conv_image(epilogue, in, 0, 0, w, bias, res, out, rows, wp, cin, cout, taps, stats, stats_rows);
 }
 
+/* flux_hip_conv_stats to fp32 over the nearest-neighbour 2x enlargement of the bordered image `in`; rows and wp are the enlargement's. conv.hip's kernel
+ * reads the source in place of it; for the tiles of smaller images it is written to `enlarged` first. Writing it took 104 us at 1024 x 1024 x 256, 53
+ * at 512 x 512 x 512 and 14 at 256 x 256 x 512, and the convolution read four times the bytes. */
+extern "C" int flux_hip_conv_enlarged(const void *in, void *enlarged, const void *w, const float *bias, float *out, int rows, int wp, int cin, int cout,
+                                      float *stats, int *stats_rows) {
+    if (!in || !enlarged || !w || !bias || !out || wp < 4 || rows % wp || rows / wp < 4 || ((rows / wp | wp) & 1) || cin <= 0 || cin & 63 || cout <= 0 || cout & 63)
+        return flux_hip_fail("flux_hip_conv_enlarged: bad argument (rows=%d wp=%d cin=%d cout=%d)", rows, wp, cin, cout);
+    if ((((uintptr_t)in | (uintptr_t)enlarged | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)out) & 15) || (stats && (!stats_rows || ((uintptr_t)stats & 7))))
+        return flux_hip_fail("flux_hip_conv_enlarged: unaligned operand");
+    GemmArgs g = conv_args(in, w, out, rows, wp, cin, cout, 9);
+    g.conv_stride = 1; g.conv_in_wp = wp;
+    g.bias = bias; g.stats = stats;
+    return conv_launch(g, FLUX_HIP_EPI_CONV_F32, stats_rows, enlarged);
+}
+
 /* flux_hip_conv_stats without its argument checks, for the VAE's own layers: the bf16 output takes a residual as well, and
  * in_wp > 0 makes it the stride-2 3x3 convolution of a bordered image in_wp wide, rows and wp being the output's. For 1x1
  * convolutions without residual or statistics on that side, packed & 1: `in`, packed & 2: `out` hold the (rows / wp - 2) * (wp - 2)
  * interior positions only. */
 extern "C" int flux_hip_conv_image(int epilogue, const void *in, int in_wp, int packed, const void *w, const float *bias, const float *res, void *out,
                                    int rows, int wp, int cin, int cout, int taps, float *stats, int *stats_rows) {
-    GemmArgs g = {};
-    g.A[0] = (const bf16 *)in;
-    g.W[0] = (const bf16 *)w;
-    g.C[0] = out;
-    g.N = cout; g.K = taps * cin; g.lda = cin; g.ldw = taps * cin; g.ldc = cout;
-    g.conv_taps = taps; g.conv_wp = wp; g.conv_rows = rows;
+    GemmArgs g = conv_args(in, w, out, rows, wp, cin, cout, taps);
     g.conv_packed_out = packed >> 1 & 1;
     g.conv_stride = packed & 1 ? 0 : in_wp > 0 ? 2 : 1; g.conv_in_wp = in_wp > 0 ? in_wp : wp;
-    g.M[0] = rows;
-    if (wp > 0) {
-        g.M[0] = wp > 2 && rows / wp > 2 ? (rows / wp - 2) * (wp - 2) : 0;
-        g.conv_magic = wp > 2 ? 0xFFFFFFFFu / (unsigned)(wp - 2) : 0;
-    }
     g.bias = bias; g.res = res; g.stats = stats;
     if (stats && (!stats_rows || ((uintptr_t)stats & 7))) return flux_hip_fail("flux_hip_conv_stats: stats needs stats_rows and 8-byte alignment");
     return conv_launch(g, epilogue, stats_rows);

@@ -304,6 +304,49 @@ def test_conv_patch_tile(hip, switches, H, W, cin, cout):
         np.testing.assert_array_equal(run(15, epi, r), run(1, epi, r))
 
 
+@pytest.mark.parametrize("h,w,cin,cout", [(1, 1, 128, 128), (3, 8, 128, 256), (8, 9, 192, 128), (17, 16, 256, 128), (135, 130, 128, 128)])
+def test_conv_of_the_enlarged_image(hip, switches, h, w, cin, cout):
+    """The 3x3 convolution over a 2x enlargement: tile 15, which reads the source, and tiles that need the enlargement written, against tile 1 over the
+    enlargement that flux_hip_upsample2x makes; whole numbers, the same bits. One position, images cut off by tiles on both sides, more tiles than
+    compute units (270 x 260: 289)."""
+    import ctypes
+    L = hip.lib()
+    H, W = 2 * h, 2 * w
+    rows, wp = (H + 2) * (W + 2), W + 2
+    rng = np.random.default_rng(73)
+    x, wt = rng.integers(-8, 9, (cin, h, w)).astype(np.float32), rng.integers(-4, 5, (cout, cin, 3, 3)).astype(np.float32)
+    dw, db = hip.DevBuf.from_array(conv_weight(wt)), hip.DevBuf.from_array(rng.integers(-9, 10, cout).astype(np.float32))
+    src, src32 = Guarded(hip, to_padded(x), w + 2), hip.DevBuf.from_array(to_padded(x))
+    big = Guarded(hip, np.full((rows, cin), 3.0, np.float32), wp)
+    vp, ci = ctypes.c_void_p, ctypes.c_int
+    L.flux_hip_conv_enlarged.argtypes = [vp, vp, vp, vp, vp, ci, ci, ci, ci, vp, vp]
+
+    def run(tile, f):
+        L.flux_hip_linear_force_tile(tile)
+        L.flux_hip_linear_enable_splitk(0)
+        out = hip.DevBuf.from_array(np.full((rows + 1, cout), 3.0, np.float32))
+        stats = hip.DevBuf.from_array(np.full(((rows // 32 + 2) * (cout // 4) * 2,), np.nan, np.float32))
+        n = ci(0)
+        L.flux_hip_linear_probe(-2)
+        hip.check(f(out, stats, ctypes.byref(n)))
+        ran = np.zeros(2, np.int32)
+        assert L.flux_hip_linear_probe_read_launches(2, ran.ctypes.data, None) == 1 and tile in (-1, ran[0]) and 0 < n.value <= rows // 32 + 2
+        got = out.to_array(np.float32, (rows + 1, cout))
+        assert border_is_zero(got[:rows], H, W) and (got[rows] == 3.0).all()
+        check_sums(stats.to_array(np.float32, (n.value, cout // 4, 2)).astype(np.float64).sum(0), got[:rows])
+        return got[:rows]
+
+    def enlarged(out, stats, n):
+        return L.flux_hip_conv_enlarged(src.ptr, big.ptr, dw.ptr, db.ptr, out.ptr, rows, wp, cin, cout, stats.ptr, n)
+
+    got = {tile: run(tile, enlarged) for tile in (15, 13, 3, -1)}
+    hip.check(L.flux_hip_upsample2x(big.ptr, src32.ptr, h + 2, w + 2, cin))
+    want = run(1, lambda out, stats, n: L.flux_hip_conv_stats(hip.EPI_CONV_F32, big.ptr, dw.ptr, db.ptr, None, out.ptr, rows, wp, cin, cout, 9, stats.ptr, n))
+    for tile in got:
+        np.testing.assert_array_equal(got[tile], want)
+    assert L.flux_hip_conv_enlarged(src.ptr, big.ptr, dw.ptr, db.ptr, src32.ptr, 5 * wp, wp, cin, cout, None, None) == 0     # an odd side
+
+
 @pytest.mark.parametrize("H,W,cin,cout", [(1, 1, 64, 128), (1, 40, 128, 128), (130, 1, 128, 128), (70, 2, 64, 128), (7, 5, 64, 256), (21, 18, 128, 256), (9, 42, 192, 128),
                                           (13, 63, 512, 128), (4, 90, 128, 384), (5, 127, 128, 128), (3, 155, 128, 128), (3, 157, 256, 128), (2, 300, 64, 64)])
 def test_conv_run_tile(hip, switches, H, W, cin, cout):
