@@ -227,7 +227,7 @@ def bench_vae(args):
             fl = np.array([2.0 * H * W * ci * co * t for _, H, W, ci, co, t in convs] * K)
             names = {0: "gemm_kernel<64,128,2,2,CONV>", 1: "gemm_kernel<128,128,2,2,CONV>", 2: "gemm4d_kernel<8,8,CONV> (256x256 tile)",
                      3: "gemm_kernel<64,64,2,2,CONV>", 12: "gemm4d_kernel<8,4,CONV> (256x128 tile)", 13: "gemm4d_kernel<4,4,CONV> (128x128 tile)", 14: "convp_kernel (128 positions x 64 channels)",
-                     15: "conv3_kernel (16x16 positions x 128 channels)", 17: "conv_out_kernel", 18: "conv_in_kernel"}
+                     15: "conv3_kernel (16x16 positions x 128 channels)", 17: "conv_out_kernel", 18: "conv_in_kernel", 19: "gn_skip_kernel (norm and 1x1 shortcut)"}
             per_tile = {int(t): (float(ms[tiles == t].sum()), float(fl[tiles == t].sum()), int((tiles == t).sum())) for t in np.unique(tiles)}
             dom = max(per_tile, key=lambda t: per_tile[t][0])
             t_ms, t_fl, t_n = per_tile[dom]

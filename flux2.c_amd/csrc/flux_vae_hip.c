@@ -40,6 +40,8 @@ int flux_hip_vae_attention(void *out, const void *q, const void *qkv, const void
 int flux_hip_vae_conv_out(uint8_t *rgb, float *rgb_f32, const void *in, const void *w, const float *bias, int H, int W);
 int flux_hip_vae_conv_in(float *out, const float *img, const void *w, const float *bias, int H, int W, float *stats, int *stats_rows);
 /* gemm.hip */
+int flux_hip_vae_group_norm_skip(void *out_bf16, void *raw_bf16, float *y, const float *x, const float *gamma, const float *beta, float *scratch, int hp, int wp, int cin,
+                                 float eps, const float *conv_stats, int conv_stats_rows, const void *w, const float *bias, int cout);
 int flux_hip_conv_enlarged(const void *in, void *enlarged, const void *w, const float *bias, float *out, int rows, int wp, int cin, int cout, float *stats,
                            int *stats_rows);
 int flux_hip_conv_image(int epilogue, const void *in, int in_wp, int packed, const void *w, const float *bias, const float *res, void *out, int rows, int wp,
@@ -447,11 +449,15 @@ static int conv_to_bf16(vstate *s, const vconv *c, const float *res, void *out_b
 static int run_res(vstate *s, const vres *r, void *out_bf16) {
     flux_hip_vae *v = s->v;
     const int differ = r->cin != r->cout;
-    if (!flux_hip_group_norm_stats(s->A, differ ? v->R : NULL, s->x, 0, r->n1g, r->n1b, v->gn, s->hp, s->wp, r->cin, v->eps, 1, v->st_x, s->x_rows)) return 0;
+    if (differ) { /* (s->y is free: the shortcut waits there for the second convolution) */
+        if (!flux_hip_vae_group_norm_skip(s->A, v->R, s->y, s->x, r->n1g, r->n1b, v->gn, s->hp, s->wp, r->cin, v->eps, v->st_x, s->x_rows, r->skip.w, r->skip.b,
+                                          r->cout)) return 0;
+    } else if (!flux_hip_group_norm_stats(s->A, NULL, s->x, 0, r->n1g, r->n1b, v->gn, s->hp, s->wp, r->cin, v->eps, 1, v->st_x, s->x_rows)) {
+        return 0;
+    }
     if (!run_conv(s, &r->c1, FLUX_HIP_EPI_CONV_BF16, s->A, NULL, v->Hb, 1, v->st_h, &s->h_rows)) return 0; /* only the next norm reads it */
     if (!flux_hip_group_norm_stats(s->A, NULL, v->Hb, 1, r->n2g, r->n2b, v->gn, s->hp, s->wp, r->cout, v->eps, 1, v->st_h, s->h_rows)) return 0;
     if (differ) {
-        if (!run_conv(s, &r->skip, FLUX_HIP_EPI_CONV_F32, v->R, NULL, s->y, 1, NULL, NULL)) return 0;
         if (out_bf16) return conv_to_bf16(s, &r->c2, s->y, out_bf16);
         if (!run_conv(s, &r->c2, FLUX_HIP_EPI_CONV_F32, s->A, s->y, s->y, 1, v->st_x, &s->x_rows)) return 0;
         float *t = s->x; s->x = s->y; s->y = t;

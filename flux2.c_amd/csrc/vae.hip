@@ -332,6 +332,79 @@ __global__ __launch_bounds__(256) void gn_fused_kernel(bf16 *__restrict__ out, b
     }
 }
 
+/* The first norm of a residual block that changes the channel count, and its 1x1 shortcut, from one read of x: out bf16 = swish(norm(x)) as in
+ * gn_apply_kernel, y fp32 [rows][cout] = bias + bf16(x) W^T, zeros on the border. What bounds it is HBM; as two kernels with the bf16 copy of x between
+ * them, that copy was written and read once more. A workgroup takes P positions, whose bf16 values stay in LDS (64 KB at most, two workgroups to a
+ * unit), a wave 16 output channels at a time; 16-byte chunk c of position p lies at c ^ p mod 16, so that a fragment's 16
+ * rows fall on different banks. Two launches against this one, us: 1024 x 1024 x 256 -> 128 654, 410 (2.15 GB, 5.2 TB/s), 512 x 512 x 512 -> 256 335, 289 (its
+ * weights are as many bytes out of the L2s as x is), 360 x 648 x 128 -> 256 123, 87, 180 x 324 x 256 -> 512 75, 50. With four waves of 32
+ * channels 481 and 334. */
+template <int CIN, int P>
+__global__ __launch_bounds__(512, 4) void gn_skip_kernel(bf16 *__restrict__ out, float *__restrict__ y, const float *__restrict__ x, const float *__restrict__ stats,
+                                                         const float *__restrict__ gamma, const float *__restrict__ beta, const bf16 *__restrict__ w,
+                                                         const float *__restrict__ bias, int rows, int cout, int hp, int wp, unsigned long long magic) {
+    constexpr int QUADS = CIN / 4, RPI = 512 / QUADS, KS = CIN / 32, PB = P / 16, U = 8;
+    __shared__ __attribute__((aligned(16))) char raw[P * CIN * 2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l15 = lane & 15, lq = lane >> 4;
+    const int q = tid % QUADS, r0 = tid / QUADS, base = blockIdx.x * P;
+    const auto inside = [&](int r) {
+        const int py = div_wp(r, magic), px = r - py * wp;
+        return py >= 1 && py < hp - 1 && px >= 1 && px < wp - 1;
+    };
+    bf16x8 fw[KS];
+    const auto weights = [&](int n) {
+#pragma unroll
+        for (int k = 0; k < KS; k++) fw[k] = *(const bf16x8 *)(w + (size_t)(n + l15) * CIN + k * 32 + lq * 8);
+    };
+    {
+        const int g = (q * 4) / (CIN >> 5);
+        const float mean = stats[g * 2], rstd = stats[g * 2 + 1];
+        const f32x4 gm = *(const f32x4 *)(gamma + q * 4), bt = *(const f32x4 *)(beta + q * 4);
+        f32x4 sc, sh;
+#pragma unroll
+        for (int e = 0; e < 4; e++) { sc[e] = gm[e] * rstd; sh[e] = bt[e] - mean * sc[e]; }
+        f32x4 v[U];
+#pragma unroll 1
+        for (int i = 0; i < P; i += U * RPI) {
+#pragma unroll
+            for (int u = 0; u < U; u++) v[u] = *(const f32x4 *)(x + (size_t)min(base + i + u * RPI + r0, rows - 1) * CIN + q * 4);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int p = i + u * RPI + r0, r = base + p;
+                const bool in = inside(r);
+                bf16x4 o, rw;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    o[e] = (bf16)(in ? silu_f(v[u][e] * sc[e] + sh[e]) : 0.0f);
+                    rw[e] = (bf16)v[u][e];
+                }
+                if (r < rows) *(bf16x4 *)(out + (size_t)r * CIN + q * 4) = o;
+                *(bf16x4 *)(raw + p * (CIN * 2) + (((q >> 1) ^ (p & 15)) << 4) + (q & 1) * 8) = rw;
+            }
+        }
+    }
+    weights(wave * 16);
+    __syncthreads();
+#pragma unroll 1
+    for (int n = wave * 16; n < cout; n += 128) {
+        if (n >= 128) weights(n);
+        const f32x4 bv = *(const f32x4 *)(bias + n + 4 * lq);
+#pragma unroll 2
+        for (int pb = 0; pb < PB; pb++) {
+            f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int k = 0; k < KS; k++)
+                a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[k], *(const bf16x8 *)(raw + (16 * pb + l15) * (CIN * 2) + (((4 * k + lq) ^ l15) << 4)), a, 0, 0, 0);
+            const int r = base + 16 * pb + l15;
+            const bool in = inside(r);
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = in ? a[e] + bv[e] : 0.0f;
+            if (r < rows) *(f32x4 *)(y + (size_t)r * cout + n + 4 * lq) = v;
+        }
+    }
+}
+
 /* nearest-neighbour 2x upsample (flux_upsample_nearest, flux_kernels.c:1017-1036): fp32 or bf16
  * [hp*wp, C] -> bf16 [(2H+2)*(2W+2), C] with a fresh zero border. One thread per bordered source position and V
  * channels, which go to the source's up to four places: interior (y, x) to rows 2y-1, 2y and columns 2x-1, 2x of the bordered output,
@@ -715,6 +788,9 @@ __global__ __launch_bounds__(256) void vae_transpose_kernel(bf16 *__restrict__ v
 
 /* ------------------------------------------------------------------ host entry points */
 
+int conv_probe_begin(int epilogue, int tile);
+void conv_probe_end(int slot);
+
 extern "C" int flux_hip_vae_latent_in(void *out_bf16, const float *latent, const float *bn_mean, const float *bn_var,
                                       const float *pq_w, const float *pq_b, int h, int w, float eps) {
     if (h <= 0 || w <= 0) return flux_hip_fail("flux_hip_vae_latent_in: bad size %d x %d", h, w);
@@ -725,21 +801,13 @@ extern "C" int flux_hip_vae_latent_in(void *out_bf16, const float *latent, const
     return 1;
 }
 
+/* mean and 1/sqrt(var + eps) of the 32 groups, at the head of the scratch */
 template <typename T>
-static int group_norm_run(void *out_bf16, void *raw_bf16, const T *x, const float *gamma, const float *beta, float *scratch, int hp, int wp,
-                          int C, float eps, int swish, const float *conv_stats, int conv_stats_rows) {
+static int group_norm_statistics(const T *x, float *scratch, int hp, int wp, int C, float eps, const float *conv_stats, int conv_stats_rows) {
     const int rows = hp * wp, nblocks = (rows + GN_ROWS - 1) / GN_ROWS;
     float *partial = scratch + 64, *stats = scratch;
     hipStream_t st = flux_hip_stream_handle();
     const double count = (double)(hp - 2) * (wp - 2) * (C / 32);
-    const unsigned long long magic = ((1ull << 40) + (unsigned)wp - 1) / (unsigned)wp;
-    if (conv_stats && conv_stats_rows <= GN_FUSED_ROWS) {
-        const int span = (rows + 63) / 64 * (C / 64) > 1024 ? 128 : 64;
-        hipLaunchKernelGGL(gn_fused_kernel<T>, dim3((rows + span - 1) / span, C / 64), dim3(256), 0, st, (bf16 *)out_bf16, (bf16 *)raw_bf16, x, conv_stats,
-                           conv_stats_rows, count, eps, gamma, beta, rows, C, hp, wp, magic, swish, span);
-        LAUNCH_OK("gn_fused_kernel");
-        return 1;
-    }
     if (conv_stats && conv_stats_rows <= GN_ONE_PASS_ROWS) {
         hipLaunchKernelGGL(gn_stats_kernel, dim3(32), dim3(256), 0, st, stats, conv_stats, conv_stats_rows, C, count, eps);
         LAUNCH_OK("gn_stats_kernel");
@@ -757,6 +825,25 @@ static int group_norm_run(void *out_bf16, void *raw_bf16, const T *x, const floa
         hipLaunchKernelGGL(gn_finalize_kernel, dim3(32), dim3(256), 0, st, stats, partial, nblocks, count, eps);
         LAUNCH_OK("gn_finalize_kernel");
     }
+    return 1;
+}
+
+template <typename T>
+static int group_norm_run(void *out_bf16, void *raw_bf16, const T *x, const float *gamma, const float *beta, float *scratch, int hp, int wp,
+                          int C, float eps, int swish, const float *conv_stats, int conv_stats_rows) {
+    const int rows = hp * wp;
+    hipStream_t st = flux_hip_stream_handle();
+    const double count = (double)(hp - 2) * (wp - 2) * (C / 32);
+    const unsigned long long magic = ((1ull << 40) + (unsigned)wp - 1) / (unsigned)wp;
+    if (conv_stats && conv_stats_rows <= GN_FUSED_ROWS) {
+        const int span = (rows + 63) / 64 * (C / 64) > 1024 ? 128 : 64;
+        hipLaunchKernelGGL(gn_fused_kernel<T>, dim3((rows + span - 1) / span, C / 64), dim3(256), 0, st, (bf16 *)out_bf16, (bf16 *)raw_bf16, x, conv_stats,
+                           conv_stats_rows, count, eps, gamma, beta, rows, C, hp, wp, magic, swish, span);
+        LAUNCH_OK("gn_fused_kernel");
+        return 1;
+    }
+    if (!group_norm_statistics(x, scratch, hp, wp, C, eps, conv_stats, conv_stats_rows)) return 0;
+    const float *stats = scratch;
     /* as many positions per workgroup as leave 2048 workgroups, at least four per thread */
     int span = GN_ROWS;
     while (span > 4 * (256 / (C / 4)) && (rows + span - 1) / span < 2048) span >>= 1;
@@ -774,6 +861,34 @@ extern "C" int flux_hip_group_norm_stats(void *out_bf16, void *raw_bf16, const v
     if (conv_stats && conv_stats_rows <= 0) return flux_hip_fail("flux_hip_group_norm_stats: conv_stats_rows=%d", conv_stats_rows);
     return x_is_bf16 ? group_norm_run(out_bf16, raw_bf16, (const bf16 *)x, gamma, beta, scratch, hp, wp, C, eps, swish, conv_stats, conv_stats_rows)
                      : group_norm_run(out_bf16, raw_bf16, (const float *)x, gamma, beta, scratch, hp, wp, C, eps, swish, conv_stats, conv_stats_rows);
+}
+
+/* The first norm (with swish) of a residual block whose channel counts differ, and its 1x1 shortcut: y = conv(bf16(x)) as flux_hip_conv's fp32 epilogue
+ * writes it. w: [cout][cin]; raw: room for a bf16 copy of x, which only the two launches of small images use. */
+extern "C" int flux_hip_vae_group_norm_skip(void *out_bf16, void *raw_bf16, float *y, const float *x, const float *gamma, const float *beta, float *scratch, int hp,
+                                            int wp, int cin, float eps, const float *conv_stats, int conv_stats_rows, const void *w, const float *bias, int cout) {
+    if (cin != 128 && cin != 256 && cin != 512) return flux_hip_fail("flux_hip_vae_group_norm_skip: %d channels (128, 256 or 512)", cin);
+    if (hp < 3 || wp < 3 || (long long)hp * wp >= 1 << 22 || wp >= 1 << 12 || cout <= 0 || cout % 128)
+        return flux_hip_fail("flux_hip_vae_group_norm_skip: bad shape (hp=%d wp=%d cout=%d)", hp, wp, cout);
+    if (!out_bf16 || !raw_bf16 || !y || !x || !gamma || !beta || !scratch || !w || !bias) return flux_hip_fail("flux_hip_vae_group_norm_skip: NULL argument");
+    if (((uintptr_t)out_bf16 | (uintptr_t)raw_bf16 | (uintptr_t)y | (uintptr_t)x | (uintptr_t)gamma | (uintptr_t)beta | (uintptr_t)w | (uintptr_t)bias) & 15)
+        return flux_hip_fail("flux_hip_vae_group_norm_skip: operands must be 16-byte aligned");
+    const int rows = hp * wp, P = cin == 512 ? 64 : 128;
+    /* Two launches of more workgroups win where this one leaves most units with none or one: decoder, 128 x 128 x 512 -> 256 (265 workgroups) 31 + 5 us for the
+     * sums against 30, 128 x 128 x 256 -> 128 (133) no difference; encoder 128 x 128 x 128 -> 256 (133) 10 us longer together with 64 x 64 x 256 -> 512,
+     * 160 x 160 (206) 8 us shorter. */
+    if ((rows + P - 1) / P < (cin == 512 ? 300 : 150))
+        return flux_hip_group_norm_stats(out_bf16, raw_bf16, x, 0, gamma, beta, scratch, hp, wp, cin, eps, 1, conv_stats, conv_stats_rows) &&
+               flux_hip_conv_stats(FLUX_HIP_EPI_CONV_F32, raw_bf16, w, bias, nullptr, y, rows, wp, cin, cout, 1, nullptr, nullptr);
+    if (!group_norm_statistics(x, scratch, hp, wp, cin, eps, conv_stats, conv_stats_rows)) return 0;
+    const unsigned long long magic = ((1ull << 40) + (unsigned)wp - 1) / (unsigned)wp;
+    auto kern = cin == 128 ? gn_skip_kernel<128, 128> : cin == 256 ? gn_skip_kernel<256, 128> : gn_skip_kernel<512, 64>;
+    const int slot = conv_probe_begin(FLUX_HIP_EPI_CONV_F32, 19);
+    hipLaunchKernelGGL(kern, dim3((rows + P - 1) / P), dim3(512), 0, flux_hip_stream_handle(), (bf16 *)out_bf16, y, x, scratch, gamma, beta, (const bf16 *)w, bias, rows,
+                       cout, hp, wp, magic);
+    conv_probe_end(slot);
+    LAUNCH_OK("gn_skip_kernel");
+    return 1;
 }
 
 extern "C" int flux_hip_group_norm(void *out_bf16, void *raw_bf16, const void *x, int x_is_bf16, const float *gamma, const float *beta,

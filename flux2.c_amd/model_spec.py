@@ -256,9 +256,9 @@ def vae_decode_convs(h, w):
     out = [("post_quant_conv", H, W, 32, 32, 1), ("conv_in", H, W, 32, 512, 9)]
 
     def res(name, i, o):
-        out.append((name + ".conv1", H, W, i, o, 9))
         if i != o:
             out.append((name + ".conv_shortcut", H, W, i, o, 1))
+        out.append((name + ".conv1", H, W, i, o, 9))
         out.append((name + ".conv2", H, W, o, o, 9))
 
     res("mid.0", 512, 512)
@@ -294,9 +294,9 @@ def vae_encode_convs(H, W):
     out = [("conv_in", H, W, 3, 128, 9)]
 
     def res(name, i, o):
-        out.append((name + ".conv1", H, W, i, o, 9))
         if i != o:
             out.append((name + ".conv_shortcut", H, W, i, o, 1))
+        out.append((name + ".conv1", H, W, i, o, 9))
         out.append((name + ".conv2", H, W, o, o, 9))
 
     prev = 128

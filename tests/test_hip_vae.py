@@ -698,6 +698,41 @@ def test_group_norm_in_one_launch(hip, H, W, C, prows, in_bf16):
     assert (got[0][0][rows] == got[0][0][rows, 0]).all() and (got[0][1][rows] == 0x4040).all()
 
 
+@pytest.mark.parametrize("H,W,cin,cout", [(5, 7, 256, 128), (181, 190, 128, 256), (180, 183, 256, 128), (9, 4000, 256, 256), (150, 131, 512, 256), (140, 141, 256, 512),
+                                          (190, 180, 128, 512), (9000, 1, 512, 128)])
+def test_group_norm_with_shortcut(hip, switches, H, W, cin, cout):
+    """The norm and the 1x1 shortcut of a widening or narrowing block in one launch, against the norm with its bf16 copy and a convolution of that: the
+    same operations in the same order, so the same bits. A small image (the two launches), a cut last workgroup, images one position wide and high,
+    the column counts of one to four trips of a wave."""
+    import ctypes
+    L = hip.lib()
+    hp, wp = H + 2, W + 2
+    rows = hp * wp
+    x = to_padded(normal_f32((cin, H, W), 81, 1))
+    dx = hip.DevBuf.from_array(x)
+    gm, bt, b = (hip.DevBuf.from_array(normal_f32((n,), 81, 2 + i)) for i, n in enumerate((cin, cin, cout)))
+    w = hip.DevBuf.from_array(f32_to_bf16(normal_f32((cout, cin), 81, 5) * 0.1))
+    scratch = hip.DevBuf(L.flux_hip_group_norm_scratch_floats(hp, wp) * 4)
+    vp, ci = ctypes.c_void_p, ctypes.c_int
+    L.flux_hip_vae_group_norm_skip.argtypes = [vp, vp, vp, vp, vp, vp, vp, ci, ci, ci, ctypes.c_float, vp, ci, vp, vp, ci]
+    got = []
+    for one in (True, False):
+        out, raw = (hip.DevBuf.from_array(np.full((rows + 1, cin), 0x4040, np.uint16)) for _ in range(2))
+        y = hip.DevBuf.from_array(np.full((rows + 1, cout), 3.0, np.float32))
+        if one:
+            hip.check(L.flux_hip_vae_group_norm_skip(out.ptr, raw.ptr, y.ptr, dx.ptr, gm.ptr, bt.ptr, scratch.ptr, hp, wp, cin, 1e-6, None, 0, w.ptr, b.ptr, cout))
+        else:
+            hip.check(L.flux_hip_group_norm_stats(out.ptr, raw.ptr, dx.ptr, 0, gm.ptr, bt.ptr, scratch.ptr, hp, wp, cin, 1e-6, 1, None, 0))
+            L.flux_hip_linear_force_tile(1)
+            L.flux_hip_linear_enable_splitk(0)
+            hip.check(L.flux_hip_conv_stats(hip.EPI_CONV_F32, raw.ptr, w.ptr, b.ptr, None, y.ptr, rows, wp, cin, cout, 1, None, None))
+        got.append((out.to_array(np.uint16, (rows + 1, cin)), y.to_array(np.float32, (rows + 1, cout))))
+    assert (got[0][0][rows] == 0x4040).all() and (got[0][1][rows] == 3.0).all()
+    assert border_is_zero(bf16_to_f32(got[0][0][:rows]), H, W) and border_is_zero(got[0][1][:rows], H, W)
+    np.testing.assert_array_equal(got[0][0], got[1][0])
+    np.testing.assert_array_equal(got[0][1], got[1][1])
+
+
 def test_upsample(hip, oracle_mod):
     C, H, W = 128, 5, 7
     x = normal_f32((C, H, W), 55, 1)
