@@ -1876,126 +1876,101 @@ struct AdalnArgs {
     float eps;
 };
 
-__device__ __forceinline__ float block_sum_256(float v, float *red) {
+/* v summed over the workgroup's waves */
+__device__ __forceinline__ float block_sum(float v, float *red, int waves) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
     __syncthreads(); /* red is free again */
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    return (red[0] + red[1]) + (red[2] + red[3]);
+    float sum = 0.0f;
+    for (int w = 0; w < waves; w++) sum += red[w];
+    return sum;
 }
 
 /* RMS = true: the norm that follows is x / sqrt(mean(x^2) + eps) * weight instead (qwen3_rms_norm,
- * flux_qwen3.c:177-197) */
-template <bool RMS>
-__global__ __launch_bounds__(256) void splitk_finish_adaln_kernel(GemmArgs g, AdalnArgs a) {
-    __shared__ float red[4];
-    const int row = blockIdx.x;
+ * flux_qwen3.c:177-197). A thread owns Q quads of columns, blockDim.x quads apart. Everything the row needs is requested at once - the first U
+ * slices, then x, gate, scale and shift - so that it costs one round trip to memory beside the further slices. With 256 threads of
+ * four quads, four slices at a time and scale and shift behind them: 67 rows of 2560 5.6 us, now 4.8; 80 rows of 3072 5.8 and 5.2; 512 rows of
+ * 2560 9.6 and 8.1; of 3072 768 rows 12.5 and 12.7, 1202 19.3 and 18.1, 2498 30.6 and 28.2. */
+template <bool RMS, int Q, int U>
+__global__ __launch_bounds__(1024 / Q) void splitk_finish_adaln_kernel(GemmArgs g, AdalnArgs a) {
+    __shared__ float red[16];
+    const int row = blockIdx.x, threads = blockDim.x, waves = threads >> 6;
     const int prob = (row >= g.moff[1]) + (row >= g.moff[2]) + (row >= g.moff[3]);
     const int m = row - g.moff[prob];
     const int N = g.N;
-    f32x4 v[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) v[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    /* What the row needs besides the partial sums is requested ahead of its use - the residual and its gate in front of
-     * the slices, scale and shift in front of the sums over the row - so that the row costs two round trips to memory
-     * rather than four in a row (with 80 to 768 rows the kernel is a few waves per compute unit that wait for memory
-     * most of their time). */
     float *xr = (float *)g.C[prob] + (size_t)m * g.ldc;
-    f32x4 x0[4], gt0[4], sc0[4], sh0[4];
+    const float *gate = g.gate[prob], *scale = a.scale[prob], *shift = RMS ? nullptr : a.shift[prob];
+    f32x4 v[Q], x0[Q], gt0[Q], sc0[Q], sh0[Q];
+    int c[Q];
+    bool mine[Q];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int c = (i * 256 + threadIdx.x) * 4;
-        if (c < N) {
-            x0[i] = *(const f32x4 *)(xr + c);
-            gt0[i] = *(const f32x4 *)(g.gate[prob] + c);
-        }
+    for (int i = 0; i < Q; i++) {
+        const int at = (i * threads + threadIdx.x) * 4;
+        mine[i] = at < N;
+        c[i] = mine[i] ? at : 0;
+        v[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    /* slices four at a time, so that a row with many short slices keeps enough loads in flight;
-     * the additions stay in slice order */
+    /* slices U at a time, the additions in slice order */
     const size_t slice = (size_t)g.ws_rows * N;
     const float *w0 = g.ws + (size_t)row * N;
-    int s = 0;
-    for (; s + 4 <= g.ksplit; s += 4) {
-        f32x4 t[4][4];
+    f32x4 t[U][Q];
+    const auto request = [&](int s) {
 #pragma unroll
-        for (int u = 0; u < 4; u++)
+        for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int c = (i * 256 + threadIdx.x) * 4;
-                if (c < N) t[u][i] = *(const f32x4 *)(w0 + (size_t)(s + u) * slice + c);
-            }
+            for (int i = 0; i < Q; i++)
+                if (s + u < g.ksplit) t[u][i] = *(const f32x4 *)(w0 + (size_t)(s + u) * slice + c[i]);
+    };
+    request(0);
 #pragma unroll
-        for (int u = 0; u < 4; u++)
+    for (int i = 0; i < Q; i++) {
+        x0[i] = *(const f32x4 *)(xr + c[i]);
+        gt0[i] = *(const f32x4 *)(gate + c[i]);
+        sc0[i] = *(const f32x4 *)(scale + c[i]);
+        if (!RMS) sh0[i] = *(const f32x4 *)(shift + c[i]);
+    }
+    for (int s = 0;;) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int c = (i * 256 + threadIdx.x) * 4;
-                if (c < N) {
+        for (int u = 0; u < U; u++)
+            if (s + u < g.ksplit) {
+#pragma unroll
+                for (int i = 0; i < Q; i++)
 #pragma unroll
                     for (int e = 0; e < 4; e++) v[i][e] += t[u][i][e];
-                }
             }
-    }
-    for (; s < g.ksplit; s++) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int c = (i * 256 + threadIdx.x) * 4;
-            if (c < N) {
-                const f32x4 t = *(const f32x4 *)(w0 + (size_t)s * slice + c);
-#pragma unroll
-                for (int e = 0; e < 4; e++) v[i][e] += t[e];
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int c = (i * 256 + threadIdx.x) * 4;
-        if (c < N) {
-            sc0[i] = *(const f32x4 *)(a.scale[prob] + c);
-            if (!RMS) sh0[i] = *(const f32x4 *)(a.shift[prob] + c);
-        }
+        s += U;
+        if (s >= g.ksplit) break;
+        request(s);
     }
     float s1 = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int c = (i * 256 + threadIdx.x) * 4;
-        if (c < N) {
-            f32x4 x = x0[i];
-            const f32x4 gt = gt0[i];
+    for (int i = 0; i < Q; i++) {
+        f32x4 x = x0[i];
 #pragma unroll
-            for (int e = 0; e < 4; e++) x[e] += gt[e] * v[i][e];
-            *(f32x4 *)(xr + c) = x;
-            v[i] = x;
+        for (int e = 0; e < 4; e++) x[e] += gt0[i][e] * v[i][e];
+        v[i] = x;
+        if (mine[i]) {
+            *(f32x4 *)(xr + c[i]) = x;
             s1 += (x[0] + x[1]) + (x[2] + x[3]);
         }
     }
-    const float mean = RMS ? 0.0f : block_sum_256(s1, red) / (float)N;
+    const float mean = RMS ? 0.0f : block_sum(s1, red, waves) / (float)N;
     float q = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int c = (i * 256 + threadIdx.x) * 4;
-        if (c < N) {
+    for (int i = 0; i < Q; i++)
+        if (mine[i]) {
 #pragma unroll
             for (int e = 0; e < 4; e++) { const float d = v[i][e] - mean; q += d * d; }
         }
-    }
-    const float inv = 1.0f / sqrtf(block_sum_256(q, red) / (float)N + a.eps);
+    const float inv = 1.0f / sqrtf(block_sum(q, red, waves) / (float)N + a.eps);
     bf16 *o = a.out[prob] + (size_t)m * a.ldo;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int c = (i * 256 + threadIdx.x) * 4;
-        if (c < N) {
-            const f32x4 sc = sc0[i];
-            bf16x4 r;
-            if (RMS) {
+    for (int i = 0; i < Q; i++) {
+        bf16x4 r;
 #pragma unroll
-                for (int e = 0; e < 4; e++) r[e] = (bf16)(v[i][e] * inv * sc[e]);
-            } else {
-                const f32x4 sh = sh0[i];
-#pragma unroll
-                for (int e = 0; e < 4; e++) r[e] = (bf16)((1.0f + sc[e]) * ((v[i][e] - mean) * inv) + sh[e]);
-            }
-            *(bf16x4 *)(o + c) = r;
-        }
+        for (int e = 0; e < 4; e++) r[e] = (bf16)(RMS ? v[i][e] * inv * sc0[i][e] : (1.0f + sc0[i][e]) * ((v[i][e] - mean) * inv) + sh0[i][e]);
+        if (mine[i]) *(bf16x4 *)(o + c[i]) = r;
     }
 }
 
@@ -2017,10 +1992,14 @@ static int launch_split(GemmArgs &g, int tile) {
 
 static int launch_split_adaln(GemmArgs &g, int tile, const AdalnArgs &a) {
     if (!launch_epi<EPI_PARTIAL>(g, tile)) return 0;
-    if (a.shift[0])
-        hipLaunchKernelGGL(splitk_finish_adaln_kernel<false>, dim3((unsigned)g.ws_rows), dim3(256), 0, flux_hip_stream_handle(), g, a);
-    else
-        hipLaunchKernelGGL(splitk_finish_adaln_kernel<true>, dim3((unsigned)g.ws_rows), dim3(256), 0, flux_hip_stream_handle(), g, a);
+    /* Few rows wait for memory: a quad a thread, four slices on their way. With more rows than units it is the bytes (768 rows in four slices: 61 MB), and
+     * small workgroups win. Whole passes, us, first form / second: prompts of 67 tokens 2633 / 2690, 128 3172 / 3227, 200 3748 / 3784,
+     * 300 4345 / 4343, 512 5167 / 5168; denoising steps of 80 tokens 2478 / 2507, 208 3313 / 3305, 320 3743 / 3720, 640 5051 / 5000. */
+    const bool few = g.ws_rows <= 200;
+    const int quads = g.N >> 2, threads = few ? (quads + 63) / 64 * 64 : (quads + 255) / 256 * 64;
+    auto kern = few ? (a.shift[0] ? splitk_finish_adaln_kernel<false, 1, 4> : splitk_finish_adaln_kernel<true, 1, 4>)
+                    : (a.shift[0] ? splitk_finish_adaln_kernel<false, 4, 2> : splitk_finish_adaln_kernel<true, 4, 2>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)g.ws_rows), dim3(threads), 0, flux_hip_stream_handle(), g, a);
     return hipGetLastError() == hipSuccess ? 1 : flux_hip_fail("split-K reduction + AdaLN launch failed");
 }
 

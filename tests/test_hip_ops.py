@@ -502,6 +502,43 @@ def test_linear_residual_then_adaln(hip, oracle_mod, shape, tile):
     hip.lib().flux_hip_linear_force_tile(-1)
 
 
+@pytest.mark.parametrize("rms", [False, True])
+@pytest.mark.parametrize("M", [1, 200, 201])
+@pytest.mark.parametrize("N,slices", [(128, 2), (384, 8), (2560, 3), (4096, 9)])
+def test_second_pass_with_norm(hip, M, N, slices, rms):
+    """The second pass that also normalises: a quad of columns a thread up to 200 rows, four beyond; columns that leave a wave half empty, one to four
+    quads, as many slices as are requested at once, fewer and more. x as the plain second pass gives it, bit for bit; the norm against float64 on that x:
+    one rounding to bf16, 2^-9 an element, and fp32 sums."""
+    L = hip.lib()
+    K = 64 * 4 * slices
+    a, W = q(normal_f32((M, K), 82, 1)), q(normal_f32((N, K), 82, 2, 0.0, 0.05))
+    res, g = normal_f32((M + 1, N), 82, 3), normal_f32((N,), 82, 4)
+    sc, sh = normal_f32((N,), 82, 5, 1.0, 0.2), normal_f32((N,), 82, 6)
+    da, dW, dg, dsc, dsh = dev_bf16(hip, a), dev_bf16(hip, W), hip.DevBuf.from_array(g), hip.DevBuf.from_array(sc), hip.DevBuf.from_array(sh)
+    dx, plain = hip.DevBuf.from_array(res), hip.DevBuf.from_array(res)
+    dn = hip.DevBuf.from_array(np.full((M + 1, N), 0x4040, np.uint16))
+    try:
+        L.flux_hip_linear_force_tile(1)
+        L.flux_hip_linear_force_split(slices)
+        assert hip.linear_resid_adaln([(da.ptr, dW.ptr, dx.ptr, dg.ptr, M)], N, K, K, K, N, [(dn.ptr, None if rms else dsh.ptr, dsc.ptr)]) == (slices in (2, 3, 8))
+        hip.linear(hip.EPI_RESID, [(da.ptr, dW.ptr, plain.ptr, dg.ptr, M)], N, K, K, K, N)
+    finally:
+        L.flux_hip_linear_force_split(0)
+        L.flux_hip_linear_force_tile(-1)
+    x, n = dx.to_array(np.float32, (M + 1, N)), dn.to_array(np.uint16, (M + 1, N))
+    np.testing.assert_array_equal(x, plain.to_array(np.float32, (M + 1, N)))
+    np.testing.assert_array_equal(x[M], res[M])
+    assert (n[M] == 0x4040).all()
+    if slices not in (2, 3, 8):
+        return
+    x = x[:M].astype(np.float64)
+    if rms:
+        want = x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-6) * sc
+    else:
+        want = (1.0 + sc) * (x - x.mean(1, keepdims=True)) / np.sqrt(x.var(1, keepdims=True) + 1e-6) + sh
+    assert rel_l2(bf16_to_f32(n[:M]), want) < 2.0 ** -9
+
+
 def test_linear_residual_then_rms_norm(hip, oracle_mod):
     """The same second pass with the text encoder's RMS norm (no shift, scale = the norm's weight)."""
     M, N, K = 96, 2560, 4096
