@@ -539,6 +539,27 @@ def test_second_pass_with_norm(hip, M, N, slices, rms):
     assert rel_l2(bf16_to_f32(n[:M]), want) < 2.0 ** -9
 
 
+@pytest.mark.parametrize("M,M2", [(1, 5), (64, 3), (257, 100)])
+def test_transposed_store_in_slices(hip, oracle_mod, M, M2):
+    """The transposed store behind K slices, two parts with outputs of their own: 3072 inputs in slices of 6 to 24 K steps against the oracle, fp32 sums in
+    another order (2e-6, as for the one-piece form); columns behind the last row stay as they were."""
+    L = hip.lib()
+    N, K, ld = 128, 3072, M + M2 + 3
+    x, W = q(normal_f32((M + M2, K), 83, 1)), q(normal_f32((N, K), 83, 2, 0.0, 0.05))
+    dx, dW = dev_bf16(hip, x), dev_bf16(hip, W)
+    want = oracle_mod.linear(x, W)
+    try:
+        for slices in (0, 2, 8):
+            L.flux_hip_linear_force_split(slices)
+            o1, o2 = (hip.DevBuf.from_array(np.full((N, ld), 7.0, np.float32)) for _ in range(2))
+            hip.linear(hip.EPI_F32_T, [(dx.ptr, dW.ptr, o1.ptr, None, M), (dx.at(M * K * 2), dW.ptr, o2.ptr, None, M2)], N, K, K, K, ld)
+            for o, m, w in ((o1, M, want[:M]), (o2, M2, want[M:])):
+                got = o.to_array(np.float32, (N, ld))
+                assert rel_l2(got[:, :m].T, w) < 2e-6 and (got[:, m:] == 7.0).all()
+    finally:
+        L.flux_hip_linear_force_split(0)
+
+
 def test_linear_residual_then_rms_norm(hip, oracle_mod):
     """The same second pass with the text encoder's RMS norm (no shift, scale = the norm's weight)."""
     M, N, K = 96, 2560, 4096
