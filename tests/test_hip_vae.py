@@ -733,6 +733,29 @@ def test_group_norm_with_shortcut(hip, switches, H, W, cin, cout):
     np.testing.assert_array_equal(got[0][1], got[1][1])
 
 
+@pytest.mark.parametrize("h,w", [(1, 1), (2, 1), (3, 5), (16, 9)])
+def test_latent_input(hip, h, w):
+    """Scaling, 2x2 unpatchify and the post-quant 1x1 convolution against float64: one rounding to bf16 (2^-9 an element) of fp32 sums; zeros on the border
+    and in channels 32 to 63, nothing behind the last position. Position counts around a workgroup's 16."""
+    import ctypes
+    z, mean, var = normal_f32((128, h, w), 91, 1), normal_f32((128,), 91, 2), np.abs(normal_f32((128,), 91, 3)) + 0.1
+    pw, pb = normal_f32((32, 32), 91, 4, 0.0, 0.2), normal_f32((32,), 91, 5)
+    rows = (2 * h + 2) * (2 * w + 2)
+    out = hip.DevBuf.from_array(np.full((rows + 1, 64), 0x4040, np.uint16))
+    d = [hip.DevBuf.from_array(np.ascontiguousarray(a, np.float32)) for a in (z, mean, var, pw, pb)]
+    f = hip.lib().flux_hip_vae_latent_in
+    f.argtypes = [ctypes.c_void_p] * 6 + [ctypes.c_int] * 2 + [ctypes.c_float]
+    hip.check(f(out.ptr, *[b.ptr for b in d], h, w, 1e-4))
+    got = out.to_array(np.uint16, (rows + 1, 64))
+    assert (got[rows] == 0x4040).all() and (got[:rows, 32:] == 0).all()
+    x = z.astype(np.float64) * np.sqrt(var.astype(np.float64) + 1e-4)[:, None, None] + mean.astype(np.float64)[:, None, None]
+    x = x.reshape(32, 2, 2, h, w).transpose(0, 3, 1, 4, 2).reshape(32, 2 * h, 2 * w)
+    want = np.einsum("oc,cyx->oyx", pw.astype(np.float64), x) + pb[:, None, None]
+    got = bf16_to_f32(got[:rows, :32])
+    assert border_is_zero(got, 2 * h, 2 * w)
+    assert rel_l2(from_padded(got, 2 * h, 2 * w), want) < 2.0 ** -9
+
+
 def test_upsample(hip, oracle_mod):
     C, H, W = 128, 5, 7
     x = normal_f32((C, H, W), 55, 1)
