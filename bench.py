@@ -665,7 +665,9 @@ def measure_workload(model, cfg, name, K, Wm, fused, args, headline):
     TILE_NAMES = {0: f"gemm_kernel<64,128,2,2,{epi_name}>", 1: f"gemm_kernel<128,128,2,2,{epi_name}>", 2: f"gemm4d_kernel<8,8,{epi_name}> (256x256 tile)",
                   3: f"gemm_kernel<64,64,2,2,{epi_name}>", 4: f"gemm4w_kernel<8,4,{epi_name},2,4> (256x256 tile, 8 waves)", 5: f"gemm4d_kernel<9,6,{epi_name}> (288x192 tile)",
                   6: f"gemm4d_kernel<6,6,{epi_name}> (192x192 tile)", 7: f"gemm4d_kernel<8,6,{epi_name}> (256x192 tile)",
-                  **{t: f"gemm_few_kernel<{bn},{epi_name}> ({bn} columns)" for t, bn in ((8, 80), (16, 96), (10, 112), (9, 128), (24, 144))},
+                  8: f"gemm_few_kernel<80,{epi_name}> (80 columns)", 16: f"gemm_few_kernel<96,{epi_name}> (96 columns)",
+                  10: f"gemm_few_kernel<112,{epi_name}> (112 columns)", 9: f"gemm_few_kernel<128,{epi_name}> (128 columns)",
+                  24: f"gemm_few_kernel<144,{epi_name}> (144 columns)",
                   12: f"gemm4d_kernel<8,4,{epi_name}> (256x128 tile)",
                   13: f"gemm4d_kernel<4,4,{epi_name}> (128x128 tile)", 14: f"gemm4d_kernel<6,8,{epi_name}> (192x256 tile)",
                   23: f"gemm4d_kernel<8,5,{epi_name}> (256x160 tile)",

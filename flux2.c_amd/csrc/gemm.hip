@@ -1611,7 +1611,7 @@ static int launch_cfg(GemmArgs &g) {
 }
 
 template <int BN, int EPI>
-static int launch_few(GemmArgs &g) {
+static int launch_cfg(GemmArgs &g) {
     constexpr int STAGE = (128 + BN) * 128, LDS = (160 * 1024 / STAGE < 6 ? 160 * 1024 / STAGE : 6) * STAGE;
     static bool attr_done = false;
     auto kern = gemm_few_kernel<BN, EPI>;
@@ -1744,11 +1744,11 @@ static int launch_epi(GemmArgs &g, int tile) {
         case 4: return launch_4w<8, 4, EPI, 2, 4>(g); /* 8 waves, two per SIMD, on the 256x256 tile */
         case 1: return launch_cfg<128, 128, 2, 2, EPI>(g);
         case 3: return launch_cfg<64, 64, 2, 2, EPI>(g);
-        case 8: return launch_few<80, EPI>(g);
-        case 9: return launch_few<128, EPI>(g);
-        case 10: return launch_few<112, EPI>(g);
-        case 16: return launch_few<96, EPI>(g);
-        case 24: return launch_few<144, EPI>(g);
+        case 8: return launch_cfg<80, EPI>(g);
+        case 9: return launch_cfg<128, EPI>(g);
+        case 10: return launch_cfg<112, EPI>(g);
+        case 16: return launch_cfg<96, EPI>(g);
+        case 24: return launch_cfg<144, EPI>(g);
         default: return launch_cfg<64, 128, 2, 2, EPI>(g);
     }
 }
@@ -2186,14 +2186,15 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
         double best = 1e30;
         static const int splits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
         /* every epilogue can run as K slices + a finishing pass; for SwiGLU the gate and up rows must be one contiguous block of the
-         * weight matrix. (The final layer's 128 columns, stored transposed, are 8 tiles of 64 x 64 at 256 tokens: 35 us in one piece, 14.5 in slices; 16 tokens 35 and 11.4.) */
+         * weight matrix. (The final layer's 128 columns, stored transposed, are 8 tiles of 64 x 64 at 256 tokens: 35 us in one piece, 14.5 in slices; 16 tokens 35 and 11.4; 12544 tokens, whose second pass
+         * takes 24 us, 49 and 56.) */
         const int N = g.N, K = g.K, w_row0 = g.w_row0, w_row1 = g.w_row1;
-        const bool can_split = g_splitk_enabled &&
-                               (epilogue == FLUX_HIP_EPI_RESID || epilogue == FLUX_HIP_EPI_BF16 || epilogue == FLUX_HIP_EPI_F32 || epilogue == FLUX_HIP_EPI_F32_T ||
-                                (epilogue == FLUX_HIP_EPI_SWIGLU && w_row1 == w_row0 + N / 2));
         double rows = 0.0;
         int most = 0;
         for (int i = 0; i < np; i++) rows += g.M[i], most = max(most, g.M[i]);
+        const bool can_split = g_splitk_enabled &&
+                               (epilogue == FLUX_HIP_EPI_RESID || epilogue == FLUX_HIP_EPI_BF16 || epilogue == FLUX_HIP_EPI_F32 || (epilogue == FLUX_HIP_EPI_F32_T && rows <= 8192) ||
+                                (epilogue == FLUX_HIP_EPI_SWIGLU && w_row1 == w_row0 + N / 2));
         int weights = 0; /* matrices of weights: sequences share them, streams do not */
         for (int i = 0; i < np; i++) {
             weights++;
