@@ -877,6 +877,7 @@ extern "C" int flux_hip_vae_group_norm_skip(void *out_bf16, void *raw_bf16, floa
     if (hp < 3 || wp < 3 || (long long)hp * wp >= 1 << 22 || wp >= 1 << 12 || cout <= 0 || cout % 128)
         return flux_hip_fail("flux_hip_vae_group_norm_skip: bad shape (hp=%d wp=%d cout=%d)", hp, wp, cout);
     if (!out_bf16 || !raw_bf16 || !y || !x || !gamma || !beta || !scratch || !w || !bias) return flux_hip_fail("flux_hip_vae_group_norm_skip: NULL argument");
+    if (conv_stats && conv_stats_rows <= 0) return flux_hip_fail("flux_hip_vae_group_norm_skip: conv_stats_rows=%d", conv_stats_rows);
     if (((uintptr_t)out_bf16 | (uintptr_t)raw_bf16 | (uintptr_t)y | (uintptr_t)x | (uintptr_t)gamma | (uintptr_t)beta | (uintptr_t)w | (uintptr_t)bias) & 15)
         return flux_hip_fail("flux_hip_vae_group_norm_skip: operands must be 16-byte aligned");
     const int rows = hp * wp, P = cin == 512 ? 64 : 128;

@@ -126,6 +126,20 @@ def test_attention_reference_samples_every_column():
     assert f(256) == 1 and f(511) == 1
 
 
+@pytest.mark.parametrize("hp,wp,cin", [(10, 12, 256), (130, 130, 256), (130, 130, 512)])
+def test_norm_with_shortcut_refuses_sums_without_rows(hp, wp, cin):
+    """flux_hip_group_norm_stats refuses sums of no rows, and so does the norm that takes the block's shortcut along, in its two launches and in its one: a
+    mean of nothing would go through as 0."""
+    L = fluxhip.lib()
+    f = L.flux_hip_vae_group_norm_skip
+    vp, ci = ctypes.c_void_p, ctypes.c_int
+    f.argtypes = [vp] * 7 + [ci, ci, ci, ctypes.c_float, vp, ci, vp, vp, ci]
+    p = 1 << 20                                                  # never read: the call ends at its checks
+    for rows in (0, -1):
+        assert f(p, p, p, p, p, p, p, hp, wp, cin, 1e-6, p, rows, p, p, 128) == 0
+        assert b"flux_hip_vae_group_norm_skip: conv_stats_rows" in L.flux_hip_last_error()
+
+
 def test_bench_names_the_kernels_that_tiles_launch():
     """bench.py's names of the tiles, which are looked up in kernel traces, have the template arguments of the launches."""
     source, bench = (open(os.path.join(ROOT, *p)).read() for p in (("flux2.c_amd", "csrc", "gemm.hip"), ("bench.py",)))
