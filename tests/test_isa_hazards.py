@@ -464,6 +464,129 @@ def test_run_convolution_waits_for_its_weights(assembly):
                     assert wait <= 2 * (8 - last_tap) - 2 * (patch[last_tap] == 0), (name, wait)
 
 
+def first_barrier(body):
+    """([LDS offset of the load, None for any other vector memory operation] in front of the kernel's first barrier, vmcnt of the wait there). A load into LDS
+    goes to what m0 holds, a wave's base plus a constant; the constant is followed through the scalar additions."""
+    constant, out, wait = {}, [], None
+    for line in body:
+        p = parse(line)
+        if not p:
+            continue
+        op, a = p
+        if op in ("s_add_i32", "s_mov_b32"):
+            constant[a[0]] = sum(int(t, 0) if re.fullmatch(r"0x[0-9a-f]+|\d+", t) else constant.get(t, 0) for t in a[1:])
+        elif a and re.fullmatch(r"s\d+", a[0]) and not op.startswith(("s_cmp", "s_bitcmp")):
+            constant.pop(a[0], None)
+        if op.startswith(("buffer_", "global_", "flat_", "scratch_")):
+            out.append(constant["m0"] if " lds" in line.split(";")[0] or "lds_" in op else None)
+        elif op == "s_waitcnt":
+            m = re.search(r"vmcnt\((\d+)\)", line)
+            wait = int(m.group(1)) if m else None
+        elif op == "s_barrier":
+            return out, wait
+
+
+def first_step_is_late(requests, wait, step):
+    """Whether the wait lets one of the first K step's loads (those to the LDS offsets `step`) be on its way still, or does not find each of them once."""
+    at = [i for i, offset in enumerate(requests) if offset in step]
+    return sorted(requests[i] for i in at) != sorted(step) or wait is None or wait > len(requests) - 1 - at[-1]
+
+
+def test_first_tiles_wait_for_their_first_step(assembly):
+    """The ring kernels and conv3_kernel start a workgroup's first tile when its first K step has landed and leave the others on their way: the wait in
+    front of the first barrier is a count. The compiler orders the loads in front of it, so what it lets through is counted in its output: never one
+    of the first step's loads, which go to the first slot of each operand's ring (in conv3_kernel to the first patch and the first slot of weights)."""
+    seen = 0
+    for src in ("gemm.hip", "conv.hip"):
+        for name, body in sorted(kernel_bodies(assembly[src][0]).items()):
+            m = re.search(r"gemm4([dx])_kernelILi(\d+)ELi(\d+)ELi\d+E(?:Li(\d)E)?", name)
+            if m:                                                    # a load of four waves takes 4 KB: TM and TN of them a step
+                tm, tn, ring = int(m.group(2)), int(m.group(3)), int(m.group(4) or 2)
+                step = [4096 * i for i in range(tm)] + [4096 * (ring * tm + i) for i in range(tn)]
+            elif "conv3_kernel" in name:                             # two patches of 48 KB, then 16 KB a slot of weights
+                step = [4096 * i for i in range(12)] + [4096 * (24 + i) for i in range(4)]
+            else:
+                continue
+            requests, wait = first_barrier(body)
+            assert not first_step_is_late(requests, wait, step), (name, requests, wait)
+            seen += 1
+    assert seen >= 60
+
+
+def test_the_first_barrier_sees_a_load_moved_behind_the_others():
+    load = ["\ts_add_i32 m0, s5, %d", "\tglobal_load_lds_dwordx4 v[0:1], off"]
+    def body(*offsets, wait=2):
+        return ["\tglobal_load_dword v9, v1, s[2:3]", "\ts_add_i32 s7, s6, 0x1000"] + [l % o if "%" in l else l for o in offsets for l in load] + [
+            "\ts_mov_b32 m0, s7", "\tbuffer_load_dwordx4 v3, s[8:11], 0 offen lds", "\ts_waitcnt vmcnt(%d) lgkmcnt(0)" % wait, "\ts_barrier"]
+    assert first_barrier(body(0, 8192, 12288)) == ([None, 0, 8192, 12288, 4096], 2)
+    assert not first_step_is_late(*first_barrier(body(0, 8192, 12288)), [0, 8192])
+    assert first_step_is_late(*first_barrier(body(0, 12288, 8192)), [0, 8192])                 # requested last but one
+    assert first_step_is_late(*first_barrier(body(0, 8192, 12288, wait=3)), [0, 8192])
+    assert first_step_is_late(*first_barrier(body(0, 12288)), [0, 8192])                       # not there at all
+
+
+def few_row_steps(body):
+    """What gemm_few_kernel has in front of its K loop (its vector memory operations, L: a load into LDS, V: any other), and the loop from its barrier round to
+    it again: L and V, j: a branch around what follows, M: an MFMA, B: the barrier, (n): a wait for all but n."""
+    labels = {m.group(1): ln for ln, line in enumerate(body) for m in [re.match(r"^(\.LBB\d+_\d+):", line)] if m}
+    back = [(labels[m.group(1)], ln) for ln, line in enumerate(body) for m in [re.search(r"\bs_c?branch\w*\s+(\.LBB\d+_\d+)", line)] if m and labels[m.group(1)] < ln]
+    first = lambda a: next((p[0] for p in map(parse, body[a:]) if p), "")
+    loops = [(a, b) for a, b in back if first(a) != "s_endpgm" and any("v_mfma" in l for l in body[a:b])]
+    a, b = min(x for x, _ in loops), max(y for _, y in loops)
+
+    def shape(lines):
+        out = []
+        for line in lines:
+            p = parse(line)
+            if not p:
+                continue
+            text = line.split(";")[0]
+            if p[0].startswith(("buffer_", "global_", "flat_", "scratch_")):
+                out.append("L" if " lds" in text or "lds_" in p[0] else "V")
+            elif p[0] == "s_waitcnt" and "vmcnt" in text:
+                out.append("(%s)" % re.search(r"vmcnt\((\d+)\)", text).group(1))
+            elif p[0] == "s_barrier":
+                out.append("B")
+            elif p[0].startswith("s_cbranch"):
+                out.append("j")
+            elif p[0].startswith("v_mfma"):
+                out.append("M")
+        return out
+    loop = shape(body[a:b + 1])
+    at = loop.index("B")
+    return [o for o in shape(body[:a]) if o in "LV"], loop[at:] + loop[:at]
+
+
+def few_row_waits_hold(front, loop, loads, stages):
+    """A wave that requests n loads a step waits for all but n (stages - 2): right if a step requests nothing else, if each of its `loads` loads but the first (every
+    wave has one) stands behind a branch, if they all stand between the barrier and the MFMAs and nothing but the stages - 1 first steps'
+    loads follows the last other operation in front of the loop."""
+    requests = "".join(o for o in loop[:loop.index("M")] if o in "LVj")
+    return (loop.count("B") == 1 and loop.count("L") == loads and "V" not in loop and requests.lstrip("j").startswith("j".join("L" * loads)) and
+            sorted(o for o in loop if o[0] == "(") == sorted("(%d)" % (n * (stages - 2)) for n in range(6)) and
+            "".join(front).endswith("L" * loads * (stages - 1)))
+
+
+def test_few_row_projections_wait_for_their_step(assembly):
+    """gemm_few_kernel's barrier waits with one of five counts, by the number of loads that the wave requests a step: counted in the compiler's output."""
+    kernels = {k: v for k, v in kernel_bodies(assembly["gemm.hip"][0]).items() if "gemm_few_kernel" in k}
+    assert len(kernels) >= 30
+    for name, body in sorted(kernels.items()):
+        bn = int(re.search(r"gemm_few_kernelILi(\d+)E", name).group(1))
+        front, loop = few_row_steps(body)
+        assert few_row_waits_hold(front, loop, (16 + bn // 8 + 7) // 8, min(6, 160 * 1024 // ((128 + bn) * 128))), (name, front, loop)
+
+
+def test_the_few_row_count_sees_a_load_too_many():
+    waits = ["(%d)" % (2 * n) for n in range(6)]
+    loop, front = ["B", "j", "L", "j", "L", "j", "M", "M"] + waits, ["V", "L"] + ["L"] * 5
+    assert few_row_waits_hold(front, loop, 2, 4)
+    assert not few_row_waits_hold(front + ["V"], loop, 2, 4) and not few_row_waits_hold(front[:-2], loop, 2, 4)
+    assert not few_row_waits_hold(front, loop[:6] + ["V"] + loop[6:], 2, 4)                     # a spilled register
+    assert not few_row_waits_hold(front, ["B", "j", "L", "L", "j", "M"] + waits, 2, 4)          # a wave with one load would request two
+    assert not few_row_waits_hold(front, loop[:-1] + ["(9)"], 2, 4)
+
+
 def test_projection_k_loops_carry_no_second_address_chain(assembly):
     """One K step of a projection in the ring kernel steps both operands along K by the same byte offset. Convolutions, which
     share the loop, need a row offset of their own for the activations; when the projections' bases went through the same
