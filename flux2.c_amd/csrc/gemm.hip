@@ -2576,6 +2576,11 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows, void *enlarge
     const int width = g.conv_wp - 2, height = g.conv_wp > 0 ? g.conv_rows / g.conv_wp - 2 : 0;
     const bool patch_ok = g_ring && g.conv_taps == 9 && g.conv_stride == 1 && !g.conv_packed_out && conv3_takes(height, width, g.lda, N);
     const bool run_ok = ring_ok && g.conv_taps == 9 && g.conv_stride == 1 && !g.conv_packed_out && M > 0 && convp_rows(width) <= 448;
+    /* Where CONV_RUN in one piece is a round at most, slices take longer against it than the model below has them: over 504 forms of 36 image sizes (8 x 8 to
+     * 128 x 128 and 24 x 320 positions) and seven pairs of channel counts the choice takes 0.8 % more than the best of up to 26 forms on average and 9 % at most; without
+     * the term for that 1.7 and 16 %, and a decode from a 4 x 4 latent 590 us of convolutions for 569. With more positions the same term took 128 x 128 in one piece where slices of
+     * 256 x 128 are faster: 32 x 132 x 512 in a decode 46 us and 37. */
+    const bool run_round = run_ok && (long)((M + 127) / 128) * (N / 64) <= 256;
     int tile = -1, split = 1;
     const auto choose = [&](bool slices) {
         double best = 1e30;
@@ -2606,7 +2611,7 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows, void *enlarge
                     est = rounds * (2.0 * conv_bm[t] * conv_bn[t] * 64.0 * per / rate[t] + (double)conv_bm[t] * conv_bn[t] * ((epilogue == FLUX_HIP_EPI_CONV_BF16 ? 2 : 4) + (g.res ? 4 : 0)) / 4.0e10) + 6.0e-6;
                 if (run) est += 0.5e-6 + (rounds - 1) * 3.5e-6;           /* (a second round's first loads meet the first one's stores) */
                 if (sp > 1) est += 4.0e-6 + 2.0 * ws / 4.0e12;
-                if (sp > 1 && run_ok) est += run ? 1.5e-6 : 3.0e-6; /* against CONV_RUN in one piece, which the images that want slices mostly take */
+                if (sp > 1 && run_round) est += run ? 1.5e-6 : 3.0e-6;
                 if (est < best) { best = est; tile = t; split = sp; }
             }
         }

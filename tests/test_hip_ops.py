@@ -504,11 +504,11 @@ def test_linear_residual_then_adaln(hip, oracle_mod, shape, tile):
 
 @pytest.mark.parametrize("rms", [False, True])
 @pytest.mark.parametrize("M", [1, 200, 201])
-@pytest.mark.parametrize("N,slices", [(128, 2), (384, 8), (2560, 3), (4096, 9)])
+@pytest.mark.parametrize("N,slices", [(128, 2), (384, 8), (2560, 3), (4096, 8), (4096, 6)])
 def test_second_pass_with_norm(hip, M, N, slices, rms):
     """The second pass that also normalises: a quad of columns a thread up to 200 rows, four beyond; columns that leave a wave half empty, one to four
-    quads, as many slices as are requested at once, fewer and more. x as the plain second pass gives it, bit for bit; the norm against float64 on that x:
-    one rounding to bf16, 2^-9 an element, and fp32 sums."""
+    quads and the widest row there is (16 waves); fewer slices than are requested at once, whole groups of them and a last group that is not full. x
+    as the plain second pass gives it, bit for bit; the norm against float64 on that x: one rounding to bf16, 2^-9 an element, and fp32 sums."""
     L = hip.lib()
     K = 64 * 4 * slices
     a, W = q(normal_f32((M, K), 82, 1)), q(normal_f32((N, K), 82, 2, 0.0, 0.05))
@@ -520,7 +520,7 @@ def test_second_pass_with_norm(hip, M, N, slices, rms):
     try:
         L.flux_hip_linear_force_tile(1)
         L.flux_hip_linear_force_split(slices)
-        assert hip.linear_resid_adaln([(da.ptr, dW.ptr, dx.ptr, dg.ptr, M)], N, K, K, K, N, [(dn.ptr, None if rms else dsh.ptr, dsc.ptr)]) == (slices in (2, 3, 8))
+        assert hip.linear_resid_adaln([(da.ptr, dW.ptr, dx.ptr, dg.ptr, M)], N, K, K, K, N, [(dn.ptr, None if rms else dsh.ptr, dsc.ptr)])
         hip.linear(hip.EPI_RESID, [(da.ptr, dW.ptr, plain.ptr, dg.ptr, M)], N, K, K, K, N)
     finally:
         L.flux_hip_linear_force_split(0)
@@ -529,14 +529,35 @@ def test_second_pass_with_norm(hip, M, N, slices, rms):
     np.testing.assert_array_equal(x, plain.to_array(np.float32, (M + 1, N)))
     np.testing.assert_array_equal(x[M], res[M])
     assert (n[M] == 0x4040).all()
-    if slices not in (2, 3, 8):
-        return
     x = x[:M].astype(np.float64)
     if rms:
         want = x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-6) * sc
     else:
         want = (1.0 + sc) * (x - x.mean(1, keepdims=True)) / np.sqrt(x.var(1, keepdims=True) + 1e-6) + sh
     assert rel_l2(bf16_to_f32(n[:M]), want) < 2.0 ** -9
+
+
+def test_slice_count_that_is_not_there(hip):
+    """Nine slices, which the dispatch does not have: the projection runs in one piece and leaves the norm to its caller."""
+    L = hip.lib()
+    M, N, K = 5, 256, 64 * 4 * 9
+    a, W = q(normal_f32((M, K), 84, 1)), q(normal_f32((N, K), 84, 2, 0.0, 0.05))
+    res, g = normal_f32((M, N), 84, 3), normal_f32((N,), 84, 4)
+    da, dW, dg = dev_bf16(hip, a), dev_bf16(hip, W), hip.DevBuf.from_array(g)
+    dx, plain, dn = hip.DevBuf.from_array(res), hip.DevBuf.from_array(res), hip.DevBuf.from_array(np.full((M, N), 0x4040, np.uint16))
+    try:
+        L.flux_hip_linear_force_tile(1)
+        L.flux_hip_linear_force_split(9)
+        assert not hip.linear_resid_adaln([(da.ptr, dW.ptr, dx.ptr, dg.ptr, M)], N, K, K, K, N, [(dn.ptr, dg.ptr, dg.ptr)])
+        L.flux_hip_linear_force_split(0)
+        L.flux_hip_linear_enable_splitk(0)
+        hip.linear(hip.EPI_RESID, [(da.ptr, dW.ptr, plain.ptr, dg.ptr, M)], N, K, K, K, N)
+    finally:
+        L.flux_hip_linear_enable_splitk(1)
+        L.flux_hip_linear_force_split(0)
+        L.flux_hip_linear_force_tile(-1)
+    np.testing.assert_array_equal(dx.to_array(np.float32, (M, N)), plain.to_array(np.float32, (M, N)))
+    assert (dn.to_array(np.uint16, (M, N)) == 0x4040).all()
 
 
 @pytest.mark.parametrize("M,M2", [(1, 5), (64, 3), (257, 100)])
@@ -666,10 +687,10 @@ def test_linear_qkv_swiglu_wide_tiles(hip, oracle_mod, tile, bm, qc, mlp, K, row
 @pytest.mark.parametrize("tile,M", [(8, 1), (8, 37), (8, 64), (9, 80), (9, 128), (10, 80), (10, 96)])
 @pytest.mark.parametrize("K", [64, 192, 320, 448, 1024])
 def test_linear_deep_ring_tiles(hip, oracle_mod, tile, M, K):
-    """Tiles 8 and 9: the 64 x 128 and 128 x 128 tiles with a ring of 6 and 5 LDS stages for parts of few rows.
+    """Tiles 8, 9 and 10: 80, 128 and 112 columns with a ring of 6, 5 and 5 LDS stages for parts of few rows (gemm_few_kernel).
     K steps from one (fewer than the ring holds) to sixteen (the ring wraps several times); bf16, fp32, gated
-    residual over two parts, SwiGLU and the fused [Q|K|V|gate|up] launch; bit for bit what the two-stage form of the
-    same tile gives (same MFMA order), and right against the oracle. The launch probe confirms which tile ran."""
+    residual over two parts, SwiGLU and the fused [Q|K|V|gate|up] launch; bit for bit what the two-stage 64 x 128 or 128 x 128
+    tile gives (same MFMA order), and right against the oracle. The launch probe confirms which tile ran."""
     import ctypes
     L = hip.lib()
     L.flux_hip_linear_qkv_swiglu.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 8
@@ -683,7 +704,7 @@ def test_linear_deep_ring_tiles(hip, oracle_mod, tile, M, K):
     outs = {}
     L.flux_hip_linear_enable_splitk(0)
     try:
-        for t in (tile, 1 if tile == 10 else tile - 8):            # tile 0 = 64 x 128 and tile 1 = 128 x 128 with two stages
+        for t in (tile, 1 if tile == 10 else tile - 8):            # tile 0 = 64 x 128 and tile 1 = 128 x 128, two stages
             L.flux_hip_linear_force_tile(t)
             L.flux_hip_linear_probe(hip.EPI_BF16)
             o16, o32 = hip.DevBuf(M * N * 2), hip.DevBuf(M * N * 4)
@@ -765,6 +786,48 @@ def test_linear_few_row_tiles(hip, tile, M, K, N):
     assert (r0[M] == res[0][M]).all() and (r1[M2] == res[1][M2]).all()
 
 
+@pytest.mark.parametrize("tile", [8, 16, 10, 9, 24])
+@pytest.mark.parametrize("M,N,K,slices", [(1, 128, 512, 2), (67, 256, 832, 3), (128, 640, 832, 2), (9, 640, 2624, 8)])
+def test_linear_few_row_tiles_in_slices(hip, tile, M, N, K, slices):
+    """gemm_few_kernel in K slices: partial sums of cut-off column tiles and of two parts behind each other in the workspace, slices of four K steps up to more than
+    any ring holds, a last slice shorter than the others and than the ring (13 steps as 5, 5 and 3; 41 for eight slices as six of 6 and one of 5). Plain
+    fp32, residual and SwiGLU: bit for bit what the two-stage 64 x 64 tile gives in as many slices; sliced it is (other bits than in
+    one piece). Rows behind the output stay as they were."""
+    L = hip.lib()
+    M2, mlp = M // 2 + 1, N // 2
+    x, x2, W = q(normal_f32((M, K), 85, 1)), q(normal_f32((M2, K), 85, 2)), q(normal_f32((2 * N, K), 85, 3, 0.0, 0.1))
+    dx, dx2, dW, dg = dev_bf16(hip, x), dev_bf16(hip, x2), dev_bf16(hip, W), hip.DevBuf.from_array(normal_f32((N,), 85, 4))
+    res = normal_f32((M + 1, N), 85, 5), normal_f32((M2 + 1, N), 85, 6)
+    outs = []
+    try:
+        for t, sp in ((tile, slices), (3, slices), (tile, 0)):
+            L.flux_hip_linear_force_tile(t)
+            L.flux_hip_linear_enable_splitk(sp > 0)
+            L.flux_hip_linear_force_split(sp)
+            L.flux_hip_linear_probe(hip.EPI_F32)
+            o32, sw = hip.DevBuf.from_array(np.full((M + 1, N), 7.0, np.float32)), hip.DevBuf.from_array(np.full((M + 1, mlp), 7, np.uint16))
+            r = [hip.DevBuf.from_array(a) for a in res]
+            hip.linear(hip.EPI_F32, [(dx.ptr, dW.ptr, o32.ptr, None, M)], N, K, K, K, N)
+            ran = np.zeros(4, np.int32)
+            assert L.flux_hip_linear_probe_read_launches(4, ran.ctypes.data, None) == 1 and ran[0] == t
+            L.flux_hip_linear_probe(-1)
+            hip.linear(hip.EPI_RESID, [(dx.ptr, dW.ptr, r[0].ptr, dg.ptr, M), (dx2.ptr, dW.at(N * K * 2), r[1].ptr, dg.ptr, M2)], N, K, K, K, N)
+            hip.linear(hip.EPI_SWIGLU, [(dx.ptr, dW.ptr, sw.ptr, None, M)], N, K, K, K, mlp, 0, mlp)
+            outs.append([o32.to_array(np.float32, (M + 1, N)), r[0].to_array(np.float32, (M + 1, N)), r[1].to_array(np.float32, (M2 + 1, N)), sw.to_array(np.uint16, (M + 1, mlp))])
+    finally:
+        L.flux_hip_linear_force_split(0)
+        L.flux_hip_linear_force_tile(-1)
+        L.flux_hip_linear_enable_splitk(1)
+        L.flux_hip_linear_probe(-1)
+    for a, b in zip(outs[0], outs[1]):
+        np.testing.assert_array_equal(a, b)
+    assert (outs[0][0] != outs[2][0]).any()
+    o32, r0, r1, sw = outs[0]
+    assert (o32[M] == 7).all() and (sw[M] == 7).all() and (r0[M] == res[0][M]).all() and (r1[M2] == res[1][M2]).all()
+    want = x.astype(np.float64) @ W[:N].astype(np.float64).T
+    assert rel_l2(o32[:M], want) < 2e-6
+
+
 @pytest.mark.parametrize("M,K", [(1, 256), (255, 320), (257, 448), (512, 2560)])
 @pytest.mark.parametrize("mlp", [64, 128, 192, 320, 9728])
 def test_linear_swiglu_160_wide_tile(hip, M, K, mlp):
@@ -798,7 +861,7 @@ def test_linear_swiglu_160_wide_tile(hip, M, K, mlp):
 @pytest.mark.parametrize("M,K", [(1, 64), (67, 192), (80, 448), (96, 1024)])
 @pytest.mark.parametrize("N", [384, 512, 640])
 def test_linear_96_wide_ring_tile(hip, oracle_mod, M, K, N):
-    """Tile 16 (96 x 96, six waves) whose last column tile is cut off after one wave's columns (512), two (640) or not at all (384): bit
+    """Tile 16 (gemm_few_kernel, 96 columns) whose last column tile is cut off after 32 columns (512), 64 (640) or not at all (384): bit
     for bit what the two-stage 128 x 128 tile gives, as bf16, fp32, gated residual, SwiGLU (whose cut lies within gate and up), the fused
     launch where 96 divides both sides, and as K slices; columns beyond N stay as they were."""
     import ctypes

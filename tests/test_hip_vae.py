@@ -412,6 +412,18 @@ def check_sums(stats, written):
     np.testing.assert_allclose(stats[:, 0], quads.sum((0, 2)), atol=2.0 ** -8 * np.abs(quads).sum((0, 2)).max() + 1e-30)
 
 
+@pytest.mark.parametrize("H,W,tile", [(32, 132, 12), (52, 80, 12), (68, 68, 12), (32, 120, 14), (12, 12, 14)])
+def test_conv_choice_around_a_round_of_runs(hip, switches, H, W, tile):
+    """512 -> 512 channels to fp32 with residual: up to 4096 positions (256 workgroups) the run tile, beyond that the slices of 256 x 128."""
+    rows, C = (H + 2) * (W + 2), 512
+    x, w, b = hip.DevBuf.from_array(np.zeros((rows, C), np.uint16)), hip.DevBuf.from_array(np.zeros((C, 9 * C), np.uint16)), hip.DevBuf.from_array(np.ones(C, np.float32))
+    out = hip.DevBuf.from_array(np.zeros((rows, C), np.float32))
+    conv_image(hip, -1, 0, hip.EPI_CONV_F32, x.ptr, 0, 0, w, b, out.ptr, out.ptr, rows, W + 2, C, C, 9)
+    ran = np.zeros(4, np.int32)
+    assert hip.lib().flux_hip_linear_probe_read_launches(4, ran.ctypes.data, None) == 1 and ran[0] == tile
+    assert out.to_array(np.float32, (rows, C)).sum() == H * W * C
+
+
 @pytest.mark.parametrize("tile,split", CONV_FORMS)
 @pytest.mark.parametrize("C,H,W", [(64, 2, 2), (128, 8, 6), (64, 2, 74), (128, 62, 2), (128, 34, 66)])
 def test_conv_with_stride_2(hip, oracle_mod, switches, tile, split, C, H, W):
