@@ -1611,7 +1611,7 @@ static int launch_cfg(GemmArgs &g) {
 }
 
 template <int BN, int EPI>
-static int launch_cfg(GemmArgs &g) {
+static int launch_few(GemmArgs &g) {
     constexpr int STAGE = (128 + BN) * 128, LDS = (160 * 1024 / STAGE < 6 ? 160 * 1024 / STAGE : 6) * STAGE;
     static bool attr_done = false;
     auto kern = gemm_few_kernel<BN, EPI>;
@@ -1744,11 +1744,11 @@ static int launch_epi(GemmArgs &g, int tile) {
         case 4: return launch_4w<8, 4, EPI, 2, 4>(g); /* 8 waves, two per SIMD, on the 256x256 tile */
         case 1: return launch_cfg<128, 128, 2, 2, EPI>(g);
         case 3: return launch_cfg<64, 64, 2, 2, EPI>(g);
-        case 8: return launch_cfg<80, EPI>(g);
-        case 9: return launch_cfg<128, EPI>(g);
-        case 10: return launch_cfg<112, EPI>(g);
-        case 16: return launch_cfg<96, EPI>(g);
-        case 24: return launch_cfg<144, EPI>(g);
+        case 8: return launch_few<80, EPI>(g);
+        case 9: return launch_few<128, EPI>(g);
+        case 10: return launch_few<112, EPI>(g);
+        case 16: return launch_few<96, EPI>(g);
+        case 24: return launch_few<144, EPI>(g);
         default: return launch_cfg<64, 128, 2, 2, EPI>(g);
     }
 }

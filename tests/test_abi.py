@@ -145,13 +145,15 @@ def test_bench_names_the_kernels_that_tiles_launch():
     source, bench = (open(os.path.join(ROOT, *p)).read() for p in (("flux2.c_amd", "csrc", "gemm.hip"), ("bench.py",)))
     body = source[source.index("static int launch_epi("):]
     body = body[:body.index("\n}\n")]
-    launched = {int(i): (kind, [a for a in args.replace(" ", "").split(",") if a != "EPI"])
-                for i, kind, args in re.findall(r"case (\d+):.*?return launch_(cfg|4d|4w|4x)<([^>]*)>", body)}
-    named = {int(i): args.split(",") for i, args in re.findall(r'(\d+): f"gemm\w*_kernel<([^>]*)>', bench)}
-    assert len(named) >= 13 and len(launched) >= 20
-    for tile, args in named.items():
+    launched = {}
+    for i, kind, args in re.findall(r"case (\d+):.*?return launch_(cfg|few|4d|4w|4x)<([^>]*)>", body):
+        launched.setdefault(int(i), {})[kind] = [a for a in args.replace(" ", "").split(",") if a != "EPI"]
+    kinds = {"gemm_kernel": "cfg", "gemm_few_kernel": "few", "gemm4d_kernel": "4d", "gemm4w_kernel": "4w", "gemm4x_kernel": "4x"}
+    named = {int(i): (kinds[kernel], args.split(",")) for i, kernel, args in re.findall(r'(\d+): f"(gemm\w*_kernel)<([^>]*)>', bench)}
+    assert len(named) >= 13 and len(launched) >= 20 and sum(kind == "few" for kind, _ in named.values()) == 5
+    for tile, (kind, args) in named.items():
         if tile in launched:                                     # (0 is the default)
-            kind, want = launched[tile]
+            want = launched[tile][kind]
             got = [a for a in args if a != "{epi_name}"]
             assert got == (want[:2] if len(got) == 2 and kind != "cfg" else want), (tile, args, want)      # (a ring's depths are left out)
 
