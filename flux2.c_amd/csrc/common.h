@@ -25,6 +25,11 @@ bool conv3_takes(int H, int W, int cin, int cout);
 long conv3_tiles(int H, int W, int cout);
 int conv3_launch(bool f32, bool up, const void *in, const void *w, const float *bias, const float *res, void *out, int H, int W, int cin, int cout, float *stats,
                  int *stats_rows, int units);
+/* gemm.hip: the launch probe's record of a convolution that another file launches */
+int conv_probe_begin(int epilogue, int tile);
+void conv_probe_end(int slot);
+/* vae.hip, for convolutions over an enlargement that is written first */
+extern "C" int flux_hip_vae_upsample2x_bf16(void *out_bf16, const void *x_bf16, int hp, int wp, int C);
 
 #define HIP_OK(call)                                                                   \
     do {                                                                               \

@@ -570,9 +570,6 @@ __global__ __launch_bounds__(256) void conv_in_kernel(float *__restrict__ out, c
 
 } // namespace
 
-int conv_probe_begin(int epilogue, int tile);
-void conv_probe_end(int slot);
-
 /* in: bf16 [(H + 2) * (W + 2)][128]; w: the first three rows of flux_hip_conv's weights; rgb 8-bit [H][W][3] and/or rgb_f32 [3][H][W] */
 extern "C" int flux_hip_vae_conv_out(uint8_t *rgb, float *rgb_f32, const void *in, const void *w, const float *bias, int H, int W) {
     if (H <= 0 || W <= 0 || !in || !w || !bias) return flux_hip_fail("flux_hip_vae_conv_out: bad argument");

@@ -36,18 +36,17 @@ int flux_hip_vae_key_bias(float *bias, int n, int keys);
 size_t flux_hip_vae_attention_work_floats(int n, int ld);
 int flux_hip_vae_attention(void *out, const void *q, const void *qkv, const void *vt, void *P, float *o32, float *work, int n, int keys, int ld, float scale,
                            int *done);
+int flux_hip_vae_latent_out(float *latent, const float *x, int ldx, const float *bn_mean, const float *bn_var, int h, int w, float eps);
+int flux_hip_vae_group_norm_skip(void *out_bf16, void *raw_bf16, float *y, const float *x, const float *gamma, const float *beta, float *scratch, int hp, int wp, int cin,
+                                 float eps, const float *conv_stats, int conv_stats_rows, const void *w, const float *bias, int cout);
 /* conv.hip */
 int flux_hip_vae_conv_out(uint8_t *rgb, float *rgb_f32, const void *in, const void *w, const float *bias, int H, int W);
 int flux_hip_vae_conv_in(float *out, const float *img, const void *w, const float *bias, int H, int W, float *stats, int *stats_rows);
 /* gemm.hip */
-int flux_hip_vae_group_norm_skip(void *out_bf16, void *raw_bf16, float *y, const float *x, const float *gamma, const float *beta, float *scratch, int hp, int wp, int cin,
-                                 float eps, const float *conv_stats, int conv_stats_rows, const void *w, const float *bias, int cout);
 int flux_hip_conv_enlarged(const void *in, void *enlarged, const void *w, const float *bias, float *out, int rows, int wp, int cin, int cout, float *stats,
                            int *stats_rows);
 int flux_hip_conv_image(int epilogue, const void *in, int in_wp, int packed, const void *w, const float *bias, const float *res, void *out, int rows, int wp,
                         int cin, int cout, int taps, float *stats, int *stats_rows);
-/* vae.hip */
-int flux_hip_vae_latent_out(float *latent, const float *x, int ldx, const float *bn_mean, const float *bn_var, int h, int w, float eps);
 
 enum { K_VEC, K_CONV3, K_CONV1, K_RAW, K_CONV3_PACKED };
 enum { SIDE_BOTH, SIDE_DECODER, SIDE_ENCODER };

@@ -794,9 +794,6 @@ __global__ __launch_bounds__(256) void vae_transpose_kernel(bf16 *__restrict__ v
 
 /* ------------------------------------------------------------------ host entry points */
 
-int conv_probe_begin(int epilogue, int tile);
-void conv_probe_end(int slot);
-
 extern "C" int flux_hip_vae_latent_in(void *out_bf16, const float *latent, const float *bn_mean, const float *bn_var,
                                       const float *pq_w, const float *pq_b, int h, int w, float eps) {
     if (h <= 0 || w <= 0) return flux_hip_fail("flux_hip_vae_latent_in: bad size %d x %d", h, w);
