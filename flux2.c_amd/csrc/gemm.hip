@@ -1384,12 +1384,13 @@ __global__ __launch_bounds__(256) void gemm4x_kernel(GemmArgs g) {
 
 /* 3x3 convolutions of images with too few 16 x 16 tiles for conv.hip's kernel: 128 positions x 64 channels per workgroup.
  * As a GEMM (the ring kernel's 128 x 128 tile) every K step fetches its 128 positions x 64 channels again, nine times what a chunk of channels
- * holds, and images this small then need K slices with a second pass to give every compute unit work. Here the positions that a tile's nine taps touch
+ * holds, and images this small need three to eight K slices with a second pass to give every compute unit work. This tile is half as wide: two to four
+ * slices up to some 40 x 40 x 512, one piece beyond. Here the positions that a tile's nine taps touch
  * lie in LDS for a whole chunk (those of the next chunk arrive meanwhile), and the ring holds the weights alone: 11 to 14 KB a step.
  *
  * GEMM rows are interior positions in row-major order, so a tile is a run of positions whatever the image's sides. Its neighbourhood is one run
  * of the bordered image, from a row above the first position to a row below the last one, as long as that is at most 448 positions, and
- * otherwise (images wider than 155) three runs, one per tap row, CONVP_BAND apart in LDS: the LDS row of position p's tap (dy, dx) is
+ * otherwise (images wider than 156) three runs, one per tap row, CONVP_BAND apart in LDS: the LDS row of position p's tap (dy, dx) is
  * p - (the tile's first position) + dy * pitch + dx either way, pitch being the image's or CONVP_BAND. NPL: loads of eight LDS rows per wave
  * and chunk, 28, 40 or 56 KB twice; the weights have the rest.
  *
@@ -1897,8 +1898,8 @@ __device__ __forceinline__ float block_sum(float v, float *red, int waves) {
 /* RMS = true: the norm that follows is x / sqrt(mean(x^2) + eps) * weight instead (qwen3_rms_norm,
  * flux_qwen3.c:177-197). A thread owns Q quads of columns, blockDim.x quads apart. Everything the row needs is requested at once - the first U
  * slices, then x, gate, scale and shift - so that it costs one round trip to memory beside the further slices. With 256 threads of
- * four quads, four slices at a time and scale and shift behind them: 67 rows of 2560 5.6 us, now 4.8; 80 rows of 3072 5.8 and 5.2; 512 rows of
- * 2560 9.6 and 8.1; of 3072 768 rows 12.5 and 12.7, 1202 19.3 and 18.1, 2498 30.6 and 28.2. */
+ * four quads, four slices at a time and scale and shift behind them / now, us: three slices of 3072, 80 rows 5.9 / 4.2, 200 6.4 / 4.9, 512 9.0 / 8.0, 768 10.9 / 10.2,
+ * 1202 17.5 / 14.9, 2498 31.0 / 26.4; four slices 768 rows 12.2 / 11.4, 2498 34.1 / 33.2; four slices of 2560, 80 rows 4.5 / 4.1, 512 7.8 / 7.5. */
 template <bool RMS, int Q, int U>
 __global__ __launch_bounds__(1024 / Q) void splitk_finish_adaln_kernel(GemmArgs g, AdalnArgs a) {
     __shared__ float red[16];
@@ -2000,7 +2001,7 @@ static int launch_split(GemmArgs &g, int tile) {
 static int launch_split_adaln(GemmArgs &g, int tile, const AdalnArgs &a) {
     if (!launch_epi<EPI_PARTIAL>(g, tile)) return 0;
     /* Few rows wait for memory: a quad a thread, four slices on their way. With more rows than units it is the bytes (768 rows in four slices: 61 MB), and
-     * small workgroups win. Whole passes, us, first form / second: prompts of 67 tokens 2633 / 2690, 128 3172 / 3227, 200 3748 / 3784,
+     * small workgroups win. Whole passes, us, a quad a thread / four: prompts of 67 tokens 2633 / 2690, 128 3172 / 3227, 200 3748 / 3784,
      * 300 4345 / 4343, 512 5167 / 5168; denoising steps of 80 tokens 2478 / 2507, 208 3313 / 3305, 320 3743 / 3720, 640 5051 / 5000. */
     const bool few = g.ws_rows <= 200;
     const int quads = g.N >> 2, threads = few ? (quads + 63) / 64 * 64 : (quads + 255) / 256 * 64;
@@ -2186,14 +2187,18 @@ static int gemm_dispatch(GemmArgs &g, int np, int epilogue, unsigned allowed, in
         double best = 1e30;
         static const int splits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
         /* every epilogue can run as K slices + a finishing pass; for SwiGLU the gate and up rows must be one contiguous block of the
-         * weight matrix. (The final layer's 128 columns, stored transposed, are 8 tiles of 64 x 64 at 256 tokens: 35 us in one piece, 14.5 in slices; 16 tokens 35 and 11.4; 12544 tokens, whose second pass
-         * takes 24 us, 49 and 56.) */
+         * weight matrix. The transposed store (the final layer's 128 columns: 8 tiles of 64 x 64 at 256 rows) does up to 8192 rows. Weights from HBM and
+         * activations just written, as in a step, us in one piece / in slices: 16 rows 24 / 13, 256 37 / 17, 2048 39 / 19, 2304 39 / 32, 4096 42 / 24, 4864 43 / 36,
+         * 6912 46 / 40, 7936 46 / 44, 8192 47 / 32, never slower over 37 row counts; beyond, a gain or none as
+         * the count falls: 8448 50 / 50, 9216 51 / 35, 11008 54 / 54, 12032 55 / 56, 12544 55 / 57. (With weights that a cache holds one piece takes 26 to 28 us
+         * and slices up to 39 from 2304 rows on; in a step 7 GB of other weights have passed.) */
         const int N = g.N, K = g.K, w_row0 = g.w_row0, w_row1 = g.w_row1;
         double rows = 0.0;
         int most = 0;
         for (int i = 0; i < np; i++) rows += g.M[i], most = max(most, g.M[i]);
         const bool can_split = g_splitk_enabled &&
-                               (epilogue == FLUX_HIP_EPI_RESID || epilogue == FLUX_HIP_EPI_BF16 || epilogue == FLUX_HIP_EPI_F32 || (epilogue == FLUX_HIP_EPI_F32_T && rows <= 8192) ||
+                               (epilogue == FLUX_HIP_EPI_RESID || epilogue == FLUX_HIP_EPI_BF16 || epilogue == FLUX_HIP_EPI_F32 ||
+                                (epilogue == FLUX_HIP_EPI_F32_T && rows <= 8192) ||
                                 (epilogue == FLUX_HIP_EPI_SWIGLU && w_row1 == w_row0 + N / 2));
         int weights = 0; /* matrices of weights: sequences share them, streams do not */
         for (int i = 0; i < np; i++) {
@@ -2558,11 +2563,11 @@ static int conv_finish(GemmArgs &g) {
 
 /* Tile and K split of a convolution by the same kind of model as gemm_dispatch's: rounds of workgroups, each a tile's time at
  * its measured rate plus the bytes of its epilogue at a compute unit's share of the memory rate (nothing overlaps those where one
- * workgroup owns the unit). K slices, which add a second pass and its partial sums, are what small images need: 32 x 32
- * positions x 512 channels are 32 tiles of 128 x 128 for 256 units, 57 us in one piece and 24 in slices (27 in a decode); at 96 x 96 positions
- * one piece wins (54 us against 69). conv.hip's kernel is ahead from about a round of its tiles on (80 x 120 x 512: 46 us against 53 of
- * 256 x 128) as long as the image's sides do not leave a second, nearly empty round (90 x 162 x 512: 264 of its tiles, 90 us; 228 of 256 x 128,
- * 59 us). Over 111 forms of 37 layers the chosen tile took 1.5 % less than the best of four timed behind it, i.e. the same. */
+ * workgroup owns the unit). K slices add a second pass and its partial sums; images that leave most units idle take them. 512 -> 512 channels with residual, us between events, operands
+ * from the memory-side cache: 16 x 16 positions are 16 run tiles in one piece, 20.1, in four slices 15.6; 32 x 32 20.4, 18.6 in two and 19.2 in four (128 x 128 tiles 36 and
+ * 23 in four); at 56 x 56 one piece wins, 22.3 against 30.2. conv.hip's kernel is ahead from about a round of its tiles on (96 x 96: 57.7, 59.4 of
+ * 256 x 128; 88 x 136 60.4 and 61.9) as long as the image's sides do not leave a second, nearly empty round (90 x 162: 264 of its tiles, 99.6 us; 228 of
+ * 256 x 128, 66.5). */
 static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows, void *enlarged = nullptr) {
     static const int occ[CONV_TILES] = {3, 2, 1, 4, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1};
     static const double rate[CONV_TILES] = {2.0e12, 3.3e12, 5.4e12, 1.5e12, 0, 0, 0, 0, 0, 0, 0, 0, 4.8e12, 4.2e12, 5.0e12, 6.2e12}; /* FLOP/s of one CU */
@@ -2594,7 +2599,8 @@ static int conv_launch(GemmArgs &g, int epilogue, int *stats_rows, void *enlarge
             if (run && !run_ok) continue;
             const long tiles = t == CONV_PATCH ? conv3_tiles(height, width, N) : (long)((M + conv_bm[t] - 1) / conv_bm[t]) * (N / conv_bn[t]);
             for (int sp : splits) {
-                const int unit = run ? 9 : 1; /* a slice is whole chunks of channels there, two at least (of one it is mostly its first loads: 15.2 us against 13.6 at 16 x 16 x 512) */
+                /* a slice of runs is whole chunks of channels, two at least (of one it is mostly its first loads: 17.3 us against 15.6 at 16 x 16 x 512) */
+                const int unit = run ? 9 : 1;
                 const int per = (kt_total / unit + sp - 1) / sp * unit, used = (kt_total + per - 1) / per, last = kt_total - (used - 1) * per;
                 if (sp > 1 && (t == CONV_PATCH || !slices || per < 4 || last < 4 || used != sp || N % 64 || (run && per < 18 && !forced))) continue;
                 if (slices && g_force_split && kt_total / g_force_split >= 4 && sp != g_force_split) continue;

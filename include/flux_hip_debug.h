@@ -16,19 +16,19 @@ extern "C" {
 #endif
 
 /* force_tile: 0/1/2/3/5/6/7 pins the GEMM tile of flux_hip_linear (64x128, 128x128, 256x256, 64x64,
- * 288x192, 192x192, 256x192; 4 = 256x256 in its 8-wave form, never chosen automatically; 8 / 9 / 10 = 64x128 / 128x128 / 96x128
- * with a ring of 6 / 5 / 5 LDS stages, only for row ranges of at most 64 / 128 / 96 rows; 11 = 256x224, whose last column
+ * 288x192, 192x192, 256x192; 4 = 256x256 in its 8-wave form, never chosen automatically; 8 / 16 / 10 / 9 / 24 = 80 / 96 / 112 /
+ * 128 / 144 columns for row ranges of at most 128 rows, whose last column tile is cut off at N and whose ring is 6 / 5 / 5 / 5 / 4
+ * LDS stages; 11 = 256x224, whose last column
  * tile is cut off at N: for the residual and bf16 epilogues with at least four 64-wide K steps and no K slices; 12 / 13 / 14 =
- * 256x128 / 128x128 / 192x256 in the ring kernel, at least four K steps; 16 = 96x96 with a ring of 6 for row ranges of at most 96 rows,
- * whose last column tile is cut off at N; 17 to 22 = 288x288, 384x224, 320x224, 320x256, 288x256, 352x224 for the fused [Q|K|V|gate|up]
- * launch alone, at least four K steps; 23 = 256x160 in the ring kernel for the SwiGLU epilogue alone, whose last column tile is cut off
- * at N, a multiple of 64, at least four K steps), -1
- * restores the automatic choice (a tile whose width does not divide N is skipped, tile 11 apart; if none is left the
- * 128x128 tile runs). Convolutions know tiles 0 to 3, 12, 13 and 15 (16x16
- * positions x 128 channels, their neighbourhood in LDS: 3x3 without stride, at least 128 input channels) and ignore one
- * that does not fit the layer. */
+ * 256x128 / 128x128 / 192x256 in the ring kernel, at least four K steps; 17 to 22 = 288x288, 384x224, 320x224, 320x256, 288x256,
+ * 352x224 for the fused [Q|K|V|gate|up] launch alone, at least four K steps; 23 = 256x160 in the ring kernel for the SwiGLU epilogue
+ * alone, whose last column tile is cut off at N, a multiple of 64, at least four K steps), -1
+ * restores the automatic choice (a tile that cuts no columns off and whose width does not divide N is skipped; if none is left the
+ * 128x128 tile runs). Convolutions know tiles 0 to 3, 12, 13, 14 (128 consecutive positions x 64 channels, their neighbourhood in LDS:
+ * 3x3 without stride; K slices of whole 64-channel chunks) and 15 (16x16 positions x 128 channels, likewise, at least 128 input channels) and
+ * ignore one that does not fit the layer. */
 void flux_hip_linear_force_tile(int tile);
-/* bit t set = the automatic choice may use tile t (default 0xFF7FEF: all but tile 4; 0 restores it) */
+/* bit t set = the automatic choice may use tile t (default 0x1FF7FEF: all but tile 4; 0 restores it) */
 void flux_hip_linear_tile_mask(unsigned mask);
 /* 0 turns the split-K path off (default 1) */
 void flux_hip_linear_enable_splitk(int on);

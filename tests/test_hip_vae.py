@@ -348,11 +348,11 @@ def test_conv_of_the_enlarged_image(hip, switches, h, w, cin, cout):
 
 
 @pytest.mark.parametrize("H,W,cin,cout", [(1, 1, 64, 128), (1, 40, 128, 128), (130, 1, 128, 128), (70, 2, 64, 128), (7, 5, 64, 256), (21, 18, 128, 256), (9, 42, 192, 128),
-                                          (13, 63, 512, 128), (4, 90, 128, 384), (5, 127, 128, 128), (3, 155, 128, 128), (3, 157, 256, 128), (2, 300, 64, 64)])
+                                          (13, 63, 512, 128), (4, 90, 128, 384), (5, 127, 128, 128), (3, 155, 128, 128), (4, 156, 128, 128), (3, 157, 256, 128), (2, 300, 64, 64)])
 def test_conv_run_tile(hip, switches, H, W, cin, cout):
     """Tile 14 (a run of 128 positions x 64 channels, its neighbourhood in LDS) against the 64 x 64 tile, on whole numbers whose sums fp32
     holds exactly (9 * 512 products of at most 8 * 4). One to eight chunks of channels; the neighbourhood as one run of up to 224, 320 and 448
-    positions (from width 156 on as three); images one pixel wide and high, cut-off tiles; in one piece and in slices of whole chunks."""
+    positions (from width 157 on as three; 156 fills the 448); images one pixel wide and high, cut-off tiles; in one piece and in slices of whole chunks."""
     import ctypes
     L = hip.lib()
     rows, wp = (H + 2) * (W + 2), W + 2
